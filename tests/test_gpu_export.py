@@ -198,8 +198,9 @@ def test_export_ply_with_connections(tmp_path):
         assert bits_equal(verts["p"].reshape(-1), d["coords"]) and bits_equal(verts["n"], normals)
         assert (verts["c"] == np.array(color, np.uint8)).all()
         assert (faces["k"] == 3).all() and np.array_equal(faces["i"].reshape(-1), conn)
-        back = oracle.ref_read_ply(path)
-        assert bits_equal(back["coords"], d["coords"]) and np.array_equal(back["connections"], d["connections"])
+        if oracle.ref_available():
+            back = oracle.ref_read_ply(path)
+            assert bits_equal(back["coords"], d["coords"]) and np.array_equal(back["connections"], d["connections"])
         if normal == kmc.VERTEX_NORMAL:
             kmc.export_ply(d, normal, tmp_path / "vn_ascii", binary=False, color=color)
             ours = open(tmp_path / "vn_ascii.ply", "rb").read()
