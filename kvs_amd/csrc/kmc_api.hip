@@ -485,6 +485,36 @@ void plan_rows(JobArgs& a)
     a.cshift = 0;
     while ((1u << a.cshift) < a.NC && a.cshift < 6) ++a.cshift;
     a.nrows = (uint64_t)a.nz * a.ny;
+    plan_emit(a, emit_steps(a));
+}
+
+/* Wave steps of 64 (row, chunk) pairs that a pass's levels hold. */
+uint64_t emit_steps(const JobArgs& a)
+{
+    const uint64_t G = 64u >> a.cshift;
+    return std::max(1u, a.nlev) * ((a.nrows + G - 1) / G * ((a.NC + 63) / 64));
+}
+
+/* Waves of a launch: 4096 (what 256 CUs hold at four waves per SIMD) up to
+ * 8192 where each then still has four full steps -- the second half lets the
+ * hardware even out a large pass's waves (512^3 float turbulence, three
+ * levels: 460 us with 4096, 411 with 8192, 464 with 16384), while in a small
+ * pass it only pays each wave's start twice (256^3 blobs: 26 us and 38).  A
+ * wave takes as many rows at a time as its lanes hold, but at most a quarter
+ * of its share of the pass: a surface lies in few neighbouring rows, and four
+ * or more steps far apart even the waves out (256^3: 37 us with two steps, 26
+ * with four, 27 with eight). */
+constexpr uint64_t kEmitWaves = 4096, kEmitWavesMax = 8192, kEmitSteps = 4;
+
+void plan_emit(JobArgs& a, uint64_t all)
+{
+    const uint64_t own = emit_steps(a), nlev = std::max(1u, a.nlev);
+    const uint64_t waves = std::min(kEmitWavesMax, std::max(kEmitWaves, all / 4));
+    const uint64_t want = std::max<uint64_t>(1, (waves * own + all - 1) / all / nlev);   // waves per level
+    a.erows = 64u >> a.cshift;
+    while (a.erows > 1 && a.nrows / a.erows < kEmitSteps * want) a.erows >>= 1;
+    const uint64_t units = (a.nrows + a.erows - 1) / a.erows;
+    a.eblocks = (uint32_t)std::max<uint64_t>(1, (std::min(units, want) + kWaves - 1) / kWaves);
 }
 
 bool flat_emit_fits(uint32_t ny, uint32_t nz)
@@ -590,6 +620,14 @@ void object_coords(const kmc_volume* v, float minc[3], float maxc[3])
 
 static inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
+/* The clamp range as floats, where that is exact (a.minv, a.maxv set). */
+void float_range(JobArgs& a)
+{
+    a.fminv = (float)a.minv;
+    a.fmaxv = (float)a.maxv;
+    a.fclamp = ((double)a.fminv == a.minv && (double)a.fmaxv == a.maxv && a.minv <= a.maxv) ? 1u : 0u;
+}
+
 /* Per-job fields of a pass of up to kMaxLevels levels. */
 void init_job(JobArgs& a, const kmc_volume* v, const void* dvals, const double* iso, uint32_t nlev, int normal_type,
               int dup, double mn, double mx, const float minc[3], const float maxc[3])
@@ -604,6 +642,7 @@ void init_job(JobArgs& a, const kmc_volume* v, const void* dvals, const double* 
     a.vnormal = (!dup && normal_type == KMC_VERTEX_NORMAL) ? 1u : 0u;
     a.minv = mn;
     a.maxv = mx;
+    float_range(a);
     for (int k = 0; k < 3; ++k) {
         a.minc[k] = minc[k];
         const float span = maxc[k] - minc[k];          // (max_coord - min_coord), float
@@ -770,7 +809,7 @@ kmc_status run_pass(const kmc_volume* v, const void* dvals, const double* iso, u
             a.toff[l + 1] = a.toff[l] + tot[l * 2 + 1];
         }
         const uint64_t nv = a.voff[nlev], nt = a.toff[nlev];
-        const size_t bytes = align_up(nv * 8, 256) + align_up(nt * 8, 256) + align_up(nt, 256) +
+        const size_t bytes = dup ? 0 : align_up(nv * 8, 256) + align_up(nt * 8, 256) + align_up(nt, 256) +
                              (a.vnormal ? align_up(nt * 12, 256) + nv * 16 : 0);
         if (bytes) {
             recs = device_alloc(bytes);

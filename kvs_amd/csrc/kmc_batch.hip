@@ -35,11 +35,14 @@ struct SegOut {
     uint64_t rb;
 };
 
-/* Flat-emit records of a pass: vertex keys, triangle records, cube indices,
- * face normals and vertex slots (VertexNormal), each 256-byte aligned. */
+/* Flat-emit records of a pass with shared vertices: vertex keys, triangle
+ * records, cube indices, face normals and vertex slots (VertexNormal), each
+ * 256-byte aligned; duplicated triangles are emitted without records. */
 __host__ __device__ inline uint64_t align256(uint64_t x) { return (x + 255) & ~255ull; }
-__host__ __device__ inline uint64_t record_bytes(uint64_t nv, uint64_t nt, bool vn)
+__host__ __device__ inline uint64_t emit_record_bytes(const JobArgs& a, uint64_t nv, uint64_t nt)
 {
+    if (a.dup) return 0;
+    const bool vn = a.vnormal != 0;
     return align256(nv * 8) + align256(nt * 8) + align256(nt) + (vn ? align256(nt * 12) + align256(nv * 16) : 0);
 }
 
@@ -172,7 +175,7 @@ __global__ __launch_bounds__(kLayoutBlock) void k_batch_layout(JobArgs* jobs, co
                         sz[i][1] += a.dup ? 0 : level_total(a, l, 0);
                         sz[i][2] += level_total(a, l, 1);
                     }
-                    sz[i][0] = record_bytes(sz[i][1], sz[i][2], a.vnormal != 0);
+                    sz[i][0] = emit_record_bytes(a, sz[i][1], sz[i][2]);
                 }
                 v[0] += sz[i][0]; v[1] += sz[i][1]; v[2] += sz[i][2];
             }
@@ -273,6 +276,7 @@ struct Group {
     uint32_t p0, p1;             // passes [p0, p1)
     uint64_t rows, units;
     uint32_t max_levels;         // the most levels of one of its passes
+    uint32_t emit_blocks;        // the most emit workgroups per level of one of its passes
     uint32_t emit_lds;
     uint32_t teams;                // emit teams per workgroup
     uint64_t* row_start_d;       // p1 - p0 + 1 entries
@@ -305,6 +309,7 @@ struct kmc_batch {
     uint32_t scan_parts;
     uint64_t* bitvol_d;
     uint64_t bitvol_words;
+    bool two_phase;                         // planned for batch_launch_front / batch_launch_emit
     bool flat;                              // flat emit (else the tile teams)
     bool flat_ok;                           // every pass's rows fit the flat records' 20-bit y / z
     uint32_t* cpre_d;                       // in-row chunk prefixes of the count pass (flat)
@@ -393,10 +398,16 @@ kmc_status plan_tiles(kmc_batch* b, uint32_t r_max, uint32_t queue_cap)
         plan_rows(p.a);
     }
     for (Group& g : b->groups) {
+        /* the graph's emit takes a group's passes in one launch; the two-phase
+         * form launches each pass by itself */
+        uint64_t steps = 0;
+        for (uint32_t i = g.p0; i < g.p1; ++i) steps += emit_steps(b->passes[i].a);
+        for (uint32_t i = g.p0; i < g.p1 && !b->two_phase; ++i) plan_emit(b->passes[i].a, steps);
         std::vector<uint64_t> rs, ts;
         uint64_t r = 0, t = 0;
         uint32_t stride = 0, teams = kEmitTeams;
         g.max_levels = 0;
+        g.emit_blocks = 1;
         for (uint32_t i = g.p0; i < g.p1; ++i) {
             rs.push_back(r);
             ts.push_back(t);
@@ -404,6 +415,7 @@ kmc_status plan_tiles(kmc_batch* b, uint32_t r_max, uint32_t queue_cap)
             t += b->passes[i].a.nunits;
             stride = std::max(stride, b->passes[i].a.team_stride);
             g.max_levels = std::max(g.max_levels, b->passes[i].a.nlev);
+            g.emit_blocks = std::max(g.emit_blocks, b->passes[i].a.eblocks);
         }
         /* one emit launch per group: every team region of a workgroup is as
          * large as the group's largest, and as many teams as 64 KiB hold */
@@ -495,6 +507,8 @@ hipError_t record_emit(kmc_batch* b, hipStream_t st, bool host_sizes)
         for (const Group& g : b->groups) {
             if (host_sizes) {
                 for (uint32_t i = g.p0; i < g.p1 && e == hipSuccess; ++i) e = launch_flat_emit(g.dtype, b->passes[i].a, st);
+            } else if (g.mode == 0) {
+                e = launch_dup_batch(g.dtype, b->jobs_d + g.p0, g.p1 - g.p0, g.emit_blocks, g.max_levels, st);
             } else {
                 e = launch_compact_batch(b->jobs_d + g.p0, g.row_start_d, g.p1 - g.p0, g.rows, st);
                 if (e == hipSuccess)
@@ -656,6 +670,7 @@ kmc_status create_impl(const kmc_job* jobs, uint32_t n_jobs, uint32_t flags, hip
     b->r_max = 16;
     b->queue_cap = 128;
     b->upload_stream = st;
+    b->two_phase = plan_only;
 
     /* jobs: device values, min/max, object coordinates */
     b->users.resize(n_jobs);
@@ -878,7 +893,7 @@ hipError_t batch_launch_emit(kmc_batch* b, hipStream_t st)
                 T += nt;
             }
             off[i] = bytes;
-            bytes += record_bytes(V, T, p.a.vnormal != 0);
+            bytes += emit_record_bytes(p.a, V, T);
             b->istart_h[i] = vsum;
             b->istart_h[np + 1 + i] = tsum;
             vsum += V;
@@ -920,14 +935,18 @@ uint64_t batch_work_bytes(const kmc_batch* b)
 
 uint64_t batch_record_arena_bytes(const kmc_batch* b) { return b->flat ? b->cap_r : 0; }
 
-/* Flat-emit record bytes surface i adds once its sizes are known. */
+/* Record bytes surface i is budgeted with once its sizes are known (8 per
+ * vertex and 9 per triangle, 28 more per vertex with VertexNormal; an upper
+ * bound of what its emit takes). */
 uint64_t batch_record_bytes(const kmc_batch* b, uint32_t i)
 {
     const uint32_t sg = b->surface_seg[i];
     if (!b->flat || sg == ~0u) return 0;
     const Pass& p = b->passes[b->seg_pass_level[sg] >> 3];
     const SegOut& so = b->segout_h[sg];
-    return record_bytes(p.a.dup ? 0 : so.nv, so.nt, p.a.vnormal != 0);
+    const uint64_t nv = p.a.dup ? 0 : so.nv;
+    return align256(nv * 8) + align256(so.nt * 8) + align256(so.nt) +
+           (p.a.vnormal ? align256(so.nt * 12) + align256(nv * 16) : 0);
 }
 
 void batch_destroy(kmc_batch* b) { destroy(b); }

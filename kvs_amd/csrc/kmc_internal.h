@@ -59,8 +59,16 @@ void init_surface(kmc_surface* s, double iso, int normal_type, int dup, double m
 void init_job(JobArgs& a, const kmc_volume* v, const void* dvals, const double* iso, uint32_t nlev, int normal_type,
               int dup, double mn, double mx, const float minc[3], const float maxc[3]);
 
+void float_range(JobArgs& a);
+
 /* Row geometry of every emit (a.nx, a.ny, a.nz set): a.NC, a.cshift, a.nrows. */
 void plan_rows(JobArgs& a);
+
+/* Split of the chunk-batch emit (rows planned; a.nlev set): a.erows and
+ * a.eblocks of a pass whose emit shares its launch with others, `all` being
+ * the sum of their emit_steps. */
+uint64_t emit_steps(const JobArgs& a);
+void plan_emit(JobArgs& a, uint64_t all);
 
 /* True when the flat emit serves a volume of these y / z sizes (its records
  * pack y and z in 20 bits) and KMC_EMIT does not ask for the tile teams. */
@@ -88,10 +96,13 @@ hipError_t launch_flat_emit(int dtype, const JobArgs& a, hipStream_t st, hipEven
  * per-item kernels over the items start[j] .. start[j + 1] of each job. */
 hipError_t launch_compact_batch(const JobArgs* jobs, const uint64_t* row_start, uint32_t njobs, uint64_t rows,
                                 hipStream_t st);
-/* the per-item kernels of one pass whose record offsets are set (after its compaction) */
-hipError_t launch_flat_items(int dtype, const JobArgs& a, hipStream_t st);
 hipError_t launch_flat_batch(int dtype, int mode, const JobArgs* jobs, const uint64_t* vstart, const uint64_t* tstart,
                              uint32_t njobs, hipStream_t st);
+/* Chunk-batch emit (kmc_emit.hip): the duplicated triangles of a pass, or of
+ * a batch group's passes (`blocks` / `levels`: the most of one of them). */
+hipError_t launch_dup(int dtype, const JobArgs& a, hipStream_t st);
+hipError_t launch_dup_batch(int dtype, const JobArgs* jobs, uint32_t njobs, uint32_t blocks, uint32_t levels,
+                            hipStream_t st);
 hipError_t launch_classify(int dtype, const JobArgs& a, hipStream_t st);
 /* SlicePlane: masks from the plane's sign (a.plane), and the duplicated emit
  * (compaction, then one thread per triangle with per-vertex colours). */

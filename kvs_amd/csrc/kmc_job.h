@@ -75,8 +75,12 @@ struct JobArgs {
     uint32_t teams;        // teams per emit workgroup (<= kEmitTeams; fewer when a team's LDS is large)
     uint32_t rec_levels;   // flat emit: bit l set when level l has records (levels without outputs get none)
     uint64_t nunits;   // nlev * nb * nslabs
+    uint32_t erows;    // chunk-batch emit: node rows per wave step (at most 64 >> cshift) ...
+    uint32_t eblocks;  // ... and workgroups per level
     uint64_t nrows;    // nz * ny: counts and prefixes are kept per node row
     double minv, maxv; // clamp range of the interpolation (volume min/max)
+    float fminv, fmaxv;    // the same as floats ...
+    uint32_t fclamp;       // ... 1: exactly, and minv <= maxv
     float minc[3];     // min object coordinate
     float sc[3];       // (max - min) / ncells, per axis (float ops, host side)
     double iso[kMaxLevels];

@@ -30,21 +30,13 @@
 #include <algorithm>
 #include <map>
 #include <mutex>
+#include "kmc_device.h"
+#include "kmc_internal.h"
 #include "kmc_job.h"
-#include "mc_tables.h"
 
 #pragma clang fp contract(off)
 
 namespace kmc {
-
-__constant__ uint64_t d_tri[256] = { KMC_TABLE_WORDS };
-
-/* Emit modes, a template parameter so that each kernel carries only its own
- * path: duplicated vertices, shared vertices with PolygonNormal, shared
- * vertices with VertexNormal. */
-enum : int { kModeDup = 0, kModePolygon = 1, kModeVertex = 2 };
-
-__host__ __device__ inline int emit_mode(const JobArgs& a) { return a.dup ? kModeDup : (a.vnormal ? kModeVertex : kModePolygon); }
 
 /* ------------------------------------------------------------------------- */
 /* classification                                                              */
@@ -78,74 +70,6 @@ struct Classify<float> {
     }
 };
 
-__device__ __forceinline__ double iso_of(const JobArgs& a, int l)
-{
-    double r = a.iso[0];
-#pragma unroll
-    for (int k = 1; k < kMaxLevels; ++k)
-        if (k == l) r = a.iso[k];
-    return r;
-}
-
-/* ------------------------------------------------------------------------- */
-/* interpolation and normals                                                   */
-/* ------------------------------------------------------------------------- */
-
-template <typename T>
-__device__ __forceinline__ void interpolate_values(const JobArgs& a, double iso, T value_a, T value_b,
-                                                   uint32_t ax, uint32_t ay, uint32_t az,
-                                                   uint32_t bx, uint32_t by, uint32_t bz, float out[3]);
-
-/* interpolate_vertex<T> + (p + min_coord) * scale_factor for the edge from
- * node a to node b (integer node coordinates). */
-template <typename T>
-__device__ __forceinline__ void interpolate(const JobArgs& a, const T* vol, double iso,
-                                            uint32_t ax, uint32_t ay, uint32_t az,
-                                            uint32_t bx, uint32_t by, uint32_t bz, float out[3])
-{
-    const uint64_t line = a.nx, slice = (uint64_t)a.nx * a.ny;
-    const uint64_t ia = ax + ay * line + az * slice;
-    const uint64_t ib = bx + by * line + bz * slice;
-    interpolate_values<T>(a, iso, vol[ia], vol[ib], ax, ay, az, bx, by, bz, out);
-}
-
-/* The interpolation of interpolate() from the two node values. */
-template <typename T>
-__device__ __forceinline__ void interpolate_values(const JobArgs& a, double iso, T value_a, T value_b,
-                                                   uint32_t ax, uint32_t ay, uint32_t az,
-                                                   uint32_t bx, uint32_t by, uint32_t bz, float out[3])
-{
-    double va = (double)value_a;
-    double vb = (double)value_b;
-    va = va <= a.minv ? a.minv : (va <= a.maxv ? va : a.maxv);
-    vb = vb <= a.minv ? a.minv : (vb <= a.maxv ? vb : a.maxv);
-    double r = (iso - va) / (vb - va);
-    r = r < 0 ? -r : r;
-    const double s = 1.0 - r;
-    const double pa[3] = { (double)(float)ax, (double)(float)ay, (double)(float)az };
-    const double pb[3] = { (double)(float)bx, (double)(float)by, (double)(float)bz };
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const double t0 = s * pa[k];
-        const double t1 = r * pb[k];
-        const float p = (float)(t0 + t1);
-        const float q = p + a.minc[k];
-        out[k] = q * a.sc[k];
-    }
-}
-
-__device__ __forceinline__ void face_normal(const float v0[3], const float v1[3], const float v2[3], float n[3])
-{
-    const float d1x = v1[0] - v0[0], d1y = v1[1] - v0[1], d1z = v1[2] - v0[2];
-    const float d2x = v2[0] - v0[0], d2y = v2[1] - v0[1], d2z = v2[2] - v0[2];
-    const float p0 = d1y * d2z, p1 = d1z * d2y;
-    const float p2 = d1z * d2x, p3 = d1x * d2z;
-    const float p4 = d1x * d2y, p5 = d1y * d2x;
-    n[0] = p0 - p1;
-    n[1] = p2 - p3;
-    n[2] = p4 - p5;
-}
-
 /* ------------------------------------------------------------------------- */
 /* tile-team emit                                                              */
 /* ------------------------------------------------------------------------- */
@@ -155,32 +79,6 @@ __device__ __forceinline__ void face_normal(const float v0[3], const float v1[3]
  * waits for another wave.  The LDS operations of one wave complete in issue
  * order; wave_sync only keeps the compiler from moving memory operations
  * across the points where lanes start reading what other lanes wrote. */
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-__device__ __forceinline__ uint32_t uniform(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
-
-__device__ __forceinline__ uint64_t uniform64(uint64_t x)
-{
-    return (uint64_t)uniform((uint32_t)(x >> 32)) << 32 | uniform((uint32_t)x);
-}
-
-__device__ __forceinline__ uint64_t readlane64(uint64_t x, int k)
-{
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, k);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(x >> 32), k);
-    return (uint64_t)hi << 32 | lo;
-}
-
-/* Set bits of the wave mask m on the lanes below this one (v_mbcnt). */
-__device__ __forceinline__ uint32_t lanes_below(uint64_t m)
-{
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
 
 /* LDS arrays of one team (layout of lds_layout) and the shared case table. */
 struct Team {
@@ -286,15 +184,6 @@ __device__ __forceinline__ uint32_t* wrow(const Team& v, int z, uint32_t ws, uin
 __device__ __forceinline__ uint32_t cidx(const Team& v, uint32_t cs, uint32_t j, uint32_t c)
 {
     return (cs * (v.R + 1) + j) * v.NC + c;
-}
-
-/* Mask of the nodes x < limit inside chunk c. */
-__device__ __forceinline__ uint64_t valid_mask(uint32_t c, uint32_t limit)
-{
-    const uint32_t x0 = c * 64u;
-    if (limit <= x0) return 0ull;
-    const uint32_t n = limit - x0;
-    return n >= 64u ? ~0ull : ((1ull << n) - 1ull);
 }
 
 /* Bits of chunk c of a row of NC chunks shifted so that bit i holds node x+1. */
@@ -421,17 +310,6 @@ __device__ __forceinline__ Span grid_span(uint64_t b, uint64_t e, uint32_t units
 /* ------------------------------------------------------------------------- */
 /* wave scan                                                                   */
 /* ------------------------------------------------------------------------- */
-
-__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x)
-{
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t t = __shfl_up(x, d);
-        if (lane >= d) x += t;
-    }
-    return x;
-}
 
 /* In-place exclusive scan of n u32 values in LDS by one wave; returns the
  * total (the same in every lane). */
@@ -585,27 +463,6 @@ __device__ __forceinline__ void node_edge_coords(const JobArgs& a, const T* vol,
     interpolate<T>(a, vol, iso, x, y, z, x + (axis == 0), y + (axis == 1), z + (axis == 2), out);
 }
 
-/* Owner node offset (dx, dy, dz) and axis of local edge e, packed as
- * dx | dy << 1 | dz << 2 | axis << 3 (connect_isopoints, :493-504), five
- * bits per edge. */
-__device__ __forceinline__ uint32_t edge_owner(uint32_t e)
-{
-    constexpr uint64_t kOwner =
-        (0x00ull << 0) | (0x09ull << 5) | (0x02ull << 10) | (0x08ull << 15) | (0x04ull << 20) | (0x0Dull << 25) |
-        (0x06ull << 30) | (0x0Cull << 35) | (0x10ull << 40) | (0x11ull << 45) | (0x13ull << 50) | (0x12ull << 55);
-    return (uint32_t)(kOwner >> (5 * e)) & 31u;
-}
-
-/* Table-orientation endpoints of local edge e as two corner offsets packed
- * bit0 x, bit1 y, bit2 z, first endpoint in the low nibble
- * (MarchingCubesTable.cpp:276-290), eight bits per edge. */
-__device__ __forceinline__ uint32_t edge_ends(uint32_t e)
-{
-    constexpr uint64_t kLo = 0x4667755402233110ull;   // edges 0..7
-    constexpr uint32_t kHi = 0x62735140u;             // edges 8..11
-    return e < 8 ? (uint32_t)(kLo >> (8 * e)) & 0xFFu : (kHi >> (8 * (e - 8))) & 0xFFu;
-}
-
 /* Output bases of tile (z, band): vertex prefixes of node rows (z-1, y0),
  * (z-1, y0+R), (z, y0), (z, y0+R) and the triangle prefix of cell row
  * (y0, z-1), relative to the first row of their segment; one lane loads each
@@ -652,22 +509,6 @@ __device__ __forceinline__ uint32_t tile_rank(const JobArgs& a, const Team& v, i
     if (axis >= 1) r += (uint32_t)((e.x >> i) & 1ull);
     if (axis >= 2) r += (uint32_t)((e.y >> i) & 1ull);
     return r;
-}
-
-/* The four cells around the edge of node (x, y, zv) along axis, in scan
- * order: offsets across the edge are -1/0 along the other two axes (low axis
- * first); the edge's local id in cell q is the q-th nibble of `around`. */
-__device__ __forceinline__ void around_cell(uint32_t axis, int q, int x, int y, int zv, int& cx, int& cy, int& cz)
-{
-    const int lo = (q & 1) ? 0 : -1, hi = (q & 2) ? 0 : -1;
-    cx = x + (axis == 0 ? 0 : lo);
-    cy = y + (axis == 0 ? lo : (axis == 1 ? 0 : hi));
-    cz = zv + (axis == 2 ? 0 : hi);
-}
-
-__device__ __forceinline__ uint32_t around_nibbles(uint32_t axis)
-{
-    return axis == 0 ? 0x0246u : (axis == 1 ? 0x3175u : 0x89BAu);
 }
 
 /* VertexNormal of the vertex on (x,y,zv,axis): the float sum, in triangle
@@ -1213,61 +1054,6 @@ __global__ __launch_bounds__(kBlock) void k_classify_batch(const JobArgs* jobs, 
 /* count pass: per-row counts from the bit volume                              */
 /* ------------------------------------------------------------------------- */
 
-/* Crossing edges and active cells of chunk c of node row (y, z) of one level,
- * read straight from the bit volume `lev` (coalesced across the lanes of a
- * row, neighbours from L1/L2).  x/y/z: crossing edges owned by the row's
- * nodes; act: active cells of cell row (y, z-1); k0/k3/k4/k7: the masks of
- * the cells' four node rows (bit i of kq is corner q of cell x = 64c + i; the
- * x+1 corners 1, 2, 5, 6 are the next bits of the same masks); next: bit 0 of
- * the next chunk's word of those four rows (corners 1, 2, 5, 6 of cell 63). */
-struct RowChunk {
-    uint64_t x, y, z, act;
-    uint64_t k0, k3, k4, k7;
-    uint32_t next;
-};
-
-__device__ __forceinline__ void row_chunk(const JobArgs& a, const uint64_t* lev, uint32_t y, uint32_t z, uint32_t c,
-                                          RowChunk& o)
-{
-    const uint64_t slice_words = (uint64_t)a.ny * a.NC;
-    const bool has_up = y + 1 < a.ny, has_next = z + 1 < a.nz, has_cells = z >= 1 && has_up;
-    /* Every load is issued (no branch around it): a neighbour row outside the
-     * volume is read as the row itself, which makes its crossings (b ^ u,
-     * b ^ n0) zero, and the cells are masked out below.  The next chunk of a
-     * row's last chunk is read as the chunk itself: its bit 0 lands only on
-     * bit 63 of the shifted words and of `next`, i.e. on node / cell 64c + 63,
-     * which lies at or past nx - 1 in a row's last chunk, so valid_mask(c,
-     * nx - 1) clears it from x and act (and corner_pairs reads `next` only for
-     * an active cell 63). */
-    const uint64_t* row = lev + (uint64_t)z * slice_words + (uint64_t)y * a.NC;
-    const uint64_t* up = has_up ? row + a.NC : row;
-    const uint64_t* nz = has_next ? row + slice_words : row;
-    const uint64_t* pr = has_cells ? row - slice_words : row;
-    const uint64_t* pu = has_cells ? pr + a.NC : row;
-    const uint32_t cn = c + 1 < a.NC ? c + 1 : c;
-    const uint64_t b = row[c], b1 = row[cn];
-    const uint64_t u = up[c], u1 = up[cn];
-    const uint64_t n0 = nz[c];
-    const uint64_t p = pr[c], p1 = pr[cn];
-    const uint64_t q = pu[c], q1 = pu[cn];
-    const uint64_t c4 = b, c5 = (b >> 1) | (b1 << 63);
-    const uint64_t c7 = u, c6 = (u >> 1) | (u1 << 63);
-    const uint64_t c1 = (p >> 1) | (p1 << 63), c2 = (q >> 1) | (q1 << 63);
-    const uint64_t vx = valid_mask(c, a.nx - 1), vn = valid_mask(c, a.nx);
-    o.x = (b ^ c5) & vx;
-    o.y = (b ^ u) & vn;
-    o.z = (b ^ n0) & vn;
-    const uint64_t or_ = p | c1 | c2 | q | c4 | c5 | c6 | c7;
-    const uint64_t an = p & c1 & c2 & q & c4 & c5 & c6 & c7;
-    o.act = has_cells ? (or_ & ~an) & vx : 0ull;
-    o.k0 = p;
-    o.k3 = q;
-    o.k4 = c4;
-    o.k7 = c7;
-    o.next = (uint32_t)(p1 & 1ull) | (uint32_t)(q1 & 1ull) << 1 | (uint32_t)(b1 & 1ull) << 2 |
-             (uint32_t)(u1 & 1ull) << 3;
-}
-
 /* (y, z) of node row g + sub of a wave that walks row groups g = g0, g0 +
  * step, ... (g0 and step are the same on all of the wave's lanes): the
  * group's first row advances by the step's quotient and remainder by ny,
@@ -1309,28 +1095,6 @@ __device__ __forceinline__ void row_next(const JobArgs& a, RowWalk& w)
         w.yg -= a.ny;
         ++w.zg;
     }
-}
-
-/* The cube index with bits 2, 3 and bits 6, 7 swapped (an involution). */
-__device__ __forceinline__ uint32_t swap_pairs(uint32_t c)
-{
-    return (c & 0x33u) | ((c & 0x44u) << 1) | ((c & 0x88u) >> 1);
-}
-
-/* swap_pairs(cube index) of cell i of a chunk: the corners (x, x+1) of each of
- * the cell's four node rows are two adjacent bits of that row's mask (k0, k3,
- * k4, k7), taken as one 2-bit window; for cell 63 the x+1 bits come from the
- * next chunk (o.next). */
-__device__ __forceinline__ uint32_t corner_pairs(const RowChunk& o, uint32_t i)
-{
-    if (i == 63u) {
-        return (uint32_t)(o.k0 >> 63) | (o.next & 1u) << 1 | (uint32_t)(o.k3 >> 63) << 2 |
-               ((o.next >> 1) & 1u) << 3 | (uint32_t)(o.k4 >> 63) << 4 | ((o.next >> 2) & 1u) << 5 |
-               (uint32_t)(o.k7 >> 63) << 6 | ((o.next >> 3) & 1u) << 7;
-    }
-    const uint32_t p0 = (uint32_t)(o.k0 >> i) & 3u, p3 = (uint32_t)(o.k3 >> i) & 3u;
-    const uint32_t p4 = (uint32_t)(o.k4 >> i) & 3u, p7 = (uint32_t)(o.k7 >> i) & 3u;
-    return p0 | p3 << 2 | p4 << 4 | p7 << 6;
 }
 
 /* x of the lane d below within its DPP row of 16 lanes (0 for the row's
@@ -1602,22 +1366,6 @@ __device__ __forceinline__ uint32_t level_at(const uint64_t* off, uint32_t nlev,
     uint32_t l = 0;
     for (uint32_t k = 1; k < nlev; ++k) l += i >= off[k] ? 1u : 0u;
     return l;
-}
-
-/* In-row prefixes (vertices, triangles) of chunk word w.  Rows of at most 64
- * chunks keep both in one word of vpc (vertices in the low, triangles in the
- * high 16 bits: at most 63 chunks of 192 and 320 come before a chunk);
- * longer rows keep them in vpc and tpc. */
-__device__ __forceinline__ void chunk_prefix(const JobArgs& a, uint64_t w, uint32_t& v, uint32_t& t)
-{
-    if (a.NC <= 64) {
-        const uint32_t p = a.vpc[w];
-        v = p & 0xFFFFu;
-        t = p >> 16;
-    } else {
-        v = a.vpc[w];
-        t = a.tpc[w];
-    }
 }
 
 /* One non-empty chunk of the compaction, queued as y | z << 20 | level << 40
@@ -1892,7 +1640,7 @@ __device__ __forceinline__ void stage_table_block(uint64_t* tri)
     __syncthreads();
 }
 
-/* Every triangle of shared vertices (duplicated ones: dup_finish): its
+/* Every triangle of shared vertices (duplicated ones: kmc_emit.hip): its
  * connectivity (connect_isopoints, :439-521) and the face normal of the
  * shared vertices' coordinates -- the PolygonNormal output
  * (calculate_normals_on_polygon, :531-559) or, with VertexNormal, kept in
@@ -1916,7 +1664,7 @@ __device__ __forceinline__ void triangle_item(const JobArgs& a, const uint64_t* 
     if (!coords) return;   // a level without outputs (not admitted)
     const uint64_t id = g - a.toff[l];
     float p[3][3], nn[3];
-    static_assert(M != kModeDup, "duplicated triangles: dup_finish");
+    static_assert(M != kModeDup, "duplicated triangles: kmc_emit.hip");
     const ChunkCross* cross_l = a.cross + (uint64_t)l * level_words;
     /* the owner chunks' crossing records of all three edges are loaded
      * before any is used, so the three loads are in flight together */
@@ -1974,146 +1722,22 @@ __device__ __forceinline__ void triangle_item(const JobArgs& a, const uint64_t* 
     dst[2] = nn[2];
 }
 
-/* A duplicated triangle in flight: its record and cube index, and the node
- * values at both ends of its three edges. */
-template <typename T>
-struct DupItem {
-    uint64_t rec;
-    uint32_t ci;
-    T va[3], vb[3];
-};
-
-/* The three edges of triangle t of cube index ci, in table order. */
-__device__ __forceinline__ void dup_edges(const uint64_t* tri, uint64_t rec, uint32_t ci, uint32_t eds[3])
-{
-    const uint32_t t = (uint32_t)(rec >> 60);
-    const uint64_t w = tri[ci];
-    eds[0] = (uint32_t)((w >> (12 * t)) & 0xF);
-    eds[1] = (uint32_t)((w >> (12 * t + 8)) & 0xF);
-    eds[2] = (uint32_t)((w >> (12 * t + 4)) & 0xF);
-}
-
-/* Issues the node-value loads of item d (its record and cube index set). */
-template <typename T>
-__device__ __forceinline__ void dup_load(const JobArgs& a, const uint64_t* tri, DupItem<T>& d)
-{
-    const T* vol = (const T*)a.values;
-    const uint64_t line = a.nx, slice = (uint64_t)a.nx * a.ny;
-    const uint64_t x = d.rec & 0xFFFFFu, y = (d.rec >> 20) & 0xFFFFFu, zc = (d.rec >> 40) & 0xFFFFFu;
-    uint32_t eds[3];
-    dup_edges(tri, d.rec, d.ci, eds);
-#pragma unroll
-    for (int jj = 0; jj < 3; ++jj) {
-        const uint32_t qq = edge_ends(eds[jj]);
-        const uint64_t ia = (x + (qq & 1u)) + (y + ((qq >> 1) & 1u)) * line + (zc + ((qq >> 2) & 1u)) * slice;
-        const uint64_t ib = (x + ((qq >> 4) & 1u)) + (y + ((qq >> 5) & 1u)) * line + (zc + ((qq >> 6) & 1u)) * slice;
-        d.va[jj] = vol[ia];
-        d.vb[jj] = vol[ib];
-    }
-}
-
-/* Duplicated triangle g from its loaded item: its three vertices in table
- * orientation and its face normal (extract_surfaces_with_duplication,
- * :155-243), as triangle_item computes them. */
-template <typename T>
-__device__ __forceinline__ void dup_finish(const JobArgs& a, const uint64_t* tri, uint64_t g, const DupItem<T>& d)
-{
-    const uint32_t l = level_at(a.toff, a.nlev, g);
-    float* coords = nullptr;
-    float* normals = nullptr;
-#pragma unroll
-    for (int k = 0; k < kMaxLevels; ++k)
-        if (k == (int)l) { coords = a.coords[k]; normals = a.normals[k]; }
-    if (!coords) return;   // a level without outputs (not admitted)
-    const uint64_t id = g - a.toff[l];
-    const double iso = iso_of(a, (int)l);
-    const uint32_t x = (uint32_t)(d.rec & 0xFFFFFu), y = (uint32_t)((d.rec >> 20) & 0xFFFFFu);
-    const uint32_t zc = (uint32_t)((d.rec >> 40) & 0xFFFFFu);
-    uint32_t eds[3];
-    dup_edges(tri, d.rec, d.ci, eds);
-    float p[3][3], nn[3];
-#pragma unroll
-    for (int jj = 0; jj < 3; ++jj) {
-        const uint32_t qq = edge_ends(eds[jj]);
-        interpolate_values<T>(a, iso, d.va[jj], d.vb[jj], x + (qq & 1u), y + ((qq >> 1) & 1u), zc + ((qq >> 2) & 1u),
-                              x + ((qq >> 4) & 1u), y + ((qq >> 5) & 1u), zc + ((qq >> 6) & 1u), p[jj]);
-    }
-    face_normal(p[0], p[1], p[2], nn);
-    float* co = coords + 9 * id;
-#pragma unroll
-    for (int jj = 0; jj < 3; ++jj) {
-        co[3 * jj + 0] = p[jj][0];
-        co[3 * jj + 1] = p[jj][1];
-        co[3 * jj + 2] = p[jj][2];
-    }
-    normals[3 * id + 0] = nn[0];
-    normals[3 * id + 1] = nn[1];
-    normals[3 * id + 2] = nn[2];
-}
-
-/* Duplicated triangles g, g + step, ... < n, software-pipelined over two
- * register sets that take turns (a copy of a loaded value would wait for its
- * load): while item g is interpolated and stored, the node values of the
- * next item and the record of the one after it are in flight (vector memory
- * operations complete in issue order, so the wait for item g's values leaves
- * the newer loads outstanding); indices past the range's end are clamped to
- * its last item, so that every iteration issues the same loads. */
-template <typename T>
-__device__ __forceinline__ void triangles_range_dup(const JobArgs& a, const uint64_t* tri, uint64_t g, uint64_t n,
-                                                    uint64_t step)
-{
-    if (g >= n) return;
-    const uint64_t last = n - 1;
-    DupItem<T> d0, d1;
-    d0.rec = a.trec[g];
-    d0.ci = a.tci[g];
-    dup_load<T>(a, tri, d0);
-    uint64_t gn = g + step < last ? g + step : last;
-    uint64_t rn = a.trec[gn];
-    uint32_t cn = a.tci[gn];
-    for (;;) {
-        d1.rec = rn;
-        d1.ci = cn;
-        dup_load<T>(a, tri, d1);
-        gn = g + 2 * step < last ? g + 2 * step : last;
-        rn = a.trec[gn];
-        cn = a.tci[gn];
-        dup_finish<T>(a, tri, g, d0);
-        g += step;
-        if (g >= n) break;
-        d0.rec = rn;
-        d0.ci = cn;
-        dup_load<T>(a, tri, d0);
-        gn = g + 2 * step < last ? g + 2 * step : last;
-        rn = a.trec[gn];
-        cn = a.tci[gn];
-        dup_finish<T>(a, tri, g, d1);
-        g += step;
-        if (g >= n) break;
-    }
-}
-
-/* Triangles g, g + step, ... < n: duplicated ones through the two-stage
- * pipeline above; with shared vertices the next item's record is loaded
- * while this one is worked on. */
+/* Triangles g, g + step, ... < n: the next item's record is loaded while this
+ * one is worked on. */
 template <typename T, int M>
 __device__ __forceinline__ void triangles_range(const JobArgs& a, const uint64_t* tri, uint64_t g, uint64_t n,
                                                 uint64_t step)
 {
-    if constexpr (M == kModeDup) {
-        triangles_range_dup<T>(a, tri, g, n, step);
-    } else {
-        uint64_t rec = g < n ? a.trec[g] : 0ull;
-        uint32_t ci = g < n ? a.tci[g] : 0u;
-        for (; g < n; g += step) {
-            const uint64_t cur = rec;
-            const uint32_t cur_ci = ci;
-            if (g + step < n) {
-                rec = a.trec[g + step];
-                ci = a.tci[g + step];
-            }
-            triangle_item<T, M>(a, tri, g, cur, cur_ci);
+    uint64_t rec = g < n ? a.trec[g] : 0ull;
+    uint32_t ci = g < n ? a.tci[g] : 0u;
+    for (; g < n; g += step) {
+        const uint64_t cur = rec;
+        const uint32_t cur_ci = ci;
+        if (g + step < n) {
+            rec = a.trec[g + step];
+            ci = a.tci[g + step];
         }
+        triangle_item<T, M>(a, tri, g, cur, cur_ci);
     }
 }
 
@@ -2393,7 +2017,6 @@ __global__ __launch_bounds__(kBlock) void k_vertex_normals_batch(const JobArgs* 
         }
     });
 }
-
 
 /* ------------------------------------------------------------------------- */
 /* SlicePlane: classification by a plane, emit with per-vertex colours         */
@@ -3216,11 +2839,10 @@ template <typename T>
 hipError_t launch_flat_t(const JobArgs& a, hipStream_t st, hipEvent_t* marks)
 {
     const uint64_t nv = a.voff[a.nlev], nt = a.toff[a.nlev];
-    if (!a.dup && nv) hipLaunchKernelGGL((k_vertices<T>), dim3(flat_blocks(nv)), dim3(kBlock), 0, st, a);
+    if (nv) hipLaunchKernelGGL((k_vertices<T>), dim3(flat_blocks(nv)), dim3(kBlock), 0, st, a);
     if (marks) (void)hipEventRecord(marks[1], st);
     if (nt) {
         switch (emit_mode(a)) {
-        case kModeDup: hipLaunchKernelGGL((k_triangles<T, kModeDup>), dim3(flat_blocks(nt)), dim3(kBlock), 0, st, a); break;
         case kModePolygon:
             hipLaunchKernelGGL((k_triangles<T, kModePolygon>), dim3(flat_blocks(nt)), dim3(kBlock), 0, st, a);
             break;
@@ -3247,30 +2869,13 @@ hipError_t launch_flat_batch_t(int mode, const JobArgs* jobs, const uint64_t* vs
 {
     /* item counts live on the device: persistent grids */
     const dim3 g(256 * 8), b(kBlock);
-    if (mode != kModeDup) hipLaunchKernelGGL((k_vertices_batch<T>), g, b, 0, st, jobs, vstart, njobs);
+    hipLaunchKernelGGL((k_vertices_batch<T>), g, b, 0, st, jobs, vstart, njobs);
     switch (mode) {
-    case kModeDup: hipLaunchKernelGGL((k_triangles_batch<T, kModeDup>), g, b, 0, st, jobs, tstart, njobs); break;
     case kModePolygon: hipLaunchKernelGGL((k_triangles_batch<T, kModePolygon>), g, b, 0, st, jobs, tstart, njobs); break;
     default: hipLaunchKernelGGL((k_triangles_batch<T, kModeVertex>), g, b, 0, st, jobs, tstart, njobs); break;
     }
     if (mode == kModeVertex) hipLaunchKernelGGL(k_vertex_normals_batch, g, b, 0, st, jobs, vstart, njobs);
     return hipGetLastError();
-}
-
-hipError_t launch_flat_items(int dtype, const JobArgs& a, hipStream_t st)
-{
-    switch (dtype) {
-    case 0: return launch_flat_t<int8_t>(a, st, nullptr);
-    case 1: return launch_flat_t<int16_t>(a, st, nullptr);
-    case 2: return launch_flat_t<int32_t>(a, st, nullptr);
-    case 3: return launch_flat_t<int64_t>(a, st, nullptr);
-    case 4: return launch_flat_t<uint8_t>(a, st, nullptr);
-    case 5: return launch_flat_t<uint16_t>(a, st, nullptr);
-    case 6: return launch_flat_t<uint32_t>(a, st, nullptr);
-    case 7: return launch_flat_t<uint64_t>(a, st, nullptr);
-    case 8: return launch_flat_t<float>(a, st, nullptr);
-    default: return launch_flat_t<double>(a, st, nullptr);
-    }
 }
 
 hipError_t launch_flat_batch(int dtype, int mode, const JobArgs* jobs, const uint64_t* vstart, const uint64_t* tstart,
@@ -3292,6 +2897,12 @@ hipError_t launch_flat_batch(int dtype, int mode, const JobArgs* jobs, const uin
 
 hipError_t launch_flat_emit(int dtype, const JobArgs& a, hipStream_t st, hipEvent_t* marks)
 {
+    if (a.dup) {
+        if (marks) { (void)hipEventRecord(marks[0], st); (void)hipEventRecord(marks[1], st); }
+        const hipError_t e = launch_dup(dtype, a, st);
+        if (marks) (void)hipEventRecord(marks[2], st);
+        return e;
+    }
     const uint64_t G = 64u >> a.cshift;
     uint64_t blocks = ((a.nrows + G - 1) / G + kWaves - 1) / kWaves;
     if (blocks > 16384) blocks = 16384;
@@ -3488,7 +3099,6 @@ hipError_t launch_emit_batch(int dtype, int mode, const JobArgs* jobs, const uin
     default: return launch_emit_batch_t<double>(mode, jobs, unit_start, njobs, units, lds_bytes, teams, st);
     }
 }
-
 
 hipError_t launch_scan(const uint32_t* counts, uint64_t n, uint32_t narr, uint64_t* partials,
                        uint64_t* prefix, uint64_t* totals, hipStream_t st)

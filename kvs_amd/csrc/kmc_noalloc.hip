@@ -147,6 +147,7 @@ kmc_status extract_noalloc(const kmc_volume* v, double iso, int32_t normal_type,
         mx = host[1];
         a.minv = mn;
         a.maxv = mx;
+        float_range(a);
     }
     init_surface(out, iso, normal_type, dup, mn, mx, minc, maxc);
     const double d = mn - mx;
@@ -183,9 +184,11 @@ kmc_status extract_noalloc(const kmc_volume* v, double iso, int32_t normal_type,
     a.voff[0] = a.toff[0] = 0;
     a.voff[1] = dup ? 0 : nv;
     a.toff[1] = nt;
-    a.vkey = cv.take<uint64_t>(a.voff[1] * 8);
-    a.trec = cv.take<uint64_t>(nt * 8);
-    a.tci = cv.take<uint8_t>(nt);
+    if (!dup) {   // duplicated triangles need no records
+        a.vkey = cv.take<uint64_t>(a.voff[1] * 8);
+        a.trec = cv.take<uint64_t>(nt * 8);
+        a.tci = cv.take<uint8_t>(nt);
+    }
     a.fn = a.vnormal ? cv.take<float>(nt * 12) : nullptr;
     a.vslot = a.vnormal ? cv.take<uint32_t>(nv * 16) : nullptr;
     a.coords[0] = coords;
