@@ -139,9 +139,9 @@ kmc_status kmc_extract_levels(const kmc_volume* volume, const double* isolevels,
  * for connections; connections may be NULL with duplication).  Every work
  * array lives in one fixed device array of KMC_NOALLOC_SCRATCH_BYTES that the
  * library holds on each GPU it runs on until the process ends:
- *   - KMC_ERR_SCRATCH when the volume's work (about 48 bytes per 64-node chunk
- *     and 24 per node row) or the emit's records (about 8 bytes per vertex and
- *     9 per triangle, 28 more per vertex with VertexNormal) do not fit;
+ *   - KMC_ERR_SCRATCH when the bytes budgeted for the volume's work (about 48
+ *     per 64-node chunk and 24 per node row) or for the emit (about 8 per vertex
+ *     and 9 per triangle, 28 more per vertex with VertexNormal) do not fit;
  *   - KMC_ERR_CAPACITY when the outputs do not fit: *out then holds the sizes
  *     (n_vertices, n_triangles, n_connections, n_normals) and nothing was written.
  * On KMC_OK *out describes the caller's arrays (release is not needed).
@@ -339,7 +339,7 @@ typedef struct kmc_timing {
     double scan_ms;              /* row prefixes */
     double emit_ms;              /* coordinates, connections, normals: the four below together */
     uint32_t passes;
-    double compact_ms;           /* vertex keys and triangle records at their output ranks */
+    double compact_ms;           /* 0 (no separate compaction pass) */
     double vertices_ms;          /* coordinates */
     double triangles_ms;         /* connections and face normals (with duplication: coordinates too) */
     double vertex_normals_ms;    /* VertexNormal sums */

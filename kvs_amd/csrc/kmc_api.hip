@@ -495,24 +495,31 @@ uint64_t emit_steps(const JobArgs& a)
     return std::max(1u, a.nlev) * ((a.nrows + G - 1) / G * ((a.NC + 63) / 64));
 }
 
-/* Waves of a launch: 4096 (what 256 CUs hold at four waves per SIMD) up to
- * 8192 where each then still has four full steps -- the second half lets the
- * hardware even out a large pass's waves (512^3 float turbulence, three
- * levels: 460 us with 4096, 411 with 8192, 464 with 16384), while in a small
- * pass it only pays each wave's start twice (256^3 blobs: 26 us and 38).  A
- * wave takes as many rows at a time as its lanes hold, but at most a quarter
- * of its share of the pass: a surface lies in few neighbouring rows, and four
- * or more steps far apart even the waves out (256^3: 37 us with two steps, 26
- * with four, 27 with eight). */
-constexpr uint64_t kEmitWaves = 4096, kEmitWavesMax = 8192, kEmitSteps = 4;
+/* Waves of a launch: as many as the device holds of the kernel at once, and up
+ * to eight times that while each still has four full steps -- the later ones
+ * even out a large pass (1024^3 float turbulence, three levels, triangles /
+ * normals: 1666 / 1240 us with one time, 1367 / 1205 with two, 1250 / 1129
+ * with eight, 1277 / 1162 with sixteen; a half-filled round costs: 512^3 CT
+ * triangles 287 us with one time, 338 with 1.6) -- and no more than one per 32
+ * outputs.  A wave takes as many rows at a time as its lanes hold, but at most a
+ * quarter of its share of the pass: a surface lies in few neighbouring rows, and
+ * four steps far apart even the waves out (256^3 blobs, duplicated: 26 us, 36
+ * with two steps).  Where every chunk holds many outputs there is nothing to
+ * even out, and two steps keep the batches full (320 x 288 x 256 CT, vertices:
+ * 38 us, 42 with four). */
+constexpr uint64_t kEmitRounds = 8, kEmitItems = 32;
 
-void plan_emit(JobArgs& a, uint64_t all)
+void plan_emit(JobArgs& a, uint64_t all, uint32_t per_cu, uint64_t items)
 {
     const uint64_t own = emit_steps(a), nlev = std::max(1u, a.nlev);
-    const uint64_t waves = std::min(kEmitWavesMax, std::max(kEmitWaves, all / 4));
+    const uint64_t resident = 256ull * kWaves * per_cu;
+    uint64_t waves = resident * std::min(kEmitRounds, std::max<uint64_t>(1, all / 4 / resident));
+    if (items) waves = std::min(waves, std::max<uint64_t>(256, items / kEmitItems));
+    else waves = std::max(waves, std::min(2 * resident, all / 4));   // a batch's uneven passes even out by themselves
     const uint64_t want = std::max<uint64_t>(1, (waves * own + all - 1) / all / nlev);   // waves per level
+    const uint64_t steps = items > 4 * nlev * a.nrows * a.NC ? 2 : 4;
     a.erows = 64u >> a.cshift;
-    while (a.erows > 1 && a.nrows / a.erows < kEmitSteps * want) a.erows >>= 1;
+    while (a.erows > 1 && a.nrows / a.erows < steps * want) a.erows >>= 1;
     const uint64_t units = (a.nrows + a.erows - 1) / a.erows;
     a.eblocks = (uint32_t)std::max<uint64_t>(1, (std::min(units, want) + kWaves - 1) / kWaves);
 }
@@ -578,7 +585,7 @@ bool plan_geometry(JobArgs& a, uint32_t* lds_bytes, uint32_t r_max, uint32_t que
 
 uint32_t levels_per_pass(const kmc_volume* v, int vnormal)
 {
-    /* the flat emit keeps no per-team LDS state: every row length fits */
+    /* the chunk-batch emit keeps no per-team LDS state: every row length fits */
     if (flat_emit_fits(v->resolution[1], v->resolution[2])) return kMaxLevels;
     for (uint32_t nl = kMaxLevels; nl >= 1; --nl) {
         JobArgs a;
@@ -671,7 +678,7 @@ struct PassTimer {
         for (int i = 0; i < 9 && on; ++i)
             if (!t_ev[i] && hipEventCreate(&t_ev[i]) != hipSuccess) { (void)hipGetLastError(); on = false; }
     }
-    /* events between the flat emit's kernels (after compaction, vertices, triangles) */
+    /* events between the chunk-batch emit's kernels (start, after vertices, after triangles) */
     hipEvent_t* flat_marks() { flat = on; return on ? &t_ev[6] : nullptr; }
     bool mark(int i)
     {
@@ -710,14 +717,13 @@ kmc_status run_pass(const kmc_volume* v, const void* dvals, const double* iso, u
 {
     JobArgs a;
     init_job(a, v, dvals, iso, nlev, normal_type, dup, mn, mx, minc, maxc);
-    /* flat emit (compaction records + one thread per item) unless the records'
-     * 20-bit y / z fields do not fit or KMC_EMIT=team asks for the tile teams
-     * (read per call); only the tile teams need their LDS state to fit */
+    /* chunk-batch emit unless its 20-bit y / z fields do not fit or
+     * KMC_EMIT=team asks for the tile teams (read per call); only the tile teams
+     * need their LDS state to fit */
     const bool flat = flat_emit_fits(a.ny, a.nz);
     uint32_t lds = 0;
     if (!plan_geometry(a, &lds) && !flat) return KMC_ERR_INVALID_ARGUMENT;
     plan_rows(a);
-    a.rec_levels = (1u << nlev) - 1u;
 
     const uint32_t narr = 2 * nlev;
     const uint64_t n = a.nrows;
@@ -728,15 +734,15 @@ kmc_status run_pass(const kmc_volume* v, const void* dvals, const double* iso, u
     uint64_t* prefix = (uint64_t*)device_alloc(prefix_bytes);
     uint64_t* aux = (uint64_t*)device_alloc((size_t)(nparts + narr) * sizeof(uint64_t));
     const size_t chunks = (size_t)nlev * a.nz * a.ny * a.NC;
-    uint64_t* bitvol = (uint64_t*)device_alloc(chunks * sizeof(uint64_t));
+    uint64_t* bitvol = (uint64_t*)device_alloc(chunks * sizeof(uint64_t) + kBitSlack);
     uint32_t* cpre = flat ? (uint32_t*)device_alloc(2 * chunks * sizeof(uint32_t)) : nullptr;
-    ChunkCross* cross = (flat && !dup) ? (ChunkCross*)device_alloc(chunks * sizeof(ChunkCross)) : nullptr;
+    uint64_t* act = (flat && a.vnormal) ? (uint64_t*)device_alloc(chunks * sizeof(uint64_t) + kBitSlack) : nullptr;
     void* recs = nullptr;
     auto cleanup = [&]() {
         device_free(counts); device_free(prefix); device_free(aux); device_free(bitvol); device_free(cpre);
-        device_free(cross); device_free(recs);
+        device_free(act); device_free(recs);
     };
-    if (!counts || !prefix || !aux || !bitvol || (flat && !cpre) || (flat && !dup && !cross)) {
+    if (!counts || !prefix || !aux || !bitvol || (flat && !cpre) || (flat && a.vnormal && !act)) {
         cleanup();
         return KMC_ERR_OUT_OF_MEMORY;
     }
@@ -744,7 +750,7 @@ kmc_status run_pass(const kmc_volume* v, const void* dvals, const double* iso, u
     if (flat) {
         a.vpc = cpre;
         a.tpc = cpre + chunks;
-        a.cross = cross;
+        a.act = act;
     }
     uint64_t* partials = aux;
     uint64_t* totals = aux + nparts;
@@ -801,35 +807,23 @@ kmc_status run_pass(const kmc_volume* v, const void* dvals, const double* iso, u
         a.cap_vertices[l] = verts;
         a.cap_triangles[l] = nt;
     }
-    if (status == KMC_OK && flat) {
-        /* records: vertex keys, triangle records and cube indices, face normals */
-        a.voff[0] = a.toff[0] = 0;
-        for (uint32_t l = 0; l < nlev; ++l) {
-            a.voff[l + 1] = a.voff[l] + (dup ? 0 : tot[l * 2 + 0]);
-            a.toff[l + 1] = a.toff[l] + tot[l * 2 + 1];
-        }
-        const uint64_t nv = a.voff[nlev], nt = a.toff[nlev];
-        const size_t bytes = dup ? 0 : align_up(nv * 8, 256) + align_up(nt * 8, 256) + align_up(nt, 256) +
-                             (a.vnormal ? align_up(nt * 12, 256) + nv * 16 : 0);
-        if (bytes) {
-            recs = device_alloc(bytes);
+    if (status == KMC_OK && flat && a.vnormal) {
+        /* face normals and cell records */
+        a.toff[0] = 0;
+        for (uint32_t l = 0; l < nlev; ++l) a.toff[l + 1] = a.toff[l] + tot[l * 2 + 1];
+        const uint64_t nt = a.toff[nlev];
+        if (nt) {
+            recs = device_alloc(align_up(nt * 12, 256) + nt * 4);
             if (!recs) status = KMC_ERR_OUT_OF_MEMORY;
-        }
-        if (recs) {
-            uint8_t* p = (uint8_t*)recs;
-            a.vkey = (uint64_t*)p; p += align_up(nv * 8, 256);
-            a.trec = (uint64_t*)p; p += align_up(nt * 8, 256);
-            a.tci = p; p += align_up(nt, 256);
-            a.fn = a.vnormal ? (float*)p : nullptr;
-            if (a.vnormal) p += align_up(nt * 12, 256);
-            a.vslot = a.vnormal ? (uint32_t*)p : nullptr;
+            a.fn = (float*)recs;
+            a.crec = (uint32_t*)((uint8_t*)recs + align_up(nt * 12, 256));
         }
     }
     if (status == KMC_OK) {
         bool any = false;
         for (uint32_t l = 0; l < nlev; ++l) any = any || outs[l].n_vertices > 0;
         timer.mark(4);
-        if (any && (flat ? launch_flat_emit(v->type, a, st, timer.flat_marks()) : launch_emit(v->type, a, lds, st)) !=
+        if (any && (flat ? launch_chunk_emit(v->type, a, st, timer.flat_marks()) : launch_emit(v->type, a, lds, st)) !=
                        hipSuccess)
             status = KMC_ERR_DEVICE;
         timer.mark(5);

@@ -28,48 +28,29 @@ namespace kmc {
 
 /* Where one surface of a run landed (element offsets into the arenas); the
  * entry after the last surface holds the totals, the overflow flag (nv) and
- * the record bytes the flat emit needs (rb). */
+ * the record bytes the emit needs (rb). */
 struct SegOut {
     uint64_t nv, nt;          // vertices (node-shared) and triangles counted
     uint64_t oc, on, ok;      // offsets of coords (floats), normals (floats), connections (uint32)
     uint64_t rb;
 };
 
-/* Flat-emit records of a pass with shared vertices: vertex keys, triangle
- * records, cube indices, face normals and vertex slots (VertexNormal), each
- * 256-byte aligned; duplicated triangles are emitted without records. */
+/* Emit records of a pass: face normals and cell records (VertexNormal), each
+ * 256-byte aligned. */
 __host__ __device__ inline uint64_t align256(uint64_t x) { return (x + 255) & ~255ull; }
-__host__ __device__ inline uint64_t emit_record_bytes(const JobArgs& a, uint64_t nv, uint64_t nt)
+__host__ __device__ inline uint64_t emit_record_bytes(const JobArgs& a, uint64_t nt)
 {
-    if (a.dup) return 0;
-    const bool vn = a.vnormal != 0;
-    return align256(nv * 8) + align256(nt * 8) + align256(nt) + (vn ? align256(nt * 12) + align256(nv * 16) : 0);
+    return a.vnormal ? align256(nt * 12) + align256(nt * 4) : 0;
 }
 
 /* Point pass a's records at base (or at nothing when base is null) and set its
- * per-level item offsets from the level totals nv[l] / nt[l]; a level given
- * zero totals gets no records, and the compaction skips it (rec_levels). */
-__host__ __device__ inline void place_records(JobArgs& a, const uint64_t* nv, const uint64_t* nt, uint8_t* base)
+ * per-level offsets from the level totals nt[l]. */
+__host__ __device__ inline void place_records(JobArgs& a, const uint64_t* nt, uint8_t* base)
 {
-    a.voff[0] = a.toff[0] = 0;
-    a.rec_levels = 0;
-    for (uint32_t l = 0; l < a.nlev; ++l) {
-        a.voff[l + 1] = a.voff[l] + (base && !a.dup ? nv[l] : 0);
-        a.toff[l + 1] = a.toff[l] + (base ? nt[l] : 0);
-        if (base && ((!a.dup && nv[l]) || nt[l])) a.rec_levels |= 1u << l;
-    }
-    if (!base) {
-        a.vkey = nullptr; a.trec = nullptr; a.tci = nullptr; a.fn = nullptr; a.vslot = nullptr;
-        return;
-    }
-    const uint64_t V = a.voff[a.nlev], T = a.toff[a.nlev];
-    uint8_t* p = base;
-    a.vkey = (uint64_t*)p; p += align256(V * 8);
-    a.trec = (uint64_t*)p; p += align256(T * 8);
-    a.tci = p; p += align256(T);
-    a.fn = a.vnormal ? (float*)p : nullptr;
-    if (a.vnormal) p += align256(T * 12);
-    a.vslot = a.vnormal ? (uint32_t*)p : nullptr;
+    a.toff[0] = 0;
+    for (uint32_t l = 0; l < a.nlev; ++l) a.toff[l + 1] = a.toff[l] + (base ? nt[l] : 0);
+    a.fn = base && a.vnormal ? (float*)base : nullptr;
+    a.crec = base && a.vnormal ? (uint32_t*)(base + align256(a.toff[a.nlev] * 12)) : nullptr;
 }
 
 constexpr uint32_t kLayoutBlock = 256;
@@ -115,7 +96,7 @@ __global__ __launch_bounds__(kLayoutBlock) void k_batch_layout(JobArgs* jobs, co
                                                                float* arena_c, float* arena_n, uint32_t* arena_k,
                                                                uint64_t cap_c, uint64_t cap_n, uint64_t cap_k,
                                                                SegOut* out, uint32_t npass, uint8_t* arena_r,
-                                                               uint64_t cap_r, uint64_t* istart)
+                                                               uint64_t cap_r, uint32_t flat)
 {
     __shared__ uint32_t overflow;
     /* one sweep per kLayoutBlock * kLayoutPer surfaces, carrying the offsets */
@@ -160,57 +141,44 @@ __global__ __launch_bounds__(kLayoutBlock) void k_batch_layout(JobArgs* jobs, co
         carry[0] += tot[0]; carry[1] += tot[1]; carry[2] += tot[2];
         __syncthreads();
     }
-    /* flat-emit records of every pass (istart: null for the tile teams) */
-    uint64_t rcarry[3] = { 0, 0, 0 };
-    if (istart) {
+    /* emit records of every pass (not with the tile teams) */
+    uint64_t rcarry = 0;
+    if (flat) {
         for (uint32_t b0 = 0; b0 < npass; b0 += kLayoutBlock * kLayoutPer) {
             const uint32_t p0 = b0 + threadIdx.x * kLayoutPer;
-            uint64_t sz[kLayoutPer][3];
+            uint64_t sz[kLayoutPer];
             uint64_t v[3] = { 0, 0, 0 };
             for (uint32_t i = 0; i < kLayoutPer; ++i) {
-                sz[i][0] = sz[i][1] = sz[i][2] = 0;
-                if (p0 + i < npass) {
+                sz[i] = 0;
+                if (p0 + i < npass && jobs[p0 + i].vnormal) {
                     const JobArgs& a = jobs[p0 + i];
-                    for (uint32_t l = 0; l < a.nlev; ++l) {
-                        sz[i][1] += a.dup ? 0 : level_total(a, l, 0);
-                        sz[i][2] += level_total(a, l, 1);
-                    }
-                    sz[i][0] = emit_record_bytes(a, sz[i][1], sz[i][2]);
+                    uint64_t nt = 0;
+                    for (uint32_t l = 0; l < a.nlev; ++l) nt += level_total(a, l, 1);
+                    sz[i] = emit_record_bytes(a, nt);
                 }
-                v[0] += sz[i][0]; v[1] += sz[i][1]; v[2] += sz[i][2];
+                v[0] += sz[i];
             }
             uint64_t tot[3];
             block_scan3(v, tot);
             for (uint32_t i = 0; i < kLayoutPer; ++i) {
-                if (p0 + i < npass) {
-                    istart[p0 + i] = rcarry[1] + v[1];                 // vertex items
-                    istart[npass + 1 + p0 + i] = rcarry[2] + v[2];     // triangle items
-                    jobs[p0 + i].voff[0] = rcarry[0] + v[0];           // record byte offset (placed below)
-                }
-                v[0] += sz[i][0]; v[1] += sz[i][1]; v[2] += sz[i][2];
+                if (p0 + i < npass) jobs[p0 + i].toff[0] = rcarry + v[0];   // record byte offset (placed below)
+                v[0] += sz[i];
             }
-            rcarry[0] += tot[0]; rcarry[1] += tot[1]; rcarry[2] += tot[2];
+            rcarry += tot[0];
             __syncthreads();
         }
     }
     if (threadIdx.x == 0)
-        overflow = (carry[0] > cap_c || carry[1] > cap_n || carry[2] > cap_k || (istart && rcarry[0] > cap_r)) ? 1u : 0u;
+        overflow = (carry[0] > cap_c || carry[1] > cap_n || carry[2] > cap_k || rcarry > cap_r) ? 1u : 0u;
     __syncthreads();
     const bool fits = overflow == 0;
-    if (istart) {
+    if (flat) {
         for (uint32_t p = threadIdx.x; p < npass; p += kLayoutBlock) {
             JobArgs& a = jobs[p];
-            uint64_t nv[kMaxLevels], nt[kMaxLevels];
-            for (uint32_t l = 0; l < a.nlev; ++l) {
-                nv[l] = level_total(a, l, 0);
-                nt[l] = level_total(a, l, 1);
-            }
-            place_records(a, nv, nt, fits ? arena_r + a.voff[0] : nullptr);
-            if (!fits) istart[p] = istart[npass + 1 + p] = 0;
-        }
-        if (threadIdx.x == 0) {
-            istart[npass] = fits ? rcarry[1] : 0;
-            istart[2 * npass + 1] = fits ? rcarry[2] : 0;
+            if (!a.vnormal) continue;
+            uint64_t nt[kMaxLevels];
+            for (uint32_t l = 0; l < a.nlev; ++l) nt[l] = level_total(a, l, 1);
+            place_records(a, nt, fits ? arena_r + a.toff[0] : nullptr);
         }
     }
     for (uint32_t s = threadIdx.x; s < nseg; s += kLayoutBlock) {
@@ -232,7 +200,7 @@ __global__ __launch_bounds__(kLayoutBlock) void k_batch_layout(JobArgs* jobs, co
         t.oc = carry[0];
         t.on = carry[1];
         t.ok = carry[2];
-        t.rb = rcarry[0];
+        t.rb = rcarry;
         out[nseg] = t;
     }
 }
@@ -310,13 +278,11 @@ struct kmc_batch {
     uint64_t* bitvol_d;
     uint64_t bitvol_words;
     bool two_phase;                         // planned for batch_launch_front / batch_launch_emit
-    bool flat;                              // flat emit (else the tile teams)
-    bool flat_ok;                           // every pass's rows fit the flat records' 20-bit y / z
+    bool flat;                              // chunk-batch emit (else the tile teams)
+    bool flat_ok;                           // every pass's rows fit its 20-bit y / z
     uint32_t* cpre_d;                       // in-row chunk prefixes of the count pass (flat)
-    ChunkCross* cross_d;                    // chunk crossing records of the compaction (flat)
-    uint64_t* istart_d;                     // per-pass first vertex / triangle item (flat)
-    std::vector<uint64_t> istart_h;
-    uint8_t* arena_r;                       // flat-emit records
+    uint64_t* act_d;                        // active cells per chunk (flat, VertexNormal passes)
+    uint8_t* arena_r;                       // emit records
     uint64_t cap_r;
     SegOut* segout_d;
     SegOut* segout_h;                       // pinned
@@ -370,8 +336,7 @@ void destroy(kmc_batch* b)
     device_free(b->scan_aux_d);
     device_free(b->bitvol_d);
     device_free(b->cpre_d);
-    device_free(b->cross_d);
-    device_free(b->istart_d);
+    device_free(b->act_d);
     device_free(b->arena_r);
     device_free(b->segout_d);
     device_free(b->arena_c);
@@ -445,7 +410,7 @@ kmc_status plan_tiles(kmc_batch* b, uint32_t r_max, uint32_t queue_cap)
     for (Pass& p : b->passes) {
         p.a.vpc = b->flat ? b->cpre_d + p.bitvol_off : nullptr;
         p.a.tpc = b->flat ? b->cpre_d + b->bitvol_words + p.bitvol_off : nullptr;
-        p.a.cross = b->flat ? b->cross_d + p.bitvol_off : nullptr;
+        p.a.act = b->flat && p.a.vnormal ? b->act_d + p.bitvol_off : nullptr;
     }
     b->jobs_h.resize(b->passes.size());
     for (size_t i = 0; i < b->passes.size(); ++i) b->jobs_h[i] = b->passes[i].a;
@@ -489,32 +454,25 @@ hipError_t record_front(kmc_batch* b, hipStream_t st, bool copy_sizes)
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_batch_layout, dim3(1), dim3(kLayoutBlock), 0, st, b->jobs_d, b->seg_map_d, nseg, b->arena_c,
                        b->arena_n, b->arena_k, b->cap_c, b->cap_n, b->cap_k, b->segout_d, (uint32_t)b->passes.size(),
-                       b->arena_r, b->cap_r, b->flat ? b->istart_d : nullptr);
+                       b->arena_r, b->cap_r, b->flat ? 1u : 0u);
     e = hipGetLastError();
     if (e != hipSuccess || !copy_sizes) return e;
     return hipMemcpyAsync(b->segout_h, b->segout_d, (nseg + 1) * sizeof(SegOut), hipMemcpyDeviceToHost, st);
 }
 
-/* Launches of the emit.  host_sizes: the passes' record offsets are set on
- * the host (the serving form's two phases), so each pass runs as the plain
- * call's compaction and per-item kernels with its arguments in the launch; in
- * a captured graph they live on the device only. */
+/* Launches of the emit.  host_sizes: the passes' outputs are set on the host
+ * (the serving form's two phases), so each pass runs as the plain call's emit
+ * with its arguments in the launch; in a captured graph they live on the
+ * device only. */
 hipError_t record_emit(kmc_batch* b, hipStream_t st, bool host_sizes)
 {
     hipError_t e = hipSuccess;
     if (b->flat) {
-        const uint32_t np = (uint32_t)b->passes.size();
         for (const Group& g : b->groups) {
-            if (host_sizes) {
-                for (uint32_t i = g.p0; i < g.p1 && e == hipSuccess; ++i) e = launch_flat_emit(g.dtype, b->passes[i].a, st);
-            } else if (g.mode == 0) {
-                e = launch_dup_batch(g.dtype, b->jobs_d + g.p0, g.p1 - g.p0, g.emit_blocks, g.max_levels, st);
-            } else {
-                e = launch_compact_batch(b->jobs_d + g.p0, g.row_start_d, g.p1 - g.p0, g.rows, st);
-                if (e == hipSuccess)
-                    e = launch_flat_batch(g.dtype, g.mode, b->jobs_d + g.p0, b->istart_d + g.p0,
-                                          b->istart_d + np + 1 + g.p0, g.p1 - g.p0, st);
-            }
+            if (host_sizes)
+                for (uint32_t i = g.p0; i < g.p1 && e == hipSuccess; ++i) e = launch_chunk_emit(g.dtype, b->passes[i].a, st);
+            else
+                e = launch_chunk_emit_batch(g.dtype, g.mode, b->jobs_d + g.p0, g.p1 - g.p0, g.emit_blocks, g.max_levels, st);
             if (e != hipSuccess) return e;
         }
         return e;
@@ -758,15 +716,16 @@ kmc_status create_impl(const kmc_job* jobs, uint32_t n_jobs, uint32_t flags, hip
         b->counts_d = (uint32_t*)device_alloc(coff * 4);
         b->prefix_d = (uint64_t*)device_alloc(coff * 8);
         b->scan_aux_d = (uint64_t*)device_alloc((b->scan_parts + 1) * 8);
-        b->bitvol_d = (uint64_t*)device_alloc(boff * 8);
+        b->bitvol_d = (uint64_t*)device_alloc(boff * 8 + kBitSlack);
         b->flat_ok = true;
         for (const Pass& p : b->passes) b->flat_ok = b->flat_ok && flat_emit_fits(p.a.ny, p.a.nz);
         b->flat = b->flat_ok;
         if (b->flat_ok) {
             b->cpre_d = (uint32_t*)device_alloc(2 * boff * 4);
-            b->cross_d = (ChunkCross*)device_alloc(boff * sizeof(ChunkCross));
-            b->istart_d = (uint64_t*)device_alloc((2 * b->passes.size() + 2) * 8);
-            if (!b->cpre_d || !b->cross_d || !b->istart_d) {
+            bool vn = false;
+            for (const Pass& p : b->passes) vn = vn || p.a.vnormal;
+            if (vn) b->act_d = (uint64_t*)device_alloc(boff * 8 + kBitSlack);
+            if (!b->cpre_d || (vn && !b->act_d)) {
                 (void)hipGetLastError();
                 destroy(b);
                 return KMC_ERR_OUT_OF_MEMORY;
@@ -871,36 +830,21 @@ hipError_t batch_launch_emit(kmc_batch* b, hipStream_t st)
 {
     if (b->passes.empty()) return hipSuccess;
     if (b->flat) {
-        /* records of every pass from the sizes of the front phase */
+        /* records of every pass from the sizes of the front phase; only
+         * surfaces with outputs (admitted by the caller) get some */
         const uint32_t np = (uint32_t)b->passes.size();
         std::vector<uint64_t> off(np);
         uint64_t bytes = 0;
-        b->istart_h.assign(2 * np + 2, 0);
-        uint64_t vsum = 0, tsum = 0;
-        /* only surfaces with outputs (admitted by the caller) get records */
-        auto level_items = [&](const Pass& p, uint32_t l, uint64_t& nv, uint64_t& nt) {
-            const bool on = p.a.coords[l] != nullptr;
-            nv = on ? b->segout_h[p.seg0 + l].nv : 0;
-            nt = on ? b->segout_h[p.seg0 + l].nt : 0;
+        auto level_triangles = [&](const Pass& p, uint32_t l) {
+            return p.a.coords[l] != nullptr ? b->segout_h[p.seg0 + l].nt : 0;
         };
         for (uint32_t i = 0; i < np; ++i) {
             const Pass& p = b->passes[i];
-            uint64_t V = 0, T = 0;
-            for (uint32_t l = 0; l < p.nlev; ++l) {
-                uint64_t nv, nt;
-                level_items(p, l, nv, nt);
-                V += p.a.dup ? 0 : nv;
-                T += nt;
-            }
+            uint64_t T = 0;
+            for (uint32_t l = 0; l < p.nlev; ++l) T += level_triangles(p, l);
             off[i] = bytes;
-            bytes += emit_record_bytes(p.a, V, T);
-            b->istart_h[i] = vsum;
-            b->istart_h[np + 1 + i] = tsum;
-            vsum += V;
-            tsum += T;
+            bytes += emit_record_bytes(p.a, T);
         }
-        b->istart_h[np] = vsum;
-        b->istart_h[2 * np + 1] = tsum;
         if (bytes > b->cap_r) {
             device_free(b->arena_r);
             b->arena_r = (uint8_t*)device_alloc(bytes);
@@ -909,13 +853,11 @@ hipError_t batch_launch_emit(kmc_batch* b, hipStream_t st)
         }
         for (uint32_t i = 0; i < np; ++i) {
             Pass& p = b->passes[i];
-            uint64_t nv[kMaxLevels], nt[kMaxLevels];
-            for (uint32_t l = 0; l < p.nlev; ++l) level_items(p, l, nv[l], nt[l]);
-            place_records(p.a, nv, nt, b->arena_r + off[i]);
+            uint64_t nt[kMaxLevels];
+            for (uint32_t l = 0; l < p.nlev; ++l) nt[l] = level_triangles(p, l);
+            place_records(p.a, nt, b->arena_r ? b->arena_r + off[i] : nullptr);
         }
-        const hipError_t e = hipMemcpyAsync(b->istart_d, b->istart_h.data(), b->istart_h.size() * 8,
-                                            hipMemcpyHostToDevice, st);
-        if (e != hipSuccess) return e;
+        return record_emit(b, st, true);
     }
     b->jobs_h.resize(b->passes.size());
     for (size_t i = 0; i < b->passes.size(); ++i) b->jobs_h[i] = b->passes[i].a;

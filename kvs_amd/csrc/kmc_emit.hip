@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <type_traits>
+#include "kmc_chunks.h"
 #include "kmc_device.h"
 #include "kmc_internal.h"
 #include "kmc_job.h"
@@ -25,111 +26,6 @@
 namespace kmc {
 
 namespace {
-
-/* One level of a pass; the same on all lanes. */
-struct EmitLevel {
-    const uint64_t* bits;    // [nz][ny][NC] chunk masks
-    const uint32_t* vp;      // in-row chunk prefixes (chunk_prefix)
-    const uint32_t* tp;
-    const uint32_t* cv;      // row counts: crossing edges, triangles
-    const uint32_t* ct;
-    const uint64_t* pv;      // row prefixes
-    const uint64_t* pt;
-    uint64_t v0, t0;         // first prefix of each (outputs index from 0)
-};
-
-__device__ __forceinline__ EmitLevel emit_level(const JobArgs& a, uint32_t l)
-{
-    const uint64_t words = (uint64_t)l * (a.nrows * a.NC);
-    EmitLevel L;
-    L.bits = a.bitvol + words;
-    L.vp = a.vpc + words;
-    L.tp = a.tpc + words;
-    L.cv = a.counts + (uint64_t)(l * 2 + 0) * a.nrows;
-    L.ct = a.counts + (uint64_t)(l * 2 + 1) * a.nrows;
-    L.pv = a.prefix + (uint64_t)(l * 2 + 0) * a.nrows;
-    L.pt = a.prefix + (uint64_t)(l * 2 + 1) * a.nrows;
-    L.v0 = L.pv[0];
-    L.t0 = L.pt[0];
-    return L;
-}
-
-/* Calls batch(n) for every group of n <= N chunks of the level with a
- * crossing edge (V) or a triangle (!V), their entries, row | chunk << 40,
- * in q[0 .. n) (q: N + 64 entries).  A wave
- * takes units of a.erows rows x up to 64 chunks; the prefixes of kScan units
- * are in flight together, since the test of a unit is one dependent load.
- * Across a batch only the units' busy masks stay live (scalars). */
-constexpr uint32_t kScan = 4;
-
-template <bool V, uint32_t N, typename F>
-__device__ __forceinline__ void busy_chunks(const JobArgs& a, const EmitLevel& L, uint64_t* q, F&& batch)
-{
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint64_t wave = (uint64_t)blockIdx.x * kWaves + uniform(threadIdx.x >> 6), nwaves = (uint64_t)a.eblocks * kWaves;
-    const uint32_t sub = lane >> a.cshift;
-    const uint64_t step = nwaves * a.erows;
-    const bool packed = a.NC <= 64;        // vertices in the low, triangles in the high half of vpc
-    const uint32_t* pre = V || packed ? L.vp : L.tp;
-    const uint32_t* row_end = V ? L.cv : L.ct;
-    const uint32_t sh = V || !packed ? 0u : 16u, mask = packed ? 0xFFFFu : ~0u;
-    uint32_t qn = 0;
-    for (uint32_t c0 = 0; c0 < a.NC; c0 += 64) {
-        const uint32_t c = c0 + (lane & ((1u << a.cshift) - 1u));
-        const bool in = sub < a.erows && c < a.NC;
-        const bool row_last = c + 1 == a.NC;
-        for (uint64_t r0 = wave * a.erows; r0 < a.nrows; r0 += step * kScan) {
-            uint32_t p0[kScan], p1[kScan];
-#pragma unroll
-            for (uint32_t k = 0; k < kScan; ++k) {
-                const uint64_t r = r0 + k * step + sub;
-                p0[k] = p1[k] = 0u;
-                if (in && r < a.nrows) {
-                    const uint64_t w = r * a.NC + c;
-                    p0[k] = (pre[w] >> sh) & mask;
-                    p1[k] = row_last ? row_end[r] : (pre[w + 1] >> sh) & mask;
-                }
-            }
-            uint64_t busy[kScan];
-#pragma unroll
-            for (uint32_t k = 0; k < kScan; ++k) busy[k] = __ballot(p0[k] != p1[k]);
-#pragma unroll 1
-            for (uint32_t k = 0; k < kScan; ++k) {
-                uint64_t bm = busy[0];
-#pragma unroll
-                for (uint32_t j = 1; j < kScan; ++j) bm = k == j ? busy[j] : bm;
-                if ((bm >> lane) & 1ull) q[qn + lanes_below(bm)] = (r0 + k * step + sub) | (uint64_t)c << 40;
-                qn += (uint32_t)__popcll(bm);
-                const bool end = r0 + step * kScan >= a.nrows && k == kScan - 1;
-                while (qn >= N || (end && qn)) {
-                    wave_sync();
-                    const uint32_t n = qn < N ? qn : N;
-                    batch(n);
-                    wave_sync();
-                    /* the rest (at most 63) moves to the front */
-                    qn -= n;
-                    const uint64_t rest = q[N + lane];
-                    wave_sync();
-                    if (lane < qn) q[lane] = rest;
-                    wave_sync();
-                }
-            }
-        }
-    }
-}
-
-/* Row and slice of row index r. */
-__device__ __forceinline__ void row_yz(const JobArgs& a, uint64_t r, uint32_t& y, uint32_t& z)
-{
-    if (a.nrows <= 0xFFFFFFFFull) {
-        z = (uint32_t)r / a.ny;
-        y = (uint32_t)r - z * a.ny;
-    } else {
-        const uint64_t zz = r / a.ny;
-        z = (uint32_t)zz;
-        y = (uint32_t)(r - zz * a.ny);
-    }
-}
 
 /* The cases as the cells' lanes need them, indexed by swap_pairs(cube index)
  * (corner_pairs).  edges: the crossing edges (bit e: edge e).  tri: the
@@ -147,9 +43,8 @@ struct alignas(16) CaseLds {
     uint16_t edges[256];
 };
 
-/* The tables, evaluated at compile time (a workgroup only copies them).  M:
- * table orientation of the edges with duplicated vertices (:276-290 of
- * MarchingCubesTable.cpp), else low to high. */
+/* The tables, evaluated at compile time (a workgroup only copies them); the
+ * edges in their table orientation (MarchingCubesTable.cpp:276-290). */
 constexpr uint64_t kTableWords[256] = { KMC_TABLE_WORDS };
 
 constexpr uint32_t bits_below(uint32_t m, uint32_t e)
@@ -159,7 +54,7 @@ constexpr uint32_t bits_below(uint32_t m, uint32_t e)
     return n;
 }
 
-constexpr CaseLds make_cases(bool table_edges)
+constexpr CaseLds make_cases()
 {
     CaseLds t{};
     for (uint32_t i = 0; i < 256; ++i) {
@@ -179,14 +74,13 @@ constexpr CaseLds make_cases(bool table_edges)
         const uint32_t o = e < 8 ? (uint32_t)(0x4667755402233110ull >> (8 * e)) & 0xFFu
                                  : (0x62735140u >> (8 * (e - 8))) & 0xFFu;   // edge_ends
         const uint32_t p = o & 7u, q = o >> 4, axis = p ^ q;
-        const uint32_t first = table_edges ? p : p & q, second = table_edges ? q : p | q;
-        t.ends[e] = EdgeEnds{ (float)(first & 1u), (float)((first >> 1) & 1u), (float)(first >> 2),
-                              first << 6 | second << 19 | ((second & axis) ? 8u : 0u) | axis };
+        t.ends[e] = EdgeEnds{ (float)(p & 1u), (float)((p >> 1) & 1u), (float)(p >> 2),
+                              p << 6 | q << 19 | ((q & axis) ? 8u : 0u) | axis };
     }
     return t;
 }
 
-static __constant__ CaseLds d_cases_dup = make_cases(true);
+static __constant__ CaseLds d_cases_dup = make_cases();
 
 __device__ __forceinline__ void stage_cases(CaseLds& t, const CaseLds& from)
 {
@@ -195,17 +89,16 @@ __device__ __forceinline__ void stage_cases(CaseLds& t, const CaseLds& from)
     __syncthreads();
 }
 
-/* LDS of one wave of the triangle kernels: 9.6 kB with values of up to 32
+/* LDS of one wave of the duplicated triangles: 9.4 kB with values of up to 32
  * bits, so that four workgroups fit a CU's 160 KiB. */
-constexpr uint32_t kChunks = 32;         // chunks worked on at a time
-constexpr uint32_t kCellList = 320;      // active cells listed at once (a chunk has at most 64)
+constexpr uint32_t kDupCells = 320;      // active cells listed at once (a chunk has at most 64)
 constexpr uint32_t kVerts = 236;         // edge crossings of the up to 64 cells in work (a cell has at most 12)
 
 struct CellPos { float x, y, z; };         // exact: coordinates lie below 2^24
 
 template <typename T>
 struct CellLds {
-    uint64_t q[kChunks + 64];    // busy queue: at most kChunks - 1 left over and 64 new
+    uint32_t q[kChunks + 64];    // busy queue: at most kChunks - 1 left over and 64 new
     uint64_t m[4][kChunks];      // k0, k3, k4, k7 of each chunk (RowChunk)
     uint64_t out[kChunks];       // output id - batch rank of each chunk's triangles (its first array's address with
     uint64_t out2[kChunks];      // duplicated vertices, the second one's here)
@@ -214,7 +107,7 @@ struct CellLds {
     uint32_t next[kChunks];
     float p[kVerts][3];          // crossing points of the cells in work
     uint16_t el[kVerts];         // crossing: cell | edge << 6
-    uint16_t cells[kCellList];   // chunk | cell << 6
+    uint16_t cells[kDupCells];   // chunk | cell << 6
     union {
         T v[8 * 64];             // node values of the cells in work (corner offset bits x, y, z)
         uint32_t tl[320];        // then their triangles: three crossings | chunk << 24
@@ -323,13 +216,7 @@ __device__ __forceinline__ void fetch_cell(const JobArgs& a, const CaseLds& tab,
     o.pos = CellPos{ (float)x, (float)y, (float)z };
     o.chunk = q;
     o.first = k == 0 || (s.cells[k - 1] & 63u) != q;
-    RowChunk m;
-    m.k0 = s.m[0][q];
-    m.k3 = s.m[1][q];
-    m.k4 = s.m[2][q];
-    m.k7 = s.m[3][q];
-    m.next = s.next[q];
-    const uint32_t pi = corner_pairs(m, i);
+    const uint32_t pi = corner_pairs_at(s.m, s.next, q, i);
     o.tri = tab.tri[pi];
     o.edges = tab.edges[pi];
     o.nt = (uint32_t)(o.tri >> 60);
@@ -353,13 +240,10 @@ __device__ __forceinline__ void chunk_triangles(const JobArgs& a, const EmitLeve
     const uint32_t lane = threadIdx.x & 63u;
     uint64_t act = 0;
     if (lane < n) {
-        const uint64_t e = s.q[lane];
-        const uint64_t r = e & 0xFFFFFFFFFFull;
-        const uint32_t c = (uint32_t)(e >> 40);
-        uint32_t y, z;
-        row_yz(a, r, y, z);
-        RowChunk o;
-        row_chunk(a, L.bits, y, z, c, o);
+        uint64_t r;
+        uint32_t y, z, c;
+        chunk_place(a, s.q[lane], r, y, z, c);
+        const CellMasks o = load_cells(a, L, y, z, c);
         const uint64_t w = r * a.NC + c;
         act = o.act;
         s.m[0][lane] = o.k0;
@@ -376,17 +260,9 @@ __device__ __forceinline__ void chunk_triangles(const JobArgs& a, const EmitLeve
     uint32_t rank = 0;
     for (uint32_t start = 0; start < total;) {
         /* chunks whose cells fit the list */
-        const uint64_t fit = __ballot(excl >= start && incl - start <= kCellList && act != 0);
+        const uint64_t fit = __ballot(excl >= start && incl - start <= kDupCells && act != 0);
         const uint32_t stop = uniform((uint32_t)__builtin_amdgcn_readlane((int)incl, 63 - __builtin_clzll(fit)));
-        if ((fit >> lane) & 1ull) {
-            uint64_t m = act;
-            uint32_t p = excl - start;
-            while (m) {
-                const uint32_t i = (uint32_t)__ffsll((unsigned long long)m) - 1u;
-                m &= m - 1ull;
-                s.cells[p++] = (uint16_t)(lane | i << 6);
-            }
-        }
+        list_bits(act, excl, start, fit, total > 8 * n, s.cells);
         wave_sync();
         const uint32_t ncells = stop - start;
         CellItem<T> cur;
@@ -519,55 +395,699 @@ __global__ __launch_bounds__(kBlock) void k_dup_batch(const JobArgs* jobs)
     dup_level<T>(a, blockIdx.y, tab, s[threadIdx.x >> 6]);
 }
 
-template <typename T>
-hipError_t launch_dup_t(const JobArgs& a, hipStream_t st)
+/* ------------------------------------------------------------------------- */
+/* shared vertices: coordinates                                                */
+/* ------------------------------------------------------------------------- */
+
+/* Crossing edges of a wave's chunks, listed in output order (nodes in scan
+ * order, x, y, z edge of each), and produced one per lane. */
+constexpr uint32_t kPointList = 512;     // crossings listed at once (a chunk has at most 192)
+
+/* N: chunks worked on at a time. */
+template <uint32_t N>
+struct PointLds {
+    uint32_t q[N + 64];          // busy queue: at most N - 1 left over and 64 new
+    uint64_t key[N];             // 64 c | y << 20 | z << 40 of each chunk's first node
+    uint64_t out[N];             // output id - batch rank of each chunk's vertices
+    uint16_t el[kPointList];     // chunk | node << 6 | axis << 12
+};
+
+/* The vertices of the n queued chunks: emit(first, count, rank) for runs of
+ * listed ones, s.el[0 .. count); a vertex's id is s.out[chunk] + its rank.
+ * chunk(row, y, z, chunk of the row) is called on a lane of its own each. */
+template <uint32_t N, typename C, typename F>
+__device__ __forceinline__ void chunk_points(const JobArgs& a, const EmitLevel& L, PointLds<N>& s, uint32_t n, C&& chunk,
+                                             F&& emit)
 {
-    hipLaunchKernelGGL((k_dup<T>), dim3(a.eblocks, a.nlev), dim3(kBlock), 0, st, a);
+    const uint32_t lane = threadIdx.x & 63u;
+    uint64_t mx = 0, my = 0, mz = 0, base = 0;
+    if (lane < n) {
+        uint64_t r;
+        uint32_t y, z, c;
+        chunk_place(a, s.q[lane], r, y, z, c);
+        /* row_chunk's crossings alone: a neighbour row outside the volume is
+         * read as the row itself */
+        const uint64_t* row = L.bits + r * a.NC;
+        uint64_t b, b1;
+        load_words(row + c, b, b1);
+        const uint64_t u = (y + 1 < a.ny ? row + a.NC : row)[c];
+        const uint64_t nz = (z + 1 < a.nz ? row + (uint64_t)a.ny * a.NC : row)[c];
+        const uint64_t vn = valid_mask(c, a.nx);
+        mx = (b ^ (b >> 1 | b1 << 63)) & valid_mask(c, a.nx - 1);
+        my = (b ^ u) & vn;
+        mz = (b ^ nz) & vn;
+        base = (L.pv[r] - L.v0) + (a.NC <= 64 ? L.vp[r * a.NC + c] & 0xFFFFu : L.vp[r * a.NC + c]);
+        s.key[lane] = (uint64_t)(c * 64u) | (uint64_t)y << 20 | (uint64_t)z << 40;
+        chunk(r, y, z, c);
+    }
+    const uint32_t cnt = (uint32_t)(__popcll(mx) + __popcll(my) + __popcll(mz));
+    const uint32_t incl = wave_incl_scan(cnt);
+    const uint32_t excl = incl - cnt;
+    const uint32_t total = uniform((uint32_t)__builtin_amdgcn_readlane((int)incl, 63));
+    if (lane < n) s.out[lane] = base - (uint64_t)excl;
+    for (uint32_t start = 0; start < total;) {
+        const uint64_t fit = __ballot(excl >= start && incl - start <= kPointList && cnt != 0);
+        const uint32_t stop = uniform((uint32_t)__builtin_amdgcn_readlane((int)incl, 63 - __builtin_clzll(fit)));
+        if (total > 16 * n) {
+            /* dense: chunk after chunk, a node per lane (list_bits) */
+            for (uint64_t f = fit; f; f &= f - 1) {
+                const int q = __builtin_ctzll(f);
+                const uint64_t x = readlane64(mx, q), y = readlane64(my, q), z = readlane64(mz, q);
+                uint32_t p = (uint32_t)__builtin_amdgcn_readlane((int)excl, q) - start + lanes_below(x) + lanes_below(y) +
+                             lanes_below(z);
+                const uint32_t e = (uint32_t)q | lane << 6;
+                if (__builtin_amdgcn_inverse_ballot_w64(x)) s.el[p++] = (uint16_t)e;
+                if (__builtin_amdgcn_inverse_ballot_w64(y)) s.el[p++] = (uint16_t)(e | 1u << 12);
+                if (__builtin_amdgcn_inverse_ballot_w64(z)) s.el[p] = (uint16_t)(e | 2u << 12);
+            }
+        } else if ((fit >> lane) & 1ull) {
+            uint64_t m = mx | my | mz;
+            uint32_t p = excl - start;
+            while (m) {
+                const uint32_t i = (uint32_t)__ffsll((unsigned long long)m) - 1u;
+                m &= m - 1ull;
+                const uint32_t e = lane | i << 6;
+                if ((mx >> i) & 1ull) s.el[p++] = (uint16_t)e;
+                if ((my >> i) & 1ull) s.el[p++] = (uint16_t)(e | 1u << 12);
+                if ((mz >> i) & 1ull) s.el[p++] = (uint16_t)(e | 2u << 12);
+            }
+        }
+        wave_sync();
+        emit(stop - start, start);
+        wave_sync();
+        start = stop;
+    }
+}
+
+/* A vertex in flight. */
+template <typename T>
+struct PointItem {
+    uint32_t x, y, z, axis;
+    uint64_t id;
+    T va, vb;
+};
+
+template <typename T>
+__device__ __forceinline__ void fetch_point(const JobArgs& a, const PointLds<64>& s, uint32_t j, uint32_t rank, PointItem<T>& o)
+{
+    const uint32_t e = s.el[j], q = e & 63u;
+    const uint64_t key = s.key[q];
+    o.x = (uint32_t)(key & 0xFFFFFu) + ((e >> 6) & 63u);
+    o.y = (uint32_t)((key >> 20) & 0xFFFFFu);
+    o.z = (uint32_t)(key >> 40);
+    o.axis = e >> 12;
+    o.id = s.out[q] + (rank + j);
+    const uint64_t line = a.nx, slice = (uint64_t)a.nx * a.ny;
+    const T* src = (const T*)a.values + (o.x + o.y * line + o.z * slice);
+    o.va = src[0];
+    o.vb = src[o.axis == 0 ? 1ull : (o.axis == 1 ? line : slice)];
+}
+
+/* Its coordinates, interpolated low -> high (calculate_isopoints, :365-437). */
+template <typename T>
+__device__ __forceinline__ void store_point(const JobArgs& a, double iso, float* coords, const PointItem<T>& o)
+{
+    constexpr bool kFloat = sizeof(T) <= 2 || std::is_same<T, float>::value;
+    const EdgeEnds e{ 0.0f, 0.0f, 0.0f, 8u | 1u << o.axis };
+    const CellPos c{ (float)o.x, (float)o.y, (float)o.z };
+    float p[3];
+    if (kFloat && a.fclamp)
+        crossing_point<T, kFloat>(a, iso, o.va, o.vb, e, c, p);
+    else
+        crossing_point<T, false>(a, iso, o.va, o.vb, e, c, p);
+    float* co = coords + 3 * o.id;
+    co[0] = p[0];
+    co[1] = p[1];
+    co[2] = p[2];
+}
+
+template <typename T>
+__device__ __forceinline__ void points_level(const JobArgs& a, uint32_t l, PointLds<64>& s)
+{
+    if (!a.cap_vertices[l]) return;        // a level without outputs
+    const uint32_t lane = threadIdx.x & 63u;
+    const EmitLevel L = emit_level(a, l);
+    const double iso = a.iso[l];
+    float* coords = a.coords[l];
+    busy_chunks<true, 64>(a, L, s.q, [&](uint32_t n) {
+        chunk_points(a, L, s, n, [](uint64_t, uint32_t, uint32_t, uint32_t) {}, [&](uint32_t cnt, uint32_t rank) {
+            /* two vertices a lane, their values in flight together; lanes
+             * past the end fetch the last one and store nothing */
+            for (uint32_t j = lane; j < cnt + lane; j += 128) {
+                PointItem<T> p0, p1;
+                fetch_point<T>(a, s, j < cnt ? j : cnt - 1, rank, p0);
+                fetch_point<T>(a, s, j + 64 < cnt ? j + 64 : cnt - 1, rank, p1);
+                if (j < cnt) store_point<T>(a, iso, coords, p0);
+                if (j + 64 < cnt) store_point<T>(a, iso, coords, p1);
+            }
+        });
+    });
+}
+
+template <typename T>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) void k_points(JobArgs a)
+{
+    __shared__ PointLds<64> s[kWaves];
+    points_level<T>(a, blockIdx.y, s[threadIdx.x >> 6]);
+}
+
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_points_batch(const JobArgs* jobs)
+{
+    __shared__ PointLds<64> s[kWaves];
+    const JobArgs& a = jobs[blockIdx.z];
+    if (blockIdx.y >= a.nlev || blockIdx.x >= a.eblocks) return;
+    points_level<T>(a, blockIdx.y, s[threadIdx.x >> 6]);
+}
+
+/* ------------------------------------------------------------------------- */
+/* shared vertices: triangles                                                  */
+/* ------------------------------------------------------------------------- */
+
+/* Crossing edges of one chunk of a node row: the id of its first vertex and
+ * the x / y / z edge masks of its nodes. */
+struct RowCross {
+    uint64_t x, y, z;
+    uint32_t base;           // vertex ids are 32-bit, as the connections are
+    uint32_t next;           // bits 0, 1: the x and y edge of the next chunk's first node
+};
+
+struct FaceCases {
+    uint64_t tri[256];       // by pair index: corners in output order (edges), count in the top nibble
+    uint16_t edge[12];       // owner row (dy | dz << 1) << 4 | dx << 3 | axis
+    uint16_t pad[4];
+};
+
+constexpr FaceCases make_face_cases()
+{
+    FaceCases t{};
+    for (uint32_t i = 0; i < 256; ++i) {
+        const uint64_t w = kTableWords[(i & 0x33u) | ((i & 0x44u) << 1) | ((i & 0x88u) >> 1)];
+        uint64_t o = w & 0xFull << 60;
+        for (uint32_t k = 0; k < 3u * (uint32_t)(w >> 60); ++k) {
+            const uint32_t c = k % 3, from = c == 1 ? k + 1 : c == 2 ? k - 1 : k;
+            o |= ((w >> (4 * from)) & 0xFull) << (4 * k);
+        }
+        t.tri[i] = o;
+    }
+    constexpr uint64_t kOwner =
+        (0x00ull << 0) | (0x09ull << 5) | (0x02ull << 10) | (0x08ull << 15) | (0x04ull << 20) | (0x0Dull << 25) |
+        (0x06ull << 30) | (0x0Cull << 35) | (0x10ull << 40) | (0x11ull << 45) | (0x13ull << 50) | (0x12ull << 55);
+    for (uint32_t e = 0; e < 12; ++e) {   // edge_owner: dx | dy << 1 | dz << 2 | axis << 3
+        const uint32_t o = (uint32_t)(kOwner >> (5 * e)) & 31u;
+        t.edge[e] = (uint16_t)((o >> 1 & 3u) << 4 | (o & 1u) << 3 | o >> 3);
+    }
+    return t;
+}
+
+static __constant__ FaceCases d_face_cases = make_face_cases();
+
+/* Node rows (y, z), (y + 1, z), (y, z + 1), (y + 1, z + 1) of a chunk's cells;
+ * 144 bytes, so that lanes reading one row of different chunks spread over the
+ * LDS banks. */
+struct ChunkRows {
+    RowCross r[4];
+    uint32_t pad[4];
+};
+
+struct FaceLds {
+    ListLds l;
+    uint64_t k0[kChunks];        // mask of each chunk's first node row
+    uint64_t act[kChunks];       // active cells (VertexNormal)
+    uint32_t tri0[kChunks];      // id of each chunk's first triangle (32-bit, VertexNormal)
+    ChunkRows row[kChunks];
+};
+
+/* corner_pairs of cell i of a chunk: the first corner's bit and the crossings
+ * of the edges that lead from it to the others. */
+__device__ __forceinline__ uint32_t pair_of(const FaceLds& s, uint32_t q, uint32_t i)
+{
+    const RowCross* r = s.row[q].r;
+    const uint32_t c0 = (uint32_t)(s.k0[q] >> i) & 1u;
+    const uint32_t c1 = c0 ^ ((uint32_t)(r[0].x >> i) & 1u), c3 = c0 ^ ((uint32_t)(r[0].y >> i) & 1u);
+    const uint32_t c4 = c0 ^ ((uint32_t)(r[0].z >> i) & 1u), c2 = c3 ^ ((uint32_t)(r[1].x >> i) & 1u);
+    const uint32_t c7 = c3 ^ ((uint32_t)(r[1].z >> i) & 1u), c5 = c4 ^ ((uint32_t)(r[2].x >> i) & 1u);
+    const uint32_t c6 = c7 ^ ((uint32_t)(r[3].x >> i) & 1u);
+    return c0 | c1 << 1 | c3 << 2 | c2 << 3 | c4 << 4 | c5 << 5 | c7 << 6 | c6 << 7;
+}
+
+/* The cells of cell row (y, z - 1), chunk c, and the crossing edges of its four
+ * node rows (all in the volume): eight mask rows, five of them with their next
+ * word. */
+__device__ __forceinline__ CellMasks load_row_cross(const JobArgs& a, const EmitLevel& L, uint32_t y, uint32_t z,
+                                                    uint32_t c, ChunkRows& o)
+{
+    const uint64_t sw = (uint64_t)a.ny * a.NC, r0 = (uint64_t)(z - 1) * a.ny + y, r2 = r0 + a.ny;
+    const uint64_t* p = L.bits + r0 * a.NC + c;
+    const uint64_t* q = p + sw;
+    const uint64_t* u = z + 1 < a.nz ? q + sw : q;      // a row past the volume is read as the one before it
+    const uint32_t y2 = y + 2 < a.ny ? 2 * a.NC : a.NC;
+    uint64_t m00, n00, m10, n10, m20, n20, m01, n01, m11, n11;
+    load_words(p, m00, n00);
+    load_words(p + a.NC, m10, n10);
+    load_words(p + y2, m20, n20);
+    load_words(q, m01, n01);
+    load_words(q + a.NC, m11, n11);
+    const uint64_t m21 = q[y2], m02 = u[0], m12 = u[a.NC];
+    uint64_t v0, v1, v2, v3;
+    load_words(L.pv + r0, v0, v1);
+    load_words(L.pv + r2, v2, v3);
+    const uint32_t* vp = L.vp + r0 * a.NC + c;
+    const uint32_t mask = a.NC <= 64 ? 0xFFFFu : ~0u;
+    const uint32_t e0 = vp[0] & mask, e1 = vp[a.NC] & mask, e2 = vp[sw] & mask, e3 = vp[sw + a.NC] & mask;
+    const uint64_t vx = valid_mask(c, a.nx - 1), vn = valid_mask(c, a.nx);
+    auto cross = [&](RowCross& k, uint64_t b, uint64_t b1, uint64_t up, uint64_t nz, uint64_t pre, uint32_t e,
+                     uint32_t next) {
+        k.x = (b ^ (b >> 1 | b1 << 63)) & vx;
+        k.y = (b ^ up) & vn;
+        k.z = (b ^ nz) & vn;
+        k.base = (uint32_t)(pre - L.v0) + e;
+        k.next = next;
+    };
+    /* x and y edge of the first node of the next chunk (read for a cell 63 only,
+     * whose node x + 1 it is; its x edge needs a node after it) */
+    const uint64_t has = 64ull * (c + 1) + 1 < a.nx ? 1ull : 0ull;
+    auto next_bits = [&](uint64_t b1, uint64_t up1) {
+        return (uint32_t)((b1 ^ b1 >> 1) & has) | (uint32_t)((b1 ^ up1) & 1ull) << 1;
+    };
+    cross(o.r[0], m00, n00, m10, m01, v0, e0, next_bits(n00, n10));
+    cross(o.r[1], m10, n10, m20, m11, v1, e1, next_bits(n10, n20));
+    cross(o.r[2], m01, n01, m11, m02, v2, e2, next_bits(n01, n11));
+    cross(o.r[3], m11, n11, m21, m12, v3, e3, 0u);
+    return cell_masks(a, c, m00, n00, m10, n10, m01, n01, m11, n11);
+}
+
+/* Vertex id on the edge along `axis` of node i (0 .. 64) of a row's chunk: its
+ * first vertex + the crossing edges of the nodes before i and of node i's
+ * lower axes. */
+__device__ __forceinline__ uint32_t cross_rank(const RowCross& o, uint32_t i, uint32_t axis)
+{
+    const uint64_t lo = i ? ~0ull >> (64u - i) : 0ull;
+    const uint32_t r = o.base + (uint32_t)(__popcll(o.x & lo) + __popcll(o.y & lo) + __popcll(o.z & lo));
+    const uint32_t bx = i < 64u ? (uint32_t)(o.x >> i) & 1u : o.next & 1u;
+    const uint32_t by = i < 64u ? (uint32_t)(o.y >> i) & 1u : o.next >> 1;
+    return r + (axis >= 1 ? bx : 0u) + (axis >= 2 ? by : 0u);
+}
+
+/* A triangle in flight: its vertices and their coordinates. */
+struct FaceItem {
+    uint64_t id;
+    uint32_t v[3];
+    float p[3][3];
+};
+
+__device__ __forceinline__ void fetch_face(const FaceCases& tab, const FaceLds& s, const float* coords,
+                                           uint32_t cell, uint32_t t, uint32_t rank, FaceItem& o)
+{
+    const uint32_t q = cell & 63u, i = (cell >> 6) & 63u;
+    o.id = s.l.out[q] + rank;
+    const uint32_t w = (uint32_t)(tab.tri[cell >> 12] >> (12 * t));
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const uint32_t d = tab.edge[(w >> (4 * j)) & 0xFu];
+        o.v[j] = cross_rank(s.row[q].r[d >> 4], i + ((d >> 3) & 1u), d & 7u);
+    }
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const float* c = coords + 3 * (uint64_t)o.v[j];
+        o.p[j][0] = c[0];
+        o.p[j][1] = c[1];
+        o.p[j][2] = c[2];
+    }
+}
+
+/* Every triangle of shared vertices: its connectivity (connect_isopoints,
+ * :439-521) and the face normal of its vertices' coordinates -- the
+ * PolygonNormal output (calculate_normals_on_polygon, :531-559) or, with
+ * VertexNormal, kept in a.fn for the per-vertex sums, which find it through
+ * the chunk's active cells (a.act) and their first triangles and cases
+ * (a.crec). */
+template <int M>
+__device__ __forceinline__ void faces_level(const JobArgs& a, uint32_t l, const FaceCases& tab, FaceLds& s)
+{
+    if (!a.cap_triangles[l]) return;       // a level without outputs
+    const uint32_t lane = threadIdx.x & 63u;
+    const EmitLevel L = emit_level(a, l);
+    const float* coords = a.coords[l];
+    uint32_t* conn = a.conn[l];
+    float* normals = M == kModeVertex ? a.fn + 3 * a.toff[l] : a.normals[l];
+    uint64_t* act_l = M == kModeVertex ? a.act + (uint64_t)l * (a.nrows * a.NC) : nullptr;
+    uint32_t* crec = M == kModeVertex ? a.crec + a.toff[l] : nullptr;
+    busy_chunks<false, kChunks>(a, L, s.l.q, [&](uint32_t n) {
+        list_triangles(a, L, tab.tri, s.l, n, [&](uint64_t r, uint32_t y, uint32_t z, uint32_t c, uint64_t base) {
+            const CellMasks o = load_row_cross(a, L, y, z, c, s.row[lane]);
+            s.k0[lane] = o.k0;
+            if constexpr (M == kModeVertex) {
+                act_l[r * a.NC + c] = o.act;
+                s.act[lane] = o.act;
+                s.tri0[lane] = (uint32_t)base;
+            }
+            return o.act;
+        }, [&](uint32_t q, uint32_t i) { return pair_of(s, q, i); }, [&](uint32_t q, uint32_t i, uint32_t pi, uint32_t rank) {
+            /* first triangle relative to the chunk's first, and the case */
+            if constexpr (M == kModeVertex) {
+                const uint32_t t0 = s.tri0[q], ord = (uint32_t)__popcll(s.act[q] & ((1ull << i) - 1ull));
+                crec[t0 + ord] = ((uint32_t)s.l.out[q] + rank - t0) | pi << 16;
+            }
+        }, [&](uint32_t cnt, uint32_t rank) {
+            /* (two triangles a lane, their loads in flight together, are
+             * slower: 349 us to 317 on the 512^3 CT volume) */
+            for (uint32_t j = lane; j < cnt; j += 64) {
+                const uint32_t e = s.l.tl[j];
+                FaceItem o;
+                fetch_face(tab, s, coords, s.l.cell[e & 63u], e >> 6, rank + j, o);
+                uint32_t* k = conn + 3 * o.id;
+                k[0] = o.v[0];
+                k[1] = o.v[1];
+                k[2] = o.v[2];
+                float nn[3];
+                face_normal(o.p[0], o.p[1], o.p[2], nn);
+                float* no = normals + 3 * o.id;
+                no[0] = nn[0];
+                no[1] = nn[1];
+                no[2] = nn[2];
+            }
+        });
+    });
+}
+
+__device__ __forceinline__ void stage_face_cases(FaceCases& t)
+{
+    static_assert(sizeof(FaceCases) % 16 == 0, "copied in 16-byte words");
+    for (uint32_t i = threadIdx.x; i < sizeof(FaceCases) / 16; i += kBlock) ((uint4*)&t)[i] = ((const uint4*)&d_face_cases)[i];
+    __syncthreads();
+}
+
+template <int M>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_faces(JobArgs a)
+{
+    __shared__ __attribute__((aligned(16))) FaceCases tab;
+    __shared__ FaceLds s[kWaves];
+    stage_face_cases(tab);
+    faces_level<M>(a, blockIdx.y, tab, s[threadIdx.x >> 6]);
+}
+
+template <int M>
+__global__ __launch_bounds__(kBlock) void k_faces_batch(const JobArgs* jobs)
+{
+    __shared__ __attribute__((aligned(16))) FaceCases tab;
+    __shared__ FaceLds s[kWaves];
+    const JobArgs& a = jobs[blockIdx.z];
+    if (blockIdx.y >= a.nlev || blockIdx.x >= a.eblocks) return;
+    stage_face_cases(tab);
+    faces_level<M>(a, blockIdx.y, tab, s[threadIdx.x >> 6]);
+}
+
+/* ------------------------------------------------------------------------- */
+/* shared vertices: vertex normals                                             */
+/* ------------------------------------------------------------------------- */
+
+/* Triangles (table order, a bit each) of a case that use an edge. */
+struct UseCases { uint8_t use[256][12]; };
+
+constexpr UseCases make_use_cases()
+{
+    UseCases t{};
+    for (uint32_t i = 0; i < 256; ++i) {
+        const uint64_t w = kTableWords[(i & 0x33u) | ((i & 0x44u) << 1) | ((i & 0x88u) >> 1)];
+        for (uint32_t k = 0; k < 3u * (uint32_t)(w >> 60); ++k) t.use[i][(w >> (4 * k)) & 0xFu] |= (uint8_t)(1u << (k / 3));
+    }
+    return t;
+}
+
+static __constant__ UseCases d_use_cases = make_use_cases();
+
+/* A cell row around a chunk of nodes: the active cells of the chunk, its first
+ * triangle, and that of the chunk before it, whose cell 63 is the x - 1 cell
+ * of node 0. */
+struct RowCells {
+    uint64_t act;
+    uint32_t tri0, prev_tri0;
+};
+
+/* The cell rows (y - 1, z - 1), (y, z - 1), (y - 1, z), (y, z) of a chunk; 72
+ * bytes, so that lanes reading one row of different chunks spread over the LDS
+ * banks.  info: 8 bits a row, the active cells of the chunk before it without
+ * its cell 63, and bit 7 set when the row lies in the volume. */
+struct ChunkCells {
+    RowCells r[4];
+    uint32_t info, pad;
+};
+
+constexpr uint32_t kNormalChunks = 48;
+
+struct NormalLds {
+    PointLds<kNormalChunks> p;
+    ChunkCells row[kNormalChunks];
+};
+
+/* VertexNormal: the float sum, in triangle order, of the face normals of the
+ * triangles that use the vertex (calculate_normals_on_vertex, :569-605) -- the
+ * four cells around its edge in cell scan order and each cell's triangles in
+ * table order.  A cell's record (a.crec) gives its case and first triangle;
+ * the face normals of the first two triangles of every cell are loaded
+ * together (most cells have one or two), further ones after.  A slot without
+ * a triangle adds +0, which changes no partial sum: the sum starts at +0 and a
+ * float sum is -0 only when both terms are. */
+struct NormalItem {
+    uint32_t around, rec[4], t0[4], m[4];
+    bool in[4];
+    uint64_t id;
+    float f[4][2][3];
+};
+
+/* The vertex's cells and their records (loads issued). */
+__device__ __forceinline__ void fetch_cells(const JobArgs& a, const NormalLds& s, const uint32_t* crec, uint32_t j,
+                                            uint32_t rank, NormalItem& o)
+{
+    const uint32_t e = s.p.el[j], q = e & 63u, i = (e >> 6) & 63u, axis = e >> 12;
+    const uint32_t c64 = (uint32_t)(s.p.key[q] & 0xFFFFFu);
+    o.around = around_nibbles(axis);
+    o.id = s.p.out[q] + (rank + j);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        int dx, dy, dz;
+        around_cell(axis, k, 0, 0, 0, dx, dy, dz);
+        const uint32_t row = (uint32_t)((dy + 1) | (dz + 1) << 1);
+        const RowCells& r = s.row[q].r[row];
+        const uint32_t info = s.row[q].info >> (8 * row);
+        const int ci = (int)i + dx;
+        o.in[k] = (info & 128u) && (int)c64 + ci >= 0 && c64 + (uint32_t)(ci + 1) < a.nx;
+        const uint64_t below = (1ull << (ci & 63)) - 1ull;
+        o.t0[k] = ci >= 0 ? r.tri0 : r.prev_tri0;
+        const uint32_t at = o.t0[k] + (ci >= 0 ? (uint32_t)__popcll(r.act & below) : info & 127u);
+        o.rec[k] = crec[o.in[k] ? at : 0u];
+    }
+}
+
+/* The first two face normals of every cell (loads issued). */
+__device__ __forceinline__ void fetch_faces(const UseCases& use, const float* fn, NormalItem& o)
+{
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        o.m[k] = o.in[k] ? (uint32_t)use.use[(o.rec[k] >> 16) & 255u][(o.around >> (4 * k)) & 0xFu] : 0u;
+        o.t0[k] += o.rec[k] & 0xFFFFu;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            o.f[k][u][0] = o.f[k][u][1] = o.f[k][u][2] = 0.0f;
+            if (o.m[k]) {
+                const uint32_t t = (uint32_t)__ffs(o.m[k]) - 1u;
+                o.m[k] &= o.m[k] - 1u;
+                const float* p = fn + 3 * (uint64_t)(o.t0[k] + t);
+                o.f[k][u][0] = p[0];
+                o.f[k][u][1] = p[1];
+                o.f[k][u][2] = p[2];
+            }
+        }
+    }
+}
+
+__device__ __forceinline__ void store_normal(const float* fn, NormalItem& o, float* normals)
+{
+    /* the starting +0 comes from an opaque move, so that the compiler does not
+     * fold the first addition into the first load's branch (which would wait
+     * for that load alone) */
+    float zero;
+    asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+    float n[3] = { zero, zero, zero };
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            n[0] = n[0] + o.f[k][u][0];
+            n[1] = n[1] + o.f[k][u][1];
+            n[2] = n[2] + o.f[k][u][2];
+        }
+        while (o.m[k]) {   // further triangles of the cell that use the edge (rare)
+            const uint32_t t = (uint32_t)__ffs(o.m[k]) - 1u;
+            o.m[k] &= o.m[k] - 1u;
+            const float* p = fn + 3 * (uint64_t)(o.t0[k] + t);
+            n[0] = n[0] + p[0];
+            n[1] = n[1] + p[1];
+            n[2] = n[2] + p[2];
+        }
+    }
+    float* no = normals + 3 * o.id;
+    no[0] = n[0];
+    no[1] = n[1];
+    no[2] = n[2];
+}
+
+__device__ __forceinline__ void normals_level(const JobArgs& a, uint32_t l, const UseCases& use, NormalLds& s)
+{
+    if (!a.cap_vertices[l]) return;        // a level without outputs
+    const uint32_t lane = threadIdx.x & 63u;
+    const EmitLevel L = emit_level(a, l);
+    float* normals = a.normals[l];
+    const bool triangles = a.cap_triangles[l] != 0;   // without one no cell of the volume is active
+    const float* fn = a.fn + 3 * a.toff[l];
+    const uint32_t* crec = triangles ? a.crec + a.toff[l] : (const uint32_t*)L.bits;   // read, not used, without one
+    const uint64_t* act_l = a.act + (uint64_t)l * (a.nrows * a.NC);
+    const uint32_t* tri_pre = a.NC <= 64 ? L.vp : L.tp;   // chunk_prefix: triangles in the high half of vp
+    const uint32_t sh = a.NC <= 64 ? 16u : 0u;
+    busy_chunks<true, kNormalChunks>(a, L, s.p.q, [&](uint32_t n) {
+        chunk_points(a, L, s.p, n, [&](uint64_t r, uint32_t y, uint32_t z, uint32_t c) {
+/* cell row (cy, cz) is kept at node row (cy, cz + 1): node rows r -
+             * 1, r and the same of the next slice; the words of this chunk and
+             * the one before it in one load each (node row r >= 1 wherever a
+             * row below or a chunk before is used) */
+            const bool y0 = triangles && y >= 1, y1 = triangles && y + 1 < a.ny, z0 = z >= 1, z1 = z + 1 < a.nz;
+            uint32_t info = 0;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const bool in = (k & 1 ? y1 : y0) && (k & 2 ? z1 : z0);
+                const uint64_t cr = in ? r - (k & 1 ? 0 : 1) + (k & 2 ? a.ny : 0) : r;
+                const uint64_t w = cr * a.NC + c, w1 = w ? w - 1 : 0;
+                const uint32_t base = (uint32_t)(L.pt[cr] - L.t0);
+                uint64_t act1, act;
+                load_words(act_l + w1, act1, act);
+                uint32_t e1, e;
+                load_pair(tri_pre + w1, e1, e);
+                e1 = base + (e1 >> sh);
+                e = base + (e >> sh);
+                if (w == 0) { act = act1; e = e1; }
+                RowCells o;
+                o.act = act;
+                o.tri0 = e;
+                o.prev_tri0 = e1;
+                s.row[lane].r[k] = o;
+                info |= ((uint32_t)__popcll(act1 & ~(1ull << 63)) | (in ? 128u : 0u)) << (8 * k);
+            }
+            s.row[lane].info = info;
+        }, [&](uint32_t cnt, uint32_t rank) {
+            for (uint32_t j = lane; j < cnt; j += 64) {
+                NormalItem o;
+                fetch_cells(a, s, crec, j, rank, o);
+                fetch_faces(use, fn, o);
+                store_normal(fn, o, normals);
+            }
+        });
+    });
+}
+
+__device__ __forceinline__ void stage_use_cases(UseCases& t)
+{
+    static_assert(sizeof(UseCases) % 16 == 0, "copied in 16-byte words");
+    for (uint32_t i = threadIdx.x; i < sizeof(UseCases) / 16; i += kBlock) ((uint4*)&t)[i] = ((const uint4*)&d_use_cases)[i];
+    __syncthreads();
+}
+
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_normals(JobArgs a)
+{
+    __shared__ __attribute__((aligned(16))) UseCases use;
+    __shared__ NormalLds s[kWaves];
+    stage_use_cases(use);
+    normals_level(a, blockIdx.y, use, s[threadIdx.x >> 6]);
+}
+
+__global__ __launch_bounds__(kBlock) void k_normals_batch(const JobArgs* jobs)
+{
+    __shared__ __attribute__((aligned(16))) UseCases use;
+    __shared__ NormalLds s[kWaves];
+    const JobArgs& a = jobs[blockIdx.z];
+    if (blockIdx.y >= a.nlev || blockIdx.x >= a.eblocks) return;
+    stage_use_cases(use);
+    normals_level(a, blockIdx.y, use, s[threadIdx.x >> 6]);
+}
+
+/* Workgroups of each kernel that a CU holds: by LDS k_dup 4 and k_faces 5, by
+ * registers k_points 7 and k_normals 5 or more. */
+constexpr uint32_t kDupBlocks = 4, kPointBlocks = 7, kFaceBlocks = 5, kNormalBlocks = 5;
+
+template <typename T>
+hipError_t launch_chunk_emit_t(JobArgs a, hipStream_t st, hipEvent_t* marks)
+{
+    const dim3 b(kBlock);
+    uint64_t nv = 0, nt = 0;
+    for (uint32_t l = 0; l < a.nlev; ++l) { nv += a.cap_vertices[l]; nt += a.cap_triangles[l]; }
+    /* each kernel's waves by the workgroups of it that a CU holds */
+    auto grid = [&](uint32_t per_cu, uint64_t items) {
+        plan_emit(a, emit_steps(a), per_cu, items);
+        return dim3(a.eblocks, a.nlev);
+    };
+    if (!a.dup) hipLaunchKernelGGL((k_points<T>), grid(kPointBlocks, nv), b, 0, st, a);
+    if (marks) (void)hipEventRecord(marks[1], st);
+    switch (emit_mode(a)) {
+    case kModeDup: hipLaunchKernelGGL((k_dup<T>), grid(kDupBlocks, nt), b, 0, st, a); break;
+    case kModePolygon: hipLaunchKernelGGL((k_faces<kModePolygon>), grid(kFaceBlocks, nt), b, 0, st, a); break;
+    default: hipLaunchKernelGGL((k_faces<kModeVertex>), grid(kFaceBlocks, nt), b, 0, st, a); break;
+    }
+    if (marks) (void)hipEventRecord(marks[2], st);
+    if (a.vnormal) hipLaunchKernelGGL(k_normals, grid(kNormalBlocks, nv), b, 0, st, a);
     return hipGetLastError();
 }
 
 template <typename T>
-hipError_t launch_dup_batch_t(const JobArgs* jobs, uint32_t njobs, uint32_t blocks, uint32_t levels, hipStream_t st)
+hipError_t launch_chunk_emit_batch_t(int mode, const JobArgs* jobs, uint32_t njobs, uint32_t blocks, uint32_t levels,
+                                     hipStream_t st)
 {
     constexpr uint32_t kMaxJobs = 32768;   // of one grid's z
-    for (uint32_t j = 0; j < njobs; j += kMaxJobs)
-        hipLaunchKernelGGL((k_dup_batch<T>), dim3(blocks, levels, std::min(kMaxJobs, njobs - j)), dim3(kBlock), 0, st,
-                           jobs + j);
+    for (uint32_t j = 0; j < njobs; j += kMaxJobs) {
+        const dim3 g(blocks, levels, std::min(kMaxJobs, njobs - j)), b(kBlock);
+        if (mode != kModeDup) hipLaunchKernelGGL((k_points_batch<T>), g, b, 0, st, jobs + j);
+        switch (mode) {
+        case kModeDup: hipLaunchKernelGGL((k_dup_batch<T>), g, b, 0, st, jobs + j); break;
+        case kModePolygon: hipLaunchKernelGGL((k_faces_batch<kModePolygon>), g, b, 0, st, jobs + j); break;
+        default: hipLaunchKernelGGL((k_faces_batch<kModeVertex>), g, b, 0, st, jobs + j); break;
+        }
+        if (mode == kModeVertex) hipLaunchKernelGGL(k_normals_batch, g, b, 0, st, jobs + j);
+    }
     return hipGetLastError();
 }
 
 }  // namespace
 
-hipError_t launch_dup(int dtype, const JobArgs& a, hipStream_t st)
+hipError_t launch_chunk_emit(int dtype, const JobArgs& a, hipStream_t st, hipEvent_t* marks)
 {
+    if (marks) (void)hipEventRecord(marks[0], st);
     switch (dtype) {
-    case 0: return launch_dup_t<int8_t>(a, st);
-    case 1: return launch_dup_t<int16_t>(a, st);
-    case 2: return launch_dup_t<int32_t>(a, st);
-    case 3: return launch_dup_t<int64_t>(a, st);
-    case 4: return launch_dup_t<uint8_t>(a, st);
-    case 5: return launch_dup_t<uint16_t>(a, st);
-    case 6: return launch_dup_t<uint32_t>(a, st);
-    case 7: return launch_dup_t<uint64_t>(a, st);
-    case 8: return launch_dup_t<float>(a, st);
-    default: return launch_dup_t<double>(a, st);
+    case 0: return launch_chunk_emit_t<int8_t>(a, st, marks);
+    case 1: return launch_chunk_emit_t<int16_t>(a, st, marks);
+    case 2: return launch_chunk_emit_t<int32_t>(a, st, marks);
+    case 3: return launch_chunk_emit_t<int64_t>(a, st, marks);
+    case 4: return launch_chunk_emit_t<uint8_t>(a, st, marks);
+    case 5: return launch_chunk_emit_t<uint16_t>(a, st, marks);
+    case 6: return launch_chunk_emit_t<uint32_t>(a, st, marks);
+    case 7: return launch_chunk_emit_t<uint64_t>(a, st, marks);
+    case 8: return launch_chunk_emit_t<float>(a, st, marks);
+    default: return launch_chunk_emit_t<double>(a, st, marks);
     }
 }
 
-hipError_t launch_dup_batch(int dtype, const JobArgs* jobs, uint32_t njobs, uint32_t blocks, uint32_t levels,
-                            hipStream_t st)
+hipError_t launch_chunk_emit_batch(int dtype, int mode, const JobArgs* jobs, uint32_t njobs, uint32_t blocks,
+                                   uint32_t levels, hipStream_t st)
 {
     switch (dtype) {
-    case 0: return launch_dup_batch_t<int8_t>(jobs, njobs, blocks, levels, st);
-    case 1: return launch_dup_batch_t<int16_t>(jobs, njobs, blocks, levels, st);
-    case 2: return launch_dup_batch_t<int32_t>(jobs, njobs, blocks, levels, st);
-    case 3: return launch_dup_batch_t<int64_t>(jobs, njobs, blocks, levels, st);
-    case 4: return launch_dup_batch_t<uint8_t>(jobs, njobs, blocks, levels, st);
-    case 5: return launch_dup_batch_t<uint16_t>(jobs, njobs, blocks, levels, st);
-    case 6: return launch_dup_batch_t<uint32_t>(jobs, njobs, blocks, levels, st);
-    case 7: return launch_dup_batch_t<uint64_t>(jobs, njobs, blocks, levels, st);
-    case 8: return launch_dup_batch_t<float>(jobs, njobs, blocks, levels, st);
-    default: return launch_dup_batch_t<double>(jobs, njobs, blocks, levels, st);
+    case 0: return launch_chunk_emit_batch_t<int8_t>(mode, jobs, njobs, blocks, levels, st);
+    case 1: return launch_chunk_emit_batch_t<int16_t>(mode, jobs, njobs, blocks, levels, st);
+    case 2: return launch_chunk_emit_batch_t<int32_t>(mode, jobs, njobs, blocks, levels, st);
+    case 3: return launch_chunk_emit_batch_t<int64_t>(mode, jobs, njobs, blocks, levels, st);
+    case 4: return launch_chunk_emit_batch_t<uint8_t>(mode, jobs, njobs, blocks, levels, st);
+    case 5: return launch_chunk_emit_batch_t<uint16_t>(mode, jobs, njobs, blocks, levels, st);
+    case 6: return launch_chunk_emit_batch_t<uint32_t>(mode, jobs, njobs, blocks, levels, st);
+    case 7: return launch_chunk_emit_batch_t<uint64_t>(mode, jobs, njobs, blocks, levels, st);
+    case 8: return launch_chunk_emit_batch_t<float>(mode, jobs, njobs, blocks, levels, st);
+    default: return launch_chunk_emit_batch_t<double>(mode, jobs, njobs, blocks, levels, st);
     }
 }
 

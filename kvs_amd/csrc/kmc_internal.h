@@ -66,11 +66,12 @@ void plan_rows(JobArgs& a);
 
 /* Split of the chunk-batch emit (rows planned; a.nlev set): a.erows and
  * a.eblocks of a pass whose emit shares its launch with others, `all` being
- * the sum of their emit_steps. */
+ * the sum of their emit_steps, for a kernel of which a CU holds per_cu
+ * workgroups and that produces `items` outputs (0: not known yet). */
 uint64_t emit_steps(const JobArgs& a);
-void plan_emit(JobArgs& a, uint64_t all);
+void plan_emit(JobArgs& a, uint64_t all, uint32_t per_cu = 4, uint64_t items = 0);
 
-/* True when the flat emit serves a volume of these y / z sizes (its records
+/* True when the chunk-batch emit serves a volume of these y / z sizes (its lists
  * pack y and z in 20 bits) and KMC_EMIT does not ask for the tile teams. */
 bool flat_emit_fits(uint32_t ny, uint32_t nz);
 
@@ -86,26 +87,18 @@ uint32_t levels_per_pass(const kmc_volume* v, int vnormal);
 
 /* Kernel launchers (kmc_kernels.hip). */
 hipError_t launch_emit(int dtype, const JobArgs& a, uint32_t lds_bytes, hipStream_t st);
-/* Flat emit of a pass (a.vpc / a.tpc written by its count pass, a.vkey /
- * a.trec / a.tci / a.fn and a.voff / a.toff set): compaction records, then
- * one thread per vertex, per triangle and (VertexNormal) per vertex normal.
- * marks: three events recorded after the compaction, the vertices and the
- * triangles (timing), or null. */
-hipError_t launch_flat_emit(int dtype, const JobArgs& a, hipStream_t st, hipEvent_t* marks = nullptr);
-/* Flat emit of a batch group: compaction over the rows of its jobs, then the
- * per-item kernels over the items start[j] .. start[j + 1] of each job. */
-hipError_t launch_compact_batch(const JobArgs* jobs, const uint64_t* row_start, uint32_t njobs, uint64_t rows,
-                                hipStream_t st);
-hipError_t launch_flat_batch(int dtype, int mode, const JobArgs* jobs, const uint64_t* vstart, const uint64_t* tstart,
-                             uint32_t njobs, hipStream_t st);
-/* Chunk-batch emit (kmc_emit.hip): the duplicated triangles of a pass, or of
- * a batch group's passes (`blocks` / `levels`: the most of one of them). */
-hipError_t launch_dup(int dtype, const JobArgs& a, hipStream_t st);
-hipError_t launch_dup_batch(int dtype, const JobArgs* jobs, uint32_t njobs, uint32_t blocks, uint32_t levels,
-                            hipStream_t st);
+/* Chunk-batch emit (kmc_emit.hip) of a pass (a.vpc / a.tpc written by its
+ * count pass, outputs and capacities set; VertexNormal: a.fn, a.crec, a.act,
+ * a.toff), or of a batch group's passes (`blocks` / `levels`: the most of one of
+ * them).  mode: 0 duplicated vertices, 1 PolygonNormal, 2 VertexNormal (shared
+ * vertices).  marks: three events recorded at the start, after the vertices and
+ * after the triangles (timing), or null. */
+hipError_t launch_chunk_emit(int dtype, const JobArgs& a, hipStream_t st, hipEvent_t* marks = nullptr);
+hipError_t launch_chunk_emit_batch(int dtype, int mode, const JobArgs* jobs, uint32_t njobs, uint32_t blocks,
+                                   uint32_t levels, hipStream_t st);
 hipError_t launch_classify(int dtype, const JobArgs& a, hipStream_t st);
-/* SlicePlane: masks from the plane's sign (a.plane), and the duplicated emit
- * (compaction, then one thread per triangle with per-vertex colours). */
+/* SlicePlane: masks from the plane's sign (a.plane), and the chunk-batch emit
+ * of its triangles with per-vertex colours. */
 hipError_t launch_classify_plane(const JobArgs& a, hipStream_t st);
 hipError_t launch_slice_emit(int dtype, const JobArgs& a, hipStream_t st);
 /* SlicePlane by node-row thresholds: thresholds (ny * nz int32) and per cell

@@ -27,9 +27,9 @@
  * Passes of one job: classify (stream the values once, write the bit volume),
  * count (per-row vertex / triangle counts and in-row chunk prefixes from the
  * bit volume), scan (row prefixes), emit (outputs at the prefixes; raw values
- * are read again only at the endpoints of crossing edges).  The emit is flat
- * (compaction records, then one thread per output item) unless y or z exceeds
- * 2^20, when the tile teams below do it.
+ * are read again only at the endpoints of crossing edges).  The emit works
+ * on batches of chunks (kmc_emit.hip) unless y or z exceeds 2^20, when the tile
+ * teams below do it.
  *
  * Within a slice, the classification bits of 64 consecutive nodes of a row
  * are held as one 64-bit mask per level (a *chunk*), built with one wave
@@ -42,19 +42,12 @@
 namespace kmc {
 
 constexpr int kMaxLevels = 8;
+constexpr uint32_t kBitSlack = 16;   // bytes allocated past a bit volume (read, not used: load_words)
 constexpr int kBlock = 256;          // threads per workgroup of the dense passes (4 waves of 64)
 constexpr int kWaves = kBlock / 64;
 constexpr int kEmitTeams = 4;        // emit workgroup: 4 independent one-wave teams
 constexpr int kEmitBlock = 64 * kEmitTeams;
 constexpr uint32_t kTableBytes = 256 * 8;   // case table at the start of the emit workgroup's LDS
-
-/* Crossing edges of one 64-node chunk with a vertex (flat emit): the
- * level-relative id of its first vertex and the x / y / z crossing-edge masks
- * of its nodes. */
-struct alignas(32) ChunkCross {
-    uint64_t base;
-    uint64_t x, y, z;
-};
 
 struct JobArgs {
     const void* values;
@@ -73,7 +66,6 @@ struct JobArgs {
     uint32_t fn_cap;   // face normals held per cell slice (VertexNormal)
     uint32_t team_stride;  // bytes of LDS per team (>= the team layout's size)
     uint32_t teams;        // teams per emit workgroup (<= kEmitTeams; fewer when a team's LDS is large)
-    uint32_t rec_levels;   // flat emit: bit l set when level l has records (levels without outputs get none)
     uint64_t nunits;   // nlev * nb * nslabs
     uint32_t erows;    // chunk-batch emit: node rows per wave step (at most 64 >> cshift) ...
     uint32_t eblocks;  // ... and workgroups per level
@@ -98,22 +90,13 @@ struct JobArgs {
     // (y, z-1) (tpc); written by the count pass when non-null
     uint32_t* vpc;
     uint32_t* tpc;
-    // records of the compaction pass (flat emit): per vertex, in output order,
-    // x | y << 20 | z << 40 | axis << 60; per triangle x | y << 20 | z << 40 |
-    // t << 60 of its cell and the cell's cube index; per triangle its face normal
-    // (VertexNormal); level l's items start at voff[l] / toff[l]
-    uint64_t* vkey;
-    uint64_t* trec;
-    uint8_t* tci;
+    // VertexNormal: per triangle its face normal, per active cell its case and
+    // first triangle (kmc_emit.hip); level l's start at toff[l]
     float* fn;
-    // per chunk (bit volume layout), written by the compaction for chunks with a vertex
-    ChunkCross* cross;
-    // VertexNormal: per vertex, for each of the four cells around its edge (in
-    // cell scan order) the item index of that cell's first triangle record;
-    // written by the triangles that use the edge (cells outside the volume:
-    // not written, not read)
-    uint32_t* vslot;
-    uint64_t voff[kMaxLevels + 1];
+    uint32_t* crec;
+    // VertexNormal: active cells of cell row (y, z-1), bit volume layout, written
+    // for chunks with one
+    uint64_t* act;
     uint64_t toff[kMaxLevels + 1];
     // per-level outputs
     float* coords[kMaxLevels];

@@ -13,11 +13,9 @@
  * ballot per level; only crossing edges and active cells do more.
  *
  * Passes: classify (values -> masks), count (per-row counts and in-row chunk
- * prefixes), scan (row prefixes), then the flat emit: a compaction writes
- * every vertex's key and every triangle's record at its output rank, and one
- * thread per vertex / triangle / vertex normal produces the outputs.  The
- * tile-team emit (each wave marching a band of rows through z with LDS rings
- * of masks) remains for volumes whose rows exceed the records' fields.
+ * prefixes), scan (row prefixes), then the emit in chunk batches (kmc_emit.hip).
+ * The tile-team emit here (each wave marching a band of rows through z with LDS
+ * rings of masks) remains for volumes whose y or z exceed its lists' fields.
  *
  * Arithmetic follows Source/Core/Visualization/Mapper/MarchingCubes.cpp bit for
  * bit: the comparison double(v) > isolevel (:299-316), the FP64 clamp / ratio /
@@ -30,6 +28,7 @@
 #include <algorithm>
 #include <map>
 #include <mutex>
+#include "kmc_chunks.h"
 #include "kmc_device.h"
 #include "kmc_internal.h"
 #include "kmc_job.h"
@@ -1356,666 +1355,10 @@ __global__ __launch_bounds__(kEmitBlock) void k_emit_batch(const JobArgs* jobs, 
     }
 }
 
-/* ------------------------------------------------------------------------- */
-/* flat emit: compaction records, then one thread per output item              */
-/* ------------------------------------------------------------------------- */
-
-/* Level of output item i given the per-level start offsets (nlev <= 8). */
-__device__ __forceinline__ uint32_t level_at(const uint64_t* off, uint32_t nlev, uint64_t i)
-{
-    uint32_t l = 0;
-    for (uint32_t k = 1; k < nlev; ++k) l += i >= off[k] ? 1u : 0u;
-    return l;
-}
-
-/* One non-empty chunk of the compaction, queued as y | z << 20 | level << 40
- * | chunk << 44. */
-__device__ __forceinline__ void compact_chunk(const JobArgs& a, const uint8_t* ntri, uint64_t e)
-{
-    const uint32_t y = (uint32_t)(e & 0xFFFFFu), z = (uint32_t)((e >> 20) & 0xFFFFFu);
-    const uint32_t l = (uint32_t)((e >> 40) & 0xFu), c = (uint32_t)(e >> 44);
-    const uint64_t level_words = (uint64_t)a.nz * a.ny * a.NC;
-    const uint64_t r = (uint64_t)z * a.ny + y;
-    const uint64_t w = (uint64_t)l * level_words + r * a.NC + c;
-    const uint64_t* pre_v = a.prefix + (uint64_t)(l * 2 + 0) * a.nrows;
-    const uint64_t* pre_t = a.prefix + (uint64_t)(l * 2 + 1) * a.nrows;
-    RowChunk o;
-    row_chunk(a, a.bitvol + (uint64_t)l * level_words, y, z, c, o);
-    uint32_t pv, pt;
-    chunk_prefix(a, w, pv, pt);
-    if (!a.dup) {
-        uint64_t m = o.x | o.y | o.z;
-        if (m) {
-            ChunkCross cc;
-            cc.base = (pre_v[r] - pre_v[0]) + pv;
-            cc.x = o.x;
-            cc.y = o.y;
-            cc.z = o.z;
-            a.cross[w] = cc;
-            uint64_t id = a.voff[l] + cc.base;
-            const uint64_t rowkey = (uint64_t)y << 20 | (uint64_t)z << 40;
-            while (m) {
-                const uint32_t i = (uint32_t)__ffsll((unsigned long long)m) - 1u;
-                m &= m - 1ull;
-                const uint64_t key = rowkey | (c * 64u + i);
-                if ((o.x >> i) & 1ull) a.vkey[id++] = key;
-                if ((o.y >> i) & 1ull) a.vkey[id++] = key | 1ull << 60;
-                if ((o.z >> i) & 1ull) a.vkey[id++] = key | 2ull << 60;
-            }
-        }
-    }
-    uint64_t m = o.act;
-    if (m) {
-        uint64_t id = a.toff[l] + (pre_t[r] - pre_t[0]) + pt;
-        const uint64_t cellkey = (uint64_t)y << 20 | (uint64_t)(z - 1) << 40;
-        while (m) {
-            const uint32_t i = (uint32_t)__ffsll((unsigned long long)m) - 1u;
-            m &= m - 1ull;
-            const uint32_t pi = corner_pairs(o, i);
-            const uint32_t ci = swap_pairs(pi);
-            const uint32_t nt = ntri[pi];
-            const uint64_t key = cellkey | (c * 64u + i);
-            for (uint32_t t = 0; t < nt; ++t, ++id) {
-                a.trec[id] = key | (uint64_t)t << 60;
-                a.tci[id] = (uint8_t)ci;
-            }
-        }
-    }
-}
-
-/* Compaction of node rows [r0, r1): every crossing edge writes its key at its
- * vertex id and every triangle its cell and table index t (plus the cell's
- * cube index) at its triangle id -- row prefix + chunk prefix within the row
- * + rank within the chunk, i.e. vertices in node scan order x {x,y,z}-edge
- * and triangles in cell scan order x table order (calculate_isopoints
- * :365-437, connect_isopoints :439-521, extract_surfaces_with_duplication
- * :155-243); chunks with a vertex also leave their crossing record.  Lanes
- * first scan (row, chunk) pairs as the count pass does, NLEV levels at a time
- * (their loads in flight together; NLEV = 0: one level at a time, any level
- * count), and queue the non-empty chunks (the chunk prefixes tell) in the
- * wave's LDS queue q (kCompactQueue entries); the work on them runs 64 chunks
- * at a time, one per lane, taken from the queue's end.  Output positions come
- * from the prefixes alone, so the queue's order does not matter. */
-constexpr uint32_t kCompactLevels = 4;
-constexpr uint32_t kCompactQueue = 64 * (kCompactLevels + 1);
-
-template <int NLEV>
-__device__ __forceinline__ void compact_rows_t(const JobArgs& a, const uint8_t* ntri, uint64_t* q, uint64_t r0, uint64_t r1,
-                                               uint64_t wave_first, uint64_t wave_step)
-{
-    constexpr uint32_t NL = NLEV ? (uint32_t)NLEV : 1u;
-    static_assert(NL <= kCompactLevels, "queue holds 63 + 64 * NL entries");
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t sub = lane >> a.cshift, cl = lane & ((1u << a.cshift) - 1u);
-    const uint32_t G = 64u >> a.cshift, CS = 1u << a.cshift;
-    const uint64_t level_words = (uint64_t)a.nz * a.ny * a.NC;
-    if (!a.trec) return;   // the records did not fit (batched form): nothing to write
-    uint32_t qn = 0;
-    RowWalk rw = row_walk(a, r0 + wave_first * G, wave_step * G);
-    for (uint64_t g = r0 + wave_first * G; g < r1; g += wave_step * G, row_next(a, rw)) {
-        const uint64_t r = g + sub;
-        const bool ok = r < r1;
-        uint32_t y, z;
-        row_at(a, rw, sub, y, z);
-        for (uint32_t l0 = 0; l0 < a.nlev; l0 += NL) {
-            for (uint32_t c0 = 0; c0 < a.NC; c0 += CS) {
-                const uint32_t c = c0 + cl;
-                bool busy[NL];
-#pragma unroll
-                for (uint32_t k = 0; k < NL; ++k) {
-                    busy[k] = false;
-                    if (ok && c < a.NC) {
-                        /* chunks without crossing edges or active cells (most of
-                         * them) are skipped on the count pass's prefixes alone */
-                        const uint32_t l = l0 + k;
-                        if (!((a.rec_levels >> l) & 1u)) continue;   // a level without records
-                        const uint64_t w = (uint64_t)l * level_words + r * a.NC + c;
-                        uint32_t v0, t0, v1, t1;
-                        chunk_prefix(a, w, v0, t0);
-                        if (c + 1 < a.NC) {
-                            chunk_prefix(a, w + 1, v1, t1);
-                        } else {
-                            v1 = a.counts[(uint64_t)(l * 2 + 0) * a.nrows + r];
-                            t1 = a.counts[(uint64_t)(l * 2 + 1) * a.nrows + r];
-                        }
-                        busy[k] = (!a.dup && v1 != v0) || t1 != t0;
-                    }
-                }
-#pragma unroll
-                for (uint32_t k = 0; k < NL; ++k) {
-                    const uint64_t bm = __ballot(busy[k]);
-                    if (busy[k])
-                        q[qn + lanes_below(bm)] =
-                            (uint64_t)y | (uint64_t)z << 20 | (uint64_t)(l0 + k) << 40 | (uint64_t)c << 44;
-                    qn += (uint32_t)__popcll(bm);
-                }
-                while (qn >= 64) {
-                    wave_sync();
-                    qn -= 64;
-                    compact_chunk(a, ntri, q[qn + lane]);
-                    wave_sync();
-                }
-            }
-        }
-    }
-    wave_sync();
-    if (lane < qn) compact_chunk(a, ntri, q[lane]);
-    wave_sync();   // the queue is reused by the next call
-}
-
-__device__ __forceinline__ void compact_rows(const JobArgs& a, const uint8_t* ntri, uint64_t* q, uint64_t r0, uint64_t r1,
-                                             uint64_t wave_first, uint64_t wave_step)
-{
-    switch (a.nlev) {
-    case 1: compact_rows_t<1>(a, ntri, q, r0, r1, wave_first, wave_step); break;
-    case 2: compact_rows_t<2>(a, ntri, q, r0, r1, wave_first, wave_step); break;
-    case 3: compact_rows_t<3>(a, ntri, q, r0, r1, wave_first, wave_step); break;
-    case 4: compact_rows_t<4>(a, ntri, q, r0, r1, wave_first, wave_step); break;
-    default: compact_rows_t<0>(a, ntri, q, r0, r1, wave_first, wave_step); break;
-    }
-}
-
-__global__ __launch_bounds__(kBlock) void k_compact(JobArgs a)
-{
-    __shared__ uint8_t ntri[256];
-    __shared__ uint64_t queue[kWaves][kCompactQueue];
-    stage_ntri(ntri);
-    const uint64_t G = 64u >> a.cshift, groups = (a.nrows + G - 1) / G;
-    const Span sp = grid_span(0, groups, kWaves, uniform(threadIdx.x >> 6));
-    const uint64_t r1 = sp.end * G < a.nrows ? sp.end * G : a.nrows;
-    compact_rows(a, ntri, queue[threadIdx.x >> 6], sp.lo * G, r1, sp.first - sp.lo, sp.step);
-}
-
-/* Compaction of a batch of jobs: the rows of all jobs in one sequence, split
- * as the count pass splits them. */
-__global__ __launch_bounds__(kBlock) void k_compact_batch(const JobArgs* jobs, const uint64_t* row_start, uint32_t njobs)
-{
-    __shared__ uint8_t ntri[256];
-    __shared__ uint64_t queue[kWaves][kCompactQueue];
-    stage_ntri(ntri);
-    const uint64_t total = row_start[njobs];
-    const uint64_t nwaves = ((uint64_t)gridDim.x * kBlock) >> 6;
-    const uint64_t wave_id = (uint64_t)blockIdx.x * kWaves + uniform(threadIdx.x >> 6);   // uniform: scalar
-    const uint64_t per = (total + nwaves - 1) / nwaves;
-    const uint64_t begin = wave_id * per;
-    const uint64_t end = begin + per < total ? begin + per : total;
-    uint64_t g = begin;
-    while (g < end) {
-        const uint32_t j = __builtin_amdgcn_readfirstlane(find_job(row_start, njobs, g));
-        const uint64_t je = row_start[j + 1] < end ? row_start[j + 1] : end;
-        compact_rows(jobs[j], ntri, queue[threadIdx.x >> 6], g - row_start[j], je - row_start[j], 0, 1);
-        g = je;
-    }
-}
-
-/* Vertex id (within its level) of the vertex on the edge along `axis` of node
- * i of a chunk, from the chunk's crossing record o: the chunk's first vertex id
- * (row prefix + chunk prefix within the row) + the crossing edges of the
- * chunk's nodes before i and of node i's lower axes. */
-__device__ __forceinline__ uint64_t cross_rank(const ChunkCross& o, uint32_t i, uint32_t axis)
-{
-    const uint64_t lo = (1ull << i) - 1ull;
-    uint64_t r = o.base;
-    r += (uint64_t)(__popcll(o.x & lo) + __popcll(o.y & lo) + __popcll(o.z & lo));
-    if (axis >= 1) r += (o.x >> i) & 1ull;
-    if (axis >= 2) r += (o.y >> i) & 1ull;
-    return r;
-}
-
-/* Node values at the two ends of the edge of vertex key `key`. */
-template <typename T>
-__device__ __forceinline__ void edge_values(const JobArgs& a, uint64_t key, T& va, T& vb)
-{
-    const T* vol = (const T*)a.values;
-    const uint64_t x = key & 0xFFFFFu, y = (key >> 20) & 0xFFFFFu, z = (key >> 40) & 0xFFFFFu;
-    const uint32_t axis = (uint32_t)(key >> 60);
-    const uint64_t line = a.nx, slice = (uint64_t)a.nx * a.ny;
-    const uint64_t ia = x + y * line + z * slice;
-    va = vol[ia];
-    vb = vol[ia + (axis == 0 ? 1ull : axis == 1 ? line : slice)];
-}
-
-/* Coordinates of vertex g (of level l, which has outputs) from its key and
- * its edge's node values (calculate_isopoints, :365-437). */
-template <typename T>
-__device__ __forceinline__ void vertex_item(const JobArgs& a, uint32_t l, uint64_t g, uint64_t key, T va, T vb)
-{
-    const uint32_t x = (uint32_t)(key & 0xFFFFFu), y = (uint32_t)((key >> 20) & 0xFFFFFu);
-    const uint32_t z = (uint32_t)((key >> 40) & 0xFFFFFu), axis = (uint32_t)(key >> 60);
-    float p[3];
-    interpolate_values<T>(a, a.iso[l], va, vb, x, y, z, x + (axis == 0), y + (axis == 1), z + (axis == 2), p);
-    float* co = a.coords[l];
-    const uint64_t id = g - a.voff[l];
-    co[3 * id + 0] = p[0];
-    co[3 * id + 1] = p[1];
-    co[3 * id + 2] = p[2];
-}
-
-/* Vertices g, g + step, ... < n of level l.  The level's isolevel, first item
- * and outputs are uniform (scalar loads, which leave the vector memory
- * operations in flight alone).  Software pipeline: while item g is finished,
- * the node values of the next item and the key of the one after it are in
- * flight (vector memory operations complete in issue order, so they are issued
- * before item g's stores; indices past the range's end are clamped to its
- * last item, so that every iteration issues the same loads). */
-template <typename T>
-__device__ __forceinline__ void vertices_level(const JobArgs& a, uint32_t l, uint64_t g, uint64_t n, uint64_t step)
-{
-    if (g >= n || !a.coords[l]) return;   // no items, or a level without outputs (not admitted)
-    const uint64_t last = n - 1;
-    /* two register sets take turns (unrolled by two), so that no loaded
-     * value is copied -- a copy would wait for its load */
-    uint64_t k0 = a.vkey[g], k1;
-    T a0, b0, a1, b1;
-    edge_values<T>(a, k0, a0, b0);
-    uint64_t kn = a.vkey[g + step < last ? g + step : last];
-    for (;;) {
-        k1 = kn;
-        edge_values<T>(a, k1, a1, b1);
-        kn = a.vkey[g + 2 * step < last ? g + 2 * step : last];
-        vertex_item<T>(a, l, g, k0, a0, b0);
-        g += step;
-        if (g >= n) break;
-        k0 = kn;
-        edge_values<T>(a, k0, a0, b0);
-        kn = a.vkey[g + 2 * step < last ? g + 2 * step : last];
-        vertex_item<T>(a, l, g, k1, a1, b1);
-        g += step;
-        if (g >= n) break;
-    }
-}
-
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_vertices(JobArgs a)
-{
-    for (uint32_t l = 0; l < a.nlev; ++l) {
-        const Span sp = grid_span(a.voff[l], a.voff[l + 1], kBlock, threadIdx.x);
-        vertices_level<T>(a, l, sp.first, sp.end, sp.step);
-    }
-}
-
 __device__ __forceinline__ void stage_table_block(uint64_t* tri)
 {
     for (uint32_t i = threadIdx.x; i < 256; i += kBlock) tri[i] = d_tri[i];
     __syncthreads();
-}
-
-/* Every triangle of shared vertices (duplicated ones: kmc_emit.hip): its
- * connectivity (connect_isopoints, :439-521) and the face normal of the
- * shared vertices' coordinates -- the PolygonNormal output
- * (calculate_normals_on_polygon, :531-559) or, with VertexNormal, kept in
- * a.fn for the per-vertex sums. */
-template <typename T, int M>
-__device__ __forceinline__ void triangle_item(const JobArgs& a, const uint64_t* tri, uint64_t g, uint64_t rec, uint32_t ci)
-{
-    const uint64_t level_words = (uint64_t)a.nz * a.ny * a.NC;
-    const uint32_t l = level_at(a.toff, a.nlev, g);
-    const uint32_t x = (uint32_t)(rec & 0xFFFFFu), y = (uint32_t)((rec >> 20) & 0xFFFFFu);
-    const uint32_t zc = (uint32_t)((rec >> 40) & 0xFFFFFu), t = (uint32_t)(rec >> 60);
-    const uint64_t w = tri[ci];
-    const uint32_t eds[3] = { (uint32_t)((w >> (12 * t)) & 0xF), (uint32_t)((w >> (12 * t + 8)) & 0xF),
-                              (uint32_t)((w >> (12 * t + 4)) & 0xF) };
-    float* coords = nullptr;
-    float* normals = nullptr;
-    uint32_t* conn = nullptr;
-#pragma unroll
-    for (int k = 0; k < kMaxLevels; ++k)
-        if (k == (int)l) { coords = a.coords[k]; normals = a.normals[k]; conn = a.conn[k]; }
-    if (!coords) return;   // a level without outputs (not admitted)
-    const uint64_t id = g - a.toff[l];
-    float p[3][3], nn[3];
-    static_assert(M != kModeDup, "duplicated triangles: kmc_emit.hip");
-    const ChunkCross* cross_l = a.cross + (uint64_t)l * level_words;
-    /* the owner chunks' crossing records of all three edges are loaded
-     * before any is used, so the three loads are in flight together */
-    const uint64_t vbase = M == kModeVertex ? a.voff[l] : 0ull;
-    ChunkCross cc[3];
-    uint32_t bit[3], axs[3];
-#pragma unroll
-    for (int jj = 0; jj < 3; ++jj) {
-        const uint32_t o = edge_owner(eds[jj]);
-        const uint32_t vx = x + (o & 1u), vy = y + ((o >> 1) & 1u), vz = zc + ((o >> 2) & 1u);
-        bit[jj] = vx & 63u;
-        axs[jj] = o >> 3;
-        cc[jj] = cross_l[((uint64_t)vz * a.ny + vy) * a.NC + (vx >> 6)];
-    }
-    uint64_t vid[3];
-#pragma unroll
-    for (int jj = 0; jj < 3; ++jj) vid[jj] = cross_rank(cc[jj], bit[jj], axs[jj]);
-    /* the vertices' coordinates are loaded before this item's stores
-     * (vector memory operations complete in issue order) */
-#pragma unroll
-    for (int jj = 0; jj < 3; ++jj) {
-        p[jj][0] = coords[3 * vid[jj] + 0];
-        p[jj][1] = coords[3 * vid[jj] + 1];
-        p[jj][2] = coords[3 * vid[jj] + 2];
-    }
-    conn[3 * id + 0] = (uint32_t)vid[0];
-    conn[3 * id + 1] = (uint32_t)vid[1];
-    conn[3 * id + 2] = (uint32_t)vid[2];
-    if constexpr (M == kModeVertex) {
-        /* the first triangle of this cell that uses an edge tells the edge's
-         * vertex where the cell's records start; the cell sits at position q
-         * around the edge (around_cell) */
-        uint32_t* slots = a.vslot + 4 * vbase;
-#pragma unroll
-        for (int jj = 0; jj < 3; ++jj) {
-            bool first = true;
-            for (uint32_t u = 0; u < t; ++u) {
-                const uint32_t f0 = (uint32_t)((w >> (12 * u)) & 0xF), f1 = (uint32_t)((w >> (12 * u + 4)) & 0xF);
-                const uint32_t f2 = (uint32_t)((w >> (12 * u + 8)) & 0xF);
-                first = first && f0 != eds[jj] && f1 != eds[jj] && f2 != eds[jj];
-            }
-            if (!first) continue;
-            const uint32_t o = edge_owner(eds[jj]);
-            const uint32_t dx = o & 1u, dy = (o >> 1) & 1u, dz = (o >> 2) & 1u, ax = o >> 3;
-            const uint32_t q = ax == 0 ? ((dy ? 0u : 1u) | (dz ? 0u : 2u))
-                             : ax == 1 ? ((dx ? 0u : 1u) | (dz ? 0u : 2u))
-                                       : ((dx ? 0u : 1u) | (dy ? 0u : 2u));
-            slots[4 * vid[jj] + q] = (uint32_t)(g - t);
-        }
-    }
-    face_normal(p[0], p[1], p[2], nn);
-    float* dst = M == kModeVertex ? a.fn + 3 * g : normals + 3 * id;
-    dst[0] = nn[0];
-    dst[1] = nn[1];
-    dst[2] = nn[2];
-}
-
-/* Triangles g, g + step, ... < n: the next item's record is loaded while this
- * one is worked on. */
-template <typename T, int M>
-__device__ __forceinline__ void triangles_range(const JobArgs& a, const uint64_t* tri, uint64_t g, uint64_t n,
-                                                uint64_t step)
-{
-    uint64_t rec = g < n ? a.trec[g] : 0ull;
-    uint32_t ci = g < n ? a.tci[g] : 0u;
-    for (; g < n; g += step) {
-        const uint64_t cur = rec;
-        const uint32_t cur_ci = ci;
-        if (g + step < n) {
-            rec = a.trec[g + step];
-            ci = a.tci[g + step];
-        }
-        triangle_item<T, M>(a, tri, g, cur, cur_ci);
-    }
-}
-
-template <typename T, int M>
-__global__ __launch_bounds__(kBlock) void k_triangles(JobArgs a)
-{
-    __shared__ uint64_t tri[256];
-    stage_table_block(tri);
-    const Span sp = grid_span(0, a.toff[a.nlev], kBlock, threadIdx.x);
-    triangles_range<T, M>(a, tri, sp.first, sp.end, sp.step);
-}
-
-/* The cells around vertex key `key`'s edge that lie in the volume: each is
- * active, and the first of its triangles that uses the edge wrote the slot. */
-__device__ __forceinline__ void vn_cells_in(const JobArgs& a, uint64_t key, bool in[4])
-{
-    const int x = (int)(key & 0xFFFFFu), y = (int)((key >> 20) & 0xFFFFFu);
-    const int zv = (int)((key >> 40) & 0xFFFFFu);
-    const uint32_t axis = (uint32_t)(key >> 60);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        int cx, cy, cz;
-        around_cell(axis, q, x, y, zv, cx, cy, cz);
-        in[q] = cx >= 0 && cy >= 0 && cz >= 0 && cx + 1 < (int)a.nx && cy + 1 < (int)a.ny && cz + 1 < (int)a.nz;
-    }
-}
-
-/* Cube indices of the cells around the edge (0 for cells outside the volume).
- * With `always`, cells outside load record 0 instead of nothing (the job has
- * triangles), so that every call issues the same loads. */
-template <bool always>
-__device__ __forceinline__ void vn_cube_indices(const JobArgs& a, uint64_t key, uint4 sl, uint32_t ci[4])
-{
-    bool in[4];
-    vn_cells_in(a, key, in);
-    const uint32_t first[4] = { sl.x, sl.y, sl.z, sl.w };
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        if constexpr (always) {
-            const uint32_t c = a.tci[in[q] ? first[q] : 0u];
-            ci[q] = in[q] ? c : 0u;
-        } else {
-            ci[q] = in[q] ? a.tci[first[q]] : 0u;
-        }
-    }
-}
-
-/* Per cell around the edge, the mask of its triangles (table order) that use
- * the edge, and the face normals of the first two such triangles of every
- * cell, loaded together (most cells have one or two). */
-struct VnGather {
-    uint32_t use[4];
-    uint32_t first[4];
-    float f[4][2][3];
-};
-
-__device__ __forceinline__ void vn_gather(const JobArgs& a, const uint64_t* tri, uint64_t key, uint4 sl,
-                                          const uint32_t ci[4], VnGather& o)
-{
-    bool in[4];
-    vn_cells_in(a, key, in);
-    const uint32_t around = around_nibbles((uint32_t)(key >> 60));
-    o.first[0] = sl.x;
-    o.first[1] = sl.y;
-    o.first[2] = sl.z;
-    o.first[3] = sl.w;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        o.use[q] = 0u;
-        if (!in[q]) continue;
-        const uint64_t w = tri[ci[q]];
-        const int nt = (int)(w >> 60);
-        const uint32_t me = (around >> (4 * q)) & 0xFu;
-        for (int t = 0; t < nt; ++t) {
-            const uint32_t e0 = (uint32_t)((w >> (12 * t)) & 0xF);
-            const uint32_t e1 = (uint32_t)((w >> (12 * t + 8)) & 0xF);
-            const uint32_t e2 = (uint32_t)((w >> (12 * t + 4)) & 0xF);
-            if (e0 == me || e1 == me || e2 == me) o.use[q] |= 1u << t;
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        uint32_t m = o.use[q];
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            o.f[q][k][0] = o.f[q][k][1] = o.f[q][k][2] = 0.0f;
-            if (m) {
-                const uint32_t t = (uint32_t)__ffs(m) - 1u;
-                m &= m - 1u;
-                const float* p = a.fn + 3 * ((uint64_t)o.first[q] + t);
-                o.f[q][k][0] = p[0];
-                o.f[q][k][1] = p[1];
-                o.f[q][k][2] = p[2];
-            }
-        }
-    }
-}
-
-/* VertexNormal of vertex g (level l, which has outputs): the float sum, in
- * triangle order, of the face normals of the triangles that use it
- * (calculate_normals_on_vertex, :569-605) -- the four cells around the edge in
- * cell scan order and each cell's triangles that use the edge in table order.
- * A slot without a triangle holds +0, and adding +0 changes no partial sum:
- * the sum starts at +0 and a float sum is -0 only when both terms are, so no
- * partial sum is -0.  The starting +0 comes from an opaque move, so that the
- * compiler does not fold the first addition into the first load's branch
- * (which would wait for that load alone). */
-__device__ __forceinline__ void vn_finish(const JobArgs& a, uint32_t l, uint64_t g, const VnGather& o)
-{
-    float zero;
-    asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
-    float nv[3] = { zero, zero, zero };
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            nv[0] = nv[0] + o.f[q][k][0];
-            nv[1] = nv[1] + o.f[q][k][1];
-            nv[2] = nv[2] + o.f[q][k][2];
-        }
-        uint32_t m = o.use[q];
-        m &= m - 1u;
-        m &= m - 1u;
-        while (m) {   // further triangles of the cell that use the edge (rare)
-            const uint32_t t = (uint32_t)__ffs(m) - 1u;
-            m &= m - 1u;
-            const float* p = a.fn + 3 * ((uint64_t)o.first[q] + t);
-            nv[0] = nv[0] + p[0];
-            nv[1] = nv[1] + p[1];
-            nv[2] = nv[2] + p[2];
-        }
-    }
-    float* normals = a.normals[l];
-    const uint64_t id = g - a.voff[l];
-    normals[3 * id + 0] = nv[0];
-    normals[3 * id + 1] = nv[1];
-    normals[3 * id + 2] = nv[2];
-}
-
-__device__ __forceinline__ void vertex_normal_item(const JobArgs& a, const uint64_t* tri, uint32_t l, uint64_t g,
-                                                   uint64_t key, uint4 sl)
-{
-    if (!a.normals[l]) return;   // a level without outputs (not admitted)
-    uint32_t ci[4];
-    vn_cube_indices<false>(a, key, sl, ci);
-    VnGather o;
-    vn_gather(a, tri, key, sl, ci, o);
-    vn_finish(a, l, g, o);
-}
-
-/* eight waves per SIMD (64 VGPRs, a few bytes of spill) beat six without */
-/* Vertex normals g, g + step, ... < n of level l (`triangles`: the job has a
- * triangle at all; without one no vertex has a cell in the volume around it).
- * Software pipeline over two register sets that take turns (a copy would
- * wait for its load): while vertex g is summed, the next vertex's cube
- * indices are in flight, and the key and slots of the one after it are
- * loaded before this vertex's store (vector memory operations complete in
- * issue order); indices past the range's end are clamped to its last item. */
-__device__ __forceinline__ void vertex_normals_level(const JobArgs& a, const uint64_t* tri, uint32_t l, bool triangles,
-                                                     uint64_t g, uint64_t n, uint64_t step)
-{
-    if (g >= n || !a.normals[l]) return;   // no items, or a level without outputs (not admitted)
-    const uint64_t last = n - 1;
-    if (!triangles) {
-        for (; g < n; g += step) vertex_normal_item(a, tri, l, g, a.vkey[g], *(const uint4*)(a.vslot + 4 * g));
-        return;
-    }
-    uint64_t k0 = a.vkey[g], k1;
-    uint4 s0 = *(const uint4*)(a.vslot + 4 * g), s1;
-    uint32_t c0[4], c1[4];
-    vn_cube_indices<true>(a, k0, s0, c0);
-    {
-        const uint64_t g1 = g + step < last ? g + step : last;
-        k1 = a.vkey[g1];
-        s1 = *(const uint4*)(a.vslot + 4 * g1);
-    }
-    VnGather o;
-    for (;;) {
-        vn_cube_indices<true>(a, k1, s1, c1);
-        vn_gather(a, tri, k0, s0, c0, o);
-        {
-            const uint64_t g2 = g + 2 * step < last ? g + 2 * step : last;
-            k0 = a.vkey[g2];
-            s0 = *(const uint4*)(a.vslot + 4 * g2);
-        }
-        vn_finish(a, l, g, o);
-        g += step;
-        if (g >= n) break;
-        vn_cube_indices<true>(a, k0, s0, c0);
-        vn_gather(a, tri, k1, s1, c1, o);
-        {
-            const uint64_t g2 = g + 2 * step < last ? g + 2 * step : last;
-            k1 = a.vkey[g2];
-            s1 = *(const uint4*)(a.vslot + 4 * g2);
-        }
-        vn_finish(a, l, g, o);
-        g += step;
-        if (g >= n) break;
-    }
-}
-
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_vertex_normals(JobArgs a)
-{
-    __shared__ uint64_t tri[256];
-    stage_table_block(tri);
-    const bool triangles = a.toff[a.nlev] > 0;
-    /* level by level (uniform per-level values) */
-    for (uint32_t l = 0; l < a.nlev; ++l) {
-        const Span sp = grid_span(a.voff[l], a.voff[l + 1], kBlock, threadIdx.x);
-        vertex_normals_level(a, tri, l, triangles, sp.first, sp.end, sp.step);
-    }
-}
-
-/* Items of a batch of jobs: start[j] is job j's first item in one sequence
- * over the launch's jobs (start[njobs]: the end).  Persistent grid: each
- * workgroup takes one contiguous part of the sequence (whole multiples of its
- * size) and runs the plain kernels' loops over the pieces of it that fall in
- * one job and one level -- no per-item job or level search. */
-struct BlockPart { uint64_t lo, hi; };
-
-__device__ __forceinline__ BlockPart block_part(uint64_t n)
-{
-    const uint64_t per = ((n + gridDim.x - 1) / gridDim.x + kBlock - 1) / kBlock * kBlock;
-    BlockPart p;
-    p.lo = (uint64_t)blockIdx.x * per < n ? (uint64_t)blockIdx.x * per : n;
-    p.hi = p.lo + per < n ? p.lo + per : n;
-    return p;
-}
-
-/* Calls f(jobs[j], lo, hi) for each job j with items in this workgroup's part,
- * [lo, hi) being those items as the job's own item indices. */
-template <typename F>
-__device__ __forceinline__ void for_part_jobs(const JobArgs* jobs, const uint64_t* start, uint32_t njobs, F&& f)
-{
-    const uint64_t base = uniform64(start[0]);
-    const BlockPart bp = block_part(uniform64(start[njobs]) - base);
-    if (bp.lo >= bp.hi) return;
-    for (uint32_t j = uniform(find_job(start, njobs, bp.lo + base)); j < njobs; ++j) {
-        const uint64_t s0 = uniform64(start[j]) - base, s1 = uniform64(start[j + 1]) - base;
-        if (s0 >= bp.hi) break;
-        const uint64_t lo = (bp.lo > s0 ? bp.lo : s0) - s0, hi = (bp.hi < s1 ? bp.hi : s1) - s0;
-        if (lo >= hi) continue;
-        f(jobs[j], lo, hi);
-    }
-}
-
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_vertices_batch(const JobArgs* jobs, const uint64_t* start, uint32_t njobs)
-{
-    for_part_jobs(jobs, start, njobs, [&](const JobArgs& a, uint64_t lo, uint64_t hi) {
-        for (uint32_t l = 0; l < a.nlev; ++l) {
-            const uint64_t l0 = lo > a.voff[l] ? lo : a.voff[l], l1 = hi < a.voff[l + 1] ? hi : a.voff[l + 1];
-            if (l0 < l1) vertices_level<T>(a, l, l0 + threadIdx.x, l1, kBlock);
-        }
-    });
-}
-
-template <typename T, int M>
-__global__ __launch_bounds__(kBlock) void k_triangles_batch(const JobArgs* jobs, const uint64_t* start, uint32_t njobs)
-{
-    __shared__ uint64_t tri[256];
-    stage_table_block(tri);
-    for_part_jobs(jobs, start, njobs, [&](const JobArgs& a, uint64_t lo, uint64_t hi) {
-        triangles_range<T, M>(a, tri, lo + threadIdx.x, hi, kBlock);
-    });
-}
-
-__global__ __launch_bounds__(kBlock) void k_vertex_normals_batch(const JobArgs* jobs, const uint64_t* start, uint32_t njobs)
-{
-    __shared__ uint64_t tri[256];
-    stage_table_block(tri);
-    for_part_jobs(jobs, start, njobs, [&](const JobArgs& a, uint64_t lo, uint64_t hi) {
-        const bool triangles = a.toff[a.nlev] > 0;
-        for (uint32_t l = 0; l < a.nlev; ++l) {
-            const uint64_t l0 = lo > a.voff[l] ? lo : a.voff[l], l1 = hi < a.voff[l + 1] ? hi : a.voff[l + 1];
-            if (l0 < l1) vertex_normals_level(a, tri, l, triangles, l0 + threadIdx.x, l1, kBlock);
-        }
-    });
 }
 
 /* ------------------------------------------------------------------------- */
@@ -2195,13 +1538,43 @@ __device__ __forceinline__ void slice_triangle(const JobArgs& a, const uint64_t*
     slice_triangle_values<T>(a, tri, rec, ci, GlobalColors{ a.ctable }, out);
 }
 
+/* Triangles of the planes the thresholds do not serve, from their chunk masks
+ * (slice_triangle's table indexed as corner_pairs gives the case). */
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_slice_triangles(JobArgs a)
 {
+    struct SliceLds {
+        ListLds l;
+        uint64_t m[4][kChunks];      // k0, k3, k4, k7 of each chunk
+        uint64_t key[kChunks];       // 64 c | y << 20 | z << 40 of each chunk's first cell
+        uint32_t next[kChunks];
+    };
     __shared__ uint64_t tri[256];
-    stage_table_block(tri);
-    const Span sp = grid_span(0, a.toff[1], kBlock, threadIdx.x);
-    for (uint64_t g = sp.first; g < sp.end; g += sp.step) slice_triangle<T>(a, tri, g, a.trec[g], a.tci[g]);
+    __shared__ SliceLds lds[kWaves];
+    for (uint32_t i = threadIdx.x; i < 256; i += kBlock) tri[i] = d_tri[swap_pairs(i)];
+    __syncthreads();
+    SliceLds& s = lds[threadIdx.x >> 6];
+    const uint32_t lane = threadIdx.x & 63u;
+    const EmitLevel L = emit_level(a, 0);
+    busy_chunks<false, kChunks>(a, L, s.l.q, [&](uint32_t n) {
+        list_triangles(a, L, tri, s.l, n, [&](uint64_t, uint32_t y, uint32_t z, uint32_t c, uint64_t) {
+            const CellMasks o = load_cells(a, L, y, z, c);
+            s.m[0][lane] = o.k0;
+            s.m[1][lane] = o.k3;
+            s.m[2][lane] = o.k4;
+            s.m[3][lane] = o.k7;
+            s.next[lane] = o.next;
+            s.key[lane] = (uint64_t)(c * 64u) | (uint64_t)y << 20 | (uint64_t)(z - 1) << 40;
+            return o.act;
+        }, [&](uint32_t q, uint32_t i) { return corner_pairs_at(s.m, s.next, q, i); },
+        [](uint32_t, uint32_t, uint32_t, uint32_t) {}, [&](uint32_t cnt, uint32_t rank) {
+            for (uint32_t j = lane; j < cnt; j += 64) {
+                const uint32_t e = s.l.tl[j], cell = s.l.cell[e & 63u], q = cell & 63u;
+                const uint64_t rec = (s.key[q] + ((cell >> 6) & 63u)) | (uint64_t)(e >> 6) << 60;
+                slice_triangle<T>(a, tri, s.l.out[q] + (rank + j), rec, cell >> 12);
+            }
+        });
+    });
 }
 
 /* SlicePlane without classifying every node.  Along a node row (y, z) the
@@ -2820,106 +2193,11 @@ hipError_t launch_count(const JobArgs& a, hipStream_t st)
     return hipGetLastError();
 }
 
-/* The VertexNormal triangle kernel runs best at four waves per SIMD: more
- * waves in flight evict the cache lines its gathers reuse (measured on the
- * 1024^3 turbulence field: 0.609 ms at its register-bound five waves, 0.587
- * at four, 0.617 at three).  A launch with this much dynamic LDS per
- * 256-thread workgroup (the kernel uses none of it) leaves room for four
- * workgroups in a CU's 160 KiB. */
-constexpr uint32_t kTriangleLdsPad = 38u << 10;
-
 /* Grid of a flat per-item kernel: up to 8 resident workgroups per CU. */
 static uint32_t flat_blocks(uint64_t items)
 {
     const uint64_t b = (items + kBlock - 1) / kBlock;
     return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(b, 256 * 8));
-}
-
-template <typename T>
-hipError_t launch_flat_t(const JobArgs& a, hipStream_t st, hipEvent_t* marks)
-{
-    const uint64_t nv = a.voff[a.nlev], nt = a.toff[a.nlev];
-    if (nv) hipLaunchKernelGGL((k_vertices<T>), dim3(flat_blocks(nv)), dim3(kBlock), 0, st, a);
-    if (marks) (void)hipEventRecord(marks[1], st);
-    if (nt) {
-        switch (emit_mode(a)) {
-        case kModePolygon:
-            hipLaunchKernelGGL((k_triangles<T, kModePolygon>), dim3(flat_blocks(nt)), dim3(kBlock), 0, st, a);
-            break;
-        default: hipLaunchKernelGGL((k_triangles<T, kModeVertex>), dim3(flat_blocks(nt)), dim3(kBlock), kTriangleLdsPad, st, a); break;
-        }
-    }
-    if (marks) (void)hipEventRecord(marks[2], st);
-    if (a.vnormal && nv) hipLaunchKernelGGL(k_vertex_normals, dim3(flat_blocks(nv)), dim3(kBlock), 0, st, a);
-    return hipGetLastError();
-}
-
-hipError_t launch_compact_batch(const JobArgs* jobs, const uint64_t* row_start, uint32_t njobs, uint64_t rows,
-                                hipStream_t st)
-{
-    uint64_t blocks = (rows / 4 + kWaves - 1) / kWaves + 1;
-    if (blocks > 16384) blocks = 16384;
-    hipLaunchKernelGGL(k_compact_batch, dim3((uint32_t)blocks), dim3(kBlock), 0, st, jobs, row_start, njobs);
-    return hipGetLastError();
-}
-
-template <typename T>
-hipError_t launch_flat_batch_t(int mode, const JobArgs* jobs, const uint64_t* vstart, const uint64_t* tstart,
-                               uint32_t njobs, hipStream_t st)
-{
-    /* item counts live on the device: persistent grids */
-    const dim3 g(256 * 8), b(kBlock);
-    hipLaunchKernelGGL((k_vertices_batch<T>), g, b, 0, st, jobs, vstart, njobs);
-    switch (mode) {
-    case kModePolygon: hipLaunchKernelGGL((k_triangles_batch<T, kModePolygon>), g, b, 0, st, jobs, tstart, njobs); break;
-    default: hipLaunchKernelGGL((k_triangles_batch<T, kModeVertex>), g, b, 0, st, jobs, tstart, njobs); break;
-    }
-    if (mode == kModeVertex) hipLaunchKernelGGL(k_vertex_normals_batch, g, b, 0, st, jobs, vstart, njobs);
-    return hipGetLastError();
-}
-
-hipError_t launch_flat_batch(int dtype, int mode, const JobArgs* jobs, const uint64_t* vstart, const uint64_t* tstart,
-                             uint32_t njobs, hipStream_t st)
-{
-    switch (dtype) {
-    case 0: return launch_flat_batch_t<int8_t>(mode, jobs, vstart, tstart, njobs, st);
-    case 1: return launch_flat_batch_t<int16_t>(mode, jobs, vstart, tstart, njobs, st);
-    case 2: return launch_flat_batch_t<int32_t>(mode, jobs, vstart, tstart, njobs, st);
-    case 3: return launch_flat_batch_t<int64_t>(mode, jobs, vstart, tstart, njobs, st);
-    case 4: return launch_flat_batch_t<uint8_t>(mode, jobs, vstart, tstart, njobs, st);
-    case 5: return launch_flat_batch_t<uint16_t>(mode, jobs, vstart, tstart, njobs, st);
-    case 6: return launch_flat_batch_t<uint32_t>(mode, jobs, vstart, tstart, njobs, st);
-    case 7: return launch_flat_batch_t<uint64_t>(mode, jobs, vstart, tstart, njobs, st);
-    case 8: return launch_flat_batch_t<float>(mode, jobs, vstart, tstart, njobs, st);
-    default: return launch_flat_batch_t<double>(mode, jobs, vstart, tstart, njobs, st);
-    }
-}
-
-hipError_t launch_flat_emit(int dtype, const JobArgs& a, hipStream_t st, hipEvent_t* marks)
-{
-    if (a.dup) {
-        if (marks) { (void)hipEventRecord(marks[0], st); (void)hipEventRecord(marks[1], st); }
-        const hipError_t e = launch_dup(dtype, a, st);
-        if (marks) (void)hipEventRecord(marks[2], st);
-        return e;
-    }
-    const uint64_t G = 64u >> a.cshift;
-    uint64_t blocks = ((a.nrows + G - 1) / G + kWaves - 1) / kWaves;
-    if (blocks > 16384) blocks = 16384;
-    hipLaunchKernelGGL(k_compact, dim3((uint32_t)blocks), dim3(kBlock), 0, st, a);
-    if (marks) (void)hipEventRecord(marks[0], st);
-    switch (dtype) {
-    case 0: return launch_flat_t<int8_t>(a, st, marks);
-    case 1: return launch_flat_t<int16_t>(a, st, marks);
-    case 2: return launch_flat_t<int32_t>(a, st, marks);
-    case 3: return launch_flat_t<int64_t>(a, st, marks);
-    case 4: return launch_flat_t<uint8_t>(a, st, marks);
-    case 5: return launch_flat_t<uint16_t>(a, st, marks);
-    case 6: return launch_flat_t<uint32_t>(a, st, marks);
-    case 7: return launch_flat_t<uint64_t>(a, st, marks);
-    case 8: return launch_flat_t<float>(a, st, marks);
-    default: return launch_flat_t<double>(a, st, marks);
-    }
 }
 
 hipError_t launch_classify_plane(const JobArgs& a, hipStream_t st)
@@ -2934,12 +2212,7 @@ hipError_t launch_classify_plane(const JobArgs& a, hipStream_t st)
 template <typename T>
 hipError_t launch_slice_emit_t(const JobArgs& a, hipStream_t st)
 {
-    const uint64_t G = 64u >> a.cshift;
-    uint64_t blocks = ((a.nrows + G - 1) / G + kWaves - 1) / kWaves;
-    if (blocks > 16384) blocks = 16384;
-    hipLaunchKernelGGL(k_compact, dim3((uint32_t)blocks), dim3(kBlock), 0, st, a);
-    const uint64_t nt = a.toff[1];
-    if (nt) hipLaunchKernelGGL((k_slice_triangles<T>), dim3(flat_blocks(nt)), dim3(kBlock), 0, st, a);
+    hipLaunchKernelGGL((k_slice_triangles<T>), dim3(a.eblocks), dim3(kBlock), 0, st, a);
     return hipGetLastError();
 }
 

@@ -73,16 +73,19 @@ struct Carve {
     }
 };
 
-/* Scratch bytes of the arrays sized by the volume alone. */
+/* Scratch bytes a volume is admitted with (the emit takes less): its work of
+ * 48 bytes per chunk with shared vertices, 16 with duplicated ones, and 24 per
+ * node row. */
 uint64_t front_bytes(const JobArgs& a, bool minmax)
 {
     const uint64_t R = a.nrows, C = a.nrows * a.NC;
     const uint64_t nparts = scan_partials_needed(R, 2);
     return up256(2 * R * 4) + up256(2 * R * 8) + up256((nparts + 2) * 8) + up256(C * 8) + up256(2 * C * 4) +
-           (a.dup ? 0 : up256(C * sizeof(ChunkCross))) + (minmax ? up256(minmax_scratch_bytes() + 16) : 0);
+           (a.dup ? 0 : up256(C * 32)) + (minmax ? up256(minmax_scratch_bytes() + 16) : 0);
 }
 
-/* Scratch bytes of the emit's records for nv vertices and nt triangles. */
+/* Scratch bytes nv vertices and nt triangles are admitted with (the emit
+ * takes at most 16 per triangle). */
 uint64_t record_bytes(const JobArgs& a, uint64_t nv, uint64_t nt)
 {
     return up256(nv * 8) + up256(nt * 8) + up256(nt) + (a.vnormal ? up256(nt * 12) + up256(nv * 16) : 0);
@@ -105,7 +108,6 @@ kmc_status extract_noalloc(const kmc_volume* v, double iso, int32_t normal_type,
     JobArgs a;
     init_job(a, v, v->values, &iso, 1, normal_type, dup, v->min_value, v->max_value, minc, maxc);
     plan_rows(a);
-    a.rec_levels = 1u;
     const uint64_t need_front = front_bytes(a, !v->has_min_max_values);
     if (need_front > KMC_NOALLOC_SCRATCH_BYTES) return KMC_ERR_SCRATCH;
 
@@ -126,7 +128,7 @@ kmc_status extract_noalloc(const kmc_volume* v, double iso, int32_t normal_type,
     a.bitvol = cv.take<uint64_t>(C * 8);
     a.vpc = cv.take<uint32_t>(2 * C * 4);
     a.tpc = a.vpc + C;
-    a.cross = dup ? nullptr : cv.take<ChunkCross>(C * sizeof(ChunkCross));
+    a.act = a.vnormal ? cv.take<uint64_t>(C * 8) : nullptr;
     a.counts = counts;
     a.prefix = prefix;
 
@@ -179,24 +181,18 @@ kmc_status extract_noalloc(const kmc_volume* v, double iso, int32_t normal_type,
     if (3 * out->n_vertices > coords_cap || 3 * out->n_normals > normals_cap || out->n_connections > conn_cap ||
         !coords || !normals || (out->n_connections && !conn))
         return KMC_ERR_CAPACITY;   // the sizes stay in *out; nothing was written
-    if (cv.used + record_bytes(a, dup ? 0 : nv, nt) > KMC_NOALLOC_SCRATCH_BYTES) return KMC_ERR_SCRATCH;
+    if (need_front + record_bytes(a, dup ? 0 : nv, nt) > KMC_NOALLOC_SCRATCH_BYTES) return KMC_ERR_SCRATCH;
 
-    a.voff[0] = a.toff[0] = 0;
-    a.voff[1] = dup ? 0 : nv;
+    a.toff[0] = 0;
     a.toff[1] = nt;
-    if (!dup) {   // duplicated triangles need no records
-        a.vkey = cv.take<uint64_t>(a.voff[1] * 8);
-        a.trec = cv.take<uint64_t>(nt * 8);
-        a.tci = cv.take<uint8_t>(nt);
-    }
     a.fn = a.vnormal ? cv.take<float>(nt * 12) : nullptr;
-    a.vslot = a.vnormal ? cv.take<uint32_t>(nv * 16) : nullptr;
+    a.crec = a.vnormal ? cv.take<uint32_t>(nt * 4) : nullptr;
     a.coords[0] = coords;
     a.normals[0] = normals;
     a.conn[0] = dup ? nullptr : conn;
     a.cap_vertices[0] = verts;
     a.cap_triangles[0] = nt;
-    if (launch_flat_emit(v->type, a, st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess) {
+    if (launch_chunk_emit(v->type, a, st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess) {
         (void)hipGetLastError();
         return KMC_ERR_DEVICE;
     }

@@ -176,7 +176,6 @@ kmc_status slice_plane_impl(const kmc_volume* v, const float coef[4], const uint
     const double iso = 0.0;
     init_job(a, v, dvals, &iso, 1, KMC_POLYGON_NORMAL, 1, mn, mx, minc, maxc);
     plan_rows(a);
-    a.rec_levels = 1u;
     for (int k = 0; k < 4; ++k) a.plane[k] = coef[k];
     if (color_range) { a.crange[0] = color_range[0]; a.crange[1] = color_range[1]; }
     else default_color_range(v->type, mn, mx, a.crange);
@@ -196,7 +195,7 @@ kmc_status slice_plane_impl(const kmc_volume* v, const float coef[4], const uint
     uint32_t* counts = (uint32_t*)alloc(2 * R * 4);
     uint64_t* prefix = (uint64_t*)alloc(2 * R * 8);
     uint64_t* aux = (uint64_t*)alloc((nparts + 2) * 8);
-    a.bitvol = (uint64_t*)alloc(C * 8);
+    a.bitvol = (uint64_t*)alloc(C * 8 + kBitSlack);
     a.vpc = (uint32_t*)alloc(2 * C * 4);
     uint8_t* dtable = (uint8_t*)alloc(3 * (size_t)res);
     if (!counts || !prefix || !aux || !a.bitvol || !a.vpc || !dtable) return finish(KMC_ERR_OUT_OF_MEMORY);
@@ -233,19 +232,15 @@ kmc_status slice_plane_impl(const kmc_volume* v, const float coef[4], const uint
         store->coords = device_alloc(9 * nt * sizeof(float));
         store->normals = device_alloc(3 * nt * sizeof(float));
         store->colors = device_alloc(9 * nt);
-        uint8_t* recs = (uint8_t*)alloc(up256(nt * 8) + nt);
-        if (!store->coords || !store->normals || !store->colors || !recs) {
+        if (!store->coords || !store->normals || !store->colors) {
             kmc_surface_release(out);
             return finish(KMC_ERR_OUT_OF_MEMORY);
         }
         out->coords = (float*)store->coords;
         out->normals = (float*)store->normals;
         out->colors = (uint8_t*)store->colors;
-        a.voff[0] = a.voff[1] = 0;
         a.toff[0] = 0;
         a.toff[1] = nt;
-        a.trec = (uint64_t*)recs;
-        a.tci = recs + up256(nt * 8);
         a.coords[0] = out->coords;
         a.normals[0] = out->normals;
         a.colors = out->colors;
