@@ -99,17 +99,24 @@ __global__ __launch_bounds__(kLayoutBlock) void k_batch_layout(JobArgs* jobs, co
                                                                uint64_t cap_r, uint32_t flat)
 {
     __shared__ uint32_t overflow;
-    /* one sweep per kLayoutBlock * kLayoutPer surfaces, carrying the offsets */
+    /* one sweep per kLayoutBlock * per surfaces, carrying the offsets; a
+     * thread's surfaces are a chain of dependent loads, so it takes one as long
+     * as there are threads for all (30 surfaces: 20 us with eight) */
+    auto per_thread = [](uint32_t n) {
+        const uint32_t p = (n + kLayoutBlock - 1) / kLayoutBlock;
+        return p < kLayoutPer ? (p ? p : 1u) : kLayoutPer;
+    };
+    const uint32_t sper = per_thread(nseg), pper = per_thread(npass);
     uint64_t carry[3] = { 0, 0, 0 };
-    for (uint32_t b0 = 0; b0 < nseg; b0 += kLayoutBlock * kLayoutPer) {
-        const uint32_t s0 = b0 + threadIdx.x * kLayoutPer;
+    for (uint32_t b0 = 0; b0 < nseg; b0 += kLayoutBlock * sper) {
+        const uint32_t s0 = b0 + threadIdx.x * sper;
         uint64_t sz[kLayoutPer][3];
         uint64_t nv[kLayoutPer], nt[kLayoutPer];
         uint64_t v[3] = { 0, 0, 0 };
         for (uint32_t i = 0; i < kLayoutPer; ++i) {
             nv[i] = nt[i] = 0;
             sz[i][0] = sz[i][1] = sz[i][2] = 0;
-            if (s0 + i < nseg) {
+            if (i < sper && s0 + i < nseg) {
                 const uint32_t m = seg_map[s0 + i];
                 const JobArgs& a = jobs[m >> 3];
                 const uint32_t l = m & 7u;
@@ -127,7 +134,7 @@ __global__ __launch_bounds__(kLayoutBlock) void k_batch_layout(JobArgs* jobs, co
         uint64_t tot[3];
         block_scan3(v, tot);
         for (uint32_t i = 0; i < kLayoutPer; ++i) {
-            if (s0 + i < nseg) {
+            if (i < sper && s0 + i < nseg) {
                 SegOut o;
                 o.nv = nv[i];
                 o.nt = nt[i];
@@ -144,13 +151,13 @@ __global__ __launch_bounds__(kLayoutBlock) void k_batch_layout(JobArgs* jobs, co
     /* emit records of every pass (not with the tile teams) */
     uint64_t rcarry = 0;
     if (flat) {
-        for (uint32_t b0 = 0; b0 < npass; b0 += kLayoutBlock * kLayoutPer) {
-            const uint32_t p0 = b0 + threadIdx.x * kLayoutPer;
+        for (uint32_t b0 = 0; b0 < npass; b0 += kLayoutBlock * pper) {
+            const uint32_t p0 = b0 + threadIdx.x * pper;
             uint64_t sz[kLayoutPer];
             uint64_t v[3] = { 0, 0, 0 };
             for (uint32_t i = 0; i < kLayoutPer; ++i) {
                 sz[i] = 0;
-                if (p0 + i < npass && jobs[p0 + i].vnormal) {
+                if (i < pper && p0 + i < npass && jobs[p0 + i].vnormal) {
                     const JobArgs& a = jobs[p0 + i];
                     uint64_t nt = 0;
                     for (uint32_t l = 0; l < a.nlev; ++l) nt += level_total(a, l, 1);
@@ -161,7 +168,7 @@ __global__ __launch_bounds__(kLayoutBlock) void k_batch_layout(JobArgs* jobs, co
             uint64_t tot[3];
             block_scan3(v, tot);
             for (uint32_t i = 0; i < kLayoutPer; ++i) {
-                if (p0 + i < npass) jobs[p0 + i].toff[0] = rcarry + v[0];   // record byte offset (placed below)
+                if (i < pper && p0 + i < npass) jobs[p0 + i].toff[0] = rcarry + v[0];   // record byte offset (placed below)
                 v[0] += sz[i];
             }
             rcarry += tot[0];
@@ -242,14 +249,14 @@ struct Group {
     int dtype;
     int mode;                    // 0 duplicated, 1 PolygonNormal, 2 VertexNormal
     uint32_t p0, p1;             // passes [p0, p1)
-    uint64_t rows, units;
+    uint64_t max_chunks, max_groups;   // the most chunks and row groups of one of its passes
+    uint64_t units;
     uint32_t max_levels;         // the most levels of one of its passes
     uint32_t emit_blocks;        // the most emit workgroups per level of one of its passes
     uint32_t emit_lds;
     uint32_t teams;                // emit teams per workgroup
-    uint64_t* row_start_d;       // p1 - p0 + 1 entries
-    uint64_t* unit_start_d;
-    std::vector<uint64_t> row_start_h, unit_start_h;   // upload sources, kept while the copies may run
+    uint64_t* unit_start_d;      // p1 - p0 + 1 entries
+    std::vector<uint64_t> unit_start_h;   // upload source, kept while the copy may run
 };
 
 }  // namespace
@@ -306,9 +313,8 @@ namespace {
 void free_plan_buffers(kmc_batch* b)
 {
     for (Group& g : b->groups) {
-        device_free(g.row_start_d);
         device_free(g.unit_start_d);
-        g.row_start_d = g.unit_start_d = nullptr;
+        g.unit_start_d = nullptr;
     }
 }
 
@@ -368,15 +374,17 @@ kmc_status plan_tiles(kmc_batch* b, uint32_t r_max, uint32_t queue_cap)
         uint64_t steps = 0;
         for (uint32_t i = g.p0; i < g.p1; ++i) steps += emit_steps(b->passes[i].a);
         for (uint32_t i = g.p0; i < g.p1 && !b->two_phase; ++i) plan_emit(b->passes[i].a, steps);
-        std::vector<uint64_t> rs, ts;
-        uint64_t r = 0, t = 0;
+        std::vector<uint64_t> ts;
+        uint64_t t = 0;
         uint32_t stride = 0, teams = kEmitTeams;
         g.max_levels = 0;
         g.emit_blocks = 1;
+        g.max_chunks = g.max_groups = 0;
         for (uint32_t i = g.p0; i < g.p1; ++i) {
-            rs.push_back(r);
+            const JobArgs& a = b->passes[i].a;
+            g.max_chunks = std::max(g.max_chunks, a.nrows * a.NC);
+            g.max_groups = std::max(g.max_groups, (a.nrows << a.cshift) / 64 + 1);
             ts.push_back(t);
-            r += b->passes[i].a.nrows;
             t += b->passes[i].a.nunits;
             stride = std::max(stride, b->passes[i].a.team_stride);
             g.max_levels = std::max(g.max_levels, b->passes[i].a.nlev);
@@ -391,19 +399,13 @@ kmc_status plan_tiles(kmc_batch* b, uint32_t r_max, uint32_t queue_cap)
         }
         g.teams = teams;
         g.emit_lds = emit_lds_bytes(stride, teams);
-        rs.push_back(r);
         ts.push_back(t);
-        g.rows = r;
         g.units = t;
         if (t > 0xFFFFFFFFull) return KMC_ERR_INVALID_ARGUMENT;
-        g.row_start_d = (uint64_t*)device_alloc(rs.size() * 8);
         g.unit_start_d = (uint64_t*)device_alloc(ts.size() * 8);
-        if (!g.row_start_d || !g.unit_start_d) return KMC_ERR_OUT_OF_MEMORY;
-        g.row_start_h = std::move(rs);
+        if (!g.unit_start_d) return KMC_ERR_OUT_OF_MEMORY;
         g.unit_start_h = std::move(ts);
-        if (hipMemcpyAsync(g.row_start_d, g.row_start_h.data(), g.row_start_h.size() * 8, hipMemcpyHostToDevice,
-                           b->upload_stream) != hipSuccess ||
-            hipMemcpyAsync(g.unit_start_d, g.unit_start_h.data(), g.unit_start_h.size() * 8, hipMemcpyHostToDevice,
+        if (hipMemcpyAsync(g.unit_start_d, g.unit_start_h.data(), g.unit_start_h.size() * 8, hipMemcpyHostToDevice,
                            b->upload_stream) != hipSuccess)
             return KMC_ERR_DEVICE;
     }
@@ -440,11 +442,11 @@ hipError_t record_front(kmc_batch* b, hipStream_t st, bool copy_sizes)
         if (e != hipSuccess) return e;
     } else {
         for (const Group& g : b->groups) {
-            e = launch_classify_batch(g.dtype, b->jobs_d + g.p0, g.row_start_d, g.p1 - g.p0, g.rows, g.max_levels, st);
+            e = launch_classify_batch(g.dtype, b->jobs_d + g.p0, g.p1 - g.p0, g.max_chunks, g.max_levels, st);
             if (e != hipSuccess) return e;
         }
         for (const Group& g : b->groups) {
-            e = launch_count_batch(b->jobs_d + g.p0, g.row_start_d, g.p1 - g.p0, g.rows, st);
+            e = launch_count_batch(b->jobs_d + g.p0, g.p1 - g.p0, g.max_groups, st);
             if (e != hipSuccess) return e;
         }
     }

@@ -116,10 +116,10 @@ size_t minmax_scratch_bytes();
 /* The unstructured form: vol[0], then vol[conn[i]] for every connection entry in order. */
 hipError_t launch_minmax_gather(int dtype, const void* vol, const uint32_t* conn, uint64_t nconn, void* scratch,
                                 double* out, hipStream_t st);
-hipError_t launch_classify_batch(int dtype, const JobArgs* jobs, const uint64_t* row_start, uint32_t njobs,
-                                 uint64_t rows, uint32_t max_levels, hipStream_t st);
-hipError_t launch_count_batch(const JobArgs* jobs, const uint64_t* row_start, uint32_t njobs, uint64_t rows,
-                              hipStream_t st);
+/* chunks / groups: the most chunks, and row groups of 64 >> cshift rows, of one job */
+hipError_t launch_classify_batch(int dtype, const JobArgs* jobs, uint32_t njobs, uint64_t chunks, uint32_t max_levels,
+                                 hipStream_t st);
+hipError_t launch_count_batch(const JobArgs* jobs, uint32_t njobs, uint64_t groups, hipStream_t st);
 /* mode: 0 duplicated vertices, 1 PolygonNormal, 2 VertexNormal (shared vertices) */
 hipError_t launch_emit_batch(int dtype, int mode, const JobArgs* jobs, const uint64_t* unit_start, uint32_t njobs,
                              uint64_t units, uint32_t lds_bytes, uint32_t teams, hipStream_t st);

@@ -827,46 +827,42 @@ __device__ __forceinline__ void classify_row(const JobArgs& a, uint64_t row)
     }
 }
 
-/* Classification of chunks [q0, q1) of a job, q = row * NC + chunk: the
- * chunks of consecutive rows follow each other, so short rows share a wave's
- * batches of loads and its windows of 64 parked masks, which leave with one
- * coalesced store per level (the masks of consecutive rows are contiguous). */
+/* Classification of 16 chunks from q0 on, then of every step-th such run below
+ * q1, q = row * NC + chunk: the chunks of consecutive rows follow each other,
+ * so that short rows share a wave's loads, and the masks of consecutive rows are
+ * contiguous (one 128-byte store per level). */
 template <typename T, int NLEV>
-__device__ __forceinline__ void classify_chunks(const JobArgs& a, uint64_t q0, uint64_t q1)
+__device__ __forceinline__ void classify_chunks(const JobArgs& a, uint64_t q0, uint64_t q1, uint64_t step)
 {
     const uint32_t lane = threadIdx.x & 63u;
     const T* vals = (const T*)a.values;
     const uint64_t level_words = (uint64_t)a.nz * a.ny * a.NC;
     constexpr uint32_t kBatch = 16;
-    for (uint64_t w0 = q0; w0 < q1; w0 += 64) {
-        const uint32_t wn = (q1 - w0) < 64 ? (uint32_t)(q1 - w0) : 64u;
+    for (; q0 < q1; q0 += step) {
+        const uint32_t wn = (q1 - q0) < kBatch ? (uint32_t)(q1 - q0) : kBatch;
+        uint64_t row = q0 / a.NC;
+        uint32_t c = (uint32_t)(q0 - row * a.NC);
+        T val[kBatch];
+        uint32_t cs[kBatch];
+#pragma unroll
+        for (uint32_t i = 0; i < kBatch; ++i) {
+            cs[i] = c;
+            const uint32_t x = c * 64u + lane;
+            val[i] = (i < wn && x < a.nx) ? __builtin_nontemporal_load(vals + row * a.nx + x) : T(0);   // read once
+            if (++c == a.NC) { c = 0; ++row; }
+        }
         uint32_t lo[NLEV], hi[NLEV];
 #pragma unroll
         for (int l = 0; l < NLEV; ++l) { lo[l] = 0; hi[l] = 0; }
-        uint64_t row = w0 / a.NC;
-        uint32_t c = (uint32_t)(w0 - row * a.NC);
-        for (uint32_t cb = 0; cb < wn; cb += kBatch) {
-            T val[kBatch];
-            uint32_t cs[kBatch];
 #pragma unroll
-            for (uint32_t i = 0; i < kBatch; ++i) {
-                cs[i] = c;
-                const uint32_t x = c * 64u + lane;
-                val[i] = (cb + i < wn && x < a.nx) ? vals[row * a.nx + x] : T(0);
-                if (++c == a.NC) { c = 0; ++row; }
-            }
+        for (uint32_t i = 0; i < kBatch; ++i) {
+            const bool in = i < wn && cs[i] * 64u + lane < a.nx;
+            const bool mine = lane == i;
 #pragma unroll
-            for (uint32_t i = 0; i < kBatch; ++i) {
-                if (cb + i < wn) {
-                    const bool in = cs[i] * 64u + lane < a.nx;
-                    const bool mine = lane == cb + i;
-#pragma unroll
-                    for (int l = 0; l < NLEV; ++l) {
-                        const uint64_t m = __ballot(in && above<T>(val[i], a, l));
-                        lo[l] = mine ? (uint32_t)m : lo[l];
-                        hi[l] = mine ? (uint32_t)(m >> 32) : hi[l];
-                    }
-                }
+            for (int l = 0; l < NLEV; ++l) {
+                const uint64_t m = __ballot(in && above<T>(val[i], a, l));
+                lo[l] = mine ? (uint32_t)m : lo[l];
+                hi[l] = mine ? (uint32_t)(m >> 32) : hi[l];
             }
         }
         /* the 8-level instance also serves passes of 5..7 levels: store only
@@ -875,7 +871,8 @@ __device__ __forceinline__ void classify_chunks(const JobArgs& a, uint64_t q0, u
 #pragma unroll
             for (int l = 0; l < NLEV; ++l)
                 if (NLEV < 8 || l < (int)a.nlev)
-                    a.bitvol[(uint64_t)l * level_words + w0 + lane] = ((uint64_t)hi[l] << 32) | lo[l];
+                    __builtin_nontemporal_store(((uint64_t)hi[l] << 32) | lo[l],
+                                                &a.bitvol[(uint64_t)l * level_words + q0 + lane]);
         }
     }
 }
@@ -996,56 +993,43 @@ __device__ __forceinline__ uint32_t find_job(const uint64_t* start, uint32_t n, 
     return lo;
 }
 
-/* Classify pass of a batch of jobs sharing the value type T: the node rows of
- * all jobs form one sequence (row_start[j] = first row of job j), cut into one
- * contiguous range per wave so that the job changes rarely along a range; a
- * wave classifies its rows of a job as one run of chunks.  kWide: some job has
- * more than four levels (the eight-level instance's registers would otherwise
- * halve the waves per SIMD of every batch). */
+/* Classify pass of a batch of jobs sharing the value type T: job z's workgroups
+ * walk its chunks in steps of the whole grid, 16 consecutive chunks a wave, so
+ * that every wave has 16 loads in flight and the grid sweeps the job in address
+ * order (one contiguous range of rows per wave took 199 us on 14 volumes of 32
+ * .. 256 per axis, 186 MB).  kWide: some job has more than four levels (the
+ * eight-level instance's registers would otherwise halve the waves per SIMD of
+ * every batch). */
 template <typename T, bool kWide>
-__global__ __launch_bounds__(kBlock) void k_classify_batch(const JobArgs* jobs, const uint64_t* row_start, uint32_t njobs)
+__global__ __launch_bounds__(kBlock) void k_classify_batch(const JobArgs* jobs)
 {
-    const uint64_t total = row_start[njobs];
-    const uint64_t wave_id = (uint64_t)blockIdx.x * kWaves + uniform(threadIdx.x >> 6);   // uniform: scalar
-    const uint64_t nwaves = ((uint64_t)gridDim.x * kBlock) >> 6;
-    const uint64_t per = (total + nwaves - 1) / nwaves;
-    uint64_t g = wave_id * per;
-    const uint64_t end = g + per < total ? g + per : total;
-    if (g >= end) return;
-    uint32_t j = __builtin_amdgcn_readfirstlane(find_job(row_start, njobs, g));
-    while (g < end) {
-        while (g >= row_start[j + 1]) ++j;
-        const JobArgs& a = jobs[j];
-        const uint64_t je = row_start[j + 1] < end ? row_start[j + 1] : end;
-        if constexpr (sizeof(T) <= 2) {
-            if (packed_rows<T>(a)) {
-                /* the wave's rows as (row, segment) items, 16 at a time */
-                const uint64_t nseg = (a.nx / (4 / sizeof(T)) + 63) / 64;
-                const uint64_t i0 = (g - row_start[j]) * nseg, i1 = (je - row_start[j]) * nseg;
-                switch (a.nlev) {
-                case 1: classify_packed_items<T, 1>(a, i0, i1, 16); break;
-                case 2: classify_packed_items<T, 2>(a, i0, i1, 16); break;
-                case 3: classify_packed_items<T, 3>(a, i0, i1, 16); break;
-                case 4: classify_packed_items<T, 4>(a, i0, i1, 16); break;
-                default:
-                    if constexpr (kWide) classify_packed_items<T, 8>(a, i0, i1, 16);
-                    break;
-                }
-                g = je;
-                continue;
+    const JobArgs& a = jobs[blockIdx.z];
+    const uint64_t wave = (uint64_t)blockIdx.x * kWaves + uniform(threadIdx.x >> 6);   // uniform: scalar
+    const uint64_t step = (uint64_t)gridDim.x * kWaves * 16;
+    if constexpr (sizeof(T) <= 2) {
+        if (packed_rows<T>(a)) {
+            const uint64_t items = a.nrows * ((a.nx / (4 / sizeof(T)) + 63) / 64);
+            switch (a.nlev) {
+            case 1: classify_packed_items<T, 1>(a, wave * 16, items, step); break;
+            case 2: classify_packed_items<T, 2>(a, wave * 16, items, step); break;
+            case 3: classify_packed_items<T, 3>(a, wave * 16, items, step); break;
+            case 4: classify_packed_items<T, 4>(a, wave * 16, items, step); break;
+            default:
+                if constexpr (kWide) classify_packed_items<T, 8>(a, wave * 16, items, step);
+                break;
             }
+            return;
         }
-        const uint64_t q0 = (g - row_start[j]) * a.NC, q1 = (je - row_start[j]) * a.NC;
-        switch (a.nlev) {
-        case 1: classify_chunks<T, 1>(a, q0, q1); break;
-        case 2: classify_chunks<T, 2>(a, q0, q1); break;
-        case 3: classify_chunks<T, 3>(a, q0, q1); break;
-        case 4: classify_chunks<T, 4>(a, q0, q1); break;
-        default:
-            if constexpr (kWide) classify_chunks<T, 8>(a, q0, q1);
-            break;
-        }
-        g = je;
+    }
+    const uint64_t chunks = a.nrows * a.NC;
+    switch (a.nlev) {
+    case 1: classify_chunks<T, 1>(a, wave * 16, chunks, step); break;
+    case 2: classify_chunks<T, 2>(a, wave * 16, chunks, step); break;
+    case 3: classify_chunks<T, 3>(a, wave * 16, chunks, step); break;
+    case 4: classify_chunks<T, 4>(a, wave * 16, chunks, step); break;
+    default:
+        if constexpr (kWide) classify_chunks<T, 8>(a, wave * 16, chunks, step);
+        break;
     }
 }
 
@@ -1240,24 +1224,16 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) voi
     count_rows(a, ntri, sp.lo * G, r1, sp.first - sp.lo, sp.step);
 }
 
-/* Count pass of a batch: the node rows of all jobs form one sequence, cut
- * into one contiguous range per wave. */
-__global__ __launch_bounds__(kBlock) void k_count_batch(const JobArgs* jobs, const uint64_t* row_start, uint32_t njobs)
+/* Count pass of a batch: job z's workgroups walk its row groups in steps of the
+ * whole grid. */
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) void k_count_batch(const JobArgs* jobs)
 {
+    const JobArgs& a = jobs[blockIdx.z];
+    const uint64_t G = 64u >> a.cshift, wave = (uint64_t)blockIdx.x * kWaves;
+    if (wave * G >= a.nrows) return;   // the whole workgroup: a job smaller than the grid
     __shared__ uint8_t ntri[256];
     stage_ntri(ntri);
-    const uint64_t total = row_start[njobs];
-    const uint64_t wave_id = (uint64_t)blockIdx.x * kWaves + uniform(threadIdx.x >> 6);   // uniform: scalar
-    const uint64_t nwaves = ((uint64_t)gridDim.x * kBlock) >> 6;
-    const uint64_t per = (total + nwaves - 1) / nwaves;
-    uint64_t g = wave_id * per;
-    const uint64_t end = g + per < total ? g + per : total;
-    while (g < end) {
-        const uint32_t j = __builtin_amdgcn_readfirstlane(find_job(row_start, njobs, g));
-        const uint64_t je = row_start[j + 1] < end ? row_start[j + 1] : end;
-        count_rows(jobs[j], ntri, g - row_start[j], je - row_start[j], 0, 1);
-        g = je;
-    }
+    count_rows(a, ntri, 0, a.nrows, wave + uniform(threadIdx.x >> 6), (uint64_t)gridDim.x * kWaves);
 }
 
 /* ------------------------------------------------------------------------- */
@@ -2292,44 +2268,52 @@ hipError_t launch_emit(int dtype, const JobArgs& a, uint32_t lds_bytes, hipStrea
     }
 }
 
-template <typename T>
-hipError_t launch_classify_batch_t(const JobArgs* jobs, const uint64_t* row_start, uint32_t njobs, uint64_t rows,
-                                   uint32_t max_levels, hipStream_t st)
+/* Grid of a batch's front passes: workgroups per job for at most `units` wave
+ * units in one of them, some 16384 in all (the workgroups that a small job does
+ * not need return at once). */
+static dim3 batch_grid(uint64_t units, uint32_t njobs)
 {
-    uint64_t blocks = (rows + kWaves - 1) / kWaves;
-    if (blocks > 65536) blocks = 65536;
-    if (max_levels > 4)
-        hipLaunchKernelGGL((k_classify_batch<T, true>), dim3((uint32_t)blocks), dim3(kBlock), 0, st, jobs, row_start,
-                           njobs);
-    else
-        hipLaunchKernelGGL((k_classify_batch<T, false>), dim3((uint32_t)blocks), dim3(kBlock), 0, st, jobs, row_start,
-                           njobs);
+    const uint64_t want = (units + kWaves - 1) / kWaves, cap = std::max<uint64_t>(64, 16384 / njobs);
+    return dim3((uint32_t)std::max<uint64_t>(1, std::min(want, cap)), 1, njobs);
+}
+
+constexpr uint32_t kMaxGridJobs = 32768;   // of one grid's z
+
+template <typename T>
+hipError_t launch_classify_batch_t(const JobArgs* jobs, uint32_t njobs, uint64_t chunks, uint32_t max_levels, hipStream_t st)
+{
+    for (uint32_t j = 0; j < njobs; j += kMaxGridJobs) {
+        const uint32_t n = std::min(kMaxGridJobs, njobs - j);
+        const dim3 g = batch_grid((chunks + 15) / 16, n);
+        if (max_levels > 4) hipLaunchKernelGGL((k_classify_batch<T, true>), g, dim3(kBlock), 0, st, jobs + j);
+        else hipLaunchKernelGGL((k_classify_batch<T, false>), g, dim3(kBlock), 0, st, jobs + j);
+    }
     return hipGetLastError();
 }
 
-hipError_t launch_classify_batch(int dtype, const JobArgs* jobs, const uint64_t* row_start, uint32_t njobs,
-                                 uint64_t rows, uint32_t max_levels, hipStream_t st)
+hipError_t launch_classify_batch(int dtype, const JobArgs* jobs, uint32_t njobs, uint64_t chunks, uint32_t max_levels,
+                                 hipStream_t st)
 {
     switch (dtype) {
-    case 0: return launch_classify_batch_t<int8_t>(jobs, row_start, njobs, rows, max_levels, st);
-    case 1: return launch_classify_batch_t<int16_t>(jobs, row_start, njobs, rows, max_levels, st);
-    case 2: return launch_classify_batch_t<int32_t>(jobs, row_start, njobs, rows, max_levels, st);
-    case 3: return launch_classify_batch_t<int64_t>(jobs, row_start, njobs, rows, max_levels, st);
-    case 4: return launch_classify_batch_t<uint8_t>(jobs, row_start, njobs, rows, max_levels, st);
-    case 5: return launch_classify_batch_t<uint16_t>(jobs, row_start, njobs, rows, max_levels, st);
-    case 6: return launch_classify_batch_t<uint32_t>(jobs, row_start, njobs, rows, max_levels, st);
-    case 7: return launch_classify_batch_t<uint64_t>(jobs, row_start, njobs, rows, max_levels, st);
-    case 8: return launch_classify_batch_t<float>(jobs, row_start, njobs, rows, max_levels, st);
-    default: return launch_classify_batch_t<double>(jobs, row_start, njobs, rows, max_levels, st);
+    case 0: return launch_classify_batch_t<int8_t>(jobs, njobs, chunks, max_levels, st);
+    case 1: return launch_classify_batch_t<int16_t>(jobs, njobs, chunks, max_levels, st);
+    case 2: return launch_classify_batch_t<int32_t>(jobs, njobs, chunks, max_levels, st);
+    case 3: return launch_classify_batch_t<int64_t>(jobs, njobs, chunks, max_levels, st);
+    case 4: return launch_classify_batch_t<uint8_t>(jobs, njobs, chunks, max_levels, st);
+    case 5: return launch_classify_batch_t<uint16_t>(jobs, njobs, chunks, max_levels, st);
+    case 6: return launch_classify_batch_t<uint32_t>(jobs, njobs, chunks, max_levels, st);
+    case 7: return launch_classify_batch_t<uint64_t>(jobs, njobs, chunks, max_levels, st);
+    case 8: return launch_classify_batch_t<float>(jobs, njobs, chunks, max_levels, st);
+    default: return launch_classify_batch_t<double>(jobs, njobs, chunks, max_levels, st);
     }
 }
 
-hipError_t launch_count_batch(const JobArgs* jobs, const uint64_t* row_start, uint32_t njobs, uint64_t rows,
-                              hipStream_t st)
+hipError_t launch_count_batch(const JobArgs* jobs, uint32_t njobs, uint64_t groups, hipStream_t st)
 {
-    uint64_t blocks = (rows / 4 + kWaves - 1) / kWaves + 1;
-    if (blocks > 16384) blocks = 16384;
-    hipLaunchKernelGGL(k_count_batch, dim3((uint32_t)blocks), dim3(kBlock), 0, st, jobs, row_start, njobs);
+    for (uint32_t j = 0; j < njobs; j += kMaxGridJobs) {
+        const uint32_t n = std::min(kMaxGridJobs, njobs - j);
+        hipLaunchKernelGGL(k_count_batch, batch_grid(groups, n), dim3(kBlock), 0, st, jobs + j);
+    }
     return hipGetLastError();
 }
 
