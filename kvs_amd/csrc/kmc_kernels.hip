@@ -1847,26 +1847,77 @@ __global__ __launch_bounds__(kBlock) void k_scan_mid(uint64_t* partials, uint32_
     }
 }
 
-/* Exclusive prefix of each count array, from the scanned partials. */
+/* Four counts in one load; an array's base is aligned to one count only. */
+struct __attribute__((packed, aligned(4))) Count4 {
+    uint32_t x, y, z, w;
+};
+struct __attribute__((packed, aligned(8))) Prefix2 {
+    uint64_t x, y;
+};
+
+/* Sum over the block's threads (the same in every thread). */
+__device__ __forceinline__ uint64_t block_sum(uint64_t s, uint64_t* sh)
+{
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) s += (uint64_t)__shfl_xor((unsigned long long)s, d);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+    __syncthreads();
+    uint64_t t = 0;
+    for (int w = 0; w < kWaves; ++w) t += sh[w];
+    __syncthreads();
+    return t;
+}
+
+/* Exclusive prefix of each count array.  Where a workgroup's segment starts:
+ * kScanCounts sums all counts before it (few segments: the whole scan is this
+ * one kernel), kScanPartials the segments' sums before it, kScanScanned reads
+ * the scanned sum (so many segments that summing them per workgroup would
+ * cost more than a kernel).  Launches are what a small scan costs: 65536
+ * counts take 15 us in three kernels, 12 in two. */
+enum : int { kScanCounts = 0, kScanPartials = 1, kScanScanned = 2 };
+
+template <int kFrom>
 __global__ __launch_bounds__(kBlock) void k_scan_apply(const uint32_t* counts, uint64_t n, uint32_t nseg,
-                                                       const uint64_t* partials, uint64_t* prefix)
+                                                       const uint64_t* partials, uint64_t* prefix, uint64_t* totals)
 {
     __shared__ uint64_t sh[kWaves];
     const uint32_t arr = blockIdx.x / nseg, seg = blockIdx.x - arr * nseg;
     const uint32_t* src = counts + (uint64_t)arr * n;
     uint64_t* dst = prefix + (uint64_t)arr * n;
-    const uint64_t base = partials[blockIdx.x];
+    uint64_t base = 0;
+    if constexpr (kFrom == kScanCounts) {
+        /* four segments' loads in flight: the sum waits for memory once per four */
+        uint64_t before = 0;
+        for (uint32_t s0 = 0; s0 < seg; s0 += 4) {
+            Count4 v[4][4];
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j)
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i)
+                    v[j][i] = s0 + j < seg ? ((const Count4*)(src + (s0 + j) * kScanTile))[i * kBlock + threadIdx.x] : Count4{};
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j)
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i) before += ((uint64_t)v[j][i].x + v[j][i].y) + ((uint64_t)v[j][i].z + v[j][i].w);
+        }
+        base = block_sum(before, sh);
+    } else if constexpr (kFrom == kScanPartials) {
+        uint64_t before = 0;
+        for (uint32_t i = threadIdx.x; i < seg; i += kBlock) before += partials[(uint64_t)arr * nseg + i];
+        base = block_sum(before, sh);
+    } else {
+        base = partials[blockIdx.x];
+    }
     const uint64_t b = (uint64_t)seg * kScanTile + (uint64_t)threadIdx.x * kScanPer;
     uint32_t vals[kScanPer];
     uint64_t s = 0;
     /* a thread's 16 counts are contiguous: 16-byte loads where they lie
-     * inside the array (the array bases are 16-byte aligned when n is a
-     * multiple of 4) */
-    const bool whole = b + kScanPer <= n && (n & 3u) == 0;
+     * inside the array */
+    const bool whole = b + kScanPer <= n;
     if (whole) {
 #pragma unroll
         for (uint32_t i = 0; i < kScanPer; i += 4) {
-            const uint4 v = *(const uint4*)(src + b + i);
+            const Count4 v = *(const Count4*)(src + b + i);
             vals[i] = v.x;
             vals[i + 1] = v.y;
             vals[i + 2] = v.z;
@@ -1894,15 +1945,17 @@ __global__ __launch_bounds__(kBlock) void k_scan_apply(const uint32_t* counts, u
     uint64_t run = base;
     for (int w = 0; w < wave; ++w) run += sh[w];
     run += incl - s;
+    /* the last segment's last thread ends at the array's total */
+    if (kFrom != kScanScanned && seg == nseg - 1 && threadIdx.x == kBlock - 1) totals[arr] = run + s;
     if (whole) {
 #pragma unroll
         for (uint32_t i = 0; i < kScanPer; i += 2) {
-            ulonglong2 o;
+            Prefix2 o;
             o.x = run;
             run += vals[i];
             o.y = run;
             run += vals[i + 1];
-            *(ulonglong2*)(dst + b + i) = o;
+            *(Prefix2*)(dst + b + i) = o;
         }
     } else {
 #pragma unroll
@@ -2357,13 +2410,27 @@ hipError_t launch_emit_batch(int dtype, int mode, const JobArgs* jobs, const uin
     }
 }
 
+/* Segments up to which a workgroup sums all counts before its own (one CU reads a
+ * segment's 16 KiB in 1.1 us: 2 segments 5.4 us, 16 segments 17-21, in two
+ * kernels 12 and a launch), and up to which it sums the segments' sums. */
+constexpr uint32_t kScanDirect = 8, kScanSummed = 4096;
+
 hipError_t launch_scan(const uint32_t* counts, uint64_t n, uint32_t narr, uint64_t* partials,
                        uint64_t* prefix, uint64_t* totals, hipStream_t st)
 {
     const uint32_t nseg = (uint32_t)((n + kScanTile - 1) / kScanTile);
-    hipLaunchKernelGGL(k_scan_partials, dim3(nseg * narr), dim3(kBlock), 0, st, counts, n, nseg, partials);
-    hipLaunchKernelGGL(k_scan_mid, dim3(1), dim3(kBlock), 0, st, partials, nseg, narr, totals);
-    hipLaunchKernelGGL(k_scan_apply, dim3(nseg * narr), dim3(kBlock), 0, st, counts, n, nseg, partials, prefix);
+    const dim3 g(nseg * narr), b(kBlock);
+    if (nseg <= kScanDirect) {
+        hipLaunchKernelGGL(k_scan_apply<kScanCounts>, g, b, 0, st, counts, n, nseg, partials, prefix, totals);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(k_scan_partials, g, b, 0, st, counts, n, nseg, partials);
+    if (nseg <= kScanSummed) {
+        hipLaunchKernelGGL(k_scan_apply<kScanPartials>, g, b, 0, st, counts, n, nseg, partials, prefix, totals);
+    } else {
+        hipLaunchKernelGGL(k_scan_mid, dim3(1), b, 0, st, partials, nseg, narr, totals);
+        hipLaunchKernelGGL(k_scan_apply<kScanScanned>, g, b, 0, st, counts, n, nseg, partials, prefix, totals);
+    }
     return hipGetLastError();
 }
 
