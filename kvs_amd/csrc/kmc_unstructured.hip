@@ -16,6 +16,7 @@
  */
 #include <hip/hip_runtime.h>
 #include <cmath>
+#include <cstddef>
 #include <cstring>
 #include <vector>
 
@@ -385,6 +386,154 @@ __global__ __launch_bounds__(kBlock) void k_coord_span_final(const CoordSpan* pa
 
 static_assert(kSpanParts % kBlock == 0, "the final merge gives every thread the same number of parts");
 
+/* The ranges as long as order does not matter: the serial scans above are
+ * plain minima and maxima unless a NaN occurs or zeros of both signs tie, and
+ * a NaN or a -0 sets `odd` (the ordered passes then decide). */
+template <typename T>
+struct CellRange {
+    T mn, mx;
+    float cmn[3], cmx[3];
+    uint32_t odd;
+};
+
+template <typename T>
+__device__ __forceinline__ bool is_odd(T) { return false; }
+template <> __device__ __forceinline__ bool is_odd<float>(float v) { return v != v || __float_as_uint(v) == 0x80000000u; }
+template <> __device__ __forceinline__ bool is_odd<double>(double v)
+{
+    return v != v || (unsigned long long)__double_as_longlong(v) == 0x8000000000000000ull;
+}
+
+template <typename T>
+__device__ __forceinline__ void range_merge(CellRange<T>& f, const CellRange<T>& g)
+{
+    f.mn = g.mn < f.mn ? g.mn : f.mn;
+    f.mx = g.mx > f.mx ? g.mx : f.mx;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        f.cmn[k] = g.cmn[k] < f.cmn[k] ? g.cmn[k] : f.cmn[k];
+        f.cmx[k] = g.cmx[k] > f.cmx[k] ? g.cmx[k] : f.cmx[k];
+    }
+    f.odd |= g.odd;
+}
+
+template <typename T>
+__device__ __forceinline__ void block_range(CellRange<T>& r, CellRange<T>* sh)
+{
+    sh[threadIdx.x] = r;
+    for (uint32_t d = kBlock / 2; d > 0; d >>= 1) {
+        __syncthreads();
+        if (threadIdx.x < d) {
+            range_merge(r, sh[threadIdx.x + d]);
+            sh[threadIdx.x] = r;
+        }
+    }
+}
+
+constexpr uint32_t kRangeParts = 2048;
+
+/* k_ucount and both ranges in one pass over the connections: three passes read
+ * them and gathered through them each (3.07 M tetrahedra: coordinate span 47 +
+ * 11 us, value range 25 + 8, count 14; together here 25 + 4). */
+template <typename T, int C, bool SLICE>
+__global__ __launch_bounds__(kBlock) void k_ucount_ranges(UArgs a, CellRange<T>* parts)
+{
+    __shared__ CellRange<T> sh[kBlock];
+    const T* vol = (const T*)a.values;
+    CellRange<T> r;
+    r.mn = r.mx = vol[0];                       // the value scan is seeded with the first value
+    r.odd = is_odd<T>(vol[0]) ? 1u : 0u;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) { r.cmn[k] = INFINITY; r.cmx[k] = -INFINITY; }
+    const uint64_t step = (uint64_t)gridDim.x * kBlock;
+    for (uint64_t cell = (uint64_t)blockIdx.x * kBlock + threadIdx.x; cell < a.ncells; cell += step) {
+        uint64_t li[8];
+        cell_nodes<C>(a, cell, li);
+#pragma unroll
+        for (int i = 0; i < Cell<C>::nodes; ++i) {
+            const T v = vol[li[i]];
+            r.mn = v < r.mn ? v : r.mn;
+            r.mx = v > r.mx ? v : r.mx;
+            bool odd = is_odd<T>(v);
+            const float* p = a.coords + 3 * li[i];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const float c = p[k];
+                r.cmn[k] = c < r.cmn[k] ? c : r.cmn[k];
+                r.cmx[k] = c > r.cmx[k] ? c : r.cmx[k];
+                odd = odd || is_odd<float>(c);
+            }
+            r.odd |= odd ? 1u : 0u;
+        }
+        const uint32_t ti = cell_case<T, C, SLICE>(a, li);
+        const bool skip = ti == 0 || ti == (uint32_t)Cell<C>::all_ones;
+        a.tidx[cell] = (uint8_t)ti;
+        a.counts[cell] = skip ? 0u : (uint32_t)(Cell<C>::tri(ti) >> 60);
+    }
+    block_range(r, sh);
+    if (threadIdx.x == 0) parts[blockIdx.x] = r;
+}
+
+/* What the host reads back. */
+struct Ranges {
+    double mm[2];
+    float cc[6];
+    uint32_t odd, pad;
+};
+
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_range_final(const CellRange<T>* parts, uint32_t n, Ranges* out)
+{
+    __shared__ CellRange<T> sh[kBlock];
+    CellRange<T> r = parts[threadIdx.x < n ? threadIdx.x : 0u];
+#pragma unroll 4
+    for (uint32_t i = threadIdx.x + kBlock; i < n; i += kBlock) range_merge(r, parts[i]);
+    block_range(r, sh);
+    if (threadIdx.x == 0) {
+        out->mm[0] = (double)r.mn;
+        out->mm[1] = (double)r.mx;
+        for (int k = 0; k < 3; ++k) { out->cc[k] = r.cmn[k]; out->cc[3 + k] = r.cmx[k]; }
+        out->odd = r.odd;
+    }
+}
+
+template <typename T, int C, bool SLICE>
+hipError_t launch_ranges_t(const UArgs& a, void* parts, Ranges* out, hipStream_t st)
+{
+    const uint32_t n = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((a.ncells + kBlock - 1) / kBlock, kRangeParts));
+    hipLaunchKernelGGL((k_ucount_ranges<T, C, SLICE>), dim3(n), dim3(kBlock), 0, st, a, (CellRange<T>*)parts);
+    hipLaunchKernelGGL((k_range_final<T>), dim3(1), dim3(kBlock), 0, st, (const CellRange<T>*)parts, n, out);
+    return hipGetLastError();
+}
+
+template <typename T, bool SLICE>
+hipError_t launch_ranges_c(int cell, const UArgs& a, void* parts, Ranges* out, hipStream_t st)
+{
+    switch (cell) {
+    case kTet: return launch_ranges_t<T, kTet, SLICE>(a, parts, out, st);
+    case kHex: return launch_ranges_t<T, kHex, SLICE>(a, parts, out, st);
+    case kPyr: return launch_ranges_t<T, kPyr, SLICE>(a, parts, out, st);
+    default: return launch_ranges_t<T, kPrism, SLICE>(a, parts, out, st);
+    }
+}
+
+template <bool SLICE>
+hipError_t launch_ranges(int dtype, int cell, const UArgs& a, void* parts, Ranges* out, hipStream_t st)
+{
+    switch (dtype) {
+    case 0: return launch_ranges_c<int8_t, SLICE>(cell, a, parts, out, st);
+    case 1: return launch_ranges_c<int16_t, SLICE>(cell, a, parts, out, st);
+    case 2: return launch_ranges_c<int32_t, SLICE>(cell, a, parts, out, st);
+    case 3: return launch_ranges_c<int64_t, SLICE>(cell, a, parts, out, st);
+    case 4: return launch_ranges_c<uint8_t, SLICE>(cell, a, parts, out, st);
+    case 5: return launch_ranges_c<uint16_t, SLICE>(cell, a, parts, out, st);
+    case 6: return launch_ranges_c<uint32_t, SLICE>(cell, a, parts, out, st);
+    case 7: return launch_ranges_c<uint64_t, SLICE>(cell, a, parts, out, st);
+    case 8: return launch_ranges_c<float, SLICE>(cell, a, parts, out, st);
+    default: return launch_ranges_c<double, SLICE>(cell, a, parts, out, st);
+    }
+}
+
 template <typename T, int C, bool SLICE>
 hipError_t launch_cells_t(const UArgs& a, bool emit, hipStream_t st)
 {
@@ -507,27 +656,31 @@ kmc_status run_cells(const kmc_unstructured_volume* v, bool slice, double iso, i
         for (int k = 0; k < 4; ++k) a.plane[k] = coef[k];
     ReadPart parts[2];
     int nparts_back = 0;
-    uint8_t ranges[40];
-    if (need_values || need_coords) {
-        uint8_t* scratch = (uint8_t*)alloc(minmax_scratch_bytes() + 64 + kSpanParts * sizeof(CoordSpan));
-        if (!scratch) return finish(KMC_ERR_OUT_OF_MEMORY);
-        double* dmm = (double*)(scratch + minmax_scratch_bytes());
-        float* dcc = (float*)(scratch + minmax_scratch_bytes() + 16);
-        CoordSpan* spans = (CoordSpan*)(scratch + minmax_scratch_bytes() + 64);
-        bool ok = true;
-        if (need_values) ok = launch_minmax_gather(v->type, dvals, dconn, nconn, scratch, dmm, st) == hipSuccess;
-        if (ok && need_coords) {
+    Ranges ranges;
+    ranges.odd = 0;
+    /* both ranges together come with the count pass; else, or when that meets
+     * a value whose order matters, from the ordered passes */
+    const bool fused = need_values && need_coords && count_now;
+    uint8_t* scratch = nullptr;
+    auto ordered_ranges = [&]() -> kmc_status {
+        if (!scratch) scratch = (uint8_t*)alloc(minmax_scratch_bytes() + sizeof(Ranges) + kSpanParts * sizeof(CoordSpan));
+        if (!scratch) return KMC_ERR_OUT_OF_MEMORY;
+        Ranges* dr = (Ranges*)(scratch + minmax_scratch_bytes());
+        CoordSpan* spans = (CoordSpan*)(dr + 1);
+        if (need_values && launch_minmax_gather(v->type, dvals, dconn, nconn, scratch, dr->mm, st) != hipSuccess)
+            return KMC_ERR_DEVICE;
+        if (need_coords) {
             hipLaunchKernelGGL(k_coord_span_partial, dim3(kSpanParts), dim3(kBlock), 0, st, dcoords, dconn, nconn,
                                spans);
-            hipLaunchKernelGGL(k_coord_span_final, dim3(1), dim3(kBlock), 0, st, spans, dcc);
-            ok = hipGetLastError() == hipSuccess;
+            hipLaunchKernelGGL(k_coord_span_final, dim3(1), dim3(kBlock), 0, st, spans, dr->cc);
         }
-        if (!ok) {
-            (void)hipGetLastError();
-            return finish(KMC_ERR_DEVICE);
-        }
-        /* the min/max (16 bytes) and the coordinate span (24) lie together */
-        parts[nparts_back++] = ReadPart{ ranges, dmm, sizeof(ranges) };
+        if (hipGetLastError() != hipSuccess) return KMC_ERR_DEVICE;
+        parts[nparts_back++] = ReadPart{ &ranges, dr, offsetof(Ranges, odd) };
+        return KMC_OK;
+    };
+    if ((need_values || need_coords) && !fused) {
+        s = ordered_ranges();
+        if (s != KMC_OK) return finish(s);
     }
     const uint32_t nparts = count_now ? scan_partials_needed(ncells, 1) : 0;
     uint64_t* prefix = nullptr;
@@ -538,10 +691,18 @@ kmc_status run_cells(const kmc_unstructured_volume* v, bool slice, double iso, i
         a.tidx = (uint8_t*)alloc(ncells);
         prefix = (uint64_t*)alloc(ncells * 8);
         aux = (uint64_t*)alloc((nparts + 1) * 8);
-        if (!a.counts || !a.tidx || !prefix || !aux) return finish(KMC_ERR_OUT_OF_MEMORY);
+        uint8_t* rp = fused ? (uint8_t*)alloc(sizeof(Ranges) + kRangeParts * sizeof(CellRange<double>)) : nullptr;
+        if (!a.counts || !a.tidx || !prefix || !aux || (fused && !rp)) return finish(KMC_ERR_OUT_OF_MEMORY);
         a.prefix = prefix;
-        const hipError_t e1 = slice ? launch_cells<true>(v->type, kind, a, false, st)
-                                    : launch_cells<false>(v->type, kind, a, false, st);
+        hipError_t e1;
+        if (fused) {
+            Ranges* dr = (Ranges*)rp;
+            e1 = slice ? launch_ranges<true>(v->type, kind, a, dr + 1, dr, st)
+                       : launch_ranges<false>(v->type, kind, a, dr + 1, dr, st);
+            parts[nparts_back++] = ReadPart{ &ranges, dr, sizeof(Ranges) };
+        } else {
+            e1 = slice ? launch_cells<true>(v->type, kind, a, false, st) : launch_cells<false>(v->type, kind, a, false, st);
+        }
         if (e1 != hipSuccess || launch_scan(a.counts, ncells, 1, aux, prefix, aux + nparts, st) != hipSuccess) {
             (void)hipGetLastError();
             return finish(KMC_ERR_DEVICE);
@@ -552,17 +713,21 @@ kmc_status run_cells(const kmc_unstructured_volume* v, bool slice, double iso, i
         (void)hipGetLastError();
         return finish(KMC_ERR_DEVICE);
     }
+    if (fused && ranges.odd) {
+        nparts_back = 0;
+        s = ordered_ranges();
+        if (s != KMC_OK) return finish(s);
+        if (read_back_parts(parts, nparts_back, st) != hipSuccess) {
+            (void)hipGetLastError();
+            return finish(KMC_ERR_DEVICE);
+        }
+    }
     if (need_values) {
-        double hmm[2];
-        std::memcpy(hmm, ranges, 16);
-        mn = hmm[0];
-        mx = hmm[1];
+        mn = ranges.mm[0];
+        mx = ranges.mm[1];
     }
-    if (need_coords) {
-        float hcc[6];
-        std::memcpy(hcc, ranges + 16, 24);
-        for (int k = 0; k < 3; ++k) { minc[k] = hcc[k]; maxc[k] = hcc[3 + k]; }
-    }
+    if (need_coords)
+        for (int k = 0; k < 3; ++k) { minc[k] = ranges.cc[k]; maxc[k] = ranges.cc[3 + k]; }
 
     /* the surface as the mapper leaves it */
     init_surface(out, slice ? 0.0 : iso, normal_type, dup, mn, mx, minc, maxc);
