@@ -1993,7 +1993,8 @@ template <> __device__ __forceinline__ bool is_nan_val<double>(double v) { retur
 
 /* Running extreme with the reference's tie rule: on equal values the earlier
  * index wins (only observable for float +0/-0). */
-constexpr uint32_t kMinMaxParts = 2048;   // partial results of the first pass
+constexpr uint32_t kMinMaxParts = 2048;   // at most so many partial results of the first pass
+static_assert(kMinMaxParts % kBlock == 0, "the final merge gives every thread the same number of parts");
 
 template <typename T>
 struct Extreme {
@@ -2098,11 +2099,21 @@ __global__ __launch_bounds__(kBlock) void k_minmax_final(const T* vol, const Ext
 {
     Extreme<T> e;
     e.mn = T(0); e.mx = T(0); e.imn = 0; e.imx = 0; e.valid = 0;
-    for (uint32_t i = threadIdx.x; i < nparts; i += kBlock) merge_extreme(e, parts[i]);
+    const T first = vol[0];
+    /* all parts of a thread in flight before the first is merged */
+    constexpr uint32_t kPer = kMinMaxParts / kBlock;
+    Extreme<T> p[kPer];
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) {
+        const uint32_t i = threadIdx.x + k * kBlock;
+        p[k] = parts[i < nparts ? i : 0u];
+        if (i >= nparts) p[k].valid = 0;
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) merge_extreme(e, p[k]);
     const Extreme<T> r = block_extreme(e);
     if (threadIdx.x == 0) {
         Extreme<T> f = r;
-        const T first = vol[0];
         if (is_nan_val<T>(first) || !f.valid) { f.mn = first; f.mx = first; }
         out[0] = (double)f.mn;
         out[1] = (double)f.mx;
@@ -2465,7 +2476,10 @@ uint32_t scan_partials_needed(uint64_t n, uint32_t narr)
 template <typename T>
 hipError_t launch_minmax_t(const void* vol, uint64_t n, void* scratch, double* out, hipStream_t st)
 {
-    const uint32_t nparts = kMinMaxParts;
+    /* a small volume in workgroups of one load a thread: 64^3 floats are 256, and
+     * the final merge then reads one part a thread, not eight */
+    const uint64_t want = (n + (uint64_t)kBlock * (16 / sizeof(T)) - 1) / ((uint64_t)kBlock * (16 / sizeof(T)));
+    const uint32_t nparts = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(want, kMinMaxParts));
     Extreme<T>* parts = (Extreme<T>*)scratch;
     hipLaunchKernelGGL((k_minmax_partial<T>), dim3(nparts), dim3(kBlock), 0, st, (const T*)vol, n, parts);
     hipLaunchKernelGGL((k_minmax_final<T>), dim3(1), dim3(kBlock), 0, st, (const T*)vol, parts, nparts, out);
