@@ -266,38 +266,6 @@ void host_pinned_free(void* p)
     if (it != g_pin_size.end()) g_pin_free.emplace(it->second, p);
 }
 
-/* n bytes (totals, sizes, min/max) from device memory into host memory,
- * through a pinned staging block, then a wait for the stream: a copy into
- * pageable memory is staged by the runtime at a higher latency, and these
- * copies sit between a pass's front and its emit. */
-hipError_t read_back_parts(const ReadPart* parts, int n, hipStream_t st)
-{
-    size_t total = 0;
-    for (int i = 0; i < n; ++i) total += (parts[i].bytes + 15) & ~size_t(15);
-    uint8_t* pin = (uint8_t*)host_pinned_alloc(total);
-    if (!pin) return hipErrorOutOfMemory;
-    hipError_t e = hipSuccess;
-    for (int i = 0, off = 0; i < n && e == hipSuccess; off += (int)((parts[i].bytes + 15) & ~size_t(15)), ++i)
-        e = hipMemcpyAsync(pin + off, parts[i].dev, parts[i].bytes, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e == hipSuccess)
-        for (int i = 0, off = 0; i < n; off += (int)((parts[i].bytes + 15) & ~size_t(15)), ++i)
-            std::memcpy(parts[i].host, pin + off, parts[i].bytes);
-    host_pinned_free(pin);
-    return e;
-}
-
-hipError_t read_back(void* host, const void* dev, size_t n, hipStream_t st)
-{
-    void* pin = host_pinned_alloc(n);
-    if (!pin) return hipErrorOutOfMemory;
-    hipError_t e = hipMemcpyAsync(pin, dev, n, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e == hipSuccess) std::memcpy(host, pin, n);
-    host_pinned_free(pin);
-    return e;
-}
-
 /* ------------------------------------------------------------------------- */
 /* surface ownership                                                           */
 /* ------------------------------------------------------------------------- */
@@ -462,18 +430,19 @@ kmc_status device_values(const kmc_volume* v, hipStream_t st, const void** dvals
 kmc_status min_max_on_device(const kmc_volume* v, const void* dvals, hipStream_t st, double* mn, double* mx)
 {
     const uint64_t n = (uint64_t)v->resolution[0] * v->resolution[1] * v->resolution[2];
-    void* scratch = device_alloc(minmax_scratch_bytes() + 16);
+    void* scratch = device_alloc(minmax_scratch_bytes());
     if (!scratch) return KMC_ERR_OUT_OF_MEMORY;
-    double* dout = (double*)((char*)scratch + minmax_scratch_bytes());
     kmc_status s = KMC_OK;
-    double host[2] = {0, 0};
-    if (launch_minmax(v->type, dvals, n, scratch, dout, st) != hipSuccess ||
-        read_back(host, dout, sizeof(host), st) != hipSuccess) {
+    *mn = *mx = 0;
+    HostResult<double> range(st, 2);
+    if (!range.get() || launch_minmax(v->type, dvals, n, scratch, range.get(), st) != hipSuccess ||
+        range.wait() != hipSuccess) {
         s = KMC_ERR_DEVICE;
+    } else {
+        *mn = range[0];
+        *mx = range[1];
     }
     device_free(scratch);
-    *mn = host[0];
-    *mx = host[1];
     return s;
 }
 
@@ -732,17 +701,17 @@ kmc_status run_pass(const kmc_volume* v, const void* dvals, const double* iso, u
     const size_t prefix_bytes = (size_t)narr * n * sizeof(uint64_t);
     uint32_t* counts = (uint32_t*)device_alloc(counts_bytes);
     uint64_t* prefix = (uint64_t*)device_alloc(prefix_bytes);
-    uint64_t* aux = (uint64_t*)device_alloc((size_t)(nparts + narr) * sizeof(uint64_t));
+    uint64_t* partials = (uint64_t*)device_alloc((size_t)nparts * sizeof(uint64_t));
     const size_t chunks = (size_t)nlev * a.nz * a.ny * a.NC;
     uint64_t* bitvol = (uint64_t*)device_alloc(chunks * sizeof(uint64_t) + kBitSlack);
     uint32_t* cpre = flat ? (uint32_t*)device_alloc(2 * chunks * sizeof(uint32_t)) : nullptr;
     uint64_t* act = (flat && a.vnormal) ? (uint64_t*)device_alloc(chunks * sizeof(uint64_t) + kBitSlack) : nullptr;
     void* recs = nullptr;
     auto cleanup = [&]() {
-        device_free(counts); device_free(prefix); device_free(aux); device_free(bitvol); device_free(cpre);
+        device_free(counts); device_free(prefix); device_free(partials); device_free(bitvol); device_free(cpre);
         device_free(act); device_free(recs);
     };
-    if (!counts || !prefix || !aux || !bitvol || (flat && !cpre) || (flat && a.vnormal && !act)) {
+    if (!counts || !prefix || !partials || !bitvol || (flat && !cpre) || (flat && a.vnormal && !act)) {
         cleanup();
         return KMC_ERR_OUT_OF_MEMORY;
     }
@@ -752,22 +721,20 @@ kmc_status run_pass(const kmc_volume* v, const void* dvals, const double* iso, u
         a.tpc = cpre + chunks;
         a.act = act;
     }
-    uint64_t* partials = aux;
-    uint64_t* totals = aux + nparts;
     a.counts = counts;
     a.prefix = prefix;
 
+    HostResult<uint64_t> tot(st, narr);
     PassTimer timer(st);
     timer.mark(0);
-    const bool front_ok = launch_classify(v->type, a, st) == hipSuccess && timer.mark(1) &&
+    const bool front_ok = tot.get() && launch_classify(v->type, a, st) == hipSuccess && timer.mark(1) &&
                           launch_count(a, st) == hipSuccess && timer.mark(2) &&
-                          launch_scan(counts, n, narr, partials, prefix, totals, st) == hipSuccess && timer.mark(3);
+                          launch_scan(counts, n, narr, partials, prefix, tot.get(), st) == hipSuccess && timer.mark(3);
     if (!front_ok) {
         cleanup();
         return KMC_ERR_DEVICE;
     }
-    std::vector<uint64_t> tot(narr, 0);
-    if (read_back(tot.data(), totals, narr * sizeof(uint64_t), st) != hipSuccess) {
+    if (tot.wait() != hipSuccess) {
         cleanup();
         return KMC_ERR_DEVICE;
     }

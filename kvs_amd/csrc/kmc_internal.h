@@ -21,16 +21,43 @@ void* host_pinned_alloc(size_t bytes);
 void host_pinned_free(void* p);
 void* host_block_alloc(size_t bytes);
 void host_block_free(void* p);
-hipError_t read_back(void* host, const void* dev, size_t n, hipStream_t st);
 /* Pageable host memory to device memory (pinned staging for large copies). */
 hipError_t upload_host(void* dst, const void* src, size_t bytes, hipStream_t st);
-/* Several device ranges into host memory with one wait for the stream. */
-struct ReadPart {
-    void* host;
-    const void* dev;
-    size_t bytes;
+/* A small result (totals, sizes, min/max) that kernels on a stream store straight
+ * into pinned host memory: a copy from device memory is one more operation on the
+ * stream between a pass's front and its emit (256^3 float with duplication: 87.1
+ * us a call with it, 85.3 without).  The block goes back to the pool only after
+ * the stream has finished with it. */
+template <typename T>
+class HostResult {
+public:
+    explicit HostResult(hipStream_t st, size_t n = 1) : st_(st), p_((T*)host_pinned_alloc(n * sizeof(T))) {}
+    ~HostResult()
+    {
+        if (p_ && !waited_) (void)hipStreamSynchronize(st_);
+        host_pinned_free(p_);
+    }
+    HostResult(const HostResult&) = delete;
+    HostResult& operator=(const HostResult&) = delete;
+    /* For kernels to write; null if the block could not be allocated. */
+    T* get()
+    {
+        waited_ = false;
+        return p_;
+    }
+    /* Wait for the stream; then [] reads what the kernels wrote. */
+    hipError_t wait()
+    {
+        waited_ = true;
+        return hipStreamSynchronize(st_);
+    }
+    const T& operator[](size_t i) const { return p_[i]; }
+
+private:
+    hipStream_t st_;
+    T* p_;
+    bool waited_ = true;   // nothing launched yet
 };
-hipError_t read_back_parts(const ReadPart* parts, int n, hipStream_t st);
 
 /* Arrays owned by a kmc_surface (its `internal` handle). */
 struct SurfaceStorage {

@@ -77,19 +77,19 @@ kmc_status slice_by_thresholds(const kmc_volume* v, JobArgs& a, hipStream_t st, 
     int32_t* thr = (int32_t*)alloc(rows * 4);
     uint32_t* counts = (uint32_t*)alloc((ncr ? ncr : 1) * 4);
     uint64_t* prefix = (uint64_t*)alloc((ncr ? ncr : 1) * 8);
-    uint64_t* aux = (uint64_t*)alloc((nparts + 1) * 8);
+    uint64_t* partials = (uint64_t*)alloc(nparts * 8);
     uint8_t* dtable = (uint8_t*)alloc(3 * (size_t)res);
-    if (!thr || !counts || !prefix || !aux || !dtable) return KMC_ERR_OUT_OF_MEMORY;
+    if (!thr || !counts || !prefix || !partials || !dtable) return KMC_ERR_OUT_OF_MEMORY;
     a.ctable = dtable;
-    uint64_t nt = 0;
-    if (hipMemcpyAsync(dtable, table, 3 * (size_t)res, hipMemcpyHostToDevice, st) != hipSuccess ||
+    HostResult<uint64_t> total(st);
+    if (hipMemcpyAsync(dtable, table, 3 * (size_t)res, hipMemcpyHostToDevice, st) != hipSuccess || !total.get() ||
         (ncr && (launch_slice_runs_front(a, thr, counts, st) != hipSuccess ||
-                 launch_scan(counts, ncr, 1, aux, prefix, aux + nparts, st) != hipSuccess ||
-                 read_back(&nt, aux + nparts, 8, st) != hipSuccess)) ||
-        hipStreamSynchronize(st) != hipSuccess) {
+                 launch_scan(counts, ncr, 1, partials, prefix, total.get(), st) != hipSuccess)) ||
+        total.wait() != hipSuccess) {
         (void)hipGetLastError();
         return KMC_ERR_DEVICE;
     }
+    const uint64_t nt = ncr ? total[0] : 0;
     init_surface(out, 0.0, KMC_POLYGON_NORMAL, 1, mn, mx, minc, maxc);
     out->color_type = 0;   // VertexColor
     SurfaceStorage* store = new SurfaceStorage();
@@ -194,11 +194,11 @@ kmc_status slice_plane_impl(const kmc_volume* v, const float coef[4], const uint
     const uint32_t nparts = scan_partials_needed(R, 2);
     uint32_t* counts = (uint32_t*)alloc(2 * R * 4);
     uint64_t* prefix = (uint64_t*)alloc(2 * R * 8);
-    uint64_t* aux = (uint64_t*)alloc((nparts + 2) * 8);
+    uint64_t* partials = (uint64_t*)alloc(nparts * 8);
     a.bitvol = (uint64_t*)alloc(C * 8 + kBitSlack);
     a.vpc = (uint32_t*)alloc(2 * C * 4);
     uint8_t* dtable = (uint8_t*)alloc(3 * (size_t)res);
-    if (!counts || !prefix || !aux || !a.bitvol || !a.vpc || !dtable) return finish(KMC_ERR_OUT_OF_MEMORY);
+    if (!counts || !prefix || !partials || !a.bitvol || !a.vpc || !dtable) return finish(KMC_ERR_OUT_OF_MEMORY);
     a.tpc = a.vpc + C;
     a.counts = counts;
     a.prefix = prefix;
@@ -206,12 +206,9 @@ kmc_status slice_plane_impl(const kmc_volume* v, const float coef[4], const uint
     if (hipMemcpyAsync(dtable, table, 3 * (size_t)res, hipMemcpyHostToDevice, st) != hipSuccess)
         return finish(KMC_ERR_DEVICE);
 
-    uint64_t* partials = aux;
-    uint64_t* totals = aux + nparts;
-    uint64_t tot[2] = { 0, 0 };
-    if (launch_classify_plane(a, st) != hipSuccess || launch_count(a, st) != hipSuccess ||
-        launch_scan(counts, R, 2, partials, prefix, totals, st) != hipSuccess ||
-        read_back(tot, totals, sizeof(tot), st) != hipSuccess) {
+    HostResult<uint64_t> tot(st, 2);
+    if (!tot.get() || launch_classify_plane(a, st) != hipSuccess || launch_count(a, st) != hipSuccess ||
+        launch_scan(counts, R, 2, partials, prefix, tot.get(), st) != hipSuccess || tot.wait() != hipSuccess) {
         (void)hipGetLastError();
         return finish(KMC_ERR_DEVICE);
     }

@@ -16,7 +16,6 @@
  */
 #include <hip/hip_runtime.h>
 #include <cmath>
-#include <cstddef>
 #include <cstring>
 #include <vector>
 
@@ -654,29 +653,28 @@ kmc_status run_cells(const kmc_unstructured_volume* v, bool slice, double iso, i
     a.iso = iso;
     if (slice)
         for (int k = 0; k < 4; ++k) a.plane[k] = coef[k];
-    ReadPart parts[2];
-    int nparts_back = 0;
-    Ranges ranges;
-    ranges.odd = 0;
+    struct Found {
+        Ranges r;
+        uint64_t nt;
+    };
+    HostResult<Found> found(st);
+    Found* const res_dev = need_values || need_coords || count_now ? found.get() : nullptr;
+    if (!res_dev && (need_values || need_coords || count_now)) return finish(KMC_ERR_OUT_OF_MEMORY);
     /* both ranges together come with the count pass; else, or when that meets
      * a value whose order matters, from the ordered passes */
     const bool fused = need_values && need_coords && count_now;
-    uint8_t* scratch = nullptr;
     auto ordered_ranges = [&]() -> kmc_status {
-        if (!scratch) scratch = (uint8_t*)alloc(minmax_scratch_bytes() + sizeof(Ranges) + kSpanParts * sizeof(CoordSpan));
+        uint8_t* scratch = (uint8_t*)alloc(minmax_scratch_bytes() + kSpanParts * sizeof(CoordSpan));
         if (!scratch) return KMC_ERR_OUT_OF_MEMORY;
-        Ranges* dr = (Ranges*)(scratch + minmax_scratch_bytes());
-        CoordSpan* spans = (CoordSpan*)(dr + 1);
-        if (need_values && launch_minmax_gather(v->type, dvals, dconn, nconn, scratch, dr->mm, st) != hipSuccess)
+        CoordSpan* spans = (CoordSpan*)(scratch + minmax_scratch_bytes());
+        if (need_values && launch_minmax_gather(v->type, dvals, dconn, nconn, scratch, res_dev->r.mm, st) != hipSuccess)
             return KMC_ERR_DEVICE;
         if (need_coords) {
             hipLaunchKernelGGL(k_coord_span_partial, dim3(kSpanParts), dim3(kBlock), 0, st, dcoords, dconn, nconn,
                                spans);
-            hipLaunchKernelGGL(k_coord_span_final, dim3(1), dim3(kBlock), 0, st, spans, dr->cc);
+            hipLaunchKernelGGL(k_coord_span_final, dim3(1), dim3(kBlock), 0, st, spans, res_dev->r.cc);
         }
-        if (hipGetLastError() != hipSuccess) return KMC_ERR_DEVICE;
-        parts[nparts_back++] = ReadPart{ &ranges, dr, offsetof(Ranges, odd) };
-        return KMC_OK;
+        return hipGetLastError() == hipSuccess ? KMC_OK : KMC_ERR_DEVICE;
     };
     if ((need_values || need_coords) && !fused) {
         s = ordered_ranges();
@@ -684,50 +682,45 @@ kmc_status run_cells(const kmc_unstructured_volume* v, bool slice, double iso, i
     }
     const uint32_t nparts = count_now ? scan_partials_needed(ncells, 1) : 0;
     uint64_t* prefix = nullptr;
-    uint64_t* aux = nullptr;
-    uint64_t nt = 0;
     if (count_now) {
         a.counts = (uint32_t*)alloc(ncells * 4);
         a.tidx = (uint8_t*)alloc(ncells);
         prefix = (uint64_t*)alloc(ncells * 8);
-        aux = (uint64_t*)alloc((nparts + 1) * 8);
-        uint8_t* rp = fused ? (uint8_t*)alloc(sizeof(Ranges) + kRangeParts * sizeof(CellRange<double>)) : nullptr;
-        if (!a.counts || !a.tidx || !prefix || !aux || (fused && !rp)) return finish(KMC_ERR_OUT_OF_MEMORY);
+        uint64_t* partials = (uint64_t*)alloc(nparts * 8);
+        void* rp = fused ? alloc(kRangeParts * sizeof(CellRange<double>)) : nullptr;
+        if (!a.counts || !a.tidx || !prefix || !partials || (fused && !rp)) return finish(KMC_ERR_OUT_OF_MEMORY);
         a.prefix = prefix;
         hipError_t e1;
         if (fused) {
-            Ranges* dr = (Ranges*)rp;
-            e1 = slice ? launch_ranges<true>(v->type, kind, a, dr + 1, dr, st)
-                       : launch_ranges<false>(v->type, kind, a, dr + 1, dr, st);
-            parts[nparts_back++] = ReadPart{ &ranges, dr, sizeof(Ranges) };
+            e1 = slice ? launch_ranges<true>(v->type, kind, a, rp, &res_dev->r, st)
+                       : launch_ranges<false>(v->type, kind, a, rp, &res_dev->r, st);
         } else {
             e1 = slice ? launch_cells<true>(v->type, kind, a, false, st) : launch_cells<false>(v->type, kind, a, false, st);
         }
-        if (e1 != hipSuccess || launch_scan(a.counts, ncells, 1, aux, prefix, aux + nparts, st) != hipSuccess) {
+        if (e1 != hipSuccess || launch_scan(a.counts, ncells, 1, partials, prefix, &res_dev->nt, st) != hipSuccess) {
             (void)hipGetLastError();
             return finish(KMC_ERR_DEVICE);
         }
-        parts[nparts_back++] = ReadPart{ &nt, aux + nparts, 8 };
     }
-    if (nparts_back && read_back_parts(parts, nparts_back, st) != hipSuccess) {
+    if (res_dev && found.wait() != hipSuccess) {
         (void)hipGetLastError();
         return finish(KMC_ERR_DEVICE);
     }
-    if (fused && ranges.odd) {
-        nparts_back = 0;
+    const uint64_t nt = count_now ? found[0].nt : 0;
+    if (fused && found[0].r.odd) {
         s = ordered_ranges();
         if (s != KMC_OK) return finish(s);
-        if (read_back_parts(parts, nparts_back, st) != hipSuccess) {
+        if (found.wait() != hipSuccess) {
             (void)hipGetLastError();
             return finish(KMC_ERR_DEVICE);
         }
     }
     if (need_values) {
-        mn = ranges.mm[0];
-        mx = ranges.mm[1];
+        mn = found[0].r.mm[0];
+        mx = found[0].r.mm[1];
     }
     if (need_coords)
-        for (int k = 0; k < 3; ++k) { minc[k] = ranges.cc[k]; maxc[k] = ranges.cc[3 + k]; }
+        for (int k = 0; k < 3; ++k) { minc[k] = found[0].r.cc[k]; maxc[k] = found[0].r.cc[3 + k]; }
 
     /* the surface as the mapper leaves it */
     init_surface(out, slice ? 0.0 : iso, normal_type, dup, mn, mx, minc, maxc);
