@@ -183,12 +183,13 @@ __device__ __forceinline__ uint32_t around_nibbles(uint32_t axis)
  * read straight from the bit volume `lev` (coalesced across the lanes of a
  * row, neighbours from L1/L2).  x/y/z: crossing edges owned by the row's
  * nodes; act: active cells of cell row (y, z-1); k0/k3/k4/k7: the masks of
- * the cells' four node rows (bit i of kq is corner q of cell x = 64c + i; the
- * x+1 corners 1, 2, 5, 6 are the next bits of the same masks); next: bit 0 of
+ * the cells' four node rows (bit i of kq is corner q of cell x = 64c + i),
+ * k1/k2/k5/k6: the x+1 corners, the next bits of the same masks; next: bit 0 of
  * the next chunk's word of those four rows (corners 1, 2, 5, 6 of cell 63). */
 struct RowChunk {
     uint64_t x, y, z, act;
     uint64_t k0, k3, k4, k7;
+    uint64_t k1, k2, k5, k6;
     uint32_t next;
 };
 
@@ -230,6 +231,10 @@ __device__ __forceinline__ void row_chunk(const JobArgs& a, const uint64_t* lev,
     o.k3 = q;
     o.k4 = c4;
     o.k7 = c7;
+    o.k1 = c1;
+    o.k2 = c2;
+    o.k5 = c5;
+    o.k6 = c6;
     o.next = (uint32_t)(p1 & 1ull) | (uint32_t)(q1 & 1ull) << 1 | (uint32_t)(b1 & 1ull) << 2 |
              (uint32_t)(u1 & 1ull) << 3;
 }

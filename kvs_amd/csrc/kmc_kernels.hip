@@ -1120,13 +1120,43 @@ __device__ __forceinline__ uint32_t group_excl_scan(uint32_t x, uint32_t cl, uin
     return inc - x;
 }
 
+/* Triangles of a chunk's cells.  The table cuts each loop of n crossed edges into
+ * n - 2 triangles, so a cell of E crossed edges and L loops has E - 2 L.  The
+ * edges are twelve popcounts; more than one loop takes a face with all four
+ * edges crossed or two opposite corners that differ from all their neighbours,
+ * and only those cells are looked up: fewer[] holds 2 (L - 1).  A lookup per
+ * active cell ran each wave as long as its fullest chunk took (512^3: 43 us, so
+ * 31.6; 256^3 7.9 and 5.5; 1024^3 at three levels, mostly empty chunks, 432 and
+ * 413; 14 volumes of up to 256^3 in a batch 42 and 34). */
+__device__ __forceinline__ uint32_t chunk_triangles(const RowChunk& o, const uint8_t* fewer)
+{
+    const uint64_t m = o.act;
+    const uint64_t x0 = (o.k0 ^ o.k1) & m, x1 = (o.k3 ^ o.k2) & m, x2 = (o.k4 ^ o.k5) & m, x3 = (o.k7 ^ o.k6) & m;
+    const uint64_t y0 = (o.k0 ^ o.k3) & m, y1 = (o.k1 ^ o.k2) & m, y2 = (o.k4 ^ o.k7) & m, y3 = (o.k5 ^ o.k6) & m;
+    const uint64_t z0 = (o.k0 ^ o.k4) & m, z1 = (o.k1 ^ o.k5) & m, z2 = (o.k3 ^ o.k7) & m, z3 = (o.k2 ^ o.k6) & m;
+    int n = __popcll(x0) + __popcll(x1) + __popcll(x2) + __popcll(x3);
+    n += __popcll(y0) + __popcll(y1) + __popcll(y2) + __popcll(y3);
+    n += __popcll(z0) + __popcll(z1) + __popcll(z2) + __popcll(z3);
+    n -= 2 * __popcll(m);
+    /* three crossed edges of a face: the fourth is crossed too */
+    uint64_t w = (x0 & x1 & y0) | (x2 & x3 & y2) | (x0 & x2 & z0) | (x1 & x3 & z2) | (y0 & y2 & z0) | (y1 & y3 & z1);
+    w |= ((x0 & y0 & z0) & (x3 & y3 & z3)) | ((x0 & y1 & z1) & (x3 & y2 & z2));
+    w |= ((x1 & y1 & z3) & (x2 & y2 & z0)) | ((x1 & y0 & z2) & (x2 & y3 & z1));
+    while (w) {
+        const uint32_t i = (uint32_t)__ffsll((unsigned long long)w) - 1u;
+        w &= w - 1ull;
+        n -= fewer[corner_pairs(o, i)];
+    }
+    return (uint32_t)n;
+}
+
 /* Counts of node rows [r0, r1) of a job: one row group of 64 >> cshift rows
  * per wave iteration, one lane per 64-node chunk, no LDS window and no
  * barrier.  Per row: the crossing edges its nodes own and the triangles of
  * cell row (y, z-1); with a.vpc / a.tpc also each chunk's exclusive prefix of
- * both within its row.  ntri: triangle count per cube index (LDS). */
+ * both within its row.  fewer: of chunk_triangles (LDS). */
 template <int NLEV>
-__device__ __forceinline__ void count_rows_t(const JobArgs& a, const uint8_t* ntri, uint64_t r0, uint64_t r1,
+__device__ __forceinline__ void count_rows_t(const JobArgs& a, const uint8_t* fewer, uint64_t r0, uint64_t r1,
                                              uint64_t wave_first, uint64_t wave_step)
 {
     const uint32_t lane = threadIdx.x & 63u;
@@ -1152,12 +1182,7 @@ __device__ __forceinline__ void count_rows_t(const JobArgs& a, const uint8_t* nt
                     RowChunk o;
                     row_chunk(a, lev, y, z, c, o);
                     cv = (uint32_t)(__popcll(o.x) + __popcll(o.y) + __popcll(o.z));
-                    uint64_t m = o.act;
-                    while (m) {
-                        const uint32_t i = (uint32_t)__ffsll((unsigned long long)m) - 1u;
-                        m &= m - 1ull;
-                        ct += ntri[corner_pairs(o, i)];
-                    }
+                    if (o.act) ct = chunk_triangles(o, fewer);
                 }
                 if (chunk_prefixes) {
                     /* both counts in one scan: a chunk holds at most 192
@@ -1202,49 +1227,54 @@ __device__ __forceinline__ void count_rows_t(const JobArgs& a, const uint8_t* nt
 
 /* Level count as a compile-time constant where it is small, so that the loads
  * of all levels can be in flight together. */
-__device__ __forceinline__ void count_rows(const JobArgs& a, const uint8_t* ntri, uint64_t r0, uint64_t r1,
+__device__ __forceinline__ void count_rows(const JobArgs& a, const uint8_t* fewer, uint64_t r0, uint64_t r1,
                                            uint64_t wave_first, uint64_t wave_step)
 {
     switch (a.nlev) {
-    case 1: count_rows_t<1>(a, ntri, r0, r1, wave_first, wave_step); break;
-    case 2: count_rows_t<2>(a, ntri, r0, r1, wave_first, wave_step); break;
-    case 3: count_rows_t<3>(a, ntri, r0, r1, wave_first, wave_step); break;
-    case 4: count_rows_t<4>(a, ntri, r0, r1, wave_first, wave_step); break;
-    default: count_rows_t<0>(a, ntri, r0, r1, wave_first, wave_step); break;
+    case 1: count_rows_t<1>(a, fewer, r0, r1, wave_first, wave_step); break;
+    case 2: count_rows_t<2>(a, fewer, r0, r1, wave_first, wave_step); break;
+    case 3: count_rows_t<3>(a, fewer, r0, r1, wave_first, wave_step); break;
+    case 4: count_rows_t<4>(a, fewer, r0, r1, wave_first, wave_step); break;
+    default: count_rows_t<0>(a, fewer, r0, r1, wave_first, wave_step); break;
     }
 }
 
-/* Triangle count per swap_pairs(cube index) (the index corner_pairs gives). */
-__device__ __forceinline__ void stage_ntri(uint8_t* ntri)
+/* 2 (loops - 1) per swap_pairs(cube index) (the index corner_pairs gives):
+ * the cell's crossed edges less its triangles, less 2. */
+__device__ __forceinline__ void stage_fewer(uint8_t* fewer)
 {
-    for (uint32_t i = threadIdx.x; i < 256; i += kBlock) ntri[i] = (uint8_t)(d_tri[swap_pairs(i)] >> 60);
+    for (uint32_t i = threadIdx.x; i < 256; i += kBlock) {
+        const uint32_t c = swap_pairs(i), lo = c & 15u, hi = c >> 4;
+        const uint32_t edges = __popc(lo ^ ((lo >> 1) | (lo & 1u) << 3)) + __popc(hi ^ ((hi >> 1) | (hi & 1u) << 3)) +
+                               __popc(lo ^ hi);
+        fewer[i] = edges ? (uint8_t)(edges - (uint32_t)(d_tri[c] >> 60) - 2u) : 0;
+    }
     __syncthreads();
 }
 
-/* seven waves per SIMD (at most 72 VGPRs): the pass is bound by VALU issue
- * and load latency, and at eight waves (64 VGPRs) its spills cost more
- * issue than the eighth wave hides */
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) void k_count(JobArgs a)
+/* four waves per SIMD: chunk_triangles takes 101 VGPRs, and spills cost more
+ * than waves hide (512^3: 31.6 us at four, 35 at five, 45 at six, 72 at seven) */
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_count(JobArgs a)
 {
-    __shared__ uint8_t ntri[256];
-    stage_ntri(ntri);
+    __shared__ uint8_t fewer[256];
+    stage_fewer(fewer);
     /* row groups of 64 >> cshift rows as the units */
     const uint64_t G = 64u >> a.cshift, groups = (a.nrows + G - 1) / G;
     const Span sp = grid_span(0, groups, kWaves, uniform(threadIdx.x >> 6));
     const uint64_t r1 = sp.end * G < a.nrows ? sp.end * G : a.nrows;
-    count_rows(a, ntri, sp.lo * G, r1, sp.first - sp.lo, sp.step);
+    count_rows(a, fewer, sp.lo * G, r1, sp.first - sp.lo, sp.step);
 }
 
 /* Count pass of a batch: job z's workgroups walk its row groups in steps of the
  * whole grid. */
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) void k_count_batch(const JobArgs* jobs)
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_count_batch(const JobArgs* jobs)
 {
     const JobArgs& a = jobs[blockIdx.z];
     const uint64_t G = 64u >> a.cshift, wave = (uint64_t)blockIdx.x * kWaves;
     if (wave * G >= a.nrows) return;   // the whole workgroup: a job smaller than the grid
-    __shared__ uint8_t ntri[256];
-    stage_ntri(ntri);
-    count_rows(a, ntri, 0, a.nrows, wave + uniform(threadIdx.x >> 6), (uint64_t)gridDim.x * kWaves);
+    __shared__ uint8_t fewer[256];
+    stage_fewer(fewer);
+    count_rows(a, fewer, 0, a.nrows, wave + uniform(threadIdx.x >> 6), (uint64_t)gridDim.x * kWaves);
 }
 
 /* ------------------------------------------------------------------------- */
