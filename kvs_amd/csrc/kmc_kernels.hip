@@ -1859,7 +1859,13 @@ __global__ __launch_bounds__(kBlock) void k_slice_triangles_runs(JobArgs a, cons
 constexpr uint32_t kScanPer = 16;                      // elements per thread
 constexpr uint32_t kScanTile = kScanPer * kBlock;      // elements per block
 
-/* Sum of each kScanTile segment of each of the narr count arrays. */
+/* Four counts in one load; an array's base is aligned to one count only. */
+struct __attribute__((packed, aligned(4))) Count4 {
+    uint32_t x, y, z, w;
+};
+
+/* Sum of each kScanTile segment of each of the narr count arrays; a whole segment's
+ * loads are in flight at once (one at a time, 256^3: 6.7 us, so 3.0). */
 __global__ __launch_bounds__(kBlock) void k_scan_partials(const uint32_t* counts, uint64_t n, uint32_t nseg, uint64_t* partials)
 {
     __shared__ uint64_t sh[kWaves];
@@ -1867,9 +1873,14 @@ __global__ __launch_bounds__(kBlock) void k_scan_partials(const uint32_t* counts
     const uint32_t* src = counts + (uint64_t)arr * n;
     const uint64_t b = (uint64_t)seg * kScanTile;
     uint64_t s = 0;
-    for (uint32_t i = threadIdx.x; i < kScanTile; i += kBlock) {
-        const uint64_t g = b + i;
-        if (g < n) s += src[g];
+    if (b + kScanTile <= n) {
+        Count4 v[kScanPer / 4];
+#pragma unroll
+        for (uint32_t i = 0; i < kScanPer / 4; ++i) v[i] = ((const Count4*)(src + b))[i * kBlock + threadIdx.x];
+#pragma unroll
+        for (uint32_t i = 0; i < kScanPer / 4; ++i) s += ((uint64_t)v[i].x + v[i].y) + ((uint64_t)v[i].z + v[i].w);
+    } else {
+        for (uint64_t g = b + threadIdx.x; g < n; g += kBlock) s += src[g];
     }
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) s += (uint64_t)__shfl_xor((unsigned long long)s, d);
@@ -1927,10 +1938,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_mid(uint64_t* partials, uint32_
     }
 }
 
-/* Four counts in one load; an array's base is aligned to one count only. */
-struct __attribute__((packed, aligned(4))) Count4 {
-    uint32_t x, y, z, w;
-};
+/* Two prefixes in one store, likewise. */
 struct __attribute__((packed, aligned(8))) Prefix2 {
     uint64_t x, y;
 };
@@ -1953,7 +1961,7 @@ __device__ __forceinline__ uint64_t block_sum(uint64_t s, uint64_t* sh)
  * one kernel), kScanPartials the segments' sums before it, kScanScanned reads
  * the scanned sum (so many segments that summing them per workgroup would
  * cost more than a kernel).  Launches are what a small scan costs: 65536
- * counts take 15 us in three kernels, 12 in two. */
+ * counts took 15 us in three kernels, 8 in two. */
 enum : int { kScanCounts = 0, kScanPartials = 1, kScanScanned = 2 };
 
 template <int kFrom>
@@ -2520,8 +2528,8 @@ hipError_t launch_emit_batch(int dtype, int mode, const JobArgs* jobs, const uin
 
 /* Segments up to which a workgroup sums all counts before its own (one CU reads a
  * segment's 16 KiB in 1.1 us: 2 segments 5.4 us, 16 segments 17-21, in two
- * kernels 12 and a launch), and up to which it sums the segments' sums. */
-constexpr uint32_t kScanDirect = 8, kScanSummed = 4096;
+ * kernels 8 and a launch), and up to which it sums the segments' sums. */
+constexpr uint32_t kScanDirect = 4, kScanSummed = 4096;
 
 hipError_t launch_scan(const uint32_t* counts, uint64_t n, uint32_t narr, uint64_t* partials,
                        uint64_t* prefix, uint64_t* totals, hipStream_t st)
