@@ -12,7 +12,7 @@ namespace kmc {
 /* One level of a pass; the same on all lanes. */
 struct EmitLevel {
     const uint64_t* bits;    // [nz][ny][NC] chunk masks
-    const uint32_t* vp;      // in-row chunk prefixes (chunk_prefix)
+    const uint32_t* vp;      // in-row chunk prefixes
     const uint32_t* tp;
     const uint32_t* cv;      // row counts: crossing edges, triangles
     const uint32_t* ct;

@@ -183,13 +183,12 @@ __device__ __forceinline__ uint32_t around_nibbles(uint32_t axis)
  * read straight from the bit volume `lev` (coalesced across the lanes of a
  * row, neighbours from L1/L2).  x/y/z: crossing edges owned by the row's
  * nodes; act: active cells of cell row (y, z-1); k0/k3/k4/k7: the masks of
- * the cells' four node rows (bit i of kq is corner q of cell x = 64c + i),
- * k1/k2/k5/k6: the x+1 corners, the next bits of the same masks; next: bit 0 of
+ * the cells' four node rows (bit i of kq is corner q of cell x = 64c + i; the
+ * x+1 corners 1, 2, 5, 6 are the next bits of the same masks); next: bit 0 of
  * the next chunk's word of those four rows (corners 1, 2, 5, 6 of cell 63). */
 struct RowChunk {
     uint64_t x, y, z, act;
     uint64_t k0, k3, k4, k7;
-    uint64_t k1, k2, k5, k6;
     uint32_t next;
 };
 
@@ -231,10 +230,6 @@ __device__ __forceinline__ void row_chunk(const JobArgs& a, const uint64_t* lev,
     o.k3 = q;
     o.k4 = c4;
     o.k7 = c7;
-    o.k1 = c1;
-    o.k2 = c2;
-    o.k5 = c5;
-    o.k6 = c6;
     o.next = (uint32_t)(p1 & 1ull) | (uint32_t)(q1 & 1ull) << 1 | (uint32_t)(b1 & 1ull) << 2 |
              (uint32_t)(u1 & 1ull) << 3;
 }
@@ -259,22 +254,6 @@ __device__ __forceinline__ uint32_t corner_pairs(const RowChunk& o, uint32_t i)
     const uint32_t p0 = (uint32_t)(o.k0 >> i) & 3u, p3 = (uint32_t)(o.k3 >> i) & 3u;
     const uint32_t p4 = (uint32_t)(o.k4 >> i) & 3u, p7 = (uint32_t)(o.k7 >> i) & 3u;
     return p0 | p3 << 2 | p4 << 4 | p7 << 6;
-}
-
-/* In-row prefixes (vertices, triangles) of chunk word w.  Rows of at most 64
- * chunks keep both in one word of vpc (vertices in the low, triangles in the
- * high 16 bits: at most 63 chunks of 192 and 320 come before a chunk);
- * longer rows keep them in vpc and tpc. */
-__device__ __forceinline__ void chunk_prefix(const JobArgs& a, uint64_t w, uint32_t& v, uint32_t& t)
-{
-    if (a.NC <= 64) {
-        const uint32_t p = a.vpc[w];
-        v = p & 0xFFFFu;
-        t = p >> 16;
-    } else {
-        v = a.vpc[w];
-        t = a.tpc[w];
-    }
 }
 
 }  // namespace kmc

@@ -2,13 +2,13 @@
  * kmc_kernels.hip -- marching-cubes kernels for gfx950 (CDNA4, wave64).
  *
  * The path is a memory-bound stencil followed by an ordered stream
- * compaction; nothing here is a contraction, so nothing goes to MFMA.
+ * emission; nothing here is a contraction, so nothing goes to MFMA.
  *
  * Classification is bit-sliced: a wave loads 64 consecutive nodes of a row,
  * compares them against every isolevel of the pass and turns each level's
  * predicate into a 64-bit chunk mask with one ballot.  Edge crossings are XORs
  * of (shifted) chunk masks, cell activity is OR & ~AND of the eight corner
- * masks, and every rank needed for the ordered compaction is a popcount.
+ * masks, and every rank the ordered emission needs is a popcount.
  * Dense per-node work is therefore one load, one compare per level and one
  * ballot per level; only crossing edges and active cells do more.
  *
@@ -290,8 +290,7 @@ __device__ __forceinline__ uint32_t cube_index_mem(const JobArgs& a, const uint6
 
 /* (Contiguous parts per XCD -- workgroups reach the eight XCDs round-robin,
  * each with an L2 of its own -- measured 3 % slower on the whole call than
- * this plain interleave: compaction and triangles lost more than count
- * gained.) */
+ * this plain interleave: the emission lost more than count gained.) */
 struct Span { uint64_t lo, first, end, step; };
 
 /* Grid-stride walk over [b, e) in units of `units` items per workgroup
@@ -1125,23 +1124,37 @@ __device__ __forceinline__ uint32_t group_excl_scan(uint32_t x, uint32_t cl, uin
  * edges are twelve popcounts; more than one loop takes a face with all four
  * edges crossed or two opposite corners that differ from all their neighbours,
  * and only those cells are looked up: fewer[] holds 2 (L - 1).  A lookup per
- * active cell ran each wave as long as its fullest chunk took (512^3: 43 us, so
- * 31.6; 256^3 7.9 and 5.5; 1024^3 at three levels, mostly empty chunks, 432 and
- * 413; 14 volumes of up to 256^3 in a batch 42 and 34). */
+ * active cell runs each wave as long as its fullest chunk takes (512^3: 43 us, so
+ * 25.5; 256^3 7.9 and 5.1; 14 volumes of up to 256^3 in a batch 42 and 36). */
 __device__ __forceinline__ uint32_t chunk_triangles(const RowChunk& o, const uint8_t* fewer)
 {
-    const uint64_t m = o.act;
-    const uint64_t x0 = (o.k0 ^ o.k1) & m, x1 = (o.k3 ^ o.k2) & m, x2 = (o.k4 ^ o.k5) & m, x3 = (o.k7 ^ o.k6) & m;
-    const uint64_t y0 = (o.k0 ^ o.k3) & m, y1 = (o.k1 ^ o.k2) & m, y2 = (o.k4 ^ o.k7) & m, y3 = (o.k5 ^ o.k6) & m;
-    const uint64_t z0 = (o.k0 ^ o.k4) & m, z1 = (o.k1 ^ o.k5) & m, z2 = (o.k3 ^ o.k7) & m, z3 = (o.k2 ^ o.k6) & m;
-    int n = __popcll(x0) + __popcll(x1) + __popcll(x2) + __popcll(x3);
-    n += __popcll(y0) + __popcll(y1) + __popcll(y2) + __popcll(y3);
-    n += __popcll(z0) + __popcll(z1) + __popcll(z2) + __popcll(z3);
-    n -= 2 * __popcll(m);
-    /* three crossed edges of a face: the fourth is crossed too */
-    uint64_t w = (x0 & x1 & y0) | (x2 & x3 & y2) | (x0 & x2 & z0) | (x1 & x3 & z2) | (y0 & y2 & z0) | (y1 & y3 & z1);
-    w |= ((x0 & y0 & z0) & (x3 & y3 & z3)) | ((x0 & y1 & z1) & (x3 & y2 & z2));
-    w |= ((x1 & y1 & z3) & (x2 & y2 & z0)) | ((x1 & y0 & z2) & (x2 & y3 & z1));
+    int n = -2 * __popcll(o.act);
+    uint32_t multi[2];
+    /* 32 cells at a time, one after the other: half the registers */
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int d = 32 * h;
+        const uint32_t m = (uint32_t)(o.act >> d);
+        /* the x + 1 corners: the next bits, the last one's from the next chunk */
+        const uint32_t nx = h ? o.next : 0u;
+        const uint32_t k0 = (uint32_t)(o.k0 >> d), k1 = (uint32_t)(o.k0 >> (d + 1)) | nx << 31;
+        const uint32_t k3 = (uint32_t)(o.k3 >> d), k2 = (uint32_t)(o.k3 >> (d + 1)) | (nx >> 1) << 31;
+        const uint32_t k4 = (uint32_t)(o.k4 >> d), k5 = (uint32_t)(o.k4 >> (d + 1)) | (nx >> 2) << 31;
+        const uint32_t k7 = (uint32_t)(o.k7 >> d), k6 = (uint32_t)(o.k7 >> (d + 1)) | (nx >> 3) << 31;
+        const uint32_t x0 = (k0 ^ k1) & m, x1 = (k3 ^ k2) & m, x2 = (k4 ^ k5) & m, x3 = (k7 ^ k6) & m;
+        const uint32_t y0 = (k0 ^ k3) & m, y1 = (k1 ^ k2) & m, y2 = (k4 ^ k7) & m, y3 = (k5 ^ k6) & m;
+        const uint32_t z0 = (k0 ^ k4) & m, z1 = (k1 ^ k5) & m, z2 = (k3 ^ k7) & m, z3 = (k2 ^ k6) & m;
+        n += __popc(x0) + __popc(x1) + __popc(x2) + __popc(x3);
+        n += __popc(y0) + __popc(y1) + __popc(y2) + __popc(y3);
+        n += __popc(z0) + __popc(z1) + __popc(z2) + __popc(z3);
+        /* three crossed edges of a face: the fourth is crossed too */
+        uint32_t w = (x0 & x1 & y0) | (x2 & x3 & y2) | (x0 & x2 & z0) | (x1 & x3 & z2) | (y0 & y2 & z0) | (y1 & y3 & z1);
+        w |= ((x0 & y0 & z0) & (x3 & y3 & z3)) | ((x0 & y1 & z1) & (x3 & y2 & z2));
+        w |= ((x1 & y1 & z3) & (x2 & y2 & z0)) | ((x1 & y0 & z2) & (x2 & y3 & z1));
+        multi[h] = w;
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    uint64_t w = (uint64_t)multi[1] << 32 | multi[0];
     while (w) {
         const uint32_t i = (uint32_t)__ffsll((unsigned long long)w) - 1u;
         w &= w - 1ull;
@@ -1154,9 +1167,10 @@ __device__ __forceinline__ uint32_t chunk_triangles(const RowChunk& o, const uin
  * per wave iteration, one lane per 64-node chunk, no LDS window and no
  * barrier.  Per row: the crossing edges its nodes own and the triangles of
  * cell row (y, z-1); with a.vpc / a.tpc also each chunk's exclusive prefix of
- * both within its row.  fewer: of chunk_triangles (LDS). */
-template <int NLEV>
-__device__ __forceinline__ void count_rows_t(const JobArgs& a, const uint8_t* fewer, uint64_t r0, uint64_t r1,
+ * both within its row.  POP: triangles by chunk_triangles, else by a lookup per
+ * active cell; tab is the table of either (LDS). */
+template <int NLEV, bool POP>
+__device__ __forceinline__ void count_rows_t(const JobArgs& a, const uint8_t* tab, uint64_t r0, uint64_t r1,
                                              uint64_t wave_first, uint64_t wave_step)
 {
     const uint32_t lane = threadIdx.x & 63u;
@@ -1182,7 +1196,16 @@ __device__ __forceinline__ void count_rows_t(const JobArgs& a, const uint8_t* fe
                     RowChunk o;
                     row_chunk(a, lev, y, z, c, o);
                     cv = (uint32_t)(__popcll(o.x) + __popcll(o.y) + __popcll(o.z));
-                    if (o.act) ct = chunk_triangles(o, fewer);
+                    if constexpr (POP) {
+                        if (o.act) ct = chunk_triangles(o, tab);
+                    } else {
+                        uint64_t m = o.act;
+                        while (m) {
+                            const uint32_t i = (uint32_t)__ffsll((unsigned long long)m) - 1u;
+                            m &= m - 1ull;
+                            ct += tab[corner_pairs(o, i)];
+                        }
+                    }
                 }
                 if (chunk_prefixes) {
                     /* both counts in one scan: a chunk holds at most 192
@@ -1195,7 +1218,7 @@ __device__ __forceinline__ void count_rows_t(const JobArgs& a, const uint8_t* fe
                         /* coalesced stream of prefixes: nontemporal (measured
                          * faster).  Rows of at most 64 chunks are one group,
                          * so the packed scan result is the chunk's in-row
-                         * prefix pair (chunk_prefix) */
+                         * prefix pair */
                         if (a.NC <= 64) {
                             __builtin_nontemporal_store(e, &a.vpc[w]);
                         } else {
@@ -1227,54 +1250,72 @@ __device__ __forceinline__ void count_rows_t(const JobArgs& a, const uint8_t* fe
 
 /* Level count as a compile-time constant where it is small, so that the loads
  * of all levels can be in flight together. */
-__device__ __forceinline__ void count_rows(const JobArgs& a, const uint8_t* fewer, uint64_t r0, uint64_t r1,
+template <bool POP>
+__device__ __forceinline__ void count_rows(const JobArgs& a, const uint8_t* tab, uint64_t r0, uint64_t r1,
                                            uint64_t wave_first, uint64_t wave_step)
 {
     switch (a.nlev) {
-    case 1: count_rows_t<1>(a, fewer, r0, r1, wave_first, wave_step); break;
-    case 2: count_rows_t<2>(a, fewer, r0, r1, wave_first, wave_step); break;
-    case 3: count_rows_t<3>(a, fewer, r0, r1, wave_first, wave_step); break;
-    case 4: count_rows_t<4>(a, fewer, r0, r1, wave_first, wave_step); break;
-    default: count_rows_t<0>(a, fewer, r0, r1, wave_first, wave_step); break;
+    case 1: count_rows_t<1, POP>(a, tab, r0, r1, wave_first, wave_step); break;
+    case 2: count_rows_t<2, POP>(a, tab, r0, r1, wave_first, wave_step); break;
+    case 3: count_rows_t<3, POP>(a, tab, r0, r1, wave_first, wave_step); break;
+    case 4: count_rows_t<4, POP>(a, tab, r0, r1, wave_first, wave_step); break;
+    default: count_rows_t<0, POP>(a, tab, r0, r1, wave_first, wave_step); break;
     }
 }
 
-/* 2 (loops - 1) per swap_pairs(cube index) (the index corner_pairs gives):
- * the cell's crossed edges less its triangles, less 2. */
-__device__ __forceinline__ void stage_fewer(uint8_t* fewer)
+/* Per swap_pairs(cube index) (the index corner_pairs gives) 2 (loops - 1), the
+ * cell's crossed edges less its triangles, less 2; without POP its triangles. */
+template <bool POP>
+__device__ __forceinline__ void stage_counts(uint8_t* tab)
 {
     for (uint32_t i = threadIdx.x; i < 256; i += kBlock) {
-        const uint32_t c = swap_pairs(i), lo = c & 15u, hi = c >> 4;
+        const uint32_t c = swap_pairs(i), lo = c & 15u, hi = c >> 4, nt = (uint32_t)(d_tri[c] >> 60);
         const uint32_t edges = __popc(lo ^ ((lo >> 1) | (lo & 1u) << 3)) + __popc(hi ^ ((hi >> 1) | (hi & 1u) << 3)) +
                                __popc(lo ^ hi);
-        fewer[i] = edges ? (uint8_t)(edges - (uint32_t)(d_tri[c] >> 60) - 2u) : 0;
+        tab[i] = (uint8_t)(!POP ? nt : (edges ? edges - nt - 2u : 0u));
     }
     __syncthreads();
 }
 
-/* four waves per SIMD: chunk_triangles takes 101 VGPRs, and spills cost more
- * than waves hide (512^3: 31.6 us at four, 35 at five, 45 at six, 72 at seven) */
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_count(JobArgs a)
+/* Row groups of 64 >> cshift rows as the units. */
+template <bool POP, int NLEV>
+__device__ __forceinline__ void count_job(const JobArgs& a, uint8_t* tab)
 {
-    __shared__ uint8_t fewer[256];
-    stage_fewer(fewer);
-    /* row groups of 64 >> cshift rows as the units */
+    stage_counts<POP>(tab);
     const uint64_t G = 64u >> a.cshift, groups = (a.nrows + G - 1) / G;
     const Span sp = grid_span(0, groups, kWaves, uniform(threadIdx.x >> 6));
     const uint64_t r1 = sp.end * G < a.nrows ? sp.end * G : a.nrows;
-    count_rows(a, fewer, sp.lo * G, r1, sp.first - sp.lo, sp.step);
+    if constexpr (NLEV == 1) count_rows_t<1, POP>(a, tab, sp.lo * G, r1, sp.first - sp.lo, sp.step);
+    else count_rows<POP>(a, tab, sp.lo * G, r1, sp.first - sp.lo, sp.step);
+}
+
+/* One level: 74 VGPRs, six waves per SIMD without a spill. */
+__global__ __launch_bounds__(kBlock) void k_count_level(JobArgs a)
+{
+    __shared__ uint8_t tab[256];
+    count_job<true, 1>(a, tab);
+}
+
+/* Several levels, all their loads in flight: seven waves per SIMD (at most 72
+ * VGPRs).  With chunk_triangles and four waves, mostly empty chunks, whose time is
+ * load latency, lose more than full ones gain (1024^3 at three levels: 357 -> 390
+ * us with smooth fields, 432 -> 413 with rough ones). */
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) void k_count(JobArgs a)
+{
+    __shared__ uint8_t tab[256];
+    count_job<false, 0>(a, tab);
 }
 
 /* Count pass of a batch: job z's workgroups walk its row groups in steps of the
  * whole grid. */
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_count_batch(const JobArgs* jobs)
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_count_batch(const JobArgs* jobs)
 {
     const JobArgs& a = jobs[blockIdx.z];
     const uint64_t G = 64u >> a.cshift, wave = (uint64_t)blockIdx.x * kWaves;
     if (wave * G >= a.nrows) return;   // the whole workgroup: a job smaller than the grid
-    __shared__ uint8_t fewer[256];
-    stage_fewer(fewer);
-    count_rows(a, fewer, 0, a.nrows, wave + uniform(threadIdx.x >> 6), (uint64_t)gridDim.x * kWaves);
+    __shared__ uint8_t tab[256];
+    stage_counts<true>(tab);
+    count_rows<true>(a, tab, 0, a.nrows, wave + uniform(threadIdx.x >> 6), (uint64_t)gridDim.x * kWaves);
 }
 
 /* ------------------------------------------------------------------------- */
@@ -2329,7 +2370,8 @@ hipError_t launch_count(const JobArgs& a, hipStream_t st)
     const uint64_t G = 64u >> a.cshift;
     uint64_t blocks = ((a.nrows + G - 1) / G + kWaves - 1) / kWaves;
     if (blocks > 16384) blocks = 16384;
-    hipLaunchKernelGGL(k_count, dim3((uint32_t)blocks), dim3(kBlock), 0, st, a);
+    if (a.nlev == 1) hipLaunchKernelGGL(k_count_level, dim3((uint32_t)blocks), dim3(kBlock), 0, st, a);
+    else hipLaunchKernelGGL(k_count, dim3((uint32_t)blocks), dim3(kBlock), 0, st, a);
     return hipGetLastError();
 }
 
