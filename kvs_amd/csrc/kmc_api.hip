@@ -447,7 +447,7 @@ kmc_status min_max_on_device(const kmc_volume* v, const void* dvals, hipStream_t
 }
 
 /* Row geometry every emit needs: 64-node chunks per row, the lane split of
- * the count and compaction passes, node rows. */
+ * the count pass, node rows. */
 void plan_rows(JobArgs& a)
 {
     a.NC = (a.nx + 63) / 64;

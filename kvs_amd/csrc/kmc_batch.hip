@@ -362,7 +362,7 @@ kmc_status plan_tiles(kmc_batch* b, uint32_t r_max, uint32_t queue_cap)
     free_plan_buffers(b);
     b->r_max = r_max;
     b->queue_cap = queue_cap;
-    /* the flat emit keeps no per-team LDS state: a pass whose team does not
+    /* the chunk-batch emit keeps no per-team LDS state: a pass whose team does not
      * fit only rules out the tile teams */
     for (Pass& p : b->passes) {
         if (!plan_geometry(p.a, &p.lds, r_max, queue_cap) && !b->flat) return KMC_ERR_INVALID_ARGUMENT;
@@ -581,8 +581,8 @@ kmc_status run(kmc_batch* b, hipStream_t st)
     return KMC_ERR_DEVICE;
 }
 
-/* Time the candidate emit forms on this batch -- the flat emit and the tile
- * teams at several band heights and queue sizes; keep the fastest. */
+/* Time the candidate emit forms on this batch -- the chunk-batch emit and the
+ * tile teams at several band heights and queue sizes; keep the fastest. */
 kmc_status autotune(kmc_batch* b, hipStream_t st)
 {
     struct Cand { uint32_t r, q; bool flat; };

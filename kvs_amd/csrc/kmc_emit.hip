@@ -943,7 +943,7 @@ __device__ __forceinline__ void normals_level(const JobArgs& a, uint32_t l, cons
     const float* fn = a.fn + 3 * a.toff[l];
     const uint32_t* crec = triangles ? a.crec + a.toff[l] : (const uint32_t*)L.bits;   // read, not used, without one
     const uint64_t* act_l = a.act + (uint64_t)l * (a.nrows * a.NC);
-    const uint32_t* tri_pre = a.NC <= 64 ? L.vp : L.tp;   // chunk_prefix: triangles in the high half of vp
+    const uint32_t* tri_pre = a.NC <= 64 ? L.vp : L.tp;   // packed: triangles in the high half of vp
     const uint32_t sh = a.NC <= 64 ? 16u : 0u;
     busy_chunks<true, kNormalChunks>(a, L, s.p.q, [&](uint32_t n) {
         chunk_points(a, L, s.p, n, [&](uint64_t r, uint32_t y, uint32_t z, uint32_t c) {

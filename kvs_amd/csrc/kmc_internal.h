@@ -107,7 +107,7 @@ bool flat_emit_fits(uint32_t ny, uint32_t nz);
  * False if not even R = 1 fits a workgroup. */
 bool plan_geometry(JobArgs& a, uint32_t* lds_bytes, uint32_t r_max = 16, uint32_t queue_cap = 0);
 
-/* Isolevels per pass over this volume: kMaxLevels with the flat emit; with
+/* Isolevels per pass over this volume: kMaxLevels with the chunk-batch emit; with
  * the tile teams (one level per team) kMaxLevels whenever a team's LDS state
  * fits at all, 0 if it does not (for VertexNormal when vnormal). */
 uint32_t levels_per_pass(const kmc_volume* v, int vnormal);
@@ -159,11 +159,11 @@ hipError_t batch_launch_front(kmc_batch* b, hipStream_t st);
 uint32_t batch_surfaces(const kmc_batch* b);
 void batch_surface_sizes(const kmc_batch* b, uint32_t i, kmc_surface* o);
 void batch_set_outputs(kmc_batch* b, uint32_t i, float* coords, float* normals, uint32_t* conn);
-/* Flat-emit record bytes surface i adds once its sizes are known. */
+/* Intermediate bytes surface i adds once its sizes are known. */
 uint64_t batch_record_bytes(const kmc_batch* b, uint32_t i);
 hipError_t batch_launch_emit(kmc_batch* b, hipStream_t st);
 uint64_t batch_work_bytes(const kmc_batch* b);
-/* Device bytes of the flat-emit record arena the last batch_launch_emit used. */
+/* Device bytes of the intermediate arena the last batch_launch_emit used. */
 uint64_t batch_record_arena_bytes(const kmc_batch* b);
 void batch_destroy(kmc_batch* b);
 

@@ -5,8 +5,8 @@
  *
  * The caller passes the volume in device memory and the output arrays with
  * their capacities.  Every work array of the call -- classification masks,
- * per-row counts and prefixes, in-row chunk prefixes, chunk crossing records,
- * the emit's records, the min/max partials -- is carved from `scratch`, a
+ * per-row counts and prefixes, in-row chunk prefixes, VertexNormal's
+ * active-cell masks, face normals and cell records, the min/max partials -- is carved from `scratch`, a
  * fixed device array of KMC_NOALLOC_SCRATCH_BYTES that each GPU the library
  * runs on holds until the process ends.  None of these arrays needs clearing:
  * every element a kernel reads was written earlier in the same call.

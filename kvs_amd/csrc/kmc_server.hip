@@ -65,8 +65,8 @@ struct Resident {
 uint64_t request_scratch(const kmc_volume& v)
 {
     /* per node row: counts and prefixes of vertices and triangles (2 x 12 B);
-     * per 64-node chunk: its mask (8 B), its two in-row prefixes (8 B) and its
-     * crossing record (32 B) */
+     * per 64-node chunk: its mask (8 B), its two in-row prefixes (8 B), its active
+     * cells (8 B, VertexNormal) and 24 B of headroom */
     const uint64_t nx = v.resolution[0], ny = v.resolution[1], nz = v.resolution[2];
     const uint64_t nrows = ny * nz, NC = (nx + 63) / 64;
     return nrows * 2 * 12 + nrows * NC * 48 + 4096;

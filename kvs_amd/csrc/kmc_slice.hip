@@ -3,9 +3,8 @@
  * (Source/Core/Visualization/Mapper/SlicePlane.cpp:97-280) on the device.
  *
  * The plane takes the place of the isosurface: nodes classify by the sign of
- * the plane equation (no value is read for that), the count / scan /
- * compaction passes of the marching-cubes path run unchanged in duplicated
- * mode, and one thread per triangle interpolates its three vertices along the
+ * the plane equation (no value is read for that), the count and scan passes
+ * of the marching-cubes path run unchanged in duplicated mode, and one thread per triangle interpolates its three vertices along the
  * plane, colours each with the value interpolated at the same ratio, and
  * writes the negated face normal -- triangles in cell scan order, the order
  * of the reference's loop.
