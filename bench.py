@@ -152,7 +152,7 @@ def main():
 
     # per-kernel device time (HIP events between the launches, on the same stream)
     lib.kmc_set_timing(1)
-    prof = {"classify": 0.0, "count": 0.0, "scan": 0.0, "compact": 0.0, "vertices": 0.0, "triangles": 0.0,
+    prof = {"classify": 0.0, "count": 0.0, "scan": 0.0, "vertices": 0.0, "triangles": 0.0,
             "vertex_normals": 0.0, "emit": 0.0}
     for _ in range(args.profile_steps):
         step()
@@ -247,28 +247,24 @@ def measured_traffic():
 
 def kernel_rooflines(prof, n, nlev, counts):
     """Algorithmic bytes and achieved bandwidth of each kernel of one step
-    (one launch each; the emit stage is compact + vertices + triangles +
-    vertex_normals).  Per launch:
+    (one launch each; the emit stage is vertices + triangles + vertex_normals).
+    Per launch:
       classify        reads the volume (4 B per node), writes the classification
                       masks (nlev bits per node, in 64-node words);
       count           reads the masks, writes 2 x 4 B per node row and level and
                       the in-row chunk prefixes (4 B per 64-node chunk and level
                       for rows of at most 64 chunks, else 2 x 4 B);
       scan            reads those row counts, writes 8 B prefixes;
-      compact         reads the chunk prefixes (as written by count) and the
-                      masks, writes the records
-                      (8 B per vertex, 8 + 1 B per triangle; the 32-byte crossing
-                      records of chunks with a vertex are not counted);
-      vertices        reads each vertex key and its edge's two values, writes its
-                      coordinates: 8 + 8 + 12 B per vertex;
-      triangles       reads each record, cube index and its three vertices'
-                      coordinates, writes connections and face normal:
-                      8 + 1 + 36 + 12 + 12 B per triangle (the cell-slot writes,
-                      about 8 B per triangle, are not counted);
-      vertex_normals  reads each vertex key, its four cell slots and the cells'
-                      cube indices, and the face normals of the triangles using it
-                      (3 per triangle, 12 B each), writes the normal: 8 + 16 + 4 + 12
-                      B per vertex + 36 B per triangle."""
+      vertices        reads the chunk prefixes and the masks and each vertex's edge's
+                      two values, writes its coordinates: 8 + 12 B per vertex;
+      triangles       reads the chunk prefixes, the masks and its three vertices'
+                      coordinates, writes connections, face normal and cell record:
+                      36 + 12 + 12 + 4 B per triangle (the active-cell masks of busy
+                      chunks are not counted);
+      vertex_normals  reads the chunk prefixes and the masks, each cell record and the
+                      face normals of the triangles using the vertex (3 per triangle,
+                      12 B each), writes the normal: 12 B per vertex + 40 B per
+                      triangle."""
     nc = (n + 63) // 64
     masks = nlev * n * n * nc * 8
     chunks = nlev * n * n * nc
@@ -280,14 +276,12 @@ def kernel_rooflines(prof, n, nlev, counts):
         "classify": n ** 3 * 4 + masks,
         "count": masks + 2 * nlev * rows * 4 + prefix_bytes,
         "scan": 2 * nlev * rows * (4 + 8),
-        "compact": prefix_bytes + masks + 8 * nv + 9 * nt,
-        "vertices": 28 * nv,
-        "triangles": 69 * nt,
-        "vertex_normals": 40 * nv + 36 * nt,
+        "vertices": prefix_bytes + masks + 20 * nv,
+        "triangles": prefix_bytes + masks + 64 * nt,
+        "vertex_normals": prefix_bytes + masks + 12 * nv + 40 * nt,
     }
-    names = {"classify": "k_classify<float, 3>", "count": "k_count", "scan": "k_scan_*", "compact": "k_compact",
-             "vertices": "k_vertices<float>", "triangles": "k_triangles<float, 2>",
-             "vertex_normals": "k_vertex_normals"}
+    names = {"classify": "k_classify<float, 3>", "count": "k_count", "scan": "k_scan_*",
+             "vertices": "k_points<float>", "triangles": "k_faces<2>", "vertex_normals": "k_normals"}
     traffic = measured_traffic()
     out = {}
     for k in names:
