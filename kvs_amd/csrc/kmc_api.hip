@@ -457,42 +457,6 @@ void plan_rows(JobArgs& a)
     plan_emit(a, emit_steps(a));
 }
 
-/* Wave steps of 64 (row, chunk) pairs that a pass's levels hold. */
-uint64_t emit_steps(const JobArgs& a)
-{
-    const uint64_t G = 64u >> a.cshift;
-    return std::max(1u, a.nlev) * ((a.nrows + G - 1) / G * ((a.NC + 63) / 64));
-}
-
-/* Waves of a launch: as many as the device holds of the kernel at once, and up
- * to eight times that while each still has four full steps -- the later ones
- * even out a large pass (1024^3 float turbulence, three levels, triangles /
- * normals: 1666 / 1240 us with one time, 1367 / 1205 with two, 1250 / 1129
- * with eight, 1277 / 1162 with sixteen; a half-filled round costs: 512^3 CT
- * triangles 287 us with one time, 338 with 1.6) -- and no more than one per 32
- * outputs.  A wave takes as many rows at a time as its lanes hold, but at most a
- * quarter of its share of the pass: a surface lies in few neighbouring rows, and
- * four steps far apart even the waves out (256^3 blobs, duplicated: 26 us, 36
- * with two steps).  Where every chunk holds many outputs there is nothing to
- * even out, and two steps keep the batches full (320 x 288 x 256 CT, vertices:
- * 38 us, 42 with four). */
-constexpr uint64_t kEmitRounds = 8, kEmitItems = 32;
-
-void plan_emit(JobArgs& a, uint64_t all, uint32_t per_cu, uint64_t items)
-{
-    const uint64_t own = emit_steps(a), nlev = std::max(1u, a.nlev);
-    const uint64_t resident = 256ull * kWaves * per_cu;
-    uint64_t waves = resident * std::min(kEmitRounds, std::max<uint64_t>(1, all / 4 / resident));
-    if (items) waves = std::min(waves, std::max<uint64_t>(256, items / kEmitItems));
-    else waves = std::max(waves, std::min(2 * resident, all / 4));   // a batch's uneven passes even out by themselves
-    const uint64_t want = std::max<uint64_t>(1, (waves * own + all - 1) / all / nlev);   // waves per level
-    const uint64_t steps = items > 4 * nlev * a.nrows * a.NC ? 2 : 4;
-    a.erows = 64u >> a.cshift;
-    while (a.erows > 1 && a.nrows / a.erows < steps * want) a.erows >>= 1;
-    const uint64_t units = (a.nrows + a.erows - 1) / a.erows;
-    a.eblocks = (uint32_t)std::max<uint64_t>(1, (std::min(units, want) + kWaves - 1) / kWaves);
-}
-
 bool flat_emit_fits(uint32_t ny, uint32_t nz)
 {
     const char* env_emit = std::getenv("KMC_EMIT");

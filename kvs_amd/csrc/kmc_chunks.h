@@ -4,6 +4,7 @@
  */
 #pragma once
 #include "kmc_device.h"
+#include "kmc_plan.h"
 
 #pragma clang fp contract(off)
 
@@ -38,78 +39,79 @@ __device__ __forceinline__ EmitLevel emit_level(const JobArgs& a, uint32_t l)
 }
 
 /* Calls batch(n) for every group of n <= N chunks of the level with a
- * crossing edge (V) or a triangle (!V), their words' indices in the
- * level (row * NC + chunk: 32 bits serve every volume whose masks fit the
- * device) in q[0 .. n) (q: N + 64 entries).  A wave
- * takes units of a.erows rows x up to 64 chunks; the prefixes of kScan units
- * are in flight together, since the test of a unit is one dependent load.
+ * crossing edge (V) or a triangle (!V), queued in q[0 .. n) (emit_queued;
+ * chunk_place tells where they lie; q: N + 64 entries).  The prefixes of
+ * kScan units are in flight together, since the test of a unit is one dependent load.
  * Across a batch only the units' busy masks stay live (scalars). */
 constexpr uint32_t kScan = 4;
+
+__device__ __forceinline__ uint32_t emit_wave() { return blockIdx.x * (uint32_t)kWaves + uniform(threadIdx.x >> 6); }
 
 template <bool V, uint32_t N, typename F>
 __device__ __forceinline__ void busy_chunks(const JobArgs& a, const EmitLevel& L, uint32_t* q, F&& batch)
 {
     const uint32_t lane = threadIdx.x & 63u;
-    const uint64_t wave = (uint64_t)blockIdx.x * kWaves + uniform(threadIdx.x >> 6), nwaves = (uint64_t)a.eblocks * kWaves;
-    const uint32_t sub = lane >> a.cshift;
-    const uint64_t step = nwaves * a.erows;
+    const uint64_t nwaves = emit_waves(a);
     const bool packed = a.NC <= 64;        // vertices in the low, triangles in the high half of vpc
     const uint32_t* pre = V || packed ? L.vp : L.tp;
     const uint32_t* row_end = V ? L.cv : L.ct;
     const uint32_t sh = V || !packed ? 0u : 16u, mask = packed ? 0xFFFFu : ~0u;
-    uint32_t qn = 0;
-    for (uint32_t c0 = 0; c0 < a.NC; c0 += 64) {
-        const uint32_t c = c0 + (lane & ((1u << a.cshift) - 1u));
-        const bool in = sub < a.erows && c < a.NC;
-        const bool row_last = c + 1 == a.NC;
-        for (uint64_t r0 = wave * a.erows; r0 < a.nrows; r0 += step * kScan) {
-            uint32_t p0[kScan], p1[kScan];
+    uint32_t qn = 0, step = 0;
+    for (uint64_t u0 = emit_wave(); u0 < a.eunits; u0 += nwaves * kScan, step += kScan) {
+        uint32_t p0[kScan], p1[kScan];
+        /* (opaque, so that nothing made of it stays in a register over the batches) */
+        uint32_t slot = lane;
+        asm volatile("" : "+v"(slot));
+        const uint32_t sub = lane_row(a, slot), cl = lane_chunk(a, slot), o = sub * a.NC + cl;
 #pragma unroll
-            for (uint32_t k = 0; k < kScan; ++k) {
-                const uint64_t r = r0 + k * step + sub;
-                p0[k] = p1[k] = 0u;
-                if (in && r < a.nrows) {
-                    const uint64_t w = r * a.NC + c;
-                    p0[k] = (pre[w] >> sh) & mask;
-                    p1[k] = row_last ? row_end[r] : (pre[w + 1] >> sh) & mask;
-                }
+        for (uint32_t k = 0; k < kScan; ++k) {
+            const uint64_t u = u0 + k * nwaves;
+            const EmitPart at = emit_part(a, u);
+            const uint64_t row = uniform64(at.row), left = u < a.eunits ? a.nrows - row : 0;
+            const uint32_t chunk = uniform(at.chunk), chunks = a.NC - chunk;
+            const uint32_t* words = pre + (row * a.NC + chunk);
+            const uint32_t* ends = row_end + row;
+            p0[k] = p1[k] = 0u;
+            if (sub < (left < a.erows ? (uint32_t)left : a.erows) && cl < chunks) {
+                p0[k] = (words[o] >> sh) & mask;
+                p1[k] = cl + 1 == chunks ? ends[sub] : (words[o + 1] >> sh) & mask;
             }
-            uint64_t busy[kScan];
+        }
+        uint64_t busy[kScan];
 #pragma unroll
-            for (uint32_t k = 0; k < kScan; ++k) busy[k] = __ballot(p0[k] != p1[k]);
+        for (uint32_t k = 0; k < kScan; ++k) busy[k] = __ballot(p0[k] != p1[k]);
+        const bool last = u0 + nwaves * kScan >= a.eunits;
 #pragma unroll 1
-            for (uint32_t k = 0; k < kScan; ++k) {
-                uint64_t bm = busy[0];
+        for (uint32_t k = 0; k < kScan; ++k) {
+            uint64_t bm = busy[0];
 #pragma unroll
-                for (uint32_t j = 1; j < kScan; ++j) bm = k == j ? busy[j] : bm;
-                if ((bm >> lane) & 1ull) q[qn + lanes_below(bm)] = (uint32_t)((r0 + k * step + sub) * a.NC + c);
-                qn += (uint32_t)__popcll(bm);
-                const bool end = r0 + step * kScan >= a.nrows && k == kScan - 1;
-                while (qn >= N || (end && qn)) {
-                    wave_sync();
-                    const uint32_t n = qn < N ? qn : N;
-                    batch(n);
-                    wave_sync();
-                    /* the rest (at most 63) moves to the front */
-                    qn -= n;
-                    const uint32_t rest = q[N + lane];
-                    wave_sync();
-                    if (lane < qn) q[lane] = rest;
-                    wave_sync();
-                }
+            for (uint32_t j = 1; j < kScan; ++j) bm = k == j ? busy[j] : bm;
+            if ((bm >> lane) & 1ull) q[qn + lanes_below(bm)] = emit_queued(step + k, lane);
+            qn += (uint32_t)__popcll(bm);
+            const bool end = last && k == kScan - 1;
+            while (qn >= N || (end && qn)) {
+                wave_sync();
+                const uint32_t n = qn < N ? qn : N;
+                batch(n);
+                wave_sync();
+                /* the rest (at most 63) moves to the front */
+                qn -= n;
+                const uint32_t rest = q[N + lane];
+                wave_sync();
+                if (lane < qn) q[lane] = rest;
+                wave_sync();
             }
         }
     }
 }
 
-/* Row, its y and z, and chunk of the row of a queued word. */
-__device__ __forceinline__ void chunk_place(const JobArgs& a, uint32_t w, uint64_t& r, uint32_t& y, uint32_t& z, uint32_t& c)
+/* Row, its y and z, and chunk of the row of a queued slot of this wave. */
+__device__ __forceinline__ void chunk_place(const JobArgs& a, uint32_t queued, uint64_t& r, uint32_t& y, uint32_t& z, uint32_t& c)
 {
-    const uint32_t row = w / a.NC;
-    c = w - row * a.NC;
-    z = row / a.ny;
-    y = row - z * a.ny;
-    r = row;
+    const EmitPart at = emit_part(a, emit_unit(a, emit_wave(), queued));
+    r = at.row + lane_row(a, queued & 63u);
+    c = at.chunk + lane_chunk(a, queued & 63u);
+    row_place(a, r, y, z);
 }
 
 /* Lists the set bits of the masks of lanes `fit` as lane | bit << 6, each lane's

@@ -8,6 +8,7 @@
 
 #include "kmc.h"
 #include "kmc_job.h"
+#include "kmc_plan.h"
 
 namespace kmc {
 
@@ -90,13 +91,6 @@ void float_range(JobArgs& a);
 
 /* Row geometry of every emit (a.nx, a.ny, a.nz set): a.NC, a.cshift, a.nrows. */
 void plan_rows(JobArgs& a);
-
-/* Split of the chunk-batch emit (rows planned; a.nlev set): a.erows and
- * a.eblocks of a pass whose emit shares its launch with others, `all` being
- * the sum of their emit_steps, for a kernel of which a CU holds per_cu
- * workgroups and that produces `items` outputs (0: not known yet). */
-uint64_t emit_steps(const JobArgs& a);
-void plan_emit(JobArgs& a, uint64_t all, uint32_t per_cu = 4, uint64_t items = 0);
 
 /* True when the chunk-batch emit serves a volume of these y / z sizes (its lists
  * pack y and z in 20 bits) and KMC_EMIT does not ask for the tile teams. */

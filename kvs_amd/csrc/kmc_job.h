@@ -67,8 +67,11 @@ struct JobArgs {
     uint32_t team_stride;  // bytes of LDS per team (>= the team layout's size)
     uint32_t teams;        // teams per emit workgroup (<= kEmitTeams; fewer when a team's LDS is large)
     uint64_t nunits;   // nlev * nb * nslabs
-    uint32_t erows;    // chunk-batch emit: node rows per wave step (at most 64 >> cshift) ...
-    uint32_t eblocks;  // ... and workgroups per level
+    uint32_t erows;    // chunk-batch emit: node rows per wave step (at most 64 >> cshift),
+    uint32_t esegs;    // ... steps per row (of more than 64 chunks),
+    uint64_t eunits;   // ... steps of all waves per level
+    uint32_t eblocks;  // ... and workgroups per level (kmc_plan.h)
+    double seg_inverse, ny_inverse;   // 1 / esegs, 1 / ny (div_by)
     uint64_t nrows;    // nz * ny: counts and prefixes are kept per node row
     double minv, maxv; // clamp range of the interpolation (volume min/max)
     float fminv, fmaxv;    // the same as floats ...
