@@ -15,8 +15,6 @@ struct EmitLevel {
     const uint64_t* bits;    // [nz][ny][NC] chunk masks
     const uint32_t* vp;      // in-row chunk prefixes
     const uint32_t* tp;
-    const uint32_t* cv;      // row counts: crossing edges, triangles
-    const uint32_t* ct;
     const uint64_t* pv;      // row prefixes
     const uint64_t* pt;
     uint64_t v0, t0;         // first prefix of each (outputs index from 0)
@@ -29,8 +27,6 @@ __device__ __forceinline__ EmitLevel emit_level(const JobArgs& a, uint32_t l)
     L.bits = a.bitvol + words;
     L.vp = a.vpc + words;
     L.tp = a.tpc + words;
-    L.cv = a.counts + (uint64_t)(l * 2 + 0) * a.nrows;
-    L.ct = a.counts + (uint64_t)(l * 2 + 1) * a.nrows;
     L.pv = a.prefix + (uint64_t)(l * 2 + 0) * a.nrows;
     L.pt = a.prefix + (uint64_t)(l * 2 + 1) * a.nrows;
     L.v0 = L.pv[0];
@@ -38,11 +34,19 @@ __device__ __forceinline__ EmitLevel emit_level(const JobArgs& a, uint32_t l)
     return L;
 }
 
+/* A chunk's in-row prefix among the bits of its word (kHalfBusy, kWordBusy). */
+__device__ __forceinline__ uint32_t prefix_mask(const JobArgs& a) { return a.NC <= 64 ? kHalfBusy - 1u : kWordBusy - 1u; }
+
+__device__ __forceinline__ uint32_t triangles_before(const JobArgs& a, const EmitLevel& L, uint64_t w)
+{
+    return (a.NC <= 64 ? L.vp[w] >> 16 : L.tp[w]) & prefix_mask(a);
+}
+
 /* Calls batch(n) for every group of n <= N chunks of the level with a
  * crossing edge (V) or a triangle (!V), queued in q[0 .. n) (emit_queued;
- * chunk_place tells where they lie; q: N + 64 entries).  The prefixes of
- * kScan units are in flight together, since the test of a unit is one dependent load.
- * Across a batch only the units' busy masks stay live (scalars). */
+ * chunk_place tells where they lie; q: N + 64 entries).  The words of kScan units
+ * are in flight together, since the test of a unit is one dependent load.
+ * Across a batch only a bit per unit stays live in a lane. */
 constexpr uint32_t kScan = 4;
 
 __device__ __forceinline__ uint32_t emit_wave() { return blockIdx.x * (uint32_t)kWaves + uniform(threadIdx.x >> 6); }
@@ -51,44 +55,48 @@ template <bool V, uint32_t N, typename F>
 __device__ __forceinline__ void busy_chunks(const JobArgs& a, const EmitLevel& L, uint32_t* q, F&& batch)
 {
     const uint32_t lane = threadIdx.x & 63u;
-    const uint64_t nwaves = emit_waves(a);
+    const uint64_t nwaves = a.ewaves, words = a.nrows * a.NC;
     const bool packed = a.NC <= 64;        // vertices in the low, triangles in the high half of vpc
     const uint32_t* pre = V || packed ? L.vp : L.tp;
-    const uint32_t* row_end = V ? L.cv : L.ct;
-    const uint32_t sh = V || !packed ? 0u : 16u, mask = packed ? 0xFFFFu : ~0u;
+    const uint32_t bit = V && packed ? kHalfBusy : kWordBusy;
+    const uint32_t wave = emit_wave();
     uint32_t qn = 0, step = 0;
-    for (uint64_t u0 = emit_wave(); u0 < a.eunits; u0 += nwaves * kScan, step += kScan) {
-        uint32_t p0[kScan], p1[kScan];
+    for (uint64_t u0 = wave < a.ewaves ? wave : a.eunits; u0 < a.eunits; u0 += nwaves * kScan, step += kScan) {
+        uint32_t p[kScan];
         /* (opaque, so that nothing made of it stays in a register over the batches) */
         uint32_t slot = lane;
         asm volatile("" : "+v"(slot));
-        const uint32_t sub = lane_row(a, slot), cl = lane_chunk(a, slot), o = sub * a.NC + cl;
+        const bool on = lane_piece(a, slot) < a.eparts && lane_chunk(a, slot) < a.NC;
+        /* a unit's first piece, whole rows: lanes lie `off` words on from it */
+        const uint64_t piece = (uint64_t)a.NC << (a.plog - a.eshift);
+        const uint64_t off = lane_piece(a, slot) * (a.edist * piece) + lane_row(a, slot) * a.NC + lane_chunk(a, slot);
+        /* steps left: most walks of a small volume have one or two */
+        uint32_t n_left = 1;
+#pragma unroll
+        for (uint32_t k = 1; k < kScan; ++k) n_left += u0 + k * nwaves < a.eunits ? 1u : 0u;
 #pragma unroll
         for (uint32_t k = 0; k < kScan; ++k) {
-            const uint64_t u = u0 + k * nwaves;
-            const EmitPart at = emit_part(a, u);
-            const uint64_t row = uniform64(at.row), left = u < a.eunits ? a.nrows - row : 0;
-            const uint32_t chunk = uniform(at.chunk), chunks = a.NC - chunk;
-            const uint32_t* words = pre + (row * a.NC + chunk);
-            const uint32_t* ends = row_end + row;
-            p0[k] = p1[k] = 0u;
-            if (sub < (left < a.erows ? (uint32_t)left : a.erows) && cl < chunks) {
-                p0[k] = (words[o] >> sh) & mask;
-                p1[k] = cl + 1 == chunks ? ends[sub] : (words[o + 1] >> sh) & mask;
+            p[k] = 0u;
+            if (k < n_left) {
+                const uint64_t u = u0 + k * nwaves;
+                uint64_t w = u * (a.ehop * piece) + off;
+                if (a.esegs > 1) {
+                    const EmitSlot s = emit_slot(a, u, slot);
+                    w = s.chunk < a.NC ? s.row * a.NC + s.chunk : words;
+                }
+                if (on && w < words) p[k] = pre[w];
             }
         }
-        uint64_t busy[kScan];
+        uint32_t busy = 0;
 #pragma unroll
-        for (uint32_t k = 0; k < kScan; ++k) busy[k] = __ballot(p0[k] != p1[k]);
+        for (uint32_t k = 0; k < kScan; ++k) busy |= (p[k] & bit) ? 1u << k : 0u;
         const bool last = u0 + nwaves * kScan >= a.eunits;
 #pragma unroll 1
-        for (uint32_t k = 0; k < kScan; ++k) {
-            uint64_t bm = busy[0];
-#pragma unroll
-            for (uint32_t j = 1; j < kScan; ++j) bm = k == j ? busy[j] : bm;
+        for (uint32_t k = 0; k < n_left; ++k) {
+            const uint64_t bm = __ballot((busy >> k) & 1u);
             if ((bm >> lane) & 1ull) q[qn + lanes_below(bm)] = emit_queued(step + k, lane);
             qn += (uint32_t)__popcll(bm);
-            const bool end = last && k == kScan - 1;
+            const bool end = last && k == n_left - 1;
             while (qn >= N || (end && qn)) {
                 wave_sync();
                 const uint32_t n = qn < N ? qn : N;
@@ -108,9 +116,9 @@ __device__ __forceinline__ void busy_chunks(const JobArgs& a, const EmitLevel& L
 /* Row, its y and z, and chunk of the row of a queued slot of this wave. */
 __device__ __forceinline__ void chunk_place(const JobArgs& a, uint32_t queued, uint64_t& r, uint32_t& y, uint32_t& z, uint32_t& c)
 {
-    const EmitPart at = emit_part(a, emit_unit(a, emit_wave(), queued));
-    r = at.row + lane_row(a, queued & 63u);
-    c = at.chunk + lane_chunk(a, queued & 63u);
+    const EmitSlot s = emit_slot(a, emit_unit(a, emit_wave(), queued), queued & 63u);
+    r = s.row;
+    c = s.chunk;
     row_place(a, r, y, z);
 }
 
@@ -235,7 +243,7 @@ __device__ __forceinline__ void list_triangles(const JobArgs& a, const EmitLevel
         uint32_t y, z, c;
         chunk_place(a, s.q[lane], r, y, z, c);
         const uint64_t w = r * a.NC + c;
-        const uint64_t base = (L.pt[r] - L.t0) + (a.NC <= 64 ? L.vp[w] >> 16 : L.tp[w]);
+        const uint64_t base = (L.pt[r] - L.t0) + triangles_before(a, L, w);
         act = masks(r, y, z, c, base);
         s.out[lane] = base;
     }

@@ -252,7 +252,7 @@ __device__ __forceinline__ void chunk_triangles(const JobArgs& a, const EmitLeve
         s.m[3][lane] = o.k7;
         s.next[lane] = o.next;
         s.key[lane] = (uint64_t)(c * 64u) | (uint64_t)y << 20 | (uint64_t)(z - 1) << 40;
-        s.out[lane] = (L.pt[r] - L.t0) + (a.NC <= 64 ? L.vp[w] >> 16 : L.tp[w]);
+        s.out[lane] = (L.pt[r] - L.t0) + triangles_before(a, L, w);
     }
     const uint32_t incl = wave_incl_scan((uint32_t)__popcll(act));
     const uint32_t excl = incl - (uint32_t)__popcll(act);
@@ -436,7 +436,7 @@ __device__ __forceinline__ void chunk_points(const JobArgs& a, const EmitLevel& 
         mx = (b ^ (b >> 1 | b1 << 63)) & valid_mask(c, a.nx - 1);
         my = (b ^ u) & vn;
         mz = (b ^ nz) & vn;
-        base = (L.pv[r] - L.v0) + (a.NC <= 64 ? L.vp[r * a.NC + c] & 0xFFFFu : L.vp[r * a.NC + c]);
+        base = (L.pv[r] - L.v0) + (L.vp[r * a.NC + c] & prefix_mask(a));
         s.key[lane] = (uint64_t)(c * 64u) | (uint64_t)y << 20 | (uint64_t)z << 40;
         chunk(r, y, z, c);
     }
@@ -653,7 +653,7 @@ __device__ __forceinline__ CellMasks load_row_cross(const JobArgs& a, const Emit
     load_words(L.pv + r0, v0, v1);
     load_words(L.pv + r2, v2, v3);
     const uint32_t* vp = L.vp + r0 * a.NC + c;
-    const uint32_t mask = a.NC <= 64 ? 0xFFFFu : ~0u;
+    const uint32_t mask = prefix_mask(a);
     const uint32_t e0 = vp[0] & mask, e1 = vp[a.NC] & mask, e2 = vp[sw] & mask, e3 = vp[sw + a.NC] & mask;
     const uint64_t vx = valid_mask(c, a.nx - 1), vn = valid_mask(c, a.nx);
     auto cross = [&](RowCross& k, uint64_t b, uint64_t b1, uint64_t up, uint64_t nz, uint64_t pre, uint32_t e,
@@ -944,7 +944,7 @@ __device__ __forceinline__ void normals_level(const JobArgs& a, uint32_t l, cons
     const uint32_t* crec = triangles ? a.crec + a.toff[l] : (const uint32_t*)L.bits;   // read, not used, without one
     const uint64_t* act_l = a.act + (uint64_t)l * (a.nrows * a.NC);
     const uint32_t* tri_pre = a.NC <= 64 ? L.vp : L.tp;   // packed: triangles in the high half of vp
-    const uint32_t sh = a.NC <= 64 ? 16u : 0u;
+    const uint32_t sh = a.NC <= 64 ? 16u : 0u, mask = prefix_mask(a);
     busy_chunks<true, kNormalChunks>(a, L, s.p.q, [&](uint32_t n) {
         chunk_points(a, L, s.p, n, [&](uint64_t r, uint32_t y, uint32_t z, uint32_t c) {
 /* cell row (cy, cz) is kept at node row (cy, cz + 1): node rows r -
@@ -963,8 +963,8 @@ __device__ __forceinline__ void normals_level(const JobArgs& a, uint32_t l, cons
                 load_words(act_l + w1, act1, act);
                 uint32_t e1, e;
                 load_pair(tri_pre + w1, e1, e);
-                e1 = base + (e1 >> sh);
-                e = base + (e >> sh);
+                e1 = base + (e1 >> sh & mask);
+                e = base + (e >> sh & mask);
                 if (w == 0) { act = act1; e = e1; }
                 RowCells o;
                 o.act = act;
@@ -992,7 +992,7 @@ __device__ __forceinline__ void stage_use_cases(UseCases& t)
     __syncthreads();
 }
 
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_normals(JobArgs a)
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_normals(JobArgs a)
 {
     __shared__ __attribute__((aligned(16))) UseCases use;
     __shared__ NormalLds s[kWaves];

@@ -49,6 +49,13 @@ constexpr int kEmitTeams = 4;        // emit workgroup: 4 independent one-wave t
 constexpr int kEmitBlock = 64 * kEmitTeams;
 constexpr uint32_t kTableBytes = 256 * 8;   // case table at the start of the emit workgroup's LDS
 
+/* In-row prefixes of a chunk: rows of at most 64 chunks keep both in a word of vpc,
+ * vertices in the low and triangles in the high half, longer rows one in vpc and one in
+ * tpc.  At most 63 chunks of 192 and 320 come before a chunk of such a row (14 and 15
+ * bits), 2^14 of any row (23 bits): the top bit of each half, or word, says whether
+ * the chunk itself has any. */
+constexpr uint32_t kHalfBusy = 1u << 15, kWordBusy = 1u << 31;
+
 struct JobArgs {
     const void* values;
     uint32_t nx, ny, nz;
@@ -67,10 +74,13 @@ struct JobArgs {
     uint32_t team_stride;  // bytes of LDS per team (>= the team layout's size)
     uint32_t teams;        // teams per emit workgroup (<= kEmitTeams; fewer when a team's LDS is large)
     uint64_t nunits;   // nlev * nb * nslabs
-    uint32_t erows;    // chunk-batch emit: node rows per wave step (at most 64 >> cshift),
-    uint32_t esegs;    // ... steps per row (of more than 64 chunks),
-    uint64_t eunits;   // ... steps of all waves per level
-    uint32_t eblocks;  // ... and workgroups per level (kmc_plan.h)
+    // chunk-batch emit (kmc_plan.h): log2 of the chunk lanes of a row and of the
+    // lanes of a piece; pieces per row and per unit; a level's units; pieces from
+    // a unit to the next and between those of a unit; the waves that share a
+    // level's units and their workgroups
+    uint32_t eshift, plog, esegs, eparts;
+    uint64_t eunits, ehop, edist;
+    uint32_t ewaves, eblocks;
     double seg_inverse, ny_inverse;   // 1 / esegs, 1 / ny (div_by)
     uint64_t nrows;    // nz * ny: counts and prefixes are kept per node row
     double minv, maxv; // clamp range of the interpolation (volume min/max)
@@ -90,7 +100,8 @@ struct JobArgs {
     uint64_t* bitvol;
     // optional, same layout as bitvol: per chunk the exclusive prefix within its
     // row of the vertex counts (vpc) and of the triangle counts of cell row
-    // (y, z-1) (tpc); written by the count pass when non-null
+    // (y, z-1) (tpc), and whether the chunk has any (chunk_words); written by the
+    // count pass when non-null
     uint32_t* vpc;
     uint32_t* tpc;
     // VertexNormal: per triangle its face normal, per active cell its case and

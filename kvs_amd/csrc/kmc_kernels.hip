@@ -1219,11 +1219,12 @@ __device__ __forceinline__ void count_rows_t(const JobArgs& a, const uint8_t* ta
                          * faster).  Rows of at most 64 chunks are one group,
                          * so the packed scan result is the chunk's in-row
                          * prefix pair */
+                        const uint32_t hv = cv ? kHalfBusy : 0u, ht = ct ? kWordBusy : 0u;
                         if (a.NC <= 64) {
-                            __builtin_nontemporal_store(e, &a.vpc[w]);
+                            __builtin_nontemporal_store(e | hv | ht, &a.vpc[w]);
                         } else {
-                            __builtin_nontemporal_store(vc + (e & 0xFFFFu), &a.vpc[w]);
-                            __builtin_nontemporal_store(tc + (e >> 16), &a.tpc[w]);
+                            __builtin_nontemporal_store((vc + (e & 0xFFFFu)) | hv << 16, &a.vpc[w]);
+                            __builtin_nontemporal_store((tc + (e >> 16)) | ht, &a.tpc[w]);
                         }
                     }
                     vc += s & 0xFFFFu;

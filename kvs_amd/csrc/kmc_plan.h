@@ -3,10 +3,11 @@
  * the waves of the chunk-batch emit.  Plain C++, shared by the host's planning,
  * the kernels and the host-side tests.
  *
- * A *unit* is what a wave looks at in one step, a slot per lane: a.erows node rows
- * of up to 64 chunks, or one of the a.esegs parts of a longer row.  Wave w takes
- * units w, w + waves, w + 2 waves, ...; a slot is known to its wave by the step
- * and the lane alone, so 32 bits name it in volumes of any number of rows.
+ * A *piece* is a run of up to 16 lanes' slots: 8 or 16 chunks of a row, or all
+ * chunks of one or more short rows.  A *unit*, what a wave looks at in one step,
+ * is a.eparts pieces, side by side or equal distances apart over the level.  Wave w
+ * takes units w, w + waves, w + 2 waves, ...; a slot is known to its wave by
+ * the step and the lane alone, so 32 bits name it in volumes of any number of rows.
  */
 #pragma once
 #include <stdint.h>
@@ -28,38 +29,38 @@ namespace kmc {
  * a device. */
 KMC_HD inline uint64_t div_by(uint64_t x, double inverse) { return (uint64_t)(((double)x + 0.5) * inverse); }
 
-KMC_HD inline uint32_t emit_waves(const JobArgs& a) { return a.eblocks * (uint32_t)kWaves; }
+/* What a lane looks at: the piece of the unit, the row of the piece and the chunk of
+ * the row's part.  Pieces from a.eparts on, chunks past the row and rows past the
+ * last hold nothing. */
+KMC_HD inline uint32_t lane_piece(const JobArgs& a, uint32_t lane) { return lane >> a.plog; }
+KMC_HD inline uint32_t lane_row(const JobArgs& a, uint32_t lane) { return (lane & ((1u << a.plog) - 1u)) >> a.eshift; }
+KMC_HD inline uint32_t lane_chunk(const JobArgs& a, uint32_t lane) { return lane & ((1u << a.eshift) - 1u); }
 
-/* First row and first chunk of a unit; the same on all lanes of its wave. */
-struct EmitPart {
+struct EmitSlot {
     uint64_t row;
     uint32_t chunk;
 };
 
-KMC_HD inline EmitPart emit_part(const JobArgs& a, uint64_t unit)
+KMC_HD inline EmitSlot emit_slot(const JobArgs& a, uint64_t unit, uint32_t lane)
 {
-    EmitPart p;
-    uint64_t group = unit;
-    p.chunk = 0;
+    EmitSlot s;
+    uint64_t group = unit * a.ehop + lane_piece(a, lane) * a.edist;
+    s.chunk = lane_chunk(a, lane);
     if (a.esegs > 1) {
-        group = div_by(unit, a.seg_inverse);
-        p.chunk = (uint32_t)(unit - group * a.esegs) << a.cshift;
+        const uint64_t piece = group;
+        group = div_by(piece, a.seg_inverse);
+        s.chunk += (uint32_t)(piece - group * a.esegs) << a.eshift;
     }
-    p.row = group * a.erows;
-    return p;
+    s.row = (group << (a.plog - a.eshift)) + lane_row(a, lane);
+    return s;
 }
-
-/* Row of the unit and chunk of the row that a lane looks at.  Rows from a.erows on,
- * and slots past the row's chunks or the last row, hold nothing. */
-KMC_HD inline uint32_t lane_row(const JobArgs& a, uint32_t lane) { return lane >> a.cshift; }
-KMC_HD inline uint32_t lane_chunk(const JobArgs& a, uint32_t lane) { return lane & ((1u << a.cshift) - 1u); }
 
 /* A slot as its wave queues it, and the unit that it came from. */
 KMC_HD inline uint32_t emit_queued(uint32_t step, uint32_t lane) { return step << 6 | lane; }
 
 KMC_HD inline uint64_t emit_unit(const JobArgs& a, uint32_t wave, uint32_t queued)
 {
-    return wave + (uint64_t)(queued >> 6) * emit_waves(a);
+    return wave + (uint64_t)(queued >> 6) * a.ewaves;
 }
 
 /* Node row -> (y, z). */
@@ -67,6 +68,16 @@ KMC_HD inline void row_place(const JobArgs& a, uint64_t row, uint32_t& y, uint32
 {
     z = (uint32_t)div_by(row, a.ny_inverse);
     y = (uint32_t)row - z * a.ny;
+}
+
+/* The largest prime <= n (n >= 2). */
+inline uint32_t prime_below(uint32_t n)
+{
+    for (;; --n) {
+        bool prime = n >= 2;
+        for (uint32_t d = 2; prime && (uint64_t)d * d <= n; ++d) prime = n % d != 0;
+        if (prime) return n;
+    }
 }
 
 /* Wave steps of 64 (row, chunk) pairs that a pass's levels hold. */
@@ -82,36 +93,67 @@ inline uint64_t emit_steps(const JobArgs& a)
  * normals: 1666 / 1240 us with one time, 1367 / 1205 with two, 1250 / 1129
  * with eight, 1277 / 1162 with sixteen; a half-filled round costs: 512^3 CT
  * triangles 287 us with one time, 338 with 1.6) -- and no more than one per 32
- * outputs.  A wave takes as many rows at a time as its lanes hold, but at most a
- * quarter of its share of the pass: a surface lies in few neighbouring rows, and
- * four steps far apart even the waves out (256^3 blobs, duplicated: 26 us, 36
- * with two steps).  Where every chunk holds many outputs there is nothing to
- * even out, and two steps keep the batches full (320 x 288 x 256 CT, vertices:
- * 38 us, 42 with four). */
-constexpr uint64_t kEmitRounds = 8, kEmitItems = 32;
+ * outputs, but as many as leave none a walk of more than 16 steps: a small
+ * surface in a large volume is all walking (a sphere of radius 4 in 1024^3,
+ * vertex normals: 3390 us a call by outputs alone, 995 with 32 steps, 890 with 16). */
+constexpr uint64_t kEmitRounds = 8, kEmitItems = 32, kEmitWalk = 16;
 
 /* Split of the chunk-batch emit (rows planned; a.nlev set) of a pass whose emit
  * shares its launch with others, `all` being the sum of their emit_steps, for a
  * kernel of which a CU holds per_cu workgroups and that produces `items` outputs
- * (0: not known yet). */
+ * (0: not known yet).
+ *
+ * A wave takes 64 slots a step, but at most a quarter of its share of the pass:
+ * four steps far apart even the waves out (256^3 blobs, duplicated: 26 us, 36
+ * with two steps).  Where every chunk holds many outputs there is nothing to
+ * even out, and two steps keep the batches full (320 x 288 x 256 CT, vertices:
+ * 38 us, 42 with four).  Rows of 64 chunks and more are cut down to 8 of them a
+ * step: few rows of full chunks are long chains of work (9000 x 40 x 33 blobs,
+ * vertex normals: 270 us a call with a row's 64 chunks a step, 190 with 16, 146
+ * with 8).
+ *
+ * Pieces far apart share a sheet out (a plane of one z in 1024^3, vertex normals:
+ * 1184 us a call with pieces side by side, 943 so), pieces side by side share
+ * cache lines of neighbouring rows and slices, which counts where those of a
+ * slice do not stay in the L2 (1024^3 turbulence, three levels: 4150 us side by
+ * side, 4670 far apart; 512^3 CT 820 and 812): side by side only in volumes of
+ * 2^22 slots and more a level with an output in every sixth of them, and in rows
+ * that are cut anyway (6000 x 150 x 120 blobs, vertex normals: 224 and 244).
+ *
+ * The number of waves is made prime where they take several steps, so that no period of
+ * the rows meets the same waves again and again (a plane of one y in 1024^3, whose rows
+ * lie 1024 apart: 128 of 32768 waves had all of it, 2990 us a call, 1360 so). */
 inline void plan_emit(JobArgs& a, uint64_t all, uint32_t per_cu = 4, uint64_t items = 0)
 {
-    const uint64_t own = emit_steps(a), nlev = std::max(1u, a.nlev);
+    const uint64_t own = emit_steps(a), nlev = std::max(1u, a.nlev), slots = a.nrows * a.NC;
     const uint64_t resident = 256ull * kWaves * per_cu;
     uint64_t waves = resident * std::min(kEmitRounds, std::max<uint64_t>(1, all / 4 / resident));
-    if (items) waves = std::min(waves, std::max<uint64_t>(256, items / kEmitItems));
+    if (items) waves = std::min(waves, std::max<uint64_t>(256, std::max(items / kEmitItems, all / kEmitWalk)));
     else waves = std::max(waves, std::min(2 * resident, all / 4));   // a batch's uneven passes even out by themselves
     const uint64_t want = std::max<uint64_t>(1, (waves * own + all - 1) / all / nlev);   // waves per level
-    const uint64_t steps = items > 4 * nlev * a.nrows * a.NC ? 2 : 4;
-    a.erows = 64u >> a.cshift;
-    while (a.erows > 1 && a.nrows / a.erows < steps * want) a.erows >>= 1;
-    a.esegs = (a.NC + 63) / 64;
+    const uint64_t steps = items > 4 * nlev * slots ? 2 : 4;
+    a.eshift = std::min(a.cshift, 4u);
+    a.plog = 4;
+    a.eparts = 4;
+    auto segs = [&] { return (a.NC + (1u << a.eshift) - 1) >> a.eshift; };
+    auto pieces = [&] { return (((a.nrows - 1) >> (a.plog - a.eshift)) + 1) * segs(); };
+    while (pieces() / a.eparts < steps * want && (a.eparts > 1 || a.plog > a.eshift)) {
+        if (a.eparts > 1) a.eparts >>= 1;
+        else --a.plog;
+    }
+    if (pieces() / a.eparts < 8 * want && a.NC >= 64) a.plog = a.eshift = 3;
+    a.esegs = segs();
     a.seg_inverse = 1.0 / a.esegs;
     a.ny_inverse = 1.0 / a.ny;
-    a.eunits = (a.nrows + a.erows - 1) / a.erows * a.esegs;
+    a.eunits = (pieces() + a.eparts - 1) / a.eparts | 1;   // odd: the pieces of a unit meet no period of the rows either
+    const bool far = a.NC < 64 && (slots < 1u << 22 || (items && items / nlev < slots / 6));
+    a.ehop = far ? 1 : a.eparts;
+    a.edist = far ? a.eunits : 1;
     /* (a step's number has 26 bits in the queue) */
-    const uint64_t least = (a.eunits >> 26) + 1;
+    const uint64_t least = (a.eunits >> 25) + 1;
     a.eblocks = (uint32_t)std::max<uint64_t>(1, (std::max(least, std::min(a.eunits, want)) + kWaves - 1) / kWaves);
+    a.ewaves = a.eblocks * (uint32_t)kWaves;
+    if (a.eunits > a.ewaves) a.ewaves = prime_below(a.ewaves);
 }
 
 }  // namespace kmc

@@ -1,5 +1,6 @@
 """The emit's plan (kmc_plan.h) on the host: what a wave queues names the slot it
-looked at, in volumes of any number of rows."""
+looked at, in volumes of any number of rows, every slot is looked at once, and small
+or flat surfaces fall to many waves."""
 import os
 import subprocess
 
@@ -16,7 +17,7 @@ def plan_check(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["slots", "places", "large"])
+@pytest.mark.parametrize("what", ["slots", "places", "large", "shares"])
 def test_emit_slots(plan_check, what):
     r = subprocess.run([plan_check, what], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout
