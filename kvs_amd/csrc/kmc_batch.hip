@@ -249,14 +249,15 @@ struct Group {
     int dtype;
     int mode;                    // 0 duplicated, 1 PolygonNormal, 2 VertexNormal
     uint32_t p0, p1;             // passes [p0, p1)
-    uint64_t max_chunks, max_groups;   // the most chunks and row groups of one of its passes
     uint64_t units;
     uint32_t max_levels;         // the most levels of one of its passes
-    uint32_t emit_blocks;        // the most emit workgroups per level of one of its passes
     uint32_t emit_lds;
     uint32_t teams;                // emit teams per workgroup
     uint64_t* unit_start_d;      // p1 - p0 + 1 entries
-    std::vector<uint64_t> unit_start_h;   // upload source, kept while the copy may run
+    BlockRef* refs_d;              // workgroups of the classification, the count and the emit
+    uint32_t ncls, ncnt, nemit;
+    std::vector<uint64_t> unit_start_h;   // upload sources, kept while the copies may run
+    std::vector<BlockRef> refs_h;
 };
 
 }  // namespace
@@ -314,7 +315,9 @@ void free_plan_buffers(kmc_batch* b)
 {
     for (Group& g : b->groups) {
         device_free(g.unit_start_d);
+        device_free(g.refs_d);
         g.unit_start_d = nullptr;
+        g.refs_d = nullptr;
     }
 }
 
@@ -374,21 +377,20 @@ kmc_status plan_tiles(kmc_batch* b, uint32_t r_max, uint32_t queue_cap)
         uint64_t steps = 0;
         for (uint32_t i = g.p0; i < g.p1; ++i) steps += emit_steps(b->passes[i].a);
         for (uint32_t i = g.p0; i < g.p1 && !b->two_phase; ++i) plan_emit(b->passes[i].a, steps);
-        std::vector<uint64_t> ts;
+        std::vector<uint64_t> ts, cls, cnt;
+        std::vector<BlockRef> emit;
         uint64_t t = 0;
         uint32_t stride = 0, teams = kEmitTeams;
         g.max_levels = 0;
-        g.emit_blocks = 1;
-        g.max_chunks = g.max_groups = 0;
         for (uint32_t i = g.p0; i < g.p1; ++i) {
             const JobArgs& a = b->passes[i].a;
-            g.max_chunks = std::max(g.max_chunks, a.nrows * a.NC);
-            g.max_groups = std::max(g.max_groups, (a.nrows << a.cshift) / 64 + 1);
+            cls.push_back(classify_blocks(a));
+            cnt.push_back(count_blocks(a));
+            for (uint32_t l = 0; l < a.nlev && !b->two_phase; ++l) add_blocks(emit, i - g.p0, l, a.eblocks);
             ts.push_back(t);
             t += b->passes[i].a.nunits;
             stride = std::max(stride, b->passes[i].a.team_stride);
             g.max_levels = std::max(g.max_levels, b->passes[i].a.nlev);
-            g.emit_blocks = std::max(g.emit_blocks, b->passes[i].a.eblocks);
         }
         /* one emit launch per group: every team region of a workgroup is as
          * large as the group's largest, and as many teams as 64 KiB hold */
@@ -406,6 +408,19 @@ kmc_status plan_tiles(kmc_batch* b, uint32_t r_max, uint32_t queue_cap)
         if (!g.unit_start_d) return KMC_ERR_OUT_OF_MEMORY;
         g.unit_start_h = std::move(ts);
         if (hipMemcpyAsync(g.unit_start_d, g.unit_start_h.data(), g.unit_start_h.size() * 8, hipMemcpyHostToDevice,
+                           b->upload_stream) != hipSuccess)
+            return KMC_ERR_DEVICE;
+        if (b->two_phase) continue;
+        g.refs_h = front_blocks(cls);
+        g.ncls = (uint32_t)g.refs_h.size();
+        const std::vector<BlockRef> count = front_blocks(cnt);
+        g.ncnt = (uint32_t)count.size();
+        g.nemit = (uint32_t)emit.size();
+        g.refs_h.insert(g.refs_h.end(), count.begin(), count.end());
+        g.refs_h.insert(g.refs_h.end(), emit.begin(), emit.end());
+        g.refs_d = (BlockRef*)device_alloc(g.refs_h.size() * sizeof(BlockRef));
+        if (!g.refs_d) return KMC_ERR_OUT_OF_MEMORY;
+        if (hipMemcpyAsync(g.refs_d, g.refs_h.data(), g.refs_h.size() * sizeof(BlockRef), hipMemcpyHostToDevice,
                            b->upload_stream) != hipSuccess)
             return KMC_ERR_DEVICE;
     }
@@ -432,8 +447,7 @@ hipError_t record_front(kmc_batch* b, hipStream_t st, bool copy_sizes)
     if (copy_sizes) {
         /* launched from the host (the serving form's two phases): each pass
          * as the plain call's classify and count, its arguments in the
-         * launch -- for the large volumes served, faster than the batch
-         * kernels' shared row ranges */
+         * launch */
         for (const Group& g : b->groups)
             for (uint32_t i = g.p0; i < g.p1 && e == hipSuccess; ++i) {
                 e = launch_classify(g.dtype, b->passes[i].a, st);
@@ -442,11 +456,11 @@ hipError_t record_front(kmc_batch* b, hipStream_t st, bool copy_sizes)
         if (e != hipSuccess) return e;
     } else {
         for (const Group& g : b->groups) {
-            e = launch_classify_batch(g.dtype, b->jobs_d + g.p0, g.p1 - g.p0, g.max_chunks, g.max_levels, st);
+            e = launch_classify_batch(g.dtype, b->jobs_d + g.p0, g.refs_d, g.ncls, g.max_levels, st);
             if (e != hipSuccess) return e;
         }
         for (const Group& g : b->groups) {
-            e = launch_count_batch(b->jobs_d + g.p0, g.p1 - g.p0, g.max_groups, st);
+            e = launch_count_batch(b->jobs_d + g.p0, g.refs_d + g.ncls, g.ncnt, st);
             if (e != hipSuccess) return e;
         }
     }
@@ -474,7 +488,7 @@ hipError_t record_emit(kmc_batch* b, hipStream_t st, bool host_sizes)
             if (host_sizes)
                 for (uint32_t i = g.p0; i < g.p1 && e == hipSuccess; ++i) e = launch_chunk_emit(g.dtype, b->passes[i].a, st);
             else
-                e = launch_chunk_emit_batch(g.dtype, g.mode, b->jobs_d + g.p0, g.p1 - g.p0, g.emit_blocks, g.max_levels, st);
+                e = launch_chunk_emit_batch(g.dtype, g.mode, b->jobs_d + g.p0, g.refs_d + g.ncls + g.ncnt, g.nemit, st);
             if (e != hipSuccess) return e;
         }
         return e;

@@ -18,9 +18,10 @@ struct EmitLevel {
     const uint64_t* pv;      // row prefixes
     const uint64_t* pt;
     uint64_t v0, t0;         // first prefix of each (outputs index from 0)
+    uint32_t wave;           // this wave among the level's
 };
 
-__device__ __forceinline__ EmitLevel emit_level(const JobArgs& a, uint32_t l)
+__device__ __forceinline__ EmitLevel emit_level(const JobArgs& a, uint32_t l, uint32_t block)
 {
     const uint64_t words = (uint64_t)l * (a.nrows * a.NC);
     EmitLevel L;
@@ -31,6 +32,7 @@ __device__ __forceinline__ EmitLevel emit_level(const JobArgs& a, uint32_t l)
     L.pt = a.prefix + (uint64_t)(l * 2 + 1) * a.nrows;
     L.v0 = L.pv[0];
     L.t0 = L.pt[0];
+    L.wave = block * (uint32_t)kWaves + uniform(threadIdx.x >> 6);
     return L;
 }
 
@@ -49,8 +51,6 @@ __device__ __forceinline__ uint32_t triangles_before(const JobArgs& a, const Emi
  * Across a batch only a bit per unit stays live in a lane. */
 constexpr uint32_t kScan = 4;
 
-__device__ __forceinline__ uint32_t emit_wave() { return blockIdx.x * (uint32_t)kWaves + uniform(threadIdx.x >> 6); }
-
 template <bool V, uint32_t N, typename F>
 __device__ __forceinline__ void busy_chunks(const JobArgs& a, const EmitLevel& L, uint32_t* q, F&& batch)
 {
@@ -59,7 +59,7 @@ __device__ __forceinline__ void busy_chunks(const JobArgs& a, const EmitLevel& L
     const bool packed = a.NC <= 64;        // vertices in the low, triangles in the high half of vpc
     const uint32_t* pre = V || packed ? L.vp : L.tp;
     const uint32_t bit = V && packed ? kHalfBusy : kWordBusy;
-    const uint32_t wave = emit_wave();
+    const uint32_t wave = L.wave;
     uint32_t qn = 0, step = 0;
     for (uint64_t u0 = wave < a.ewaves ? wave : a.eunits; u0 < a.eunits; u0 += nwaves * kScan, step += kScan) {
         uint32_t p[kScan];
@@ -114,9 +114,9 @@ __device__ __forceinline__ void busy_chunks(const JobArgs& a, const EmitLevel& L
 }
 
 /* Row, its y and z, and chunk of the row of a queued slot of this wave. */
-__device__ __forceinline__ void chunk_place(const JobArgs& a, uint32_t queued, uint64_t& r, uint32_t& y, uint32_t& z, uint32_t& c)
+__device__ __forceinline__ void chunk_place(const JobArgs& a, const EmitLevel& L, uint32_t queued, uint64_t& r, uint32_t& y, uint32_t& z, uint32_t& c)
 {
-    const EmitSlot s = emit_slot(a, emit_unit(a, emit_wave(), queued), queued & 63u);
+    const EmitSlot s = emit_slot(a, emit_unit(a, L.wave, queued), queued & 63u);
     r = s.row;
     c = s.chunk;
     row_place(a, r, y, z);
@@ -241,7 +241,7 @@ __device__ __forceinline__ void list_triangles(const JobArgs& a, const EmitLevel
     if (lane < n) {
         uint64_t r;
         uint32_t y, z, c;
-        chunk_place(a, s.q[lane], r, y, z, c);
+        chunk_place(a, L, s.q[lane], r, y, z, c);
         const uint64_t w = r * a.NC + c;
         const uint64_t base = (L.pt[r] - L.t0) + triangles_before(a, L, w);
         act = masks(r, y, z, c, base);

@@ -242,7 +242,7 @@ __device__ __forceinline__ void chunk_triangles(const JobArgs& a, const EmitLeve
     if (lane < n) {
         uint64_t r;
         uint32_t y, z, c;
-        chunk_place(a, s.q[lane], r, y, z, c);
+        chunk_place(a, L, s.q[lane], r, y, z, c);
         const CellMasks o = load_cells(a, L, y, z, c);
         const uint64_t w = r * a.NC + c;
         act = o.act;
@@ -335,11 +335,11 @@ __device__ __forceinline__ void chunk_triangles(const JobArgs& a, const EmitLeve
 /* ------------------------------------------------------------------------- */
 
 template <typename T>
-__device__ __forceinline__ void dup_level(const JobArgs& a, uint32_t l, const CaseLds& tab, CellLds<T>& s)
+__device__ __forceinline__ void dup_level(const JobArgs& a, uint32_t l, uint32_t block, const CaseLds& tab, CellLds<T>& s)
 {
     if (!a.cap_triangles[l]) return;       // a level without outputs
     const uint32_t lane = threadIdx.x & 63u;
-    const EmitLevel L = emit_level(a, l);
+    const EmitLevel L = emit_level(a, l, block);
     const double iso = a.iso[l];
     float* coords = a.coords[l];
     float* normals = a.normals[l];
@@ -381,18 +381,18 @@ __global__ __launch_bounds__(kBlock) void k_dup(JobArgs a)
     __shared__ CaseLds tab;
     __shared__ CellLds<T> s[kWaves];
     stage_cases(tab, d_cases_dup);
-    dup_level<T>(a, blockIdx.y, tab, s[threadIdx.x >> 6]);
+    dup_level<T>(a, blockIdx.y, blockIdx.x, tab, s[threadIdx.x >> 6]);
 }
 
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_dup_batch(const JobArgs* jobs)
+__global__ __launch_bounds__(kBlock) void k_dup_batch(const JobArgs* jobs, const BlockRef* refs)
 {
     __shared__ CaseLds tab;
     __shared__ CellLds<T> s[kWaves];
-    const JobArgs& a = jobs[blockIdx.z];
-    if (blockIdx.y >= a.nlev || blockIdx.x >= a.eblocks) return;
+    const BlockRef r = refs[blockIdx.x];
+    const JobArgs& a = jobs[r.job];
     stage_cases(tab, d_cases_dup);
-    dup_level<T>(a, blockIdx.y, tab, s[threadIdx.x >> 6]);
+    dup_level<T>(a, r.level, r.block, tab, s[threadIdx.x >> 6]);
 }
 
 /* ------------------------------------------------------------------------- */
@@ -424,7 +424,7 @@ __device__ __forceinline__ void chunk_points(const JobArgs& a, const EmitLevel& 
     if (lane < n) {
         uint64_t r;
         uint32_t y, z, c;
-        chunk_place(a, s.q[lane], r, y, z, c);
+        chunk_place(a, L, s.q[lane], r, y, z, c);
         /* row_chunk's crossings alone: a neighbour row outside the volume is
          * read as the row itself */
         const uint64_t* row = L.bits + r * a.NC;
@@ -522,11 +522,11 @@ __device__ __forceinline__ void store_point(const JobArgs& a, double iso, float*
 }
 
 template <typename T>
-__device__ __forceinline__ void points_level(const JobArgs& a, uint32_t l, PointLds<64>& s)
+__device__ __forceinline__ void points_level(const JobArgs& a, uint32_t l, uint32_t block, PointLds<64>& s)
 {
     if (!a.cap_vertices[l]) return;        // a level without outputs
     const uint32_t lane = threadIdx.x & 63u;
-    const EmitLevel L = emit_level(a, l);
+    const EmitLevel L = emit_level(a, l, block);
     const double iso = a.iso[l];
     float* coords = a.coords[l];
     busy_chunks<true, 64>(a, L, s.q, [&](uint32_t n) {
@@ -548,16 +548,16 @@ template <typename T>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) void k_points(JobArgs a)
 {
     __shared__ PointLds<64> s[kWaves];
-    points_level<T>(a, blockIdx.y, s[threadIdx.x >> 6]);
+    points_level<T>(a, blockIdx.y, blockIdx.x, s[threadIdx.x >> 6]);
 }
 
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_points_batch(const JobArgs* jobs)
+__global__ __launch_bounds__(kBlock) void k_points_batch(const JobArgs* jobs, const BlockRef* refs)
 {
     __shared__ PointLds<64> s[kWaves];
-    const JobArgs& a = jobs[blockIdx.z];
-    if (blockIdx.y >= a.nlev || blockIdx.x >= a.eblocks) return;
-    points_level<T>(a, blockIdx.y, s[threadIdx.x >> 6]);
+    const BlockRef r = refs[blockIdx.x];
+    const JobArgs& a = jobs[r.job];
+    points_level<T>(a, r.level, r.block, s[threadIdx.x >> 6]);
 }
 
 /* ------------------------------------------------------------------------- */
@@ -723,11 +723,11 @@ __device__ __forceinline__ void fetch_face(const FaceCases& tab, const FaceLds& 
  * the chunk's active cells (a.act) and their first triangles and cases
  * (a.crec). */
 template <int M>
-__device__ __forceinline__ void faces_level(const JobArgs& a, uint32_t l, const FaceCases& tab, FaceLds& s)
+__device__ __forceinline__ void faces_level(const JobArgs& a, uint32_t l, uint32_t block, const FaceCases& tab, FaceLds& s)
 {
     if (!a.cap_triangles[l]) return;       // a level without outputs
     const uint32_t lane = threadIdx.x & 63u;
-    const EmitLevel L = emit_level(a, l);
+    const EmitLevel L = emit_level(a, l, block);
     const float* coords = a.coords[l];
     uint32_t* conn = a.conn[l];
     float* normals = M == kModeVertex ? a.fn + 3 * a.toff[l] : a.normals[l];
@@ -784,18 +784,18 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
     __shared__ __attribute__((aligned(16))) FaceCases tab;
     __shared__ FaceLds s[kWaves];
     stage_face_cases(tab);
-    faces_level<M>(a, blockIdx.y, tab, s[threadIdx.x >> 6]);
+    faces_level<M>(a, blockIdx.y, blockIdx.x, tab, s[threadIdx.x >> 6]);
 }
 
 template <int M>
-__global__ __launch_bounds__(kBlock) void k_faces_batch(const JobArgs* jobs)
+__global__ __launch_bounds__(kBlock) void k_faces_batch(const JobArgs* jobs, const BlockRef* refs)
 {
     __shared__ __attribute__((aligned(16))) FaceCases tab;
     __shared__ FaceLds s[kWaves];
-    const JobArgs& a = jobs[blockIdx.z];
-    if (blockIdx.y >= a.nlev || blockIdx.x >= a.eblocks) return;
+    const BlockRef r = refs[blockIdx.x];
+    const JobArgs& a = jobs[r.job];
     stage_face_cases(tab);
-    faces_level<M>(a, blockIdx.y, tab, s[threadIdx.x >> 6]);
+    faces_level<M>(a, r.level, r.block, tab, s[threadIdx.x >> 6]);
 }
 
 /* ------------------------------------------------------------------------- */
@@ -933,11 +933,11 @@ __device__ __forceinline__ void store_normal(const float* fn, NormalItem& o, flo
     no[2] = n[2];
 }
 
-__device__ __forceinline__ void normals_level(const JobArgs& a, uint32_t l, const UseCases& use, NormalLds& s)
+__device__ __forceinline__ void normals_level(const JobArgs& a, uint32_t l, uint32_t block, const UseCases& use, NormalLds& s)
 {
     if (!a.cap_vertices[l]) return;        // a level without outputs
     const uint32_t lane = threadIdx.x & 63u;
-    const EmitLevel L = emit_level(a, l);
+    const EmitLevel L = emit_level(a, l, block);
     float* normals = a.normals[l];
     const bool triangles = a.cap_triangles[l] != 0;   // without one no cell of the volume is active
     const float* fn = a.fn + 3 * a.toff[l];
@@ -997,17 +997,17 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
     __shared__ __attribute__((aligned(16))) UseCases use;
     __shared__ NormalLds s[kWaves];
     stage_use_cases(use);
-    normals_level(a, blockIdx.y, use, s[threadIdx.x >> 6]);
+    normals_level(a, blockIdx.y, blockIdx.x, use, s[threadIdx.x >> 6]);
 }
 
-__global__ __launch_bounds__(kBlock) void k_normals_batch(const JobArgs* jobs)
+__global__ __launch_bounds__(kBlock) void k_normals_batch(const JobArgs* jobs, const BlockRef* refs)
 {
     __shared__ __attribute__((aligned(16))) UseCases use;
     __shared__ NormalLds s[kWaves];
-    const JobArgs& a = jobs[blockIdx.z];
-    if (blockIdx.y >= a.nlev || blockIdx.x >= a.eblocks) return;
+    const BlockRef r = refs[blockIdx.x];
+    const JobArgs& a = jobs[r.job];
     stage_use_cases(use);
-    normals_level(a, blockIdx.y, use, s[threadIdx.x >> 6]);
+    normals_level(a, r.level, r.block, use, s[threadIdx.x >> 6]);
 }
 
 /* Workgroups of each kernel that a CU holds: by LDS k_dup 4 and k_faces 5, by
@@ -1038,20 +1038,16 @@ hipError_t launch_chunk_emit_t(JobArgs a, hipStream_t st, hipEvent_t* marks)
 }
 
 template <typename T>
-hipError_t launch_chunk_emit_batch_t(int mode, const JobArgs* jobs, uint32_t njobs, uint32_t blocks, uint32_t levels,
-                                     hipStream_t st)
+hipError_t launch_chunk_emit_batch_t(int mode, const JobArgs* jobs, const BlockRef* refs, uint32_t nrefs, hipStream_t st)
 {
-    constexpr uint32_t kMaxJobs = 32768;   // of one grid's z
-    for (uint32_t j = 0; j < njobs; j += kMaxJobs) {
-        const dim3 g(blocks, levels, std::min(kMaxJobs, njobs - j)), b(kBlock);
-        if (mode != kModeDup) hipLaunchKernelGGL((k_points_batch<T>), g, b, 0, st, jobs + j);
-        switch (mode) {
-        case kModeDup: hipLaunchKernelGGL((k_dup_batch<T>), g, b, 0, st, jobs + j); break;
-        case kModePolygon: hipLaunchKernelGGL((k_faces_batch<kModePolygon>), g, b, 0, st, jobs + j); break;
-        default: hipLaunchKernelGGL((k_faces_batch<kModeVertex>), g, b, 0, st, jobs + j); break;
-        }
-        if (mode == kModeVertex) hipLaunchKernelGGL(k_normals_batch, g, b, 0, st, jobs + j);
+    const dim3 g(nrefs), b(kBlock);
+    if (mode != kModeDup) hipLaunchKernelGGL((k_points_batch<T>), g, b, 0, st, jobs, refs);
+    switch (mode) {
+    case kModeDup: hipLaunchKernelGGL((k_dup_batch<T>), g, b, 0, st, jobs, refs); break;
+    case kModePolygon: hipLaunchKernelGGL((k_faces_batch<kModePolygon>), g, b, 0, st, jobs, refs); break;
+    default: hipLaunchKernelGGL((k_faces_batch<kModeVertex>), g, b, 0, st, jobs, refs); break;
     }
+    if (mode == kModeVertex) hipLaunchKernelGGL(k_normals_batch, g, b, 0, st, jobs, refs);
     return hipGetLastError();
 }
 
@@ -1074,20 +1070,20 @@ hipError_t launch_chunk_emit(int dtype, const JobArgs& a, hipStream_t st, hipEve
     }
 }
 
-hipError_t launch_chunk_emit_batch(int dtype, int mode, const JobArgs* jobs, uint32_t njobs, uint32_t blocks,
-                                   uint32_t levels, hipStream_t st)
+hipError_t launch_chunk_emit_batch(int dtype, int mode, const JobArgs* jobs, const BlockRef* refs, uint32_t nrefs,
+                                   hipStream_t st)
 {
     switch (dtype) {
-    case 0: return launch_chunk_emit_batch_t<int8_t>(mode, jobs, njobs, blocks, levels, st);
-    case 1: return launch_chunk_emit_batch_t<int16_t>(mode, jobs, njobs, blocks, levels, st);
-    case 2: return launch_chunk_emit_batch_t<int32_t>(mode, jobs, njobs, blocks, levels, st);
-    case 3: return launch_chunk_emit_batch_t<int64_t>(mode, jobs, njobs, blocks, levels, st);
-    case 4: return launch_chunk_emit_batch_t<uint8_t>(mode, jobs, njobs, blocks, levels, st);
-    case 5: return launch_chunk_emit_batch_t<uint16_t>(mode, jobs, njobs, blocks, levels, st);
-    case 6: return launch_chunk_emit_batch_t<uint32_t>(mode, jobs, njobs, blocks, levels, st);
-    case 7: return launch_chunk_emit_batch_t<uint64_t>(mode, jobs, njobs, blocks, levels, st);
-    case 8: return launch_chunk_emit_batch_t<float>(mode, jobs, njobs, blocks, levels, st);
-    default: return launch_chunk_emit_batch_t<double>(mode, jobs, njobs, blocks, levels, st);
+    case 0: return launch_chunk_emit_batch_t<int8_t>(mode, jobs, refs, nrefs, st);
+    case 1: return launch_chunk_emit_batch_t<int16_t>(mode, jobs, refs, nrefs, st);
+    case 2: return launch_chunk_emit_batch_t<int32_t>(mode, jobs, refs, nrefs, st);
+    case 3: return launch_chunk_emit_batch_t<int64_t>(mode, jobs, refs, nrefs, st);
+    case 4: return launch_chunk_emit_batch_t<uint8_t>(mode, jobs, refs, nrefs, st);
+    case 5: return launch_chunk_emit_batch_t<uint16_t>(mode, jobs, refs, nrefs, st);
+    case 6: return launch_chunk_emit_batch_t<uint32_t>(mode, jobs, refs, nrefs, st);
+    case 7: return launch_chunk_emit_batch_t<uint64_t>(mode, jobs, refs, nrefs, st);
+    case 8: return launch_chunk_emit_batch_t<float>(mode, jobs, refs, nrefs, st);
+    default: return launch_chunk_emit_batch_t<double>(mode, jobs, refs, nrefs, st);
     }
 }
 

@@ -110,13 +110,12 @@ uint32_t levels_per_pass(const kmc_volume* v, int vnormal);
 hipError_t launch_emit(int dtype, const JobArgs& a, uint32_t lds_bytes, hipStream_t st);
 /* Chunk-batch emit (kmc_emit.hip) of a pass (a.vpc / a.tpc written by its
  * count pass, outputs and capacities set; VertexNormal: a.fn, a.crec, a.act,
- * a.toff), or of a batch group's passes (`blocks` / `levels`: the most of one of
- * them).  mode: 0 duplicated vertices, 1 PolygonNormal, 2 VertexNormal (shared
+ * a.toff), or of a batch group's passes (a workgroup per ref).  mode: 0 duplicated vertices, 1 PolygonNormal, 2 VertexNormal (shared
  * vertices).  marks: three events recorded at the start, after the vertices and
  * after the triangles (timing), or null. */
 hipError_t launch_chunk_emit(int dtype, const JobArgs& a, hipStream_t st, hipEvent_t* marks = nullptr);
-hipError_t launch_chunk_emit_batch(int dtype, int mode, const JobArgs* jobs, uint32_t njobs, uint32_t blocks,
-                                   uint32_t levels, hipStream_t st);
+hipError_t launch_chunk_emit_batch(int dtype, int mode, const JobArgs* jobs, const BlockRef* refs, uint32_t nrefs,
+                                   hipStream_t st);
 hipError_t launch_classify(int dtype, const JobArgs& a, hipStream_t st);
 /* SlicePlane: masks from the plane's sign (a.plane), and the chunk-batch emit
  * of its triangles with per-vertex colours. */
@@ -137,10 +136,10 @@ size_t minmax_scratch_bytes();
 /* The unstructured form: vol[0], then vol[conn[i]] for every connection entry in order. */
 hipError_t launch_minmax_gather(int dtype, const void* vol, const uint32_t* conn, uint64_t nconn, void* scratch,
                                 double* out, hipStream_t st);
-/* chunks / groups: the most chunks, and row groups of 64 >> cshift rows, of one job */
-hipError_t launch_classify_batch(int dtype, const JobArgs* jobs, uint32_t njobs, uint64_t chunks, uint32_t max_levels,
+/* Front passes of a batch group, a workgroup per ref (front_blocks). */
+hipError_t launch_classify_batch(int dtype, const JobArgs* jobs, const BlockRef* refs, uint32_t nrefs, uint32_t max_levels,
                                  hipStream_t st);
-hipError_t launch_count_batch(const JobArgs* jobs, uint32_t njobs, uint64_t groups, hipStream_t st);
+hipError_t launch_count_batch(const JobArgs* jobs, const BlockRef* refs, uint32_t nrefs, hipStream_t st);
 /* mode: 0 duplicated vertices, 1 PolygonNormal, 2 VertexNormal (shared vertices) */
 hipError_t launch_emit_batch(int dtype, int mode, const JobArgs* jobs, const uint64_t* unit_start, uint32_t njobs,
                              uint64_t units, uint32_t lds_bytes, uint32_t teams, hipStream_t st);

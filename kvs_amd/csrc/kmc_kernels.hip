@@ -1003,19 +1003,20 @@ __device__ __forceinline__ uint32_t find_job(const uint64_t* start, uint32_t n, 
     return lo;
 }
 
-/* Classify pass of a batch of jobs sharing the value type T: job z's workgroups
- * walk its chunks in steps of the whole grid, 16 consecutive chunks a wave, so
- * that every wave has 16 loads in flight and the grid sweeps the job in address
+/* Classify pass of a batch of jobs sharing the value type T: a job's workgroups
+ * (front_blocks) walk its chunks in steps of them all, 16 consecutive chunks a
+ * wave, so that every wave has 16 loads in flight and they sweep the job in address
  * order (one contiguous range of rows per wave took 199 us on 14 volumes of 32
  * .. 256 per axis, 186 MB).  kWide: some job has more than four levels (the
  * eight-level instance's registers would otherwise halve the waves per SIMD of
  * every batch). */
 template <typename T, bool kWide>
-__global__ __launch_bounds__(kBlock) void k_classify_batch(const JobArgs* jobs)
+__global__ __launch_bounds__(kBlock) void k_classify_batch(const JobArgs* jobs, const BlockRef* refs)
 {
-    const JobArgs& a = jobs[blockIdx.z];
-    const uint64_t wave = (uint64_t)blockIdx.x * kWaves + uniform(threadIdx.x >> 6);   // uniform: scalar
-    const uint64_t step = (uint64_t)gridDim.x * kWaves * 16;
+    const BlockRef ref = refs[blockIdx.x];
+    const JobArgs& a = jobs[ref.job];
+    const uint64_t wave = (uint64_t)ref.block * kWaves + uniform(threadIdx.x >> 6);   // uniform: scalar
+    const uint64_t step = (uint64_t)ref.blocks * kWaves * 16;
     if constexpr (sizeof(T) <= 2) {
         if (packed_rows<T>(a)) {
             const uint64_t items = a.nrows * ((a.nx / (4 / sizeof(T)) + 63) / 64);
@@ -1307,16 +1308,17 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) voi
     count_job<false, 0>(a, tab);
 }
 
-/* Count pass of a batch: job z's workgroups walk its row groups in steps of the
- * whole grid. */
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_count_batch(const JobArgs* jobs)
+/* Count pass of a batch: a job's workgroups walk its row groups in steps of them
+ * all. */
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_count_batch(const JobArgs* jobs,
+                                                                                              const BlockRef* refs)
 {
-    const JobArgs& a = jobs[blockIdx.z];
-    const uint64_t G = 64u >> a.cshift, wave = (uint64_t)blockIdx.x * kWaves;
-    if (wave * G >= a.nrows) return;   // the whole workgroup: a job smaller than the grid
+    const BlockRef ref = refs[blockIdx.x];
+    const JobArgs& a = jobs[ref.job];
+    const uint64_t wave = (uint64_t)ref.block * kWaves;
     __shared__ uint8_t tab[256];
     stage_counts<true>(tab);
-    count_rows<true>(a, tab, 0, a.nrows, wave + uniform(threadIdx.x >> 6), (uint64_t)gridDim.x * kWaves);
+    count_rows<true>(a, tab, 0, a.nrows, wave + uniform(threadIdx.x >> 6), (uint64_t)ref.blocks * kWaves);
 }
 
 /* ------------------------------------------------------------------------- */
@@ -1626,7 +1628,7 @@ __global__ __launch_bounds__(kBlock) void k_slice_triangles(JobArgs a)
     __syncthreads();
     SliceLds& s = lds[threadIdx.x >> 6];
     const uint32_t lane = threadIdx.x & 63u;
-    const EmitLevel L = emit_level(a, 0);
+    const EmitLevel L = emit_level(a, 0, blockIdx.x);
     busy_chunks<false, kChunks>(a, L, s.l.q, [&](uint32_t n) {
         list_triangles(a, L, tri, s.l, n, [&](uint64_t, uint32_t y, uint32_t z, uint32_t c, uint64_t) {
             const CellMasks o = load_cells(a, L, y, z, c);
@@ -2480,52 +2482,34 @@ hipError_t launch_emit(int dtype, const JobArgs& a, uint32_t lds_bytes, hipStrea
     }
 }
 
-/* Grid of a batch's front passes: workgroups per job for at most `units` wave
- * units in one of them, some 16384 in all (the workgroups that a small job does
- * not need return at once). */
-static dim3 batch_grid(uint64_t units, uint32_t njobs)
-{
-    const uint64_t want = (units + kWaves - 1) / kWaves, cap = std::max<uint64_t>(64, 16384 / njobs);
-    return dim3((uint32_t)std::max<uint64_t>(1, std::min(want, cap)), 1, njobs);
-}
-
-constexpr uint32_t kMaxGridJobs = 32768;   // of one grid's z
-
 template <typename T>
-hipError_t launch_classify_batch_t(const JobArgs* jobs, uint32_t njobs, uint64_t chunks, uint32_t max_levels, hipStream_t st)
+hipError_t launch_classify_batch_t(const JobArgs* jobs, const BlockRef* refs, uint32_t nrefs, uint32_t max_levels, hipStream_t st)
 {
-    for (uint32_t j = 0; j < njobs; j += kMaxGridJobs) {
-        const uint32_t n = std::min(kMaxGridJobs, njobs - j);
-        const dim3 g = batch_grid((chunks + 15) / 16, n);
-        if (max_levels > 4) hipLaunchKernelGGL((k_classify_batch<T, true>), g, dim3(kBlock), 0, st, jobs + j);
-        else hipLaunchKernelGGL((k_classify_batch<T, false>), g, dim3(kBlock), 0, st, jobs + j);
-    }
+    if (max_levels > 4) hipLaunchKernelGGL((k_classify_batch<T, true>), dim3(nrefs), dim3(kBlock), 0, st, jobs, refs);
+    else hipLaunchKernelGGL((k_classify_batch<T, false>), dim3(nrefs), dim3(kBlock), 0, st, jobs, refs);
     return hipGetLastError();
 }
 
-hipError_t launch_classify_batch(int dtype, const JobArgs* jobs, uint32_t njobs, uint64_t chunks, uint32_t max_levels,
+hipError_t launch_classify_batch(int dtype, const JobArgs* jobs, const BlockRef* refs, uint32_t nrefs, uint32_t max_levels,
                                  hipStream_t st)
 {
     switch (dtype) {
-    case 0: return launch_classify_batch_t<int8_t>(jobs, njobs, chunks, max_levels, st);
-    case 1: return launch_classify_batch_t<int16_t>(jobs, njobs, chunks, max_levels, st);
-    case 2: return launch_classify_batch_t<int32_t>(jobs, njobs, chunks, max_levels, st);
-    case 3: return launch_classify_batch_t<int64_t>(jobs, njobs, chunks, max_levels, st);
-    case 4: return launch_classify_batch_t<uint8_t>(jobs, njobs, chunks, max_levels, st);
-    case 5: return launch_classify_batch_t<uint16_t>(jobs, njobs, chunks, max_levels, st);
-    case 6: return launch_classify_batch_t<uint32_t>(jobs, njobs, chunks, max_levels, st);
-    case 7: return launch_classify_batch_t<uint64_t>(jobs, njobs, chunks, max_levels, st);
-    case 8: return launch_classify_batch_t<float>(jobs, njobs, chunks, max_levels, st);
-    default: return launch_classify_batch_t<double>(jobs, njobs, chunks, max_levels, st);
+    case 0: return launch_classify_batch_t<int8_t>(jobs, refs, nrefs, max_levels, st);
+    case 1: return launch_classify_batch_t<int16_t>(jobs, refs, nrefs, max_levels, st);
+    case 2: return launch_classify_batch_t<int32_t>(jobs, refs, nrefs, max_levels, st);
+    case 3: return launch_classify_batch_t<int64_t>(jobs, refs, nrefs, max_levels, st);
+    case 4: return launch_classify_batch_t<uint8_t>(jobs, refs, nrefs, max_levels, st);
+    case 5: return launch_classify_batch_t<uint16_t>(jobs, refs, nrefs, max_levels, st);
+    case 6: return launch_classify_batch_t<uint32_t>(jobs, refs, nrefs, max_levels, st);
+    case 7: return launch_classify_batch_t<uint64_t>(jobs, refs, nrefs, max_levels, st);
+    case 8: return launch_classify_batch_t<float>(jobs, refs, nrefs, max_levels, st);
+    default: return launch_classify_batch_t<double>(jobs, refs, nrefs, max_levels, st);
     }
 }
 
-hipError_t launch_count_batch(const JobArgs* jobs, uint32_t njobs, uint64_t groups, hipStream_t st)
+hipError_t launch_count_batch(const JobArgs* jobs, const BlockRef* refs, uint32_t nrefs, hipStream_t st)
 {
-    for (uint32_t j = 0; j < njobs; j += kMaxGridJobs) {
-        const uint32_t n = std::min(kMaxGridJobs, njobs - j);
-        hipLaunchKernelGGL(k_count_batch, batch_grid(groups, n), dim3(kBlock), 0, st, jobs + j);
-    }
+    hipLaunchKernelGGL(k_count_batch, dim3(nrefs), dim3(kBlock), 0, st, jobs, refs);
     return hipGetLastError();
 }
 

@@ -12,6 +12,7 @@
 #pragma once
 #include <stdint.h>
 #include <algorithm>
+#include <vector>
 #include "kmc_job.h"
 
 #if defined(__HIPCC__)
@@ -154,6 +155,43 @@ inline void plan_emit(JobArgs& a, uint64_t all, uint32_t per_cu = 4, uint64_t it
     a.eblocks = (uint32_t)std::max<uint64_t>(1, (std::max(least, std::min(a.eunits, want)) + kWaves - 1) / kWaves);
     a.ewaves = a.eblocks * (uint32_t)kWaves;
     if (a.eunits > a.ewaves) a.ewaves = prime_below(a.ewaves);
+}
+
+/* One workgroup of a launch over a batch's passes: its pass, its level (emit) and
+ * which of the pass's (level's) workgroups it is. */
+struct BlockRef {
+    uint32_t job, level, block, blocks;
+};
+
+inline void add_blocks(std::vector<BlockRef>& out, uint32_t job, uint32_t level, uint64_t blocks)
+{
+    for (uint32_t i = 0; i < blocks; ++i) out.push_back(BlockRef{ job, level, i, (uint32_t)blocks });
+}
+
+/* Workgroups of a batch's front passes: as many as each pass has work for, or some
+ * 16384 in all, dealt by that work.  (The same number for every pass left one
+ * 512^3 volume among 255 of 32^3 to 64 workgroups: duplicated vertices, 645 us a run
+ * when rows were cut evenly over all waves, 1707 so.) */
+constexpr uint64_t kFrontBlocks = 16384;
+
+inline std::vector<BlockRef> front_blocks(const std::vector<uint64_t>& wants)
+{
+    uint64_t sum = 0;
+    for (uint64_t w : wants) sum += w;
+    std::vector<BlockRef> out;
+    for (uint32_t j = 0; j < wants.size(); ++j)
+        add_blocks(out, j, 0, sum <= kFrontBlocks ? wants[j] : std::max<uint64_t>(1, wants[j] * kFrontBlocks / sum));
+    return out;
+}
+
+/* Workgroups that a pass's classification (16 chunks a wave at a time) and count
+ * (row groups of 64 >> cshift rows) have work for. */
+inline uint64_t classify_blocks(const JobArgs& a) { return (a.nrows * a.NC + 16 * kWaves - 1) / (16 * kWaves); }
+
+inline uint64_t count_blocks(const JobArgs& a)
+{
+    const uint64_t G = 64u >> a.cshift;
+    return ((a.nrows + G - 1) / G + kWaves - 1) / kWaves;
 }
 
 }  // namespace kmc

@@ -1,4 +1,4 @@
-/* Host program over the emit's plan (kmc_plan.h): plan_check slots | places | large | shares. */
+/* Host program over the emit's plan (kmc_plan.h): plan_check slots | places | large | shares | unequal. */
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -158,6 +158,33 @@ static void shares()
         fail("long rows", a);
 }
 
+/* A large volume among small ones keeps its share of a batch's workgroups. */
+static void unequal()
+{
+    for (uint32_t small : { 0u, 1u, 13u, 255u, 5000u }) {
+        std::vector<JobArgs> jobs(1, volume(512, 512, 512, 1));
+        jobs.resize(small + 1, volume(32, 32, 32, 1));
+        for (int count = 0; count < 2; ++count) {
+            std::vector<uint64_t> wants;
+            uint64_t sum = 0;
+            for (const JobArgs& a : jobs) {
+                wants.push_back(count ? count_blocks(a) : classify_blocks(a));
+                sum += wants.back();
+            }
+            const std::vector<BlockRef> refs = front_blocks(wants);
+            std::vector<uint64_t> has(jobs.size(), 0);
+            for (const BlockRef& r : refs) {
+                if (r.block != has[r.job] || r.block >= r.blocks || r.blocks > wants[r.job]) fail("workgroups of a job", jobs[r.job]);
+                ++has[r.job];
+            }
+            for (uint64_t n : has)
+                if (n == 0) fail("a job without a workgroup", jobs[0]);
+            if (refs.size() > kFrontBlocks + jobs.size()) fail("too many workgroups", jobs[0]);
+            if (has[0] * sum * 2 < wants[0] * std::min(sum, kFrontBlocks)) fail("the large volume's share", jobs[0]);
+        }
+    }
+}
+
 int main(int argc, char** argv)
 {
     if (argc < 2) return 2;
@@ -165,6 +192,7 @@ int main(int argc, char** argv)
     else if (!std::strcmp(argv[1], "large")) large();
     else if (!std::strcmp(argv[1], "places")) places();
     else if (!std::strcmp(argv[1], "shares")) shares();
+    else if (!std::strcmp(argv[1], "unequal")) unequal();
     else return 2;
     std::printf("ok\n");
     return 0;

@@ -1,0 +1,38 @@
+"""Batches of very unequal volumes -- one large among many small ones, of one node row
+among them, with several levels and both classification forms -- against the
+oracle, bit for bit."""
+
+import numpy as np
+import pytest
+
+import oracle
+from kvs_amd import kmc
+from tests.conftest import assert_same_surface
+
+pytestmark = pytest.mark.gpu
+
+
+def _volume(dims, seed, dtype):
+    nx, ny, nz = dims
+    rng = np.random.default_rng(seed)
+    z, y, x = np.meshgrid(*(np.linspace(0, 3, n) for n in (nz, ny, nx)), indexing="ij")
+    f = np.sin(2 * x + seed) + np.cos(3 * y) + np.sin(z * 2 + x) + 0.05 * rng.random((nz, ny, nx))
+    return f.astype(np.float32) if dtype == np.float32 else ((f + 3) * 40).astype(dtype)
+
+
+@pytest.mark.parametrize("normal,dup", [(kmc.POLYGON_NORMAL, True), (kmc.POLYGON_NORMAL, False), (kmc.VERTEX_NORMAL, False)])
+@pytest.mark.parametrize("large_at,small", [(0, 300), (40, 40)])
+def test_one_large_volume(normal, dup, large_at, small):
+    specs = []
+    for i in range(small + 1):
+        dtype = np.uint8 if i % 5 == 3 else np.float32
+        if i == large_at:
+            dims, dtype = (300, 170, 130), np.float32
+        else:
+            dims = [(5, 6, 7), (8, 3, 2), (2, 2, 2), (65, 4, 3), (4, 1, 9), (16, 8, 4)][i % 6]
+        levels = [0.3, -0.2] if i % 4 == 1 else [0.3]
+        specs.append((_volume(dims, i, dtype), [120.5 + 20 * l for l in levels] if dtype == np.uint8 else levels, normal, dup))
+    got = kmc.batch_extract(specs)
+    for (v, levels, _, _), surfaces in zip(specs, got):
+        for l, s in zip(levels, surfaces):
+            assert_same_surface(s, oracle.extract(v, l, normal, dup), f"{v.shape} {v.dtype} {l}")

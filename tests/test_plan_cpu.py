@@ -1,6 +1,7 @@
 """The emit's plan (kmc_plan.h) on the host: what a wave queues names the slot it
 looked at, in volumes of any number of rows, every slot is looked at once, and small
-or flat surfaces fall to many waves."""
+or flat surfaces fall to many waves, and a large volume among many small ones in a
+batch keeps its share of the workgroups."""
 import os
 import subprocess
 
@@ -17,7 +18,7 @@ def plan_check(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["slots", "places", "large", "shares"])
+@pytest.mark.parametrize("what", ["slots", "places", "large", "shares", "unequal"])
 def test_emit_slots(plan_check, what):
     r = subprocess.run([plan_check, what], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout
