@@ -409,22 +409,28 @@ __global__ __launch_bounds__(kBlock) void k_coord_span_final(const CoordSpan* pa
 
 static_assert(kSpanParts % kBlock == 0, "the final merge gives every thread the same number of parts");
 
-/* The ranges as long as order does not matter: the serial scans above are
- * plain minima and maxima unless a NaN occurs or zeros of both signs tie, and
- * a NaN or a -0 sets `odd` (the ordered passes then decide). */
+/* The ranges in one pass: the serial scans above are plain minima and maxima (a NaN
+ * value compares false and is passed over, and one that seeds the scan stays)
+ * unless a coordinate is NaN, or an extreme is zero and zeros of both signs occur:
+ * its sign is then the first zero value's, or the last zero coordinate's, of the scan.
+ * Only then, and only for the values or the coordinates, the ordered passes decide.
+ * (Keeping the zeros' places in this pass instead costs every mesh: 3.07 M
+ * tetrahedra 80.3 us a call, 88.1 so.) */
+enum : uint32_t { kNegZeroValue = 1, kNegZeroCoord = 2 /* << axis */, kNanCoord = 16 };
+
 template <typename T>
 struct CellRange {
     T mn, mx;
     float cmn[3], cmx[3];
-    uint32_t odd;
+    uint32_t seen;
 };
 
 template <typename T>
-__device__ __forceinline__ bool is_odd(T) { return false; }
-template <> __device__ __forceinline__ bool is_odd<float>(float v) { return v != v || __float_as_uint(v) == 0x80000000u; }
-template <> __device__ __forceinline__ bool is_odd<double>(double v)
+__device__ __forceinline__ bool is_neg_zero(T) { return false; }
+template <> __device__ __forceinline__ bool is_neg_zero<float>(float v) { return __float_as_uint(v) == 0x80000000u; }
+template <> __device__ __forceinline__ bool is_neg_zero<double>(double v)
 {
-    return v != v || (unsigned long long)__double_as_longlong(v) == 0x8000000000000000ull;
+    return (unsigned long long)__double_as_longlong(v) == 0x8000000000000000ull;
 }
 
 template <typename T>
@@ -437,7 +443,7 @@ __device__ __forceinline__ void range_merge(CellRange<T>& f, const CellRange<T>&
         f.cmn[k] = g.cmn[k] < f.cmn[k] ? g.cmn[k] : f.cmn[k];
         f.cmx[k] = g.cmx[k] > f.cmx[k] ? g.cmx[k] : f.cmx[k];
     }
-    f.odd |= g.odd;
+    f.seen |= g.seen;
 }
 
 template <typename T>
@@ -465,7 +471,7 @@ __global__ __launch_bounds__(kBlock) void k_ucount_ranges(UArgs a, CellRange<T>*
     const T* vol = (const T*)a.values;
     CellRange<T> r;
     r.mn = r.mx = vol[0];                       // the value scan is seeded with the first value
-    r.odd = is_odd<T>(vol[0]) ? 1u : 0u;
+    bool nan = false, zero_v = is_neg_zero<T>(vol[0]), zero_c[3] = { false, false, false };
 #pragma unroll
     for (int k = 0; k < 3; ++k) { r.cmn[k] = INFINITY; r.cmx[k] = -INFINITY; }
     const uint64_t step = (uint64_t)gridDim.x * kBlock;
@@ -477,22 +483,25 @@ __global__ __launch_bounds__(kBlock) void k_ucount_ranges(UArgs a, CellRange<T>*
             const T v = vol[li[i]];
             r.mn = v < r.mn ? v : r.mn;
             r.mx = v > r.mx ? v : r.mx;
-            bool odd = is_odd<T>(v);
+            zero_v = zero_v || is_neg_zero<T>(v);
             const float* p = a.coords + 3 * li[i];
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
                 const float c = p[k];
                 r.cmn[k] = c < r.cmn[k] ? c : r.cmn[k];
                 r.cmx[k] = c > r.cmx[k] ? c : r.cmx[k];
-                odd = odd || is_odd<float>(c);
+                zero_c[k] = zero_c[k] || is_neg_zero<float>(c);
+                nan = nan || c != c;
             }
-            r.odd |= odd ? 1u : 0u;
         }
         const uint32_t ti = cell_case<T, C, SLICE>(a, li);
         const bool skip = ti == 0 || ti == (uint32_t)Cell<C>::all_ones;
         a.tidx[cell] = (uint8_t)ti;
         a.counts[cell] = skip ? 0u : (uint32_t)(Cell<C>::tri(ti) >> 60);
     }
+    r.seen = (zero_v ? kNegZeroValue : 0u) | (nan ? kNanCoord : 0u);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) r.seen |= zero_c[k] ? kNegZeroCoord << k : 0u;
     block_range(r, sh);
     if (threadIdx.x == 0) parts[blockIdx.x] = r;
 }
@@ -501,7 +510,7 @@ __global__ __launch_bounds__(kBlock) void k_ucount_ranges(UArgs a, CellRange<T>*
 struct Ranges {
     double mm[2];
     float cc[6];
-    uint32_t odd, pad;
+    uint32_t values_again, coords_again;   // not 0: the ordered pass decides
 };
 
 template <typename T>
@@ -515,8 +524,14 @@ __global__ __launch_bounds__(kBlock) void k_range_final(const CellRange<T>* part
     if (threadIdx.x == 0) {
         out->mm[0] = (double)r.mn;
         out->mm[1] = (double)r.mx;
-        for (int k = 0; k < 3; ++k) { out->cc[k] = r.cmn[k]; out->cc[3 + k] = r.cmx[k]; }
-        out->odd = r.odd;
+        out->values_again = (r.seen & kNegZeroValue) && (r.mn == T(0) || r.mx == T(0)) ? 1u : 0u;
+        uint32_t again = r.seen & kNanCoord;
+        for (int k = 0; k < 3; ++k) {
+            out->cc[k] = r.cmn[k];
+            out->cc[3 + k] = r.cmx[k];
+            again |= (r.seen & kNegZeroCoord << k) && (r.cmn[k] == 0.0f || r.cmx[k] == 0.0f) ? 1u : 0u;
+        }
+        out->coords_again = again;
     }
 }
 
@@ -694,16 +709,16 @@ kmc_status run_cells(const kmc_unstructured_volume* v, bool slice, double iso, i
     HostResult<Found> found(st);
     Found* const res_dev = need_values || need_coords || count_now ? found.get() : nullptr;
     if (!res_dev && (need_values || need_coords || count_now)) return finish(KMC_ERR_OUT_OF_MEMORY);
-    /* both ranges together come with the count pass; else, or when that meets
-     * a value whose order matters, from the ordered passes */
+    /* both ranges together come with the count pass; else, and where order turns out
+     * to matter, from the ordered passes */
     const bool fused = need_values && need_coords && count_now;
-    auto ordered_ranges = [&]() -> kmc_status {
+    auto ordered_ranges = [&](bool values, bool coords) -> kmc_status {
         uint8_t* scratch = (uint8_t*)alloc(minmax_scratch_bytes() + kSpanParts * sizeof(CoordSpan));
         if (!scratch) return KMC_ERR_OUT_OF_MEMORY;
         CoordSpan* spans = (CoordSpan*)(scratch + minmax_scratch_bytes());
-        if (need_values && launch_minmax_gather(v->type, dvals, dconn, nconn, scratch, res_dev->r.mm, st) != hipSuccess)
+        if (values && launch_minmax_gather(v->type, dvals, dconn, nconn, scratch, res_dev->r.mm, st) != hipSuccess)
             return KMC_ERR_DEVICE;
-        if (need_coords) {
+        if (coords) {
             hipLaunchKernelGGL(k_coord_span_partial, dim3(kSpanParts), dim3(kBlock), 0, st, dcoords, dconn, nconn,
                                spans);
             hipLaunchKernelGGL(k_coord_span_final, dim3(1), dim3(kBlock), 0, st, spans, res_dev->r.cc);
@@ -711,7 +726,7 @@ kmc_status run_cells(const kmc_unstructured_volume* v, bool slice, double iso, i
         return hipGetLastError() == hipSuccess ? KMC_OK : KMC_ERR_DEVICE;
     };
     if ((need_values || need_coords) && !fused) {
-        s = ordered_ranges();
+        s = ordered_ranges(need_values, need_coords);
         if (s != KMC_OK) return finish(s);
     }
     const uint32_t nparts = count_now ? scan_partials_needed(ncells, 1) : 0;
@@ -741,8 +756,10 @@ kmc_status run_cells(const kmc_unstructured_volume* v, bool slice, double iso, i
         return finish(KMC_ERR_DEVICE);
     }
     const uint64_t nt = count_now ? found[0].nt : 0;
-    if (fused && found[0].r.odd) {
-        s = ordered_ranges();
+    if (fused && (found[0].r.values_again || found[0].r.coords_again)) {
+        const bool values = found[0].r.values_again != 0, coords = found[0].r.coords_again != 0;
+        (void)found.get();   // kernels write to it again
+        s = ordered_ranges(values, coords);
         if (s != KMC_OK) return finish(s);
         if (found.wait() != hipSuccess) {
             (void)hipGetLastError();
