@@ -891,10 +891,8 @@ __global__ __launch_bounds__(kBlock) void k_classify(JobArgs a)
     for (uint64_t row = wave_id; row < nrows; row += nwaves) classify_row<T, NLEV>(a, row);
 }
 
-/* The same for rows shorter than 16 chunks, 16 chunks of consecutive rows a wave:
- * a row a wave would leave it fewer loads in flight (256^3 float: 23.5 us, runs
- * 15.0; 301 x 257 x 199 double at two levels 22.7 and 21.6).  Rows of 16 chunks
- * keep a wave busy (1024^3 float at three levels: 790 us, runs 1160). */
+/* The same for many short rows (classify_by_runs), 16 chunks of consecutive rows a
+ * wave: 256^3 float 23.5 us a row a wave, 15.0 so. */
 template <typename T, int NLEV>
 __global__ __launch_bounds__(kBlock) void k_classify_runs(JobArgs a)
 {
@@ -2324,7 +2322,7 @@ hipError_t launch_classify_t(const JobArgs& a, hipStream_t st)
         /* rows of whole dwords: one dword of nodes per lane */
         if (packed_rows<T>(a)) return launch_classify_packed_t<T>(a, st);
     }
-    if (a.NC < 16) {
+    if (classify_by_runs(a, sizeof(T))) {
         const uint64_t want = ((a.nrows * a.NC + 15) / 16 + kWaves - 1) / kWaves;
         const dim3 g((uint32_t)std::min<uint64_t>(want, 1u << 20)), b(kBlock);
         switch (a.nlev) {

@@ -157,6 +157,22 @@ inline void plan_emit(JobArgs& a, uint64_t all, uint32_t per_cu = 4, uint64_t it
     if (a.eunits > a.ewaves) a.ewaves = prime_below(a.ewaves);
 }
 
+/* Classification: 16 chunks of consecutive rows a wave (runs) or a row a wave.  A row
+ * a wave leaves short rows few loads in flight, and with more rows than the device
+ * holds waves that is what it waits for; runs spend some instructions per chunk
+ * and level and store their masks in shorter pieces.  Row / run form, us:
+ *   float, one level, 65536 rows of 4 / 8 / 12 / 16 chunks  25.2 / 30.2 / 39.0, 16.6 / 26.9 / 36.9; 86.8 and 87.3 at 2 GiB
+ *   three levels, 4 / 5 / 6 / 12 chunks  28.6 / 30.6 / 32.4 / 45.9 and 25.0 / 29.8 / 34.4 / 61.8
+ *   double, one level, 4 / 5 / 6 / 8 chunks  27.2 / 32.2 / 34.6 / 43.8 and 24.9 / 30.0 / 34.6 / 46.0
+ *   uint16 (odd rows), three levels, 3 / 4 / 6 / 8 chunks  38.7 / 43.6 / 56.6 / 67.5 and 31.1 / 41.5 / 56.9 / 75.4
+ *   five levels, 262144 rows of 4 chunks  float 300 and 351, double 163 and 183 (at 2^28 bytes a volume of 3 chunks 7 % slower, of 2 faster)
+ *   one level, 1024 .. 8192 rows: the same within 0.5 us, uint16 6.6 and 7.5 */
+inline bool classify_by_runs(const JobArgs& a, uint32_t value_size)
+{
+    constexpr uint32_t most[3][5] = { { 8, 6, 4, 2, 2 }, { 12, 6, 5, 4, 2 }, { 5, 5, 5, 4, 2 } };   // by levels, the last for five and more
+    return a.nrows > 8192 && a.NC <= most[value_size <= 2 ? 0 : value_size / 4][std::min(a.nlev, 5u) - 1];
+}
+
 /* One workgroup of a launch over a batch's passes: its pass, its level (emit) and
  * which of the pass's (level's) workgroups it is. */
 struct BlockRef {
