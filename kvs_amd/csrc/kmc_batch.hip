@@ -376,7 +376,8 @@ kmc_status plan_tiles(kmc_batch* b, uint32_t r_max, uint32_t queue_cap)
          * form launches each pass by itself */
         uint64_t steps = 0;
         for (uint32_t i = g.p0; i < g.p1; ++i) steps += emit_steps(b->passes[i].a);
-        for (uint32_t i = g.p0; i < g.p1 && !b->two_phase; ++i) plan_emit(b->passes[i].a, steps);
+        for (uint32_t i = g.p0; i < g.p1 && !b->two_phase; ++i)
+            plan_emit(b->passes[i].a, steps, g.mode == 0 ? dup_blocks((uint32_t)type_size(g.dtype)) : 4);
         std::vector<uint64_t> ts, cls, cnt;
         std::vector<BlockRef> emit;
         uint64_t t = 0;

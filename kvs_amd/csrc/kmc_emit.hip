@@ -89,8 +89,8 @@ __device__ __forceinline__ void stage_cases(CaseLds& t, const CaseLds& from)
     __syncthreads();
 }
 
-/* LDS of one wave of the duplicated triangles: 9.4 kB with values of up to 32
- * bits, so that four workgroups fit a CU's 160 KiB. */
+/* LDS of one wave of the duplicated triangles: 9.1 kB with values of up to 32
+ * bits, so that four workgroups fit a CU's 160 KiB; 11.1 kB with 64 bits, three. */
 constexpr uint32_t kDupCells = 320;      // active cells listed at once (a chunk has at most 64)
 constexpr uint32_t kVerts = 236;         // edge crossings of the up to 64 cells in work (a cell has at most 12)
 
@@ -1010,13 +1010,14 @@ __global__ __launch_bounds__(kBlock) void k_normals_batch(const JobArgs* jobs, c
     normals_level(a, r.level, r.block, use, s[threadIdx.x >> 6]);
 }
 
-/* Workgroups of each kernel that a CU holds: by LDS k_dup 4 and k_faces 5, by
- * registers k_points 7 and k_normals 5 or more. */
-constexpr uint32_t kDupBlocks = 4, kPointBlocks = 7, kFaceBlocks = 5, kNormalBlocks = 5;
+/* Workgroups of each kernel that a CU holds: by LDS k_dup dup_blocks and k_faces 5,
+ * by registers k_points 7 and k_normals 5 or more. */
+constexpr uint32_t kPointBlocks = 7, kFaceBlocks = 5, kNormalBlocks = 5;
 
 template <typename T>
 hipError_t launch_chunk_emit_t(JobArgs a, hipStream_t st, hipEvent_t* marks)
 {
+    static_assert((160u << 10) / (sizeof(CaseLds) + kWaves * sizeof(CellLds<T>)) == dup_blocks(sizeof(T)), "workgroups a CU holds");
     const dim3 b(kBlock);
     uint64_t nv = 0, nt = 0;
     for (uint32_t l = 0; l < a.nlev; ++l) { nv += a.cap_vertices[l]; nt += a.cap_triangles[l]; }
@@ -1028,7 +1029,7 @@ hipError_t launch_chunk_emit_t(JobArgs a, hipStream_t st, hipEvent_t* marks)
     if (!a.dup) hipLaunchKernelGGL((k_points<T>), grid(kPointBlocks, nv), b, 0, st, a);
     if (marks) (void)hipEventRecord(marks[1], st);
     switch (emit_mode(a)) {
-    case kModeDup: hipLaunchKernelGGL((k_dup<T>), grid(kDupBlocks, nt), b, 0, st, a); break;
+    case kModeDup: hipLaunchKernelGGL((k_dup<T>), grid(dup_blocks(sizeof(T)), nt), b, 0, st, a); break;
     case kModePolygon: hipLaunchKernelGGL((k_faces<kModePolygon>), grid(kFaceBlocks, nt), b, 0, st, a); break;
     default: hipLaunchKernelGGL((k_faces<kModeVertex>), grid(kFaceBlocks, nt), b, 0, st, a); break;
     }

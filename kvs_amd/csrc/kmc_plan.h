@@ -99,6 +99,11 @@ inline uint64_t emit_steps(const JobArgs& a)
  * vertex normals: 3390 us a call by outputs alone, 995 with 32 steps, 890 with 16). */
 constexpr uint64_t kEmitRounds = 8, kEmitItems = 32, kEmitWalk = 16;
 
+/* Workgroups of the duplicated triangles' kernel that a CU's LDS holds, by the size of
+ * the values it stages (kmc_emit.hip checks it).  A grid for four of them where three
+ * fit takes a round and a third: 512^3 double CT 770 us a call, so 705. */
+constexpr uint32_t dup_blocks(uint32_t value_size) { return value_size == 8 ? 3u : 4u; }
+
 /* Split of the chunk-batch emit (rows planned; a.nlev set) of a pass whose emit
  * shares its launch with others, `all` being the sum of their emit_steps, for a
  * kernel of which a CU holds per_cu workgroups and that produces `items` outputs
