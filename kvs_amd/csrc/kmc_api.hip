@@ -599,7 +599,7 @@ void init_job(JobArgs& a, const kmc_volume* v, const void* dvals, const double* 
 namespace {
 thread_local bool t_timing = false;
 thread_local kmc_timing t_last;
-thread_local hipEvent_t t_ev[9] = { nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr };
+thread_local hipEvent_t t_ev[8] = { nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr };
 }
 
 struct PassTimer {
@@ -608,10 +608,10 @@ struct PassTimer {
     bool flat = false;
     explicit PassTimer(hipStream_t s) : st(s), on(t_timing)
     {
-        for (int i = 0; i < 9 && on; ++i)
+        for (int i = 0; i < 8 && on; ++i)
             if (!t_ev[i] && hipEventCreate(&t_ev[i]) != hipSuccess) { (void)hipGetLastError(); on = false; }
     }
-    /* events between the chunk-batch emit's kernels (start, after vertices, after triangles) */
+    /* events between the chunk-batch emit's kernels (after vertices, after triangles) */
     hipEvent_t* flat_marks() { flat = on; return on ? &t_ev[6] : nullptr; }
     bool mark(int i)
     {
@@ -629,15 +629,13 @@ struct PassTimer {
         t_last.emit_ms += ms[4];
         t_last.passes += 1;
         if (flat) {
-            float f[4] = { 0, 0, 0, 0 };
+            float f[3] = { 0, 0, 0 };
             (void)hipEventElapsedTime(&f[0], t_ev[4], t_ev[6]);
             (void)hipEventElapsedTime(&f[1], t_ev[6], t_ev[7]);
-            (void)hipEventElapsedTime(&f[2], t_ev[7], t_ev[8]);
-            (void)hipEventElapsedTime(&f[3], t_ev[8], t_ev[5]);
-            t_last.compact_ms += f[0];
-            t_last.vertices_ms += f[1];
-            t_last.triangles_ms += f[2];
-            t_last.vertex_normals_ms += f[3];
+            (void)hipEventElapsedTime(&f[2], t_ev[7], t_ev[5]);
+            t_last.vertices_ms += f[0];
+            t_last.triangles_ms += f[1];
+            t_last.vertex_normals_ms += f[2];
         }
     }
 };

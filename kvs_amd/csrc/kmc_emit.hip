@@ -1027,13 +1027,13 @@ hipError_t launch_chunk_emit_t(JobArgs a, hipStream_t st, hipEvent_t* marks)
         return dim3(a.eblocks, a.nlev);
     };
     if (!a.dup) hipLaunchKernelGGL((k_points<T>), grid(kPointBlocks, nv), b, 0, st, a);
-    if (marks) (void)hipEventRecord(marks[1], st);
+    if (marks) (void)hipEventRecord(marks[0], st);
     switch (emit_mode(a)) {
     case kModeDup: hipLaunchKernelGGL((k_dup<T>), grid(dup_blocks(sizeof(T)), nt), b, 0, st, a); break;
     case kModePolygon: hipLaunchKernelGGL((k_faces<kModePolygon>), grid(kFaceBlocks, nt), b, 0, st, a); break;
     default: hipLaunchKernelGGL((k_faces<kModeVertex>), grid(kFaceBlocks, nt), b, 0, st, a); break;
     }
-    if (marks) (void)hipEventRecord(marks[2], st);
+    if (marks) (void)hipEventRecord(marks[1], st);
     if (a.vnormal) hipLaunchKernelGGL(k_normals, grid(kNormalBlocks, nv), b, 0, st, a);
     return hipGetLastError();
 }
@@ -1056,7 +1056,6 @@ hipError_t launch_chunk_emit_batch_t(int mode, const JobArgs* jobs, const BlockR
 
 hipError_t launch_chunk_emit(int dtype, const JobArgs& a, hipStream_t st, hipEvent_t* marks)
 {
-    if (marks) (void)hipEventRecord(marks[0], st);
     switch (dtype) {
     case 0: return launch_chunk_emit_t<int8_t>(a, st, marks);
     case 1: return launch_chunk_emit_t<int16_t>(a, st, marks);

@@ -110,9 +110,9 @@ uint32_t levels_per_pass(const kmc_volume* v, int vnormal);
 hipError_t launch_emit(int dtype, const JobArgs& a, uint32_t lds_bytes, hipStream_t st);
 /* Chunk-batch emit (kmc_emit.hip) of a pass (a.vpc / a.tpc written by its
  * count pass, outputs and capacities set; VertexNormal: a.fn, a.crec, a.act,
- * a.toff), or of a batch group's passes (a workgroup per ref).  mode: 0 duplicated vertices, 1 PolygonNormal, 2 VertexNormal (shared
- * vertices).  marks: three events recorded at the start, after the vertices and
- * after the triangles (timing), or null. */
+ * a.toff), or of a batch group's passes (a workgroup per ref).  mode: 0
+ * duplicated vertices, 1 PolygonNormal, 2 VertexNormal (shared vertices).  marks: two
+ * events recorded after the vertices and after the triangles (timing), or null. */
 hipError_t launch_chunk_emit(int dtype, const JobArgs& a, hipStream_t st, hipEvent_t* marks = nullptr);
 hipError_t launch_chunk_emit_batch(int dtype, int mode, const JobArgs* jobs, const BlockRef* refs, uint32_t nrefs,
                                    hipStream_t st);
