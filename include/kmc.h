@@ -141,7 +141,8 @@ kmc_status kmc_extract_levels(const kmc_volume* volume, const double* isolevels,
  * library holds on each GPU it runs on until the process ends:
  *   - KMC_ERR_SCRATCH when the bytes budgeted for the volume's work (about 48
  *     per 64-node chunk and 24 per node row) or for the emit (about 8 per vertex
- *     and 9 per triangle, 28 more per vertex with VertexNormal) do not fit;
+ *     and 9 per triangle; with VertexNormal 16 more per vertex and 12 more per
+ *     triangle) do not fit;
  *   - KMC_ERR_CAPACITY when the outputs do not fit: *out then holds the sizes
  *     (n_vertices, n_triangles, n_connections, n_normals) and nothing was written.
  * On KMC_OK *out describes the caller's arrays (release is not needed).

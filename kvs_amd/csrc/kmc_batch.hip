@@ -895,8 +895,8 @@ uint64_t batch_work_bytes(const kmc_batch* b)
 uint64_t batch_record_arena_bytes(const kmc_batch* b) { return b->flat ? b->cap_r : 0; }
 
 /* Record bytes surface i is budgeted with once its sizes are known (8 per
- * vertex and 9 per triangle, 28 more per vertex with VertexNormal; an upper
- * bound of what its emit takes). */
+ * vertex and 9 per triangle; with VertexNormal 16 more per vertex and 12 more per
+ * triangle; an upper bound of what its emit takes). */
 uint64_t batch_record_bytes(const kmc_batch* b, uint32_t i)
 {
     const uint32_t sg = b->surface_seg[i];
