@@ -3,11 +3,12 @@
  *
  * After the count pass and the scan, the output position of everything a
  * 64-node chunk holds is known: row prefix + chunk prefix within the row.  A
- * wave walks the (row, chunk) pairs of one level, queues the chunks that hold
- * something in LDS and works on 64 of them at a time: each lane takes one
- * chunk's masks, the wave lists the chunks' active cells in LDS, and the
- * listed triangles are produced one per lane -- every lane busy whatever the
- * chunks hold, nothing but the outputs written.
+ * wave walks its share of a level's (row, chunk) slots (kmc_plan.h), queues the
+ * chunks that hold something in LDS and works on 32, 48 or 64 of them at a time:
+ * each lane takes one chunk's masks, the wave lists the chunks' active cells or
+ * crossing edges in LDS, and the listed items are produced one per lane -- every lane
+ * busy whatever the chunks hold; only the vertex normals need more than the
+ * outputs written (face normals and cell records).
  *
  * Output order: cells in scan order, triangles in table order
  * (extract_surfaces_with_duplication,
@@ -947,7 +948,7 @@ __device__ __forceinline__ void normals_level(const JobArgs& a, uint32_t l, uint
     const uint32_t sh = a.NC <= 64 ? 16u : 0u, mask = prefix_mask(a);
     busy_chunks<true, kNormalChunks>(a, L, s.p.q, [&](uint32_t n) {
         chunk_points(a, L, s.p, n, [&](uint64_t r, uint32_t y, uint32_t z, uint32_t c) {
-/* cell row (cy, cz) is kept at node row (cy, cz + 1): node rows r -
+            /* cell row (cy, cz) is kept at node row (cy, cz + 1): node rows r -
              * 1, r and the same of the next slice; the words of this chunk and
              * the one before it in one load each (node row r >= 1 wherever a
              * row below or a chunk before is used) */

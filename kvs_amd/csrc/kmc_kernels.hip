@@ -1255,7 +1255,10 @@ __device__ __forceinline__ void count_rows(const JobArgs& a, const uint8_t* tab,
                                            uint64_t wave_first, uint64_t wave_step)
 {
     switch (a.nlev) {
-    case 1: count_rows_t<1, POP>(a, tab, r0, r1, wave_first, wave_step); break;
+    case 1:
+        /* a plain pass of one level has a kernel of its own (k_count_level) */
+        if constexpr (POP) count_rows_t<1, POP>(a, tab, r0, r1, wave_first, wave_step);
+        break;
     case 2: count_rows_t<2, POP>(a, tab, r0, r1, wave_first, wave_step); break;
     case 3: count_rows_t<3, POP>(a, tab, r0, r1, wave_first, wave_step); break;
     case 4: count_rows_t<4, POP>(a, tab, r0, r1, wave_first, wave_step); break;

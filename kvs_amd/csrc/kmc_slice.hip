@@ -4,10 +4,10 @@
  *
  * The plane takes the place of the isosurface: nodes classify by the sign of
  * the plane equation (no value is read for that), the count and scan passes
- * of the marching-cubes path run unchanged in duplicated mode, and one thread per triangle interpolates its three vertices along the
- * plane, colours each with the value interpolated at the same ratio, and
- * writes the negated face normal -- triangles in cell scan order, the order
- * of the reference's loop.
+ * of the marching-cubes path run unchanged in duplicated mode, and one thread
+ * per triangle interpolates its three vertices along the plane, colours each
+ * with the value interpolated at the same ratio, and writes the negated face
+ * normal -- triangles in cell scan order, the order of the reference's loop.
  */
 #include <hip/hip_runtime.h>
 #include <cmath>
@@ -23,8 +23,6 @@
 namespace kmc {
 
 namespace {
-
-inline size_t up256(size_t x) { return (x + 255) & ~size_t(255); }
 
 /* MapperBase::setRange (MapperBase.cpp:54-83) for a transfer function
  * without a range of its own. */
