@@ -471,27 +471,39 @@ __global__ __launch_bounds__(kBlock) void k_ucount_ranges(UArgs a, CellRange<T>*
     const T* vol = (const T*)a.values;
     CellRange<T> r;
     r.mn = r.mx = vol[0];                       // the value scan is seeded with the first value
-    bool nan = false, zero_v = is_neg_zero<T>(vol[0]), zero_c[3] = { false, false, false };
+    r.seen = is_neg_zero<T>(vol[0]) ? kNegZeroValue : 0u;
 #pragma unroll
     for (int k = 0; k < 3; ++k) { r.cmn[k] = INFINITY; r.cmx[k] = -INFINITY; }
     const uint64_t step = (uint64_t)gridDim.x * kBlock;
     for (uint64_t cell = (uint64_t)blockIdx.x * kBlock + threadIdx.x; cell < a.ncells; cell += step) {
         uint64_t li[8];
         cell_nodes<C>(a, cell, li);
+        uint32_t odd = 0;
 #pragma unroll
         for (int i = 0; i < Cell<C>::nodes; ++i) {
             const T v = vol[li[i]];
             r.mn = v < r.mn ? v : r.mn;
             r.mx = v > r.mx ? v : r.mx;
-            zero_v = zero_v || is_neg_zero<T>(v);
+            bool o = is_neg_zero<T>(v);
             const float* p = a.coords + 3 * li[i];
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
                 const float c = p[k];
                 r.cmn[k] = c < r.cmn[k] ? c : r.cmn[k];
                 r.cmx[k] = c > r.cmx[k] ? c : r.cmx[k];
-                zero_c[k] = zero_c[k] || is_neg_zero<float>(c);
-                nan = nan || c != c;
+                o = o || is_neg_zero<float>(c) || c != c;
+            }
+            odd |= o ? 1u : 0u;
+        }
+        if (odd) {   // rare: one test a cell, which and where after it
+#pragma unroll 1
+            for (int i = 0; i < Cell<C>::nodes; ++i) {
+                const uint64_t n = a.conn[cell * Cell<C>::nodes + i];
+                r.seen |= is_neg_zero<T>(vol[n]) ? kNegZeroValue : 0u;
+                for (int k = 0; k < 3; ++k) {
+                    const float c = a.coords[3 * n + k];
+                    r.seen |= (is_neg_zero<float>(c) ? kNegZeroCoord << k : 0u) | (c != c ? kNanCoord : 0u);
+                }
             }
         }
         const uint32_t ti = cell_case<T, C, SLICE>(a, li);
@@ -499,9 +511,6 @@ __global__ __launch_bounds__(kBlock) void k_ucount_ranges(UArgs a, CellRange<T>*
         a.tidx[cell] = (uint8_t)ti;
         a.counts[cell] = skip ? 0u : (uint32_t)(Cell<C>::tri(ti) >> 60);
     }
-    r.seen = (zero_v ? kNegZeroValue : 0u) | (nan ? kNanCoord : 0u);
-#pragma unroll
-    for (int k = 0; k < 3; ++k) r.seen |= zero_c[k] ? kNegZeroCoord << k : 0u;
     block_range(r, sh);
     if (threadIdx.x == 0) parts[blockIdx.x] = r;
 }
