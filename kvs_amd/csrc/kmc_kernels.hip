@@ -1124,7 +1124,7 @@ __device__ __forceinline__ uint32_t group_excl_scan(uint32_t x, uint32_t cl, uin
  * edges crossed or two opposite corners that differ from all their neighbours,
  * and only those cells are looked up: fewer[] holds 2 (L - 1).  A lookup per
  * active cell runs each wave as long as its fullest chunk takes (512^3: 43 us, so
- * 25.5; 256^3 7.9 and 5.1; 14 volumes of up to 256^3 in a batch 42 and 36). */
+ * 27; 256^3 7.9 and 5.5; 14 volumes of up to 256^3 in a batch 42 and 33). */
 __device__ __forceinline__ uint32_t chunk_triangles(const RowChunk& o, const uint8_t* fewer)
 {
     int n = -2 * __popcll(o.act);
