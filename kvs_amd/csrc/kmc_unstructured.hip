@@ -474,11 +474,11 @@ __global__ __launch_bounds__(kBlock) void k_ucount_ranges(UArgs a, CellRange<T>*
     r.seen = is_neg_zero<T>(vol[0]) ? kNegZeroValue : 0u;
 #pragma unroll
     for (int k = 0; k < 3; ++k) { r.cmn[k] = INFINITY; r.cmx[k] = -INFINITY; }
-    const uint64_t step = (uint64_t)gridDim.x * kBlock;
-    for (uint64_t cell = (uint64_t)blockIdx.x * kBlock + threadIdx.x; cell < a.ncells; cell += step) {
+    const uint64_t first = (uint64_t)blockIdx.x * kBlock + threadIdx.x, step = (uint64_t)gridDim.x * kBlock;
+    uint32_t odd = 0;
+    for (uint64_t cell = first; cell < a.ncells; cell += step) {
         uint64_t li[8];
         cell_nodes<C>(a, cell, li);
-        uint32_t odd = 0;
 #pragma unroll
         for (int i = 0; i < Cell<C>::nodes; ++i) {
             const T v = vol[li[i]];
@@ -495,10 +495,18 @@ __global__ __launch_bounds__(kBlock) void k_ucount_ranges(UArgs a, CellRange<T>*
             }
             odd |= o ? 1u : 0u;
         }
-        if (odd) {   // rare: one test a cell, which and where after it
-#pragma unroll 1
-            for (int i = 0; i < Cell<C>::nodes; ++i) {
-                const uint64_t n = a.conn[cell * Cell<C>::nodes + i];
+        const uint32_t ti = cell_case<T, C, SLICE>(a, li);
+        const bool skip = ti == 0 || ti == (uint32_t)Cell<C>::all_ones;
+        a.tidx[cell] = (uint8_t)ti;
+        a.counts[cell] = skip ? 0u : (uint32_t)(Cell<C>::tri(ti) >> 60);
+    }
+    /* which and where, over this thread's cells once more and only then: a test and a
+     * branch in the loop keep the next loads waiting (3.4 M prisms: 31.3 us, 36.2) */
+    if (odd) {
+        const uint64_t per = Cell<C>::nodes;
+        for (uint64_t cell = first; cell < a.ncells; cell += step) {
+            for (uint64_t i = cell * per; i < (cell + 1) * per; ++i) {
+                const uint64_t n = a.conn[i];
                 r.seen |= is_neg_zero<T>(vol[n]) ? kNegZeroValue : 0u;
                 for (int k = 0; k < 3; ++k) {
                     const float c = a.coords[3 * n + k];
@@ -506,10 +514,6 @@ __global__ __launch_bounds__(kBlock) void k_ucount_ranges(UArgs a, CellRange<T>*
                 }
             }
         }
-        const uint32_t ti = cell_case<T, C, SLICE>(a, li);
-        const bool skip = ti == 0 || ti == (uint32_t)Cell<C>::all_ones;
-        a.tidx[cell] = (uint8_t)ti;
-        a.counts[cell] = skip ? 0u : (uint32_t)(Cell<C>::tri(ti) >> 60);
     }
     block_range(r, sh);
     if (threadIdx.x == 0) parts[blockIdx.x] = r;
