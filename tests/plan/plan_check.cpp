@@ -63,7 +63,7 @@ static void check_slot(const JobArgs& a, uint32_t wave, uint64_t step, uint32_t 
 /* Every slot of a small volume belongs to exactly one wave, step and lane. */
 static void slots()
 {
-    const uint32_t shapes[][3] = { { 2, 1, 1 }, { 2, 70, 3 }, { 64, 9, 7 }, { 65, 33, 5 }, { 300, 40, 11 }, { 1024, 30, 4 },
+    const uint32_t shapes[][3] = { { 2, 1, 1 }, { 2, 70, 3 }, { 64, 9, 7 }, { 65, 33, 5 }, { 300, 40, 11 }, { 1024, 30, 4 }, { 1100, 40, 11 }, { 2000, 90, 70 }, { 4032, 9, 8 },
                                    { 4096, 5, 3 }, { 4097, 5, 3 }, { 9000, 7, 2 }, { 17, 700, 600 }, { 1024, 512, 520 } };
     for (auto& d : shapes)
         for (uint32_t nlev = 1; nlev <= 3; nlev += 2)

@@ -22,7 +22,7 @@ def _planes(shape):
     return v
 
 
-@pytest.mark.parametrize("shape", [(33, 257, 513), (64, 64, 4096), (9, 20, 4161), (5, 7, 9000), (3, 2, 20000), (260, 130, 2),
+@pytest.mark.parametrize("shape", [(33, 257, 513), (64, 64, 4096), (40, 33, 1100), (9, 50, 2049), (9, 20, 4161), (5, 7, 9000), (3, 2, 20000), (260, 130, 2),
                                    (70, 1, 64), (1, 70, 65)])
 @pytest.mark.parametrize("normal,dup", MODES)
 def test_planes(shape, normal, dup):
