@@ -621,6 +621,8 @@ kmc_status autotune(kmc_batch* b, hipStream_t st)
     b->flat = best_c.flat;
     kmc_status s = plan_tiles(b, best_c.r, best_c.q);
     if (s == KMC_OK) { destroy_graph(b); s = capture(b); }
+    /* the plan's tables are on the device before a run on any other stream */
+    if (s == KMC_OK && hipStreamSynchronize(b->upload_stream) != hipSuccess) s = KMC_ERR_DEVICE;
     return s;
 }
 

@@ -4,6 +4,7 @@ oracle, bit for bit."""
 
 import numpy as np
 import pytest
+import torch
 
 import oracle
 from kvs_amd import kmc
@@ -36,3 +37,21 @@ def test_one_large_volume(normal, dup, large_at, small):
     for (v, levels, _, _), surfaces in zip(specs, got):
         for l, s in zip(levels, surfaces):
             assert_same_surface(s, oracle.extract(v, l, normal, dup), f"{v.shape} {v.dtype} {l}")
+
+
+def test_autotuned_plan_runs_on_another_stream():
+    # planned on one stream, its tables on the device before a run on a second
+    made, used = torch.cuda.Stream(), torch.cuda.Stream()
+    vols = [_volume((40 + i, 33, 20), i, np.float32) for i in range(12)]
+    dev = [torch.from_numpy(v).cuda() for v in vols]
+    torch.cuda.synchronize()
+    specs = [(kmc.make_volume(t.data_ptr(), dims=v.shape[::-1], memory=kmc.MEMORY_DEVICE, dtype=np.float32,
+                              min_max=(float(v.min()), float(v.max()))), [0.3], kmc.POLYGON_NORMAL, True)
+             for t, v in zip(dev, vols)]
+    b = kmc.Batch(specs, autotune=True, stream=made.cuda_stream)
+    try:
+        b.run(stream=used.cuda_stream)
+        for v, s in zip(vols, b.surfaces()):
+            assert_same_surface(kmc.device_surface_to_numpy(s), oracle.extract(v, 0.3, kmc.POLYGON_NORMAL, True), f"{v.shape}")
+    finally:
+        b.close()
