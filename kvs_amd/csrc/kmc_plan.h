@@ -1,7 +1,8 @@
 /*
  * kmc_plan.h -- how the slots (node row, 64-node chunk) of a level are dealt to
- * the waves of the chunk-batch emit.  Plain C++, shared by the host's planning,
- * the kernels and the host-side tests.
+ * the waves of the chunk-batch emit, which form classifies a volume, and how a
+ * batch's workgroups are dealt to its passes.  Plain C++, shared by the host's
+ * planning, the kernels and the host-side tests.
  *
  * A *piece* is a run of up to 16 lanes' slots: 8 or 16 chunks of a row, or all
  * chunks of one or more short rows.  A *unit*, what a wave looks at in one step,
